@@ -9,13 +9,14 @@
 // with float atomics whose order varies run to run), per-row work runs one
 // 64-lane wavefront per row (FWHT across lanes) instead of one thread per row
 // with 2 KB of private arrays, and the dense products of the attention-aware
-// loss are LDS-tiled batched matrix products.  Results match the reference's
+// loss are LDS-tiled batched matrix products on the fp32 matrix cores.  Results match the reference's
 // algorithm up to float rounding; the steps that pick a discrete winner
 // (tournaments, argmins) do so with the reference's tie rules.
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <vector>
@@ -702,57 +703,109 @@ __global__ __launch_bounds__(256) void wtrm_bwd_kernel(const float* __restrict__
     *reinterpret_cast<float4*>(grec + n * D + 4 * lane) = make_float4(o[0], o[1], o[2], o[3]);
 }
 
-// C[b] (M x N) = alpha * op(A[b]) B[b] (+ C[b] when acc); row-major B (K x N,
-// ldb) and C (ldc); op(A) = A (M x K, lda) or A^T (A stored K x M, lda).
-// 64 x 64 tiles, 16-deep K slabs in LDS, 4 x 4 outputs per thread.
-__global__ __launch_bounds__(256) void gemm_kernel(const float* __restrict__ A,
-                                                   const float* __restrict__ B,
-                                                   float* __restrict__ C, int M, int N, int K,
-                                                   long lda, long ldb, long ldc, long sa, long sb,
-                                                   long sc, int trans_a, float alpha, int acc) {
-    __shared__ float sA[16][65];
-    __shared__ float sB[16][65];
-    const int b = blockIdx.z;
-    A += b * sa;
-    B += b * sb;
-    C += b * sc;
+// C[b] (M x N) = alpha * op(A[b]) B[b]; row-major B (K x N, ldb) and C (ldc);
+// op(A) = A (M x K, lda) or A^T (A stored K x M, lda).
+// fp32 MFMA 32x32x2: a block owns a 64 x 64 tile, each of its four wavefronts a
+// 32 x 32 quarter; 32-deep K slabs, double-buffered in LDS, the next slab's
+// loads in flight under the current one's 16 MFMAs.  The matrix cores take one
+// LDS word per lane and operand for 64 cycles of work, where the vector form
+// this replaces read eight words for 16 fused multiply-adds and was bound by
+// the LDS.  Scalar loads: T, and so lda, may be any size.  Grid z = batch x
+// splits; a split covers k_per of K and writes its own C (the partials are
+// added by gemm_reduce_kernel).
+// A 512-token calibration: 24 x (512 x 256 x 512) forward 376 us in four
+// launches of 94 -> 59 us (108 TFLOP/s of the 154 a large fp32 matrix product
+// reaches here); 4 x (512 x 256 x 3072) backward 2450 us in four launches of
+// 32 blocks -> 53 us with 8 splits and 5 us for their sum.
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+constexpr int GK = 32;   // K slab
+constexpr int GLD = 65;  // words per LDS row: the transposing stores hit 32 banks
+struct GemmArgs {
+    const float *A, *B;
+    float* C;
+    int M, N, K;
+    long lda, ldb, ldc, sa, sb, sc;
+    int trans_a, batch, b_div, splits, k_per;  // B's batch index is b / b_div
+    float alpha;
+    double* sumsq;  // when set, the sum of C's squares is added to it
+};
+__global__ __launch_bounds__(256) void gemm_kernel(GemmArgs g) {
+    __shared__ float sA[2][GK][GLD];
+    __shared__ float sB[2][GK][GLD];
+    const int b = blockIdx.z % g.batch, split = blockIdx.z / g.batch;
+    const float* A = g.A + b * g.sa;
+    const float* B = g.B + (b / g.b_div) * g.sb;
+    float* C = g.C + (long)blockIdx.z * g.sc;
     const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-    float c[4][4] = {};
-    for (int k0 = 0; k0 < K; k0 += 16) {
-        for (int i = threadIdx.x; i < 16 * 64; i += 256) {
-            const int kk = i >> 6, mm = i & 63;  // A slab: [k][m]
-            const int gm = m0 + mm, gk = k0 + kk;
-            float av = 0.0f;
-            if (gm < M && gk < K) av = trans_a ? A[(long)gk * lda + gm] : A[(long)gm * lda + gk];
-            sA[kk][mm] = av;
-            const int gn = n0 + mm;
-            sB[kk][mm] = (gn < N && gk < K) ? B[(long)gk * ldb + gn] : 0.0f;
+    const int k_lo = split * g.k_per, k_hi = min(g.K, k_lo + g.k_per);
+    const int t = threadIdx.x, wv = t >> 6, lane = t & 63, ln = lane & 31, hh = lane >> 5;
+    const int wm = 32 * (wv & 1), wn = 32 * (wv >> 1);
+    float ra[8], rb[8];
+    auto load = [&](int k0) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int kt = k0 + (t >> 6) + 4 * i, kr = k0 + (t & 31);
+            const int mt = m0 + (t & 63), mr = m0 + (t >> 5) + 8 * i, gn = n0 + (t & 63);
+            if (g.trans_a)
+                ra[i] = (mt < g.M && kt < k_hi) ? A[(long)kt * g.lda + mt] : 0.0f;
+            else
+                ra[i] = (mr < g.M && kr < k_hi) ? A[(long)mr * g.lda + kr] : 0.0f;
+            rb[i] = (gn < g.N && kt < k_hi) ? B[(long)kt * g.ldb + gn] : 0.0f;
         }
-        __syncthreads();
+    };
+    auto store = [&](int buf) {
 #pragma unroll
-        for (int kk = 0; kk < 16; kk++) {
-            float a4[4], b4[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                a4[i] = sA[kk][ty * 4 + i];
-                b4[i] = sB[kk][tx * 4 + i];
-            }
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-#pragma unroll
-                for (int j = 0; j < 4; j++) c[i][j] = fmaf(a4[i], b4[j], c[i][j]);
+        for (int i = 0; i < 8; i++) {
+            if (g.trans_a)
+                sA[buf][(t >> 6) + 4 * i][t & 63] = ra[i];
+            else
+                sA[buf][t & 31][(t >> 5) + 8 * i] = ra[i];
+            sB[buf][(t >> 6) + 4 * i][t & 63] = rb[i];
         }
-        __syncthreads();
+    };
+    f32x16 acc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    load(k_lo);
+    store(0);
+    int buf = 0;
+    for (int k0 = k_lo; k0 < k_hi; k0 += GK, buf ^= 1) {
+        __syncthreads();  // slab `buf` is staged, the other one is read out
+        const bool more = k0 + GK < k_hi;
+        if (more) load(k0 + GK);
+#pragma unroll
+        for (int kk = 0; kk < GK; kk += 2)
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(sA[buf][kk + hh][wm + ln],
+                                                       sB[buf][kk + hh][wn + ln], acc, 0, 0, 0);
+        if (more) store(buf ^ 1);
     }
-    for (int i = 0; i < 4; i++)
-        for (int j = 0; j < 4; j++) {
-            const int gm = m0 + ty * 4 + i, gn = n0 + tx * 4 + j;
-            if (gm < M && gn < N) {
-                float* cp = C + (long)gm * ldc + gn;
-                *cp = alpha * c[i][j] + (acc ? *cp : 0.0f);
-            }
+    double sq = 0.0;
+#pragma unroll
+    for (int r = 0; r < 16; r++) {  // row 8 (r / 4) + 4 hh + r % 4, column ln
+        const int gm = m0 + wm + 8 * (r >> 2) + 4 * hh + (r & 3), gn = n0 + wn + ln;
+        const float v = g.alpha * acc[r];
+        if (gm < g.M && gn < g.N) {
+            C[(long)gm * g.ldc + gn] = v;
+            sq += (double)v * v;
         }
+    }
+    if (g.sumsq) {
+        __shared__ double s_sq[4];
+        for (int o = 32; o >= 1; o >>= 1) sq += __shfl_xor(sq, o, 64);
+        if (lane == 0) s_sq[wv] = sq;
+        __syncthreads();
+        if (t == 0) atomicAdd(g.sumsq, (s_sq[0] + s_sq[1]) + (s_sq[2] + s_sq[3]));
+    }
+}
+
+// out[i] = alpha * (part[0][i] + part[1][i] + ...), in split order
+__global__ __launch_bounds__(256) void gemm_reduce_kernel(const float* __restrict__ part,
+                                                          float* __restrict__ out, long n,
+                                                          int splits, float alpha) {
+    const long i = (long)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    float s = 0.0f;
+#pragma unroll 8
+    for (int k = 0; k < splits; k++) s += part[k * n + i];
+    out[i] = alpha * s;
 }
 
 // sum of squares (or of (a - b)^2, and the gradient 2 (a - b) / n) into a double
@@ -1081,7 +1134,7 @@ struct Svq {
     const float* rp;    // [64][16]
     int N, T, H_q, H_kv;
     hipStream_t st;
-    Buf rot, rec, recf, dlt, wbuf, idx, dict, y, gdl, grec, gw, gq, swg, gcb, gwa, gwb, loss;
+    Buf rot, rec, recf, dlt, wbuf, idx, dict, y, gdl, grec, gw, gq, swg, gcb, gwa, gwb, loss, part;
     int init() {
         const size_t nd = (size_t)N * D * 4;
         for (Buf* b : {&rot, &rec, &recf, &dlt, &grec, &gdl}) CAL_TRY(b->alloc(nd));
@@ -1095,13 +1148,42 @@ struct Svq {
         CAL_TRY(gwa.alloc(2048 * 4));
         CAL_TRY(gwb.alloc(2048 * 4));
         CAL_TRY(loss.alloc(2 * sizeof(double)));
-        if (attn) CAL_TRY(y.alloc((size_t)H_q * T * D * 4));
+        if (attn) {
+            CAL_TRY(y.alloc((size_t)H_q * T * D * 4));
+            int kp;
+            const size_t p1 = (size_t)gemm_splits(T, D, H_q / H_kv * T, H_kv, &kp) * H_kv * T * D;
+            const size_t p2 = (size_t)gemm_splits(D, D, N, 1, &kp) * D * D;
+            CAL_TRY(part.alloc(std::max(p1, p2) * 4));
+        }
         return 0;
     }
+    // Splits of K: enough blocks for four a CU (a block's LDS and registers
+    // let four share one and cover each other's barriers), at least 128 of K,
+    // four slabs, each, and at most 16 partials to add.  The transform
+    // gradient, 16 tiles of K 2048: 410 us unsplit, 11 + 5 us in 16 splits.
+    static int gemm_splits(int M, int Nn, int K, int batch, int* k_per) {
+        const int tiles = ((Nn + 63) / 64) * ((M + 63) / 64) * batch;
+        int s = std::max(1, std::min({1024 / tiles, K / 128, 16}));
+        *k_per = ((K + s - 1) / s + GK - 1) / GK * GK;
+        return (K + *k_per - 1) / *k_per;
+    }
+    // dense C (ldc = Nn, batches sc apart = M Nn); sumsq only without splits
     void gemm(const float* A, const float* B, float* C, int M, int Nn, int K, long lda, long ldb,
-              long ldc, long sa, long sb, long sc, int batch, int ta, float alpha) {
-        hipLaunchKernelGGL(gemm_kernel, dim3((Nn + 63) / 64, (M + 63) / 64, batch), dim3(256), 0,
-                           st, A, B, C, M, Nn, K, lda, ldb, ldc, sa, sb, sc, ta, alpha, 0);
+              long sa, long sb, int batch, int b_div, int ta, float alpha, double* sumsq) {
+        GemmArgs g{A, B, C, M, Nn, K, lda, ldb, Nn, sa, sb, (long)M * Nn, ta, batch, b_div, 1, K, alpha,
+                   sumsq};
+        if (!sumsq) g.splits = gemm_splits(M, Nn, K, batch, &g.k_per);
+        if (g.splits > 1) {
+            g.C = part.as<float>();
+            g.alpha = 1.0f;
+        }
+        hipLaunchKernelGGL(gemm_kernel, dim3((Nn + 63) / 64, (M + 63) / 64, batch * g.splits),
+                           dim3(256), 0, st, g);
+        if (g.splits > 1) {
+            const long n = (long)batch * M * Nn;
+            hipLaunchKernelGGL(gemm_reduce_kernel, dim3(blocks(n, 256)), dim3(256), 0, st,
+                               part.as<float>(), C, n, g.splits, alpha);
+        }
     }
     // One pass at temperature temp (ref .cu:2436-2467 forward, :2470-2530
     // with gradients): losses[0] = reconstruction (attention-weighted MSE of
@@ -1124,25 +1206,21 @@ struct Svq {
             hipLaunchKernelGGL(wtrm_fwd_kernel, dim3(blocks(N, 4)), dim3(256), 0, st,
                                recf.as<float>(), s.wa.as<float>(), s.wb.as<float>(), v,
                                dlt.as<float>(), N);
-            for (int kv = 0; kv < H_kv; kv++)  // y_h = A_h dlt_kv for the group's heads
-                gemm(attn + (long)kv * n_rep * T * T, dlt.as<float>() + (long)kv * T * D,
-                     y.as<float>() + (long)kv * n_rep * T * D, T, D, T, T, D, D, (long)T * T, 0,
-                     (long)T * D, n_rep, 0, 1.0f);
             const long ny = (long)H_q * T * D;
             denom = (double)ny;
-            hipLaunchKernelGGL(sumsq_kernel, dim3(256), dim3(256), 0, st, y.as<float>(), nullptr,
-                               nullptr, ny, 0.0f, loss.as<double>(), 1);
+            // y_h = A_h dlt_kv, every head in one launch
+            gemm(attn, dlt.as<float>(), y.as<float>(), T, D, T, T, D, (long)T * T, (long)T * D,
+                 H_q, n_rep, 0, 1.0f, loss.as<double>());
             if (grad) {
                 const float g = 2.0f / (float)ny;
-                for (int kv = 0; kv < H_kv; kv++)  // gdlt_kv = g sum_h A_h^T y_h
-                    gemm(attn + (long)kv * n_rep * T * T, y.as<float>() + (long)kv * n_rep * T * D,
-                         gdl.as<float>() + (long)kv * T * D, T, D, n_rep * T, T, D, D, 0, 0, 0, 1,
-                         1, g);
+                // gdlt_kv = g sum_h A_h^T y_h: the group's heads stacked along K
+                gemm(attn, y.as<float>(), gdl.as<float>(), T, D, n_rep * T, T, D,
+                     (long)n_rep * T * T, (long)n_rep * T * D, H_kv, 1, 1, g, nullptr);
                 hipLaunchKernelGGL(wtrm_bwd_kernel, dim3(blocks(N, 4)), dim3(256), 0, st,
                                    gdl.as<float>(), s.wa.as<float>(), s.wb.as<float>(),
                                    grec.as<float>(), N);
-                gemm(recf.as<float>(), gdl.as<float>(), gw.as<float>(), D, D, N, D, D, D, 0, 0, 0,
-                     1, 1, 1.0f);  // gW = recf^T gdlt
+                gemm(recf.as<float>(), gdl.as<float>(), gw.as<float>(), D, D, N, D, D, 0, 0, 1, 1, 1,
+                     1.0f, nullptr);  // gW = recf^T gdlt
                 hipLaunchKernelGGL(gwab_kernel, dim3(16), dim3(256), 0, st, gw.as<float>(),
                                    s.wa.as<float>(), s.wb.as<float>(), gwa.as<float>(),
                                    gwb.as<float>());

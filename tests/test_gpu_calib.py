@@ -231,6 +231,26 @@ def test_svq_pass_vs_restatement(device, mode):
         np.testing.assert_allclose(a, w, rtol=1e-3, atol=1e-4 * max(np.abs(w).max(), 1e-30))
 
 
+@pytest.mark.parametrize("T_,H_kv,H_q", [(1, 1, 1), (31, 2, 6), (65, 1, 5), (130, 2, 4)])
+def test_svq_pass_sizes(device, T_, H_kv, H_q):
+    """The pass at sizes around the 64-wide matrix-product tiles, its 32-deep
+    slabs, the K splits (from 256 stacked rows on) and the 64-row blocks of the
+    codebook gradient, to the tolerance of test_svq_pass_vs_restatement."""
+    v, rp, cb, attn, N, Tn, H_q, H_kv = _svq_margin_case(T=T_, H_kv=H_kv, H_q=H_q, seed=31)
+    rng = np.random.default_rng(32)
+    wa = (rng.standard_normal((256, 8)) / 16).astype(np.float32)
+    wb = (rng.standard_normal((8, 256)) / 64).astype(np.float32)
+    g, l = new(49152 + 4096), new(2)
+    calib.svq_pass(T(v), T(attn), T(cb), T(wa), T(wb), T(rp), g, l, N=N, T=Tn, H_q=H_q,
+                   H_kv=H_kv, temp=0.3)
+    rl, dl, gcb, gwa, gwb = R.svq_pass(v, attn, cb, wa, wb, rp, Tn, H_q, H_kv, 0.3)
+    got = g.cpu().numpy()
+    np.testing.assert_allclose(l.cpu().numpy(), [rl, dl], rtol=1e-4)
+    for a, w in ((got[:49152], gcb.ravel()), (got[49152:51200], gwa.ravel()),
+                 (got[51200:], gwb.ravel())):
+        np.testing.assert_allclose(a, w, rtol=1e-3, atol=1e-4 * max(np.abs(w).max(), 1e-30))
+
+
 def test_svq_train_vs_restatement(device):
     """The whole trainer (3 seeds, Adam steps, best tracking, the proxy
     tournament) against the float64 restatement; with no rate the output
