@@ -599,48 +599,62 @@ __global__ void round_fp16_kernel(float* __restrict__ p, int n) {
 // nearest codeword forward, softmax(-dist / temp) weights backward).  Rows are
 // head-major V projections (row = kv_head * T + t).
 
-// per (row, patch): nearest codeword (first minimum), rec dims 0..2 = that
-// codeword, soft weights w[k] = softmax(-|v - c_k|^2 / temp), dict term
-// |c_best - v|^2.  One thread per (row, patch); the patch's codebook in LDS.
-__global__ __launch_bounds__(256) void vq_ste_kernel(const float* __restrict__ rot,
-                                                     const float* __restrict__ cb,
-                                                     float* __restrict__ rec,
-                                                     float* __restrict__ wbuf,
-                                                     int* __restrict__ idx,
-                                                     float* __restrict__ dict, int rows,
-                                                     float temp, int need_w) {
-    __shared__ float s_cb[768];
-    const int p = blockIdx.y;
-    for (int i = threadIdx.x; i < 768; i += 256) s_cb[i] = cb[p * 768 + i];
+// Per (row, patch): nearest codeword (first minimum), rec dims 0..2 = that
+// codeword, dict term |c_best - v|^2.  Block = 64 rows of one patch, four
+// threads a row on every fourth codeword each (2048 blocks at 2048 rows; one
+// thread a row left two wavefronts a SIMD), the codebook in LDS as float4 so a
+// codeword is one read.
+constexpr int SR = 64;  // rows per block
+__device__ __forceinline__ void load_codebook(float4* s_cb, const float* __restrict__ cb, int p) {
+    const float* c = cb + p * 768 + threadIdx.x * 3;
+    s_cb[threadIdx.x] = make_float4(c[0], c[1], c[2], 0.0f);
+}
+__device__ __forceinline__ float dist3(const float4& c, float v0, float v1, float v2) {
+    const float d0 = v0 - c.x, d1 = v1 - c.y, d2 = v2 - c.z;
+    return d0 * d0 + d1 * d1 + d2 * d2;
+}
+__global__ __launch_bounds__(256) void vq_hard_kernel(const float* __restrict__ rot,
+                                                      const float* __restrict__ cb,
+                                                      float* __restrict__ rec,
+                                                      int* __restrict__ idx,
+                                                      float* __restrict__ dict, int rows) {
+    __shared__ float4 s_cb[256];
+    const int p = blockIdx.y, q = threadIdx.x & 3;
+    load_codebook(s_cb, cb, p);
     __syncthreads();
-    const long n = (long)blockIdx.x * 256 + threadIdx.x;
-    if (n >= rows) return;
-    const float* v = rot + n * D + p * 4;
+    const long n = (long)blockIdx.x * SR + (threadIdx.x >> 2);
+    const float* v = rot + min(n, (long)rows - 1) * D + p * 4;
     const float v0 = v[0], v1 = v[1], v2 = v[2];
-    float bd;
-    const int bk = nearest(s_cb, v0, v1, v2, &bd);
-    idx[n * NP + p] = bk;
-    float dd = 0.0f;
-    for (int c = 0; c < 3; c++) {
-        const float df = s_cb[bk * 3 + c] - v[c];
-        dd += df * df;
-        rec[n * D + p * 4 + c] = s_cb[bk * 3 + c];
-    }
-    dict[n * NP + p] = dd;
-    if (need_w) {
-        // max of -dist / temp is -bd / temp (bd is the minimum distance)
-        const float zmax = -bd / temp;
-        float* w = wbuf + (n * NP + p) * 256;
-        float z = 0.0f;
-        for (int k = 0; k < 256; k++) {
-            const float d0 = v0 - s_cb[k * 3], d1 = v1 - s_cb[k * 3 + 1], d2 = v2 - s_cb[k * 3 + 2];
-            const float e = expf(-(d0 * d0 + d1 * d1 + d2 * d2) / temp - zmax);
-            w[k] = e;
-            z += e;
+    float bd = 1e30f;
+    int bk = q;
+#pragma unroll 8
+    for (int k = q; k < 256; k += 4) {
+        const float dd = dist3(s_cb[k], v0, v1, v2);
+        if (dd < bd) {
+            bd = dd;
+            bk = k;
         }
-        const float zi = 1.0f / z;
-        for (int k = 0; k < 256; k++) w[k] *= zi;
     }
+#pragma unroll
+    for (int m = 1; m <= 2; m <<= 1) {
+        const float od = __shfl_xor(bd, m, 64);
+        const int ok = __shfl_xor(bk, m, 64);
+        if (od < bd || (od == bd && ok < bk)) {
+            bd = od;
+            bk = ok;
+        }
+    }
+    if (n >= rows || q != 0) return;
+    idx[n * NP + p] = bk;
+    const float4 c = s_cb[bk];
+    float dd = 0.0f;
+    const float df[3] = {c.x - v0, c.y - v1, c.z - v2};
+    for (int i = 0; i < 3; i++) dd += df[i] * df[i];
+    dict[n * NP + p] = dd;
+    float* r = rec + n * D + p * 4;
+    r[0] = c.x;
+    r[1] = c.y;
+    r[2] = c.z;
 }
 
 // dim 3 of rec: round half to even of rot * 16, / 16
@@ -840,59 +854,86 @@ __global__ void rotbwd_kernel(const float* __restrict__ grec, const float* __res
         gq[i * 3 + c] = g[0] * rp[p * 16 + c] + g[1] * rp[p * 16 + 4 + c] + g[2] * rp[p * 16 + 8 + c];
 }
 
-// swg[n][p] = sum_k w[n][p][k] (gq . c_k).  One wavefront per (row, patch).
-__global__ __launch_bounds__(256) void swg_kernel(const float* __restrict__ gq,
-                                                  const float* __restrict__ cb,
-                                                  const float* __restrict__ wbuf,
-                                                  float* __restrict__ swg, int rows) {
-    const int lane = threadIdx.x & 63;
-    const long np = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (np >= (long)rows * NP) return;
-    const int p = (int)(np & 63);
-    const float g0 = gq[np * 3], g1 = gq[np * 3 + 1], g2 = gq[np * 3 + 2];
-    const float* w = wbuf + np * 256;
-    float s = 0.0f;
-    for (int k = lane; k < 256; k += 64) {
-        const float* c = cb + p * 768 + k * 3;
-        s += w[k] * (g0 * c[0] + g1 * c[1] + g2 * c[2]);
-    }
-    s = wsum(s);
-    if (lane == 0) swg[np] = s;
-}
-
-// Codebook gradient (ref .cu:2339-2371), summed over rows without atomics:
-// block = patch, thread = codeword k; for every row n
+// Codebook gradient (ref .cu:2339-2371) with w_k = softmax(-|v - c_k|^2 / temp)
+// and swg = sum_k w_k (gq . c_k): for every row
 //   gC[k] += w_k gq + (-w_k (gq . c_k - swg) / temp) * 2 (c_k - v)
 // plus, at the row's hard codeword, the dict term 2 / (N 64 3) (c_bk - v).
-__global__ __launch_bounds__(256) void cgrad_kernel(const float* __restrict__ wbuf,
-                                                    const float* __restrict__ swg,
-                                                    const float* __restrict__ gq,
-                                                    const float* __restrict__ rot,
-                                                    const float* __restrict__ cb,
-                                                    const int* __restrict__ idx,
-                                                    float* __restrict__ gcb, int rows, float temp) {
-    const int p = blockIdx.x, k = threadIdx.x;
-    const float c0 = cb[p * 768 + k * 3], c1 = cb[p * 768 + k * 3 + 1], c2 = cb[p * 768 + k * 3 + 2];
+// Block = one patch and a range of rows, 64 at a time: four threads a row find
+// the row's softmax sum and swg (their codewords interleaved), then thread k
+// adds the 64 rows' terms of codeword k.  The weights are formed twice from the
+// rows and the codebook in LDS and never stored: the buffer they took (64 x 256
+// floats a row, 134 MB at 2048 rows) was written once, scaled once and read
+// twice, the last time by 64 blocks in all.  Each block writes its own partial
+// gradient, added in row order by gemm_reduce_kernel.  2048 rows: 970 us in
+// three kernels -> 37 us and 5 for the sum, bound by the vector ALUs.
+__global__ __launch_bounds__(256) void soft_grad_kernel(const float* __restrict__ rot,
+                                                        const float* __restrict__ cb,
+                                                        const float* __restrict__ gq,
+                                                        const int* __restrict__ idx,
+                                                        float* __restrict__ part, int rows,
+                                                        int rows_per, float temp) {
+    __shared__ float4 s_cb[256];
+    __shared__ float4 s_v[SR];  // v, 1 / softmax sum
+    __shared__ float4 s_g[SR];  // gq, swg
+    __shared__ float2 s_h[SR];  // distance of the hard codeword, its index
+    const int p = blockIdx.x, t = threadIdx.x;
+    load_codebook(s_cb, cb, p);
     const float dn = 2.0f / (float)((long)rows * NP * 3);
+    const float sharp = 1.44269504f / temp;  // weights as powers of two
+    const float gs = -2.0f / temp;
+    const int lo = blockIdx.y * rows_per, hi = min(rows, lo + rows_per);
     float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f;
-    for (int n = 0; n < rows; n++) {
-        const long np = (long)n * NP + p;
-        const float w = wbuf[np * 256 + k];
-        const float g0 = gq[np * 3], g1 = gq[np * 3 + 1], g2 = gq[np * 3 + 2];
-        const float* v = rot + (long)n * D + p * 4;
-        const float gd = -(w * ((g0 * c0 + g1 * c1 + g2 * c2) - swg[np])) / temp;
-        a0 += w * g0 + gd * 2.0f * (c0 - v[0]);
-        a1 += w * g1 + gd * 2.0f * (c1 - v[1]);
-        a2 += w * g2 + gd * 2.0f * (c2 - v[2]);
-        if (idx[np] == k) {
-            a0 += dn * (c0 - v[0]);
-            a1 += dn * (c1 - v[1]);
-            a2 += dn * (c2 - v[2]);
+    for (int n0 = lo; n0 < hi; n0 += SR) {
+        __syncthreads();
+        const int r = t >> 2, q = t & 3;
+        if (n0 + r < hi) {  // uniform over a row's four lanes
+            const long np = (long)(n0 + r) * NP + p;
+            const float* v = rot + (long)(n0 + r) * D + p * 4;
+            const float v0 = v[0], v1 = v[1], v2 = v[2];
+            const float g0 = gq[np * 3], g1 = gq[np * 3 + 1], g2 = gq[np * 3 + 2];
+            const int bk = idx[np];
+            const float bd = dist3(s_cb[bk], v0, v1, v2);
+            float z = 0.0f, sw = 0.0f;
+#pragma unroll 8
+            for (int k = q; k < 256; k += 4) {
+                const float4 c = s_cb[k];
+                const float e = __builtin_amdgcn_exp2f((bd - dist3(c, v0, v1, v2)) * sharp);
+                z += e;
+                sw = fmaf(e, fmaf(g2, c.z, fmaf(g1, c.y, g0 * c.x)), sw);
+            }
+#pragma unroll
+            for (int m = 1; m <= 2; m <<= 1) {
+                z += __shfl_xor(z, m, 64);
+                sw += __shfl_xor(sw, m, 64);
+            }
+            if (q == 0) {
+                const float zi = 1.0f / z;
+                s_v[r] = make_float4(v0, v1, v2, zi);
+                s_g[r] = make_float4(g0, g1, g2, sw * zi);
+                s_h[r] = make_float2(bd, __int_as_float(bk));
+            }
+        }
+        __syncthreads();
+        const float4 c = s_cb[t];
+        const int nr = min(SR, hi - n0);
+#pragma unroll 4
+        for (int i = 0; i < nr; i++) {
+            const float4 v = s_v[i], g = s_g[i];
+            const float2 h = s_h[i];
+            const float d0 = c.x - v.x, d1 = c.y - v.y, d2 = c.z - v.z;
+            const float w =
+                __builtin_amdgcn_exp2f((h.x - (d0 * d0 + d1 * d1 + d2 * d2)) * sharp) * v.w;
+            float gd = gs * w * (fmaf(g.z, c.z, fmaf(g.y, c.y, g.x * c.x)) - g.w);
+            if (__float_as_int(h.y) == t) gd += dn;
+            a0 = fmaf(gd, d0, fmaf(w, g.x, a0));
+            a1 = fmaf(gd, d1, fmaf(w, g.y, a1));
+            a2 = fmaf(gd, d2, fmaf(w, g.z, a2));
         }
     }
-    gcb[p * 768 + k * 3] = a0;
-    gcb[p * 768 + k * 3 + 1] = a1;
-    gcb[p * 768 + k * 3 + 2] = a2;
+    float* o = part + (size_t)blockIdx.y * CB + p * 768 + t * 3;
+    o[0] = a0;
+    o[1] = a1;
+    o[2] = a2;
 }
 
 // gA = gW B^T (256 x 8), gB = A^T gW (8 x 256)
@@ -1134,27 +1175,27 @@ struct Svq {
     const float* rp;    // [64][16]
     int N, T, H_q, H_kv;
     hipStream_t st;
-    Buf rot, rec, recf, dlt, wbuf, idx, dict, y, gdl, grec, gw, gq, swg, gcb, gwa, gwb, loss, part;
+    Buf rot, rec, recf, dlt, idx, dict, y, gdl, grec, gw, gq, gcb, gwa, gwb, loss, part;
     int init() {
         const size_t nd = (size_t)N * D * 4;
         for (Buf* b : {&rot, &rec, &recf, &dlt, &grec, &gdl}) CAL_TRY(b->alloc(nd));
-        CAL_TRY(wbuf.alloc((size_t)N * NP * 256 * 4));
         CAL_TRY(idx.alloc((size_t)N * NP * 4));
         CAL_TRY(dict.alloc((size_t)N * NP * 4));
         CAL_TRY(gq.alloc((size_t)N * NP * 3 * 4));
-        CAL_TRY(swg.alloc((size_t)N * NP * 4));
         CAL_TRY(gw.alloc(D * D * 4));
         CAL_TRY(gcb.alloc(CB * 4));
         CAL_TRY(gwa.alloc(2048 * 4));
         CAL_TRY(gwb.alloc(2048 * 4));
         CAL_TRY(loss.alloc(2 * sizeof(double)));
+        int kp;
+        size_t np = (size_t)soft_ranges(N, &kp) * CB;
         if (attn) {
             CAL_TRY(y.alloc((size_t)H_q * T * D * 4));
-            int kp;
             const size_t p1 = (size_t)gemm_splits(T, D, H_q / H_kv * T, H_kv, &kp) * H_kv * T * D;
             const size_t p2 = (size_t)gemm_splits(D, D, N, 1, &kp) * D * D;
-            CAL_TRY(part.alloc(std::max(p1, p2) * 4));
+            np = std::max({np, p1, p2});
         }
+        CAL_TRY(part.alloc(np * 4));
         return 0;
     }
     // Splits of K: enough blocks for four a CU (a block's LDS and registers
@@ -1166,6 +1207,14 @@ struct Svq {
         int s = std::max(1, std::min({1024 / tiles, K / 128, 16}));
         *k_per = ((K + s - 1) / s + GK - 1) / GK * GK;
         return (K + *k_per - 1) / *k_per;
+    }
+    // Row ranges of the codebook gradient: one block of 64 rows each while that
+    // is at most 64 ranges (4096 blocks), longer ranges beyond, so the partial
+    // gradients stay under 13 MB.
+    static int soft_ranges(int N, int* per) {
+        const int r = std::min(64, (N + SR - 1) / SR);
+        *per = ((N + r - 1) / r + SR - 1) / SR * SR;
+        return (N + *per - 1) / *per;
     }
     // dense C (ldc = Nn, batches sc apart = M Nn); sumsq only without splits
     void gemm(const float* A, const float* B, float* C, int M, int Nn, int K, long lda, long ldb,
@@ -1193,9 +1242,9 @@ struct Svq {
         CAL_TRY(hipMemsetAsync(loss.p, 0, 2 * sizeof(double), st));
         hipLaunchKernelGGL(rotate_kernel, dim3(blocks((long)N * NP, 256)), dim3(256), 0, st, v, rp,
                            rot.as<float>(), N);
-        hipLaunchKernelGGL(vq_ste_kernel, dim3(blocks(N, 256), NP), dim3(256), 0, st,
-                           rot.as<float>(), s.cb.as<float>(), rec.as<float>(), wbuf.as<float>(),
-                           idx.as<int>(), dict.as<float>(), N, temp, grad ? 1 : 0);
+        hipLaunchKernelGGL(vq_hard_kernel, dim3(blocks(N, SR), NP), dim3(256), 0, st,
+                           rot.as<float>(), s.cb.as<float>(), rec.as<float>(), idx.as<int>(),
+                           dict.as<float>(), N);
         hipLaunchKernelGGL(dim3_kernel, dim3(blocks((long)N * NP, 256)), dim3(256), 0, st,
                            rot.as<float>(), rec.as<float>(), N);
         hipLaunchKernelGGL(invrot_kernel, dim3(blocks((long)N * NP, 256)), dim3(256), 0, st,
@@ -1235,12 +1284,13 @@ struct Svq {
         if (grad) {
             hipLaunchKernelGGL(rotbwd_kernel, dim3(blocks((long)N * NP, 256)), dim3(256), 0, st,
                                grec.as<float>(), rp, gq.as<float>(), N);
-            hipLaunchKernelGGL(swg_kernel, dim3(blocks((long)N * NP, 4)), dim3(256), 0, st,
-                               gq.as<float>(), s.cb.as<float>(), wbuf.as<float>(),
-                               swg.as<float>(), N);
-            hipLaunchKernelGGL(cgrad_kernel, dim3(NP), dim3(256), 0, st, wbuf.as<float>(),
-                               swg.as<float>(), gq.as<float>(), rot.as<float>(), s.cb.as<float>(),
-                               idx.as<int>(), gcb.as<float>(), N, temp);
+            int per;
+            const int ranges = soft_ranges(N, &per);
+            hipLaunchKernelGGL(soft_grad_kernel, dim3(NP, ranges), dim3(256), 0, st,
+                               rot.as<float>(), s.cb.as<float>(), gq.as<float>(), idx.as<int>(),
+                               part.as<float>(), N, per, temp);
+            hipLaunchKernelGGL(gemm_reduce_kernel, dim3(blocks(CB, 256)), dim3(256), 0, st,
+                               part.as<float>(), gcb.as<float>(), (long)CB, ranges, 1.0f);
         }
         double h[2];
         CAL_TRY(hipMemcpyAsync(h, loss.p, sizeof(h), hipMemcpyDeviceToHost, st));
