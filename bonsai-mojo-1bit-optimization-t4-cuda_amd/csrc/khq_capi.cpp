@@ -171,7 +171,20 @@ int compressed_parts(int c_len, int n_rep, int h_kv, int L_q) {
     return std::max(1, std::min(256, (c_len + 31) / 32));
 }
 
-int window_parts(int win_len) { return std::max(1, std::min(64, (win_len + 3) / 4)); }
+// fp16 window work: 16-slot tiles, one per wavefront at a time.  While the
+// tiles fit two a CU each is a block of its own (one CU loads a tile's 16 KB
+// far slower than 256 do), at most max_parts a KV head; beyond that blocks of
+// 4 wavefronts, two a CU.
+int window_waves(int win_len, int h_kv) {
+    return (win_len + 15) / 16 * h_kv <= 2 * khq::device_cu_count() ? 1 : 4;
+}
+int window_parts(int win_len, int h_kv, int waves, int max_parts = 1024) {
+    const int groups = ((win_len + 15) / 16 + waves - 1) / waves;
+    const int cap = waves == 1 ? groups : 2 * khq::device_cu_count() / h_kv;
+    const int want = std::max(1, std::min({groups, cap, max_parts}));
+    const int per = (groups + want - 1) / want * waves;  // tiles a part
+    return ((win_len + 15) / 16 + per - 1) / per;
+}
 
 khq::AttnArgs attn_args(const void* q, const void* k_payload, const void* v_payload,
                         const void* v_shared_meta, const void* k_mask, const void* k_norms,
@@ -351,9 +364,11 @@ int launch_khq_window_attn_fp16(const void* q, const void* ring_k, const void* r
     if (d != 256 || H_kv <= 0 || H_q % H_kv != 0 || H_q / H_kv > 8 || ring_cap <= 0 ||
         win_len > ring_cap || win_start < 0)
         return -100;
-    const int np = window_parts(win_len);
-    float* ws = nullptr;
-    hipError_t e = workspace((size_t)H_q * np * 258 * sizeof(float), stream, &ws);
+    const int waves = window_waves(win_len, H_kv);
+    const int np = window_parts(win_len, H_kv, waves);
+    float* ws = static_cast<float*>(out_attn);  // one part: the triple itself
+    hipError_t e = hipSuccess;
+    if (np > 1) e = workspace((size_t)H_q * np * 258 * sizeof(float), stream, &ws);
     if (e != hipSuccess) return rc_of(e);
     khq::WinArgs w{};
     w.q = static_cast<const __half*>(q);
@@ -368,8 +383,8 @@ int launch_khq_window_attn_fp16(const void* q, const void* ring_k, const void* r
     w.part_stride = np;
     w.part_offset = 0;
     w.sc = scale;
-    e = khq::launch_window_parts(w, H_q / H_kv, dim3(np, H_kv), stream);
-    if (e != hipSuccess) return rc_of(e);
+    e = khq::launch_window_parts(w, H_q / H_kv, H_kv, waves, stream);
+    if (e != hipSuccess || np == 1) return rc_of(e);
     return rc_of(khq::launch_lse_reduce(ws, static_cast<float*>(out_attn), H_q, np, stream));
 }
 
@@ -424,8 +439,8 @@ int launch_khq_gqa_attn_fp16(const void* q_gate, const void* k_cache, const void
     if (head_dim != 256 || seq_len <= 0 || H_q <= 0 || H_kv <= 0 || H_q % H_kv != 0 ||
         H_q / H_kv > 8)
         return -100;
-    // 8 positions per part (two per wavefront): 512 positions fill 256 blocks
-    const int np = std::max(1, std::min(256, (seq_len + 7) / 8));
+    const int waves = window_waves(seq_len, H_kv);
+    const int np = window_parts(seq_len, H_kv, waves);
     float* ws = nullptr;
     hipError_t e = workspace((size_t)H_q * np * 258 * sizeof(float), stream, &ws);
     if (e != hipSuccess) return rc_of(e);
@@ -442,7 +457,7 @@ int launch_khq_gqa_attn_fp16(const void* q_gate, const void* k_cache, const void
     w.part_stride = np;
     w.part_offset = 0;
     w.sc = scale;
-    e = khq::launch_window_parts(w, H_q / H_kv, dim3(np, H_kv), stream);
+    e = khq::launch_window_parts(w, H_q / H_kv, H_kv, waves, stream);
     if (e != hipSuccess) return rc_of(e);
     // merge of the parts with every load issued up front (the window is all parts)
     khq::FinishArgs f{};
@@ -516,7 +531,8 @@ static int attn_step_impl(const void* q_gate, const void* k_payload, const void*
     const bool win_in_ws = fused_tail && npc > 0 && win_len > 0 &&
                            g_kernel_choice.load(std::memory_order_relaxed) == 0 &&
                            use_mfma(n_rep, H_kv, 1);
-    const int npw = (win_len > 0 && !fused_tail) ? window_parts(win_len) : (win_in_ws ? 1 : 0);
+    // (64 window parts at most: the fixed array of the no-allocation step holds those)
+    const int npw = (win_len > 0 && !fused_tail) ? window_parts(win_len, H_kv, 4, 64) : (win_in_ws ? 1 : 0);
     const int np = npc + npw;
     const size_t ws_bytes = (size_t)H_q * std::max(np, 1) * 258 * sizeof(float);
     float* ws = nullptr;
@@ -589,7 +605,7 @@ static int attn_step_impl(const void* q_gate, const void* k_payload, const void*
         w.part_stride = np;
         w.part_offset = npc;
         w.sc = scale;
-        e = khq::launch_window_parts(w, n_rep, dim3(npw, H_kv), stream);
+        e = khq::launch_window_parts(w, n_rep, H_kv, 4, stream);
         if (e != hipSuccess) return rc_of(e);
     }
     return rc_of(khq::launch_combine_gate(ws, static_cast<const __half*>(q_gate),

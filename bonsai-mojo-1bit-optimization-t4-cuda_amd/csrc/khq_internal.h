@@ -108,7 +108,8 @@ hipError_t launch_compress(const __half* x, const __half* d_vec, const __half* r
                            uint8_t* out_sm, int n, float ts, float alpha, int is_v,
                            hipStream_t st);
 hipError_t launch_attn_parts(const AttnArgs& a, int n_rep, dim3 grid, hipStream_t st);
-hipError_t launch_window_parts(const WinArgs& a, int n_rep, dim3 grid, hipStream_t st);
+// waves: wavefronts per block, 1 or 4.
+hipError_t launch_window_parts(const WinArgs& a, int n_rep, int h_kv, int waves, hipStream_t st);
 hipError_t launch_lse_reduce(const float* part, float* out, int n_q, int n_parts,
                              hipStream_t st);
 hipError_t launch_combine_gate(const float* part, const __half* q_gate, __half* out, int H_q,

@@ -291,109 +291,194 @@ __global__ __launch_bounds__(256) void attn_part_kernel(AttnArgs a) {
 }
 
 // --------------------------------------------------------- fp16 window parts
-// One 256-thread block per (window part, KV head); each wavefront walks every
-// fourth slot of the part, lane p holding dims 4p..4p+3 of K and V, and the
-// n_rep heads of the group share each K/V row.
-template <int NREP>
-__global__ __launch_bounds__(256) void window_part_kernel(WinArgs a) {
-    __shared__ float s_acc[4][NREP][256];
-    __shared__ float s_ml[4][NREP][2];
-    const int wave = threadIdx.x >> 6;
-    const int p = threadIdx.x & 63;
-    const int part = blockIdx.x;
-    const int hkv = blockIdx.y;
-    const int per = (a.win_len + a.n_parts - 1) / a.n_parts;
-    const int lo = min(part * per, a.win_len);
-    const int hi = min(lo + per, a.win_len);
-    float q[NREP][4];
+// One block of NW wavefronts per (window part, KV head); a wavefront takes
+// every NW-th 16-slot tile of the part.  HBM-bound (4 KB a slot over the four
+// KV heads), so each wavefront keeps a tile of K and one of V in flight: the
+// next K rows are requested when the scores have used the current ones, the
+// next V rows after P x V.
+//   scores: S^T (16 slots x heads) on 16x16x32 MFMA, exact fp16 operands
+//     straight from global memory (lane (slot li, lg) holds dims 32 st + 8 lg);
+//     the lane-per-patch form this replaces spent a six-step wavefront sum on
+//     every (slot, head).  Lane (head li, lg) gets slots 4 lg .. + 3.
+//   softmax: per-head reference maximum, raised only when a tile exceeds it by
+//     more than 8; the state lives in the head's lanes.
+//   P x V: fp32 weights broadcast through LDS (one read of the slot's heads),
+//     lane p owning dims 4 p .. + 3 of every V row (512 contiguous bytes a row);
+//     24 multiply-adds a slot leave the vector ALUs a quarter busy.
+// NW = 1 while a tile can be a block of its own: one CU reads 16 KB in well
+// under a round trip, but four tiles in 7 us and a whole 185-slot window, 190 KB,
+// in 11 (8 wavefronts a block).  24 / 4 heads: 512 positions 7.8 -> 5.3 us,
+// 16,001 positions 43.7 -> 16.0 us (4.1 TB/s of the 4.9 a large copy reaches).
+constexpr int WIN_TILE = 16;
+template <int NREP, int NW>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)))
+void window_part_kernel(WinArgs a) {
+    __shared__ float s_acc[NW > 1 ? NW / 2 : 1][NREP][256];
+    __shared__ float s_ml[NW][NREP][2];
+    __shared__ __align__(16) float s_w[NW][WIN_TILE][8];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int li = lane & 15, lg = lane >> 4;
+    const int part = blockIdx.x, hkv = blockIdx.y;
+    const int n_tiles = (a.win_len + WIN_TILE - 1) / WIN_TILE;
+    const int per = (n_tiles + a.n_parts - 1) / a.n_parts;
+    const int t_hi = min(n_tiles, (part + 1) * per);
+    const int w_start = a.win_start % a.ring_cap;
+    const size_t row = (size_t)a.h_kv * 256;
+    const __half* kbase = a.ring_k + (size_t)hkv * 256 + 8 * lg;
+    const __half* vbase = a.ring_v + (size_t)hkv * 256 + 4 * lane;
+    auto slot_of = [&](int s) {  // slots past the window read its last one
+        const int x = w_start + min(s, a.win_len - 1);
+        return (size_t)(x >= a.ring_cap ? x - a.ring_cap : x);
+    };
+    mu::h8 q[8];  // column li of Q^T: head li, the columns past NREP repeat the last
+    {
+        const __half* qp = a.q + (size_t)(hkv * NREP + min(li, NREP - 1)) * 512 + 8 * lg;
 #pragma unroll
-    for (int i = 0; i < NREP; i++) {
-        const __half* qp = a.q + (size_t)(hkv * NREP + i) * 512 + p * 4;
-#pragma unroll
-        for (int c = 0; c < 4; c++) q[i][c] = h2f(qp[c]);
+        for (int st = 0; st < 8; st++)
+            q[st] = __builtin_bit_cast(mu::h8, *reinterpret_cast<const uint4*>(qp + 32 * st));
     }
-    float acc[NREP][4], mx[NREP], sm[NREP];
+    uint4 kr[8];
+    uint2 vr[WIN_TILE];
+    auto load_k = [&](int t) {
+        const __half* kp = kbase + slot_of(WIN_TILE * t + li) * row;
 #pragma unroll
-    for (int i = 0; i < NREP; i++) {
-        mx[i] = -1e20f;
-        sm[i] = 0.0f;
+        for (int st = 0; st < 8; st++) kr[st] = *reinterpret_cast<const uint4*>(kp + 32 * st);
+    };
+    auto load_v = [&](int t) {
+#pragma unroll
+        for (int i = 0; i < WIN_TILE; i++)
+            vr[i] = *reinterpret_cast<const uint2*>(vbase + slot_of(WIN_TILE * t + i) * row);
+    };
+    float acc[NREP][4];
+#pragma unroll
+    for (int i = 0; i < NREP; i++)
 #pragma unroll
         for (int c = 0; c < 4; c++) acc[i][c] = 0.0f;
+    float m_ref = -INFINITY, l_part = 0.0f;
+    auto from_lane = [](float v, int l) {
+        return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+    };
+
+    int t = part * per + wave;
+    if (t < t_hi) {
+        load_k(t);
+        load_v(t);
     }
-    // the wavefront's slots lo + wave + 4 j in groups of WG, every load of a
-    // group issued before the first is used (same slot order as one at a time)
-    constexpr int WG = 4;
-    for (int s0 = lo + wave; s0 < hi; s0 += 4 * WG) {
-        uint2 kraw[WG], vraw[WG];
+    for (; t < t_hi; t += NW) {
+        mu::f4 s = mu::f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int j = 0; j < WG; j++) {
-            const int s = min(s0 + 4 * j, hi - 1);
-            const int slot = (a.win_start + s) % a.ring_cap;
-            const size_t off = ((size_t)slot * a.h_kv + hkv) * 256 + p * 4;
-            kraw[j] = *reinterpret_cast<const uint2*>(a.ring_k + off);
-            vraw[j] = *reinterpret_cast<const uint2*>(a.ring_v + off);
+        for (int st = 0; st < 8; st++) s = mu::mfma32(__builtin_bit_cast(mu::h8, kr[st]), q[st], s);
+        if (t + NW < t_hi) load_k(t + NW);
+        float sc[4], mx = -INFINITY;
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            sc[c] = WIN_TILE * t + 4 * lg + c < a.win_len ? s[c] * a.sc : -INFINITY;
+            mx = fmaxf(mx, sc[c]);
         }
-#pragma unroll
-        for (int j = 0; j < WG; j++) {
-            if (s0 + 4 * j >= hi) break;  // uniform per wavefront
-            const __half* kh = reinterpret_cast<const __half*>(&kraw[j]);
-            const __half* vh = reinterpret_cast<const __half*>(&vraw[j]);
-            float k[4], v[4];
-#pragma unroll
-            for (int c = 0; c < 4; c++) { k[c] = h2f(kh[c]); v[c] = h2f(vh[c]); }
+        const auto p16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(mx), __float_as_uint(mx),
+                                                          false, false);
+        mx = fmaxf(__uint_as_float(p16[0]), __uint_as_float(p16[1]));
+        const auto p32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx),
+                                                          false, false);
+        mx = fmaxf(__uint_as_float(p32[0]), __uint_as_float(p32[1]));
+        const bool need = mx > m_ref + 8.0f;
+        if (__ballot(need) != 0ull) {
+            const float fac = need ? mu::fexp(m_ref - mx) : 1.0f;  // 0 when m_ref = -inf
+            m_ref = need ? mx : m_ref;
+            l_part *= fac;
 #pragma unroll
             for (int i = 0; i < NREP; i++) {
-                float t = q[i][0] * k[0];
-                t = fmaf(q[i][1], k[1], t);
-                t = fmaf(q[i][2], k[2], t);
-                t = fmaf(q[i][3], k[3], t);
-                const float sv = wave_sum(t) * a.sc;
-                float e;
-                if (sv > mx[i]) {
-                    const float fac = expf(mx[i] - sv);
-                    sm[i] = fmaf(sm[i], fac, 1.0f);
+                const float f = from_lane(fac, i);
 #pragma unroll
-                    for (int c = 0; c < 4; c++) acc[i][c] *= fac;
-                    mx[i] = sv;
-                    e = 1.0f;
-                } else {
-                    e = expf(sv - mx[i]);
-                    sm[i] += e;
-                }
-#pragma unroll
-                for (int c = 0; c < 4; c++) acc[i][c] = fmaf(e, v[c], acc[i][c]);
+                for (int c = 0; c < 4; c++) acc[i][c] *= f;
             }
         }
-    }
 #pragma unroll
-    for (int i = 0; i < NREP; i++) {
-#pragma unroll
-        for (int c = 0; c < 4; c++) s_acc[wave][i][p * 4 + c] = acc[i][c];
-        if (p == 0) {
-            s_ml[wave][i][0] = mx[i];
-            s_ml[wave][i][1] = sm[i];
+        for (int c = 0; c < 4; c++) {
+            const float w = sc[c] == -INFINITY ? 0.0f : mu::fexp(sc[c] - m_ref);
+            l_part += w;
+            if (li < NREP) s_w[wave][4 * lg + c][li] = w;
         }
+        mu::wave_sync();
+#pragma unroll
+        for (int p = 0; p < WIN_TILE; p++) {
+            const mu::h4 v = __builtin_bit_cast(mu::h4, vr[p]);
+            mu::f4 w[2];
+            w[0] = *reinterpret_cast<const mu::f4*>(&s_w[wave][p][0]);
+            if (NREP > 4) w[1] = *reinterpret_cast<const mu::f4*>(&s_w[wave][p][4]);
+#pragma unroll
+            for (int i = 0; i < NREP; i++)
+#pragma unroll
+                for (int c = 0; c < 4; c++)
+                    acc[i][c] = fmaf((float)v[c], w[i >> 2][i & 3], acc[i][c]);
+            // sums of four slots complete before the next slots' weights are
+            // read (all sixteen at once take 254 registers and spill at 8 heads)
+            if ((p & 3) == 3)
+#pragma unroll
+                for (int i = 0; i < NREP; i++)
+                    asm volatile("" : "+v"(acc[i][0]), "+v"(acc[i][1]), "+v"(acc[i][2]), "+v"(acc[i][3])
+                                 : : "memory");
+        }
+        mu::wave_sync();  // read before the next tile's weights
+        if (t + NW < t_hi) load_v(t + NW);
+    }
+
+    // ---- merge the wavefronts, upper half into lower half; one without a
+    // score (m_ref = -inf) weighs nothing
+    float l_row = l_part + __shfl_xor(l_part, 16, 64);
+    l_row += __shfl_xor(l_row, 32, 64);
+    if (lane < NREP) {
+        s_ml[wave][lane][0] = m_ref;
+        s_ml[wave][lane][1] = l_row;
     }
     __syncthreads();
-    for (int i = wave; i < NREP; i += 4) {
-        float M = -1e20f;
+    float M[NREP], den[NREP];
 #pragma unroll
-        for (int w = 0; w < 4; w++) M = fmaxf(M, s_ml[w][i][0]);
-        float den = 0.0f, o[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < NREP; i++) {
+        M[i] = -INFINITY;
 #pragma unroll
-        for (int w = 0; w < 4; w++) {
-            const float f = expf(s_ml[w][i][0] - M);
-            den = fmaf(s_ml[w][i][1], f, den);
+        for (int w = 0; w < NW; w++) M[i] = fmaxf(M[i], s_ml[w][i][0]);
+        den[i] = 0.0f;
 #pragma unroll
-            for (int c = 0; c < 4; c++) o[c] = fmaf(s_acc[w][i][p * 4 + c], f, o[c]);
+        for (int w = 0; w < NW; w++) {
+            const float m = s_ml[w][i][0];
+            den[i] = fmaf(s_ml[w][i][1], m == M[i] ? 1.0f : mu::fexp(m - M[i]), den[i]);
         }
+        const float m = s_ml[wave][i][0];
+        const float f = m == M[i] ? 1.0f : mu::fexp(m - M[i]);
+#pragma unroll
+        for (int c = 0; c < 4; c++) acc[i][c] *= f;
+    }
+#pragma unroll
+    for (int half = NW / 2; half >= 1; half /= 2) {
+        if (wave >= half && wave < 2 * half)
+#pragma unroll
+            for (int i = 0; i < NREP; i++)
+                *reinterpret_cast<float4*>(&s_acc[wave - half][i][4 * lane]) =
+                    make_float4(acc[i][0], acc[i][1], acc[i][2], acc[i][3]);
+        __syncthreads();
+        if (wave < half)
+#pragma unroll
+            for (int i = 0; i < NREP; i++) {
+                const float4 o = *reinterpret_cast<const float4*>(&s_acc[wave][i][4 * lane]);
+                acc[i][0] += o.x;
+                acc[i][1] += o.y;
+                acc[i][2] += o.z;
+                acc[i][3] += o.w;
+            }
+        __syncthreads();
+    }
+    if (wave != 0) return;
+#pragma unroll
+    for (int i = 0; i < NREP; i++) {
         const int h = hkv * NREP + i;
         float* out = a.part + ((size_t)h * a.part_stride + a.part_offset + part) * 258;
-#pragma unroll
-        for (int c = 0; c < 4; c++) out[p * 4 + c] = o[c];
-        if (p == 0) {
-            out[256] = M;
-            out[257] = den;
+        const bool empty = M[i] == -INFINITY;
+        *reinterpret_cast<float2*>(out + 4 * lane) = make_float2(acc[i][0], acc[i][1]);
+        *reinterpret_cast<float2*>(out + 4 * lane + 2) = make_float2(acc[i][2], acc[i][3]);
+        if (lane == 0) {
+            out[256] = empty ? -1e20f : M[i];
+            out[257] = empty ? 0.0f : den[i];
         }
     }
 }
@@ -623,10 +708,16 @@ hipError_t launch_attn_parts(const AttnArgs& a, int n_rep, dim3 grid, hipStream_
     return hipGetLastError();
 }
 
-hipError_t launch_window_parts(const WinArgs& a, int n_rep, dim3 grid, hipStream_t st) {
+hipError_t launch_window_parts(const WinArgs& a, int n_rep, int h_kv, int waves, hipStream_t st) {
+    const dim3 grid(a.n_parts, h_kv);
     switch (n_rep) {
-#define KHQ_CASE(N) \
-    case N: hipLaunchKernelGGL(window_part_kernel<N>, grid, dim3(256), 0, st, a); break;
+#define KHQ_CASE(N)                                                                          \
+    case N:                                                                                  \
+        if (waves == 1)                                                                      \
+            hipLaunchKernelGGL((window_part_kernel<N, 1>), grid, dim3(64), 0, st, a);        \
+        else                                                                                 \
+            hipLaunchKernelGGL((window_part_kernel<N, 4>), grid, dim3(256), 0, st, a);       \
+        break;
         KHQ_CASE(1) KHQ_CASE(2) KHQ_CASE(3) KHQ_CASE(4)
         KHQ_CASE(5) KHQ_CASE(6) KHQ_CASE(7) KHQ_CASE(8)
 #undef KHQ_CASE

@@ -473,9 +473,8 @@ def test_c3_precision_margin(device, data):
 def test_gqa_baseline_reference_cases(device):
     from test_oracle_pins import _modular_inputs, gqa_fp64
 
-    # 512 positions: 64 parts of 8 (two slots per wavefront); 3000 and 5000:
-    # 256 parts of 12 and 20 (a wavefront's slots in one part-filled group,
-    # and in a full group of four plus one)
+    # 512 positions: 32 one-tile parts a KV head; 3000 and 5000: parts of 4
+    # wavefronts, one tile each
     for H_q, H_kv, seq, max_seq in [(24, 4, 8, 16), (4, 2, 16, 16), (4, 2, 1, 16), (24, 4, 512, 512),
                                     (24, 4, 3000, 3000), (24, 4, 5000, 5000)]:
         qg, k, v = _modular_inputs(H_q, H_kv, 256, max_seq)
@@ -493,6 +492,62 @@ def test_gqa_baseline_reference_cases(device):
     assert ops.gqa_attn(t(qg16.reshape(H_q, 512)), t(k16.reshape(max_seq, H_kv, D)),
                         t(v16.reshape(max_seq, H_kv, D)), out, seq_len=4, H_q=4, H_kv=2,
                         head_dim=128, scale=0.1, check=False) == -100
+
+
+def _window_want(q, k, v, scale):
+    """float64 softmax attention of q [H_q, 256] over k, v [T, H_kv, 256] and its
+    logsumexp."""
+    n_rep = q.shape[0] // k.shape[1]
+    kr, vr = (np.repeat(x.astype(np.float64), n_rep, axis=1) for x in (k, v))
+    s = np.einsum("hd,thd->ht", q.astype(np.float64), kr) * scale
+    m = s.max(1, keepdims=True)
+    p = np.exp(s - m)
+    return np.einsum("ht,thd->hd", p, vr) / p.sum(1, keepdims=True), (m + np.log(p.sum(1, keepdims=True)))[:, 0]
+
+
+@pytest.mark.parametrize("H_q,H_kv,length", [
+    (24, 4, 15), (24, 4, 17), (24, 4, 2048), (24, 4, 2049), (24, 4, 9001),  # one / four wavefronts
+    (8, 1, 16), (7, 1, 33), (6, 2, 100), (1, 1, 8200), (40, 8, 300)])
+def test_fp16_attention_sizes(device, H_q, H_kv, length):
+    """The fp16 kernel around its 16-slot tiles, the switch from one to four
+    wavefronts a block (2 tiles a CU) and every group size, as the baseline
+    entry (gated fp16) and as the window entry (triple, wrapped ring)."""
+    rng = np.random.default_rng(length)
+    qg = rng.standard_normal((H_q, 512)).astype(np.float16)
+    k, v = (rng.standard_normal((length, H_kv, D)).astype(np.float16) for _ in range(2))
+    want, lse = _window_want(qg[:, :D], k, v, SCALE)
+    out = torch.zeros((H_q, D), device=device, dtype=torch.float16)
+    ops.gqa_attn(t(qg), t(k), t(v), out, seq_len=length, H_q=H_q, H_kv=H_kv, scale=SCALE)
+    gated = want / (1.0 + np.exp(-qg[:, D:].astype(np.float64)))
+    # fp16 rounding of the output (2^-11 of it) and fp32 arithmetic of scores
+    # up to ~6: exp amplifies their error, 256 products of 2^-24 each, to ~1e-5
+    err = np.abs(out.cpu().numpy() - gated) - 2.0 ** -11 * np.abs(gated)
+    assert err.max() <= 2e-5
+    start = length // 3
+    ring = [np.roll(x, start, axis=0) for x in (k, v)]
+    tri = torch.zeros((H_q, D + 2), device=device, dtype=torch.float32)
+    ops.window_attn(t(qg), t(ring[0]), t(ring[1]), tri, win_start=start + length, win_len=length,
+                    ring_cap=length, H_q=H_q, H_kv=H_kv, scale=SCALE)
+    got, got_lse = npref.triple_to_out(tri.cpu().numpy())
+    assert np.abs(got - want).max() <= 2e-5 and np.abs(got_lse - lse).max() <= 2e-5
+
+
+def test_fp16_attention_minus_inf_scores(device):
+    """A key whose score is -inf takes no part, also where a whole tile of 16
+    (the last one here) has nothing else."""
+    rng = np.random.default_rng(3)
+    qg = rng.standard_normal((24, 512)).astype(np.float16)
+    qg[:, 0] = -np.abs(qg[:, 0]) - np.float16(0.1)
+    k, v = (rng.standard_normal((70, 4, D)).astype(np.float16) for _ in range(2))
+    hidden = [21, *range(64, 70)]
+    want, lse = _window_want(qg[:, :D], np.delete(k, hidden, axis=0), np.delete(v, hidden, axis=0),
+                             SCALE)
+    k[hidden, :, 0] = np.inf
+    tri = torch.zeros((24, D + 2), device=device, dtype=torch.float32)
+    ops.window_attn(t(qg), t(k), t(v), tri, win_start=0, win_len=70, ring_cap=70, H_q=24, H_kv=4,
+                    scale=SCALE)
+    got, got_lse = npref.triple_to_out(tri.cpu().numpy())
+    assert np.abs(got - want).max() <= 2e-5 and np.abs(got_lse - lse).max() <= 2e-5
 
 
 def test_partial_rope_matches_oracle(device):
