@@ -248,13 +248,20 @@ int launch_khq_compress_fp16(const void* x, const void* d_vec, const void* rotor
                              void* out_shared_meta, int n, int d, float threshold_scale,
                              float alpha, int is_v, hipStream_t stream) {
     if (n <= 0 || d != 256) return -100;
-    return rc_of(khq::launch_compress(
-        static_cast<const __half*>(x), static_cast<const __half*>(d_vec),
-        static_cast<const __half*>(rotor), static_cast<const __half*>(centroids),
-        static_cast<const __half*>(vq_centroids), static_cast<uint32_t*>(out_mask),
-        static_cast<__half*>(out_norms), static_cast<__half*>(out_r_norms),
-        static_cast<uint8_t*>(out_payload), static_cast<uint8_t*>(out_shared_meta), n,
-        threshold_scale, alpha, is_v ? 1 : 0, stream));
+    const khq::CompressJob job{khq::RowSrc{static_cast<const __half*>(x), nullptr, 0, 0, 1},
+                               static_cast<const __half*>(d_vec),
+                               static_cast<const __half*>(rotor),
+                               static_cast<const __half*>(centroids),
+                               static_cast<const __half*>(vq_centroids),
+                               static_cast<uint32_t*>(out_mask),
+                               static_cast<__half*>(out_norms),
+                               static_cast<__half*>(out_r_norms),
+                               static_cast<uint8_t*>(out_payload),
+                               static_cast<uint8_t*>(out_shared_meta),
+                               n,
+                               threshold_scale,
+                               alpha};
+    return rc_of(khq::launch_compress(job, is_v ? 1 : 0, stream));
 }
 
 int launch_khq_attn_fp16(const void* q, const void* k_payload, const void* v_payload,

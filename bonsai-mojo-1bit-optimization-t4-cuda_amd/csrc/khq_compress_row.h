@@ -114,7 +114,7 @@ __device__ __forceinline__ void fold_sum2(const float* a, const float* b, int n,
 // Row r of the job is (token r / h_kv, KV head r % h_kv) of da.
 template <bool DEC = false>
 __device__ __forceinline__ void compress_block(
-    const __half* __restrict__ x, const __half* __restrict__ d_vec,
+    const RowSrc& x, const __half* __restrict__ d_vec,
     const __half* __restrict__ rotor, const __half* __restrict__ cents,
     const __half* __restrict__ vq, uint32_t* __restrict__ out_mask,
     __half* __restrict__ out_norms, __half* __restrict__ out_rn,
@@ -153,7 +153,7 @@ __device__ __forceinline__ void compress_block(
     const bool own_row = !is_v || wave == 0;  // uniform per wavefront
     float xv[4] = {0.f, 0.f, 0.f, 0.f};
     if (valid && own_row) {
-        const __half* xr = x + (size_t)row * 256 + lane * 4;
+        const __half* xr = x.row(row) + lane * 4;
 #pragma unroll
         for (int c = 0; c < 4; c++) xv[c] = h2f(xr[c]);
     }
@@ -390,6 +390,357 @@ __device__ __forceinline__ void compress_block(
         for (int c = 0; c < 4; c++)
             vt[((size_t)h * 256 + 4 * lane + c) * da->ld_vt + da->key0 + tok] = (_Float16)y[c];
     }
+}
+
+// ------------------------------------------------- compress, many rows
+// The same rows and the same bits, several rows a wavefront, for launches long
+// enough to fill the chip that way (compress_block spreads one V row over four
+// wavefronts and folds each row's sums in every lane: good for an event's few
+// hundred rows, 2-4 times the work for thousands).
+//   * The sequential folds run one row per lane: the 256 dependent steps serve
+//     all of a wavefront's rows at once.
+//   * V: the block's four wavefronts search a quarter of the codebook each for
+//     all VR rows, so a codeword is loaded and widened once per VR rows; each
+//     chunk of 8 codes costs a minimum (no index), and the winning chunk's
+//     distances are formed again at the end to find the first code equal to
+//     the minimum.  Distances, order and strict < are compress_block's, so the
+//     first minimum wins as there.
+// 8,000 rows: V 106 -> 39 us, bound by the vector ALUs (seven instructions a
+// (row, patch, code), six of them the distance: 31 us at full issue);
+// K 20.6 -> 15.7 us, 32,768 rows 66 -> 40 us, bound by its folds' latency.
+constexpr int CR_LD = 260;  // floats per LDS row: rows 4 banks apart, 16-byte aligned
+constexpr int VR = 8;       // V rows per block (two a wavefront for projection and packing)
+constexpr int KR = 4;       // K rows per wavefront
+
+__device__ __forceinline__ float row_value(float v, int r) {  // lane r's value, to all
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), r));
+}
+
+// xv: the lane's 4 dims of one row; its projection (ref .cu:1289-1312)
+__device__ __forceinline__ void project_row(const float (&xv)[4], const float (&dv4)[4],
+                                            const float (&rot)[16], float norm,
+                                            float (&proj)[4]) {
+    const float f_s = 0.0625f;
+    float r[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) r[c] = (xv[c] * dv4[c]) / (norm + 1e-8f);
+    fwht256(r);
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        float acc = r[0] * rot[0 * 4 + c];
+        acc = fmaf(r[1], rot[1 * 4 + c], acc);
+        acc = fmaf(r[2], rot[2 * 4 + c], acc);
+        acc = fmaf(r[3], rot[3 * 4 + c], acc);
+        proj[c] = acc * f_s;
+    }
+}
+
+// distances of the 8 codes in c (3 x 16 bytes) to (v0, v1, v2)
+__device__ __forceinline__ void dist8(const float (&c)[24], float alpha, float v0, float v1,
+                                      float v2, float (&d)[8]) {
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        const float d0 = fmaf(-c[3 * j], alpha, v0);
+        const float d1 = fmaf(-c[3 * j + 1], alpha, v1);
+        const float d2 = fmaf(-c[3 * j + 2], alpha, v2);
+        d[j] = fmaf(d2, d2, fmaf(d1, d1, d0 * d0));
+    }
+}
+__device__ __forceinline__ void widen8(const uint4 (&w)[3], float (&c)[24]) {
+    const uint16_t* h = reinterpret_cast<const uint16_t*>(w);
+#pragma unroll
+    for (int i = 0; i < 24; i++) c[i] = h2f(__ushort_as_half(h[i]));
+}
+
+__device__ __forceinline__ void compress_v_rows(const CompressJob& jb, int bid) {
+    __shared__ __align__(16) float s_x[VR][CR_LD];
+    __shared__ __align__(16) float s_pj[VR][256];
+    __shared__ float s_bd[4][VR][64];
+    __shared__ unsigned s_bc[4][VR][64];
+    constexpr int RW = VR / 4;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int row0 = bid * VR + wave * RW;  // the wavefront's rows to project and pack
+    float dv4[4], rot[16];
+#pragma unroll
+    for (int c = 0; c < 4; c++) dv4[c] = h2f(jb.d_vec[lane * 4 + c]);
+#pragma unroll
+    for (int i = 0; i < 16; i++) rot[i] = h2f(jb.rotor[lane * 16 + i]);
+    const float cv0 = h2f(jb.cents[lane * 4 + 3]), cv1 = h2f(jb.cents[256 + lane * 4 + 3]);
+    const uint4* cb4 = reinterpret_cast<const uint4*>(jb.vq + (size_t)lane * 768) + 24 * wave;
+    uint4 cur[3], nxt[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) cur[k] = cb4[k];
+
+    float xv[RW][4];
+#pragma unroll
+    for (int r = 0; r < RW; r++) {
+        const __half* xr = jb.x.row(min(row0 + r, jb.n - 1)) + lane * 4;
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            xv[r][c] = h2f(xr[c]);
+            s_x[wave * RW + r][lane * 4 + c] = xv[r][c];
+        }
+    }
+    mu::wave_sync();
+    const int my = lane % RW;  // the row this lane folds
+    const float norm = sqrtf(fold_sq256(s_x[wave * RW + my]) + 1e-8f);
+    if (lane < RW && row0 + lane < jb.n) jb.out_norms[row0 + lane] = __float2half(norm);
+#pragma unroll
+    for (int r = 0; r < RW; r++) {
+        float pj[4];
+        project_row(xv[r], dv4, rot, row_value(norm, r), pj);
+        *reinterpret_cast<float4*>(&s_pj[wave * RW + r][4 * lane]) =
+            make_float4(pj[0], pj[1], pj[2], pj[3]);
+    }
+    __syncthreads();
+
+    // ---- the wavefront's codebook quarter (codes 64 wave .. + 63), all VR rows
+    float v[VR][3], bd[VR];
+    unsigned bc[VR];
+#pragma unroll
+    for (int r = 0; r < VR; r++) {
+        const float4 p = *reinterpret_cast<const float4*>(&s_pj[r][4 * lane]);
+        v[r][0] = p.x;
+        v[r][1] = p.y;
+        v[r][2] = p.z;
+        bd[r] = 1e20f;
+        bc[r] = 0;
+    }
+#pragma unroll 1
+    for (unsigned ch = 0; ch < 8; ch++) {
+        if (ch < 7) {
+#pragma unroll
+            for (int k = 0; k < 3; k++) nxt[k] = cb4[3 * (ch + 1) + k];
+        }
+        float c[24];
+        widen8(cur, c);
+#pragma unroll
+        for (int r = 0; r < VR; r++) {
+            float d[8];
+            dist8(c, jb.alpha, v[r][0], v[r][1], v[r][2], d);
+            const float mn = fminf(fminf(fminf(fminf(d[0], d[1]), d[2]), fminf(fminf(d[3], d[4]), d[5])),
+                                   fminf(d[6], d[7]));
+            if (mn < bd[r]) {
+                bd[r] = mn;
+                bc[r] = ch;
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 3; k++) cur[k] = nxt[k];
+    }
+#pragma unroll
+    for (int r = 0; r < VR; r++) {
+        s_bd[wave][r][lane] = bd[r];
+        s_bc[wave][r][lane] = 8 * wave + bc[r];
+    }
+    __syncthreads();
+
+    // ---- the wavefront's own rows: winning chunk, first code at the minimum
+    uint4 win[RW][3];
+    float best_d[RW];
+    unsigned chunk[RW];
+    const uint4* cb0 = reinterpret_cast<const uint4*>(jb.vq + (size_t)lane * 768);
+#pragma unroll
+    for (int r = 0; r < RW; r++) {
+        const int br = wave * RW + r;
+        best_d[r] = s_bd[0][br][lane];
+        chunk[r] = s_bc[0][br][lane];
+#pragma unroll
+        for (int w = 1; w < 4; w++)
+            if (s_bd[w][br][lane] < best_d[r]) {
+                best_d[r] = s_bd[w][br][lane];
+                chunk[r] = s_bc[w][br][lane];
+            }
+#pragma unroll
+        for (int k = 0; k < 3; k++) win[r][k] = cb0[3 * chunk[r] + k];
+    }
+    uint32_t* s_pv = reinterpret_cast<uint32_t*>(s_bc);  // [4][RW][64]; own wavefront's part of
+                                                         // s_x holds the energies
+    __syncthreads();  // s_bd / s_bc read out
+    float max_res[RW];
+    uint64_t hi[RW];
+#pragma unroll
+    for (int r = 0; r < RW; r++) {
+        const int br = wave * RW + r;
+        const float4 pj = *reinterpret_cast<const float4*>(&s_pj[br][4 * lane]);
+        float c[24], d[8];
+        widen8(win[r], c);
+        dist8(c, jb.alpha, pj.x, pj.y, pj.z, d);
+        unsigned j = 0;
+        float h0 = c[0], h1 = c[1], h2 = c[2];
+#pragma unroll
+        for (int k = 7; k >= 0; k--)
+            if (d[k] == best_d[r] && best_d[r] < 1e20f) {
+                j = k;
+                h0 = c[3 * k];
+                h1 = c[3 * k + 1];
+                h2 = c[3 * k + 2];
+            }
+        // no code below the initial 1e20: chunk 0 and code 0, as the search leaves it
+        const unsigned best = 8 * chunk[r] + j;
+        const float c0 = h0 * jb.alpha, c1 = h1 * jb.alpha, c2 = h2 * jb.alpha;
+        s_x[br][lane] = fmaf(pj.z, pj.z, fmaf(pj.y, pj.y, pj.x * pj.x));
+        s_x[br][64 + lane] = fmaf(c2, c2, fmaf(c1, c1, c0 * c0));
+        const float dd0 = fabsf(fmaf(-cv0, jb.alpha, pj.w));
+        const float dd1 = fabsf(fmaf(-cv1, jb.alpha, pj.w));
+        unsigned bs = 0;
+        float best_s = 1e20f;
+        if (dd0 < best_s) { best_s = dd0; bs = 0; }
+        if (dd1 < best_s) { best_s = dd1; bs = 1; }
+        const float resid = fmaf(-(bs ? cv1 : cv0), jb.alpha, pj.w);
+        max_res[r] = wave_max(fabsf(resid));
+        const float res_scale = fmaxf(max_res[r], 1e-4f);
+        const float scaled = fmaf(resid / res_scale, 7.0f, 8.0f);
+        const unsigned dump = (unsigned)fmaxf(0.0f, fminf(15.0f, roundf(scaled)));
+        s_pv[br * 64 + lane] = (best & 0x7Fu) | ((bs & 1u) << 7) | ((dump & 0xFu) << 8);
+        hi[r] = __ballot(((best >> 7) & 1u) != 0u);
+    }
+    mu::wave_sync();
+    float st, sv;
+    fold_sum2(s_x[wave * RW + my], s_x[wave * RW + my] + 64, 64, st, sv);
+    if (lane < RW && row0 + lane < jb.n) jb.out_rn[row0 + lane] = __float2half(sqrtf(st / (sv + 1e-8f)));
+#pragma unroll
+    for (int r = 0; r < RW; r++) {
+        const int row = row0 + r;
+        if (row >= jb.n) break;  // uniform per wavefront
+        uint32_t* op = reinterpret_cast<uint32_t*>(jb.out_pay + (size_t)row * 104);
+        if (lane < 8) {
+            const uint32_t* p = &s_pv[(wave * RW + r) * 64 + lane * 8];
+            op[lane * 3 + 0] = p[0] | (p[1] << 12) | ((p[2] & 0xFFu) << 24);
+            op[lane * 3 + 1] = (p[2] >> 8) | (p[3] << 4) | (p[4] << 16) | ((p[5] & 0xFu) << 28);
+            op[lane * 3 + 2] = (p[5] >> 4) | (p[6] << 8) | (p[7] << 20);
+        } else if (lane == 8) {
+            op[24] = (uint32_t)(hi[r] & 0xFFFFFFFFull);
+            op[25] = (uint32_t)(hi[r] >> 32);
+        } else if (lane == 9) {
+            *reinterpret_cast<float*>(jb.out_sm + (size_t)row * 4) = max_res[r];
+        }
+    }
+}
+
+__device__ __forceinline__ void compress_k_rows(const CompressJob& jb, int bid) {
+    __shared__ __align__(16) float s_a[4][KR][CR_LD];
+    __shared__ __align__(16) float s_b[4][KR][CR_LD];
+    __shared__ uint32_t s_w[4][KR][32];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int row0 = (bid * 4 + wave) * KR;
+    const float f_s = 0.0625f;
+    float dv4[4], rot[16], cbk[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        dv4[c] = h2f(jb.d_vec[lane * 4 + c]);
+        cbk[c] = h2f(jb.cents[2 * 256 + lane * 4 + c]);
+    }
+#pragma unroll
+    for (int i = 0; i < 16; i++) rot[i] = h2f(jb.rotor[lane * 16 + i]);
+    float pj[KR][4];  // the rows, then their projections
+#pragma unroll
+    for (int r = 0; r < KR; r++) {
+        const __half* xr = jb.x.row(min(row0 + r, jb.n - 1)) + lane * 4;
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            pj[r][c] = h2f(xr[c]);
+            s_a[wave][r][lane * 4 + c] = pj[r][c];
+        }
+        if (lane < 32) s_w[wave][r][lane] = 0u;
+    }
+    mu::wave_sync();
+    const int my = lane % KR;  // the row this lane folds
+    const float norm = sqrtf(fold_sq256(s_a[wave][my]) + 1e-8f);
+    mu::wave_sync();  // s_a is reused
+    unsigned code[KR], ord[KR], n_out[KR];  // codes as the mask byte; first ordinal
+    const uint64_t lt = lanemask_lt();
+#pragma unroll
+    for (int r = 0; r < KR; r++) {
+        const float x[4] = {pj[r][0], pj[r][1], pj[r][2], pj[r][3]};
+        project_row(x, dv4, rot, row_value(norm, r), pj[r]);
+        bool cand[4];
+        unsigned base = 0, total = 0;
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            cand[c] = fabsf(pj[r][c]) > 1.60f * f_s;
+            const uint64_t b = __ballot(cand[c]);
+            base += (unsigned)__popcll(b & lt);
+            total += (unsigned)__popcll(b);
+        }
+        n_out[r] = total < 50u ? total : 50u;
+        ord[r] = base;
+        code[r] = 0;
+        unsigned run = base;
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            float sa = 0.0f, sb = 0.0f;
+            unsigned cd;
+            if (cand[c]) {
+                cd = (run < 50u) ? 3u : (pj[r][c] > 0.0f ? 2u : 1u);
+                run++;
+            } else {
+                cd = pj[r][c] > 0.47f * f_s ? 2u : (pj[r][c] < -0.47f * f_s ? 1u : 0u);
+                if (cd != 0u) {
+                    sa = fabsf(pj[r][c]);
+                    sb = cbk[c];
+                }
+            }
+            code[r] |= cd << (2 * c);
+            s_a[wave][r][lane * 4 + c] = sa;
+            s_b[wave][r][lane * 4 + c] = sb;
+        }
+        atomicOr(&s_w[wave][r][16 + (lane >> 2)], code[r] << (8 * (lane & 3)));
+    }
+    mu::wave_sync();
+    float sum_normals, sum_cbase;
+    fold_sum2(s_a[wave][my], s_b[wave][my], 256, sum_normals, sum_cbase);
+    float mult_my = (sum_cbase > 1e-5f) ? (sum_normals / sum_cbase) : 1.0f;
+    if (mult_my < 0.1f || mult_my > 10.0f || isnan(mult_my)) mult_my = 1.0f;
+    float rs[KR];
+#pragma unroll
+    for (int r = 0; r < KR; r++) {
+        const float mult = row_value(mult_my, r);
+        float res[4] = {0.f, 0.f, 0.f, 0.f};
+        float my_max = 0.0f;
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+            if (((code[r] >> (2 * c)) & 3u) == 3u) {
+                res[c] = fmaxf(0.0f, fmaf(-cbk[c], mult, fabsf(pj[r][c] * jb.ts)));
+                my_max = fmaxf(my_max, res[c]);
+            }
+        const float max_res = wave_max(my_max);
+        rs[r] = (n_out[r] > 0u) ? (fmaxf(max_res, 1e-4f) / 15.0f) : 0.0f;
+        unsigned j = ord[r];
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+            if (((code[r] >> (2 * c)) & 3u) == 3u) {
+                if (rs[r] > 0.0f) {
+                    const float r4 = roundf(res[c] / rs[r]);
+                    const unsigned rv = (unsigned)(uint8_t)fmaxf(0.0f, fminf(15.0f, r4));
+                    const unsigned by = 4u + j / 2u;
+                    atomicOr(&s_w[wave][r][by >> 2], rv << (8u * (by & 3u) + 4u * (j & 1u)));
+                }
+                if (pj[r][c] > 0.0f) {
+                    const unsigned by = 29u + j / 8u;
+                    atomicOr(&s_w[wave][r][by >> 2], 1u << (8u * (by & 3u) + (j & 7u)));
+                }
+                j++;
+            }
+        if (lane == 0) {
+            atomicOr(&s_w[wave][r][0], (unsigned)(mult * 1000.0f));
+            atomicOr(&s_w[wave][r][9], 0x02u);
+        }
+    }
+    mu::wave_sync();
+#pragma unroll
+    for (int r = 0; r < KR; r++) {
+        const int row = row0 + r;
+        if (row >= jb.n) break;  // uniform per wavefront
+        if (lane < 16) jb.out_mask[(size_t)row * 16 + lane] = s_w[wave][r][16 + lane];
+        if (lane < 10)
+            reinterpret_cast<uint32_t*>(jb.out_pay + (size_t)row * 40)[lane] = s_w[wave][r][lane];
+        if (lane == 0) {
+            jb.out_rn[row] = __float2half(rs[r]);
+            if (jb.out_sm) *reinterpret_cast<uint32_t*>(jb.out_sm + (size_t)row * 4) = 0u;
+        }
+    }
+    if (lane < KR && row0 + lane < jb.n) jb.out_norms[row0 + lane] = __float2half(norm);
 }
 
 }  // namespace khq

@@ -85,9 +85,21 @@ hipError_t launch_meta_upload(const void* host_src, void* dst, size_t bytes, hip
 hipError_t launch_step_finish_batched(const FinishArgs* args, int n_seq, int H_q,
                                       hipStream_t st);
 
-// One compressor job (the arguments of launch_compress without is_v).
+// Rows of 256 halves to compress: the first n_ring from a ring buffer of
+// ring_rows rows starting at row ring_row0 (wrapping), the rest from src.
+struct RowSrc {
+    const __half* src;
+    const __half* ring;
+    int n_ring, ring_row0, ring_rows;
+    __device__ __forceinline__ const __half* row(int r) const {
+        if (r >= n_ring) return src + (size_t)(r - n_ring) * 256;
+        const int s = ring_row0 + r;
+        return ring + (size_t)(s >= ring_rows ? s - ring_rows : s) * 256;
+    }
+};
+// One compressor job.
 struct CompressJob {
-    const __half* x;
+    RowSrc x;
     const __half* d_vec;
     const __half* rotor;
     const __half* cents;
@@ -102,11 +114,7 @@ struct CompressJob {
 };
 // The K and V jobs of one compression event in one launch.
 hipError_t launch_compress_pair(const CompressJob& k, const CompressJob& v, hipStream_t st);
-hipError_t launch_compress(const __half* x, const __half* d_vec, const __half* rotor,
-                           const __half* cents, const __half* vq, uint32_t* out_mask,
-                           __half* out_norms, __half* out_rn, uint8_t* out_pay,
-                           uint8_t* out_sm, int n, float ts, float alpha, int is_v,
-                           hipStream_t st);
+hipError_t launch_compress(const CompressJob& job, int is_v, hipStream_t st);
 hipError_t launch_attn_parts(const AttnArgs& a, int n_rep, dim3 grid, hipStream_t st);
 // waves: wavefronts per block, 1 or 4.
 hipError_t launch_window_parts(const WinArgs& a, int n_rep, int h_kv, int waves, hipStream_t st);

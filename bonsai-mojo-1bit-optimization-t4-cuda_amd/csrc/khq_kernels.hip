@@ -18,15 +18,15 @@
 
 namespace khq {
 
-__global__ __launch_bounds__(256) void compress_kernel(
-    const __half* __restrict__ x, const __half* __restrict__ d_vec,
-    const __half* __restrict__ rotor, const __half* __restrict__ cents,
-    const __half* __restrict__ vq, uint32_t* __restrict__ out_mask,
-    __half* __restrict__ out_norms, __half* __restrict__ out_rn,
-    uint8_t* __restrict__ out_pay, uint8_t* __restrict__ out_sm, int n, float ts,
-    float alpha, int is_v) {
-    compress_block(x, d_vec, rotor, cents, vq, out_mask, out_norms, out_rn, out_pay, out_sm, n, ts,
-                   alpha, is_v, (int)blockIdx.x);
+__global__ __launch_bounds__(256) void compress_kernel(CompressJob j, int is_v) {
+    compress_block(j.x, j.d_vec, j.rotor, j.cents, j.vq, j.out_mask, j.out_norms, j.out_rn,
+                   j.out_pay, j.out_sm, j.n, j.ts, j.alpha, is_v, (int)blockIdx.x);
+}
+__global__ __launch_bounds__(256) void compress_v_rows_kernel(CompressJob j) {
+    compress_v_rows(j, (int)blockIdx.x);
+}
+__global__ __launch_bounds__(256) void compress_k_rows_kernel(CompressJob j) {
+    compress_k_rows(j, (int)blockIdx.x);
 }
 
 // K and V of one compression event in one launch: blocks [0, nb_k) run the K
@@ -726,14 +726,21 @@ hipError_t launch_window_parts(const WinArgs& a, int n_rep, int h_kv, int waves,
     return hipGetLastError();
 }
 
-hipError_t launch_compress(const __half* x, const __half* d_vec, const __half* rotor,
-                           const __half* cents, const __half* vq, uint32_t* out_mask,
-                           __half* out_norms, __half* out_rn, uint8_t* out_pay,
-                           uint8_t* out_sm, int n, float ts, float alpha, int is_v,
-                           hipStream_t st) {
-    const int blocks = is_v ? n : (n + 3) / 4;
-    hipLaunchKernelGGL(compress_kernel, dim3(blocks), dim3(256), 0, st, x, d_vec, rotor, cents,
-                       vq, out_mask, out_norms, out_rn, out_pay, out_sm, n, ts, alpha, is_v);
+hipError_t launch_compress(const CompressJob& j, int is_v, hipStream_t st) {
+    // Where several rows a wavefront overtake one (their blocks take 14 us
+    // however few there are): V between 512 rows (12.1 us one row a block, 14.6
+    // eight) and 1024 (19.1, 14.8); K between 4096 (12.6, 14.2) and 8000
+    // (20.6, 15.7).
+    const int n_cu = device_cu_count();
+    if (j.n >= (is_v ? 3 : 20) * n_cu) {
+        if (is_v)
+            hipLaunchKernelGGL(compress_v_rows_kernel, dim3((j.n + VR - 1) / VR), dim3(256), 0, st, j);
+        else
+            hipLaunchKernelGGL(compress_k_rows_kernel, dim3((j.n + 4 * KR - 1) / (4 * KR)), dim3(256),
+                               0, st, j);
+    } else {
+        hipLaunchKernelGGL(compress_kernel, dim3(is_v ? j.n : (j.n + 3) / 4), dim3(256), 0, st, j, is_v);
+    }
     return hipGetLastError();
 }
 

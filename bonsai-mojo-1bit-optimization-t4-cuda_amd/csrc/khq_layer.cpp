@@ -76,10 +76,10 @@ void compress_jobs(const khq_layer* L, khq::CompressJob* kj, khq::CompressJob* v
     const size_t r0 = (size_t)L->boundary * L->H_kv;
     const int n = kChunk * L->H_kv;
     auto h = [](const void* p) { return static_cast<const __half*>(p); };
-    *kj = khq::CompressJob{L->ring_u + (size_t)s0 * kv, h(L->d_k), h(L->rotor_k), h(L->cents_k),
+    *kj = khq::CompressJob{khq::RowSrc{L->ring_u + (size_t)s0 * kv, nullptr, 0, 0, 1}, h(L->d_k), h(L->rotor_k), h(L->cents_k),
                            h(L->cents_k), L->kmask + r0 * 16, L->knorm + r0, L->krn + r0,
                            L->kpay + r0 * 40, nullptr, n, L->ts_k, L->alpha_k};
-    *vj = khq::CompressJob{L->ring_v + (size_t)s0 * kv, h(L->d_v), h(L->rotor_v), h(L->cents_v),
+    *vj = khq::CompressJob{khq::RowSrc{L->ring_v + (size_t)s0 * kv, nullptr, 0, 0, 1}, h(L->d_v), h(L->rotor_v), h(L->cents_v),
                            h(L->vq), L->kmask + r0 * 16, L->vnorm + r0, L->vrn + r0,
                            L->vpay + r0 * 104, L->vsm + r0 * 4, n, L->ts_v, L->alpha_v};
 }

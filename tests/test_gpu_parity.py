@@ -127,6 +127,30 @@ def test_compress_bitexact_scaled_codebook(device):
     assert np.array_equal(pay.vrn.cpu().numpy().view(np.uint16), vrn.view(np.uint16))
 
 
+@pytest.mark.parametrize("n", [767, 768, 5119, 5125])
+def test_compress_many_rows_bitexact(device, n):
+    """Both sides of the row counts from which a wavefront takes several rows
+    (V 768, K 5120 on 256 CUs), ragged against 8 V rows a block and 16 K rows,
+    with zero and all-outlier rows among them."""
+    lc, h = layer_consts()
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal((n, D)).astype(np.float16)
+    x[n - 1] = 0.0
+    x[n - 2, ::2] = 6.0
+    x[17] = np.float16(1e-4) * x[17]
+    pay, cents = ops.Payload(n, device), cents_dev(lc, device)
+    ops.compress(t(x), cents, pay, 0, is_v=False)
+    ops.compress(t(x), cents, pay, 0, is_v=True)
+    torch.cuda.synchronize()
+    _, mask, nrm, rn, kp, _ = oracle.compress(x, h["d_k"], h["rotor_k"], h["cents_k"], h["cents_k"],
+                                              ts=lc.ts_k, alpha=lc.alpha_k, is_v=False)
+    _, _, vn, ve, vp, sm = oracle.compress(x, h["d_v"], h["rotor_v"], h["cents_v"], h["vq"],
+                                           ts=lc.ts_v, alpha=lc.alpha_v, is_v=True)
+    for got, want in ((pay.kmask, mask), (pay.knorm, nrm), (pay.krn, rn), (pay.kpay, kp),
+                      (pay.vnorm, vn), (pay.vrn, ve), (pay.vpay, vp), (pay.vsm, sm)):
+        assert got.cpu().numpy().tobytes() == np.ascontiguousarray(want).tobytes()
+
+
 def test_compress_error_codes(device):
     lib = __import__("khq._lib", fromlist=["lib"])
     rc = lib.call("launch_khq_compress_fp16", *([None] * 10), 0, 256, 1.0, 1.0, 0, None,
