@@ -112,6 +112,14 @@ __device__ __forceinline__ void fold_sum2(const float* a, const float* b, int n,
 // at key key0 + token, V^T column key0 + token of da), from the fields just
 // packed, rounded as they are stored, so the result is the decode launch's.
 // Row r of the job is (token r / h_kv, KV head r % h_kv) of da.
+//
+// lds: the block's CompressLds (passed in: a launch whose blocks do different
+// jobs gives them the same LDS).
+struct __align__(16) CompressLds {
+    float a[4][256], b[4][256], pj[256], bd[4][64];
+    unsigned bi[4][64];
+    uint32_t w[4][32], pv[4][64];
+};
 template <bool DEC = false>
 __device__ __forceinline__ void compress_block(
     const RowSrc& x, const __half* __restrict__ d_vec,
@@ -119,10 +127,11 @@ __device__ __forceinline__ void compress_block(
     const __half* __restrict__ vq, uint32_t* __restrict__ out_mask,
     __half* __restrict__ out_norms, __half* __restrict__ out_rn,
     uint8_t* __restrict__ out_pay, uint8_t* __restrict__ out_sm, int n, float ts,
-    float alpha, int is_v, int bid, const DecompArgs* da = nullptr) {
-    __shared__ float s_a[4][256];
-    __shared__ float s_b[4][256];
-    __shared__ uint32_t s_w[4][32];
+    float alpha, int is_v, int bid, void* lds, const DecompArgs* da = nullptr) {
+    CompressLds& L = *static_cast<CompressLds*>(lds);
+    auto& s_a = L.a;
+    auto& s_b = L.b;
+    auto& s_w = L.w;
     const int wave = threadIdx.x >> 6;
     const int lane = threadIdx.x & 63;
     // K: one row per wavefront.  V: one row per block, the four wavefronts
@@ -149,7 +158,7 @@ __device__ __forceinline__ void compress_block(
     // A V row's four wavefronts share one row: wavefront 0 computes its
     // projection and hands it to the others through LDS (the search below
     // is what needs all four).
-    __shared__ float s_pj[256];
+    auto& s_pj = L.pj;
     const bool own_row = !is_v || wave == 0;  // uniform per wavefront
     float xv[4] = {0.f, 0.f, 0.f, 0.f};
     if (valid && own_row) {
@@ -320,8 +329,8 @@ __device__ __forceinline__ void compress_block(
         for (int k = 0; k < 12; k++) cur[k] = nxt[k];
     }
     {
-        __shared__ float s_bd[4][64];
-        __shared__ unsigned s_bi[4][64];
+        auto& s_bd = L.bd;
+        auto& s_bi = L.bi;
         s_bd[wave][lane] = best_d;
         s_bi[wave][lane] = best;
         __syncthreads();
@@ -358,7 +367,7 @@ __device__ __forceinline__ void compress_block(
     const uint64_t hi = __ballot(((best >> 7) & 1u) != 0u);
     s_a[wave][lane] = te;
     s_b[wave][lane] = ve;
-    __shared__ uint32_t s_pv[4][64];
+    auto& s_pv = L.pv;
     s_pv[wave][lane] = pv;
     __syncthreads();
     if (!live) return;
@@ -452,11 +461,16 @@ __device__ __forceinline__ void widen8(const uint4 (&w)[3], float (&c)[24]) {
     for (int i = 0; i < 24; i++) c[i] = h2f(__ushort_as_half(h[i]));
 }
 
-__device__ __forceinline__ void compress_v_rows(const CompressJob& jb, int bid) {
-    __shared__ __align__(16) float s_x[VR][CR_LD];
-    __shared__ __align__(16) float s_pj[VR][256];
-    __shared__ float s_bd[4][VR][64];
-    __shared__ unsigned s_bc[4][VR][64];
+struct __align__(16) VRowsLds {
+    float x[VR][CR_LD], pj[VR][256], bd[4][VR][64];
+    unsigned bc[4][VR][64];
+};
+__device__ __forceinline__ void compress_v_rows(const CompressJob& jb, int bid, void* lds) {
+    VRowsLds& L = *static_cast<VRowsLds*>(lds);
+    auto& s_x = L.x;
+    auto& s_pj = L.pj;
+    auto& s_bd = L.bd;
+    auto& s_bc = L.bc;
     constexpr int RW = VR / 4;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int row0 = bid * VR + wave * RW;  // the wavefront's rows to project and pack
@@ -618,10 +632,15 @@ __device__ __forceinline__ void compress_v_rows(const CompressJob& jb, int bid) 
     }
 }
 
-__device__ __forceinline__ void compress_k_rows(const CompressJob& jb, int bid) {
-    __shared__ __align__(16) float s_a[4][KR][CR_LD];
-    __shared__ __align__(16) float s_b[4][KR][CR_LD];
-    __shared__ uint32_t s_w[4][KR][32];
+struct __align__(16) KRowsLds {
+    float a[4][KR][CR_LD], b[4][KR][CR_LD];
+    uint32_t w[4][KR][32];
+};
+__device__ __forceinline__ void compress_k_rows(const CompressJob& jb, int bid, void* lds) {
+    KRowsLds& L = *static_cast<KRowsLds*>(lds);
+    auto& s_a = L.a;
+    auto& s_b = L.b;
+    auto& s_w = L.w;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int row0 = (bid * 4 + wave) * KR;
     const float f_s = 0.0625f;

@@ -115,6 +115,9 @@ struct CompressJob {
 // The K and V jobs of one compression event in one launch.
 hipError_t launch_compress_pair(const CompressJob& k, const CompressJob& v, hipStream_t st);
 hipError_t launch_compress(const CompressJob& job, int is_v, hipStream_t st);
+// Whether a launch over n rows uses the several-rows-a-wavefront form.
+bool compress_v_many(int n);
+bool compress_k_many(int n);
 hipError_t launch_attn_parts(const AttnArgs& a, int n_rep, dim3 grid, hipStream_t st);
 // waves: wavefronts per block, 1 or 4.
 hipError_t launch_window_parts(const WinArgs& a, int n_rep, int h_kv, int waves, hipStream_t st);
@@ -191,67 +194,91 @@ struct DecompArgs {
     int h_kv, tok0, n_tok, start_pos, key0, ld_vt;
     float a_k, a_v, rope_base;
 };
-// Ring slots (win_start + t) % ring_cap, t < n -> the same key layout at key0 + t.
+// n raw tokens (rows token * h_kv + head of k / v) -> the same key layout at
+// key0 + t (key0 a multiple of 32; V^T columns up to the next multiple of 32
+// are written too).
 struct GatherArgs {
-    const __half* ring_k;
-    const __half* ring_v;
+    RowSrc k, v;
     __half* out_k;
     __half* out_vt;
-    int h_kv, win_start, n, ring_cap, key0, ld_vt;
-    // Chunk mode (src_k != null): token t comes from src_k / src_v / src_u
-    // rows [t][h_kv][256] instead of the ring, and is also written to ring
-    // slot (win_start + t) % ring_cap of wr_k / wr_v / wr_u (wr_u optional).
+    int h_kv, n, key0, ld_vt;
+};
+// n tokens of src_k / src_v / src_u [t][h_kv][256] -> ring slots
+// (slot0 + t) % ring_cap (n <= ring_cap).
+struct RingArgs {
     const __half* src_k;
     const __half* src_v;
     const __half* src_u;
-    __half* wr_k;
-    __half* wr_v;
-    __half* wr_u;
-    // Second job (grid z = 1, chunk mode only): side_n tokens whose first
-    // side_from_src come from ring slots (side_start + t) % ring_cap and the
-    // rest from src rows t - side_from_src, written to keys side_key0 + t.
-    int side_n, side_start, side_from_src, side_key0;
+    __half* ring_k;
+    __half* ring_v;
+    __half* ring_u;
+    int h_kv, n, slot0, ring_cap;
 };
-// n_q queries (q_gate rows [n_q][H_q][512]) over dense keys [0, n_k); query j
-// sees keys [0, min(n_k, vis0 + j)).  Partial triple of (query j, head hq,
-// split s) at part[((j * H_q + hq) * n_split + s) * 258].
+// n_q queries (q_gate rows [n_q][H_q][512]) over two runs of dense keys:
+// decoded tokens at key indices [0, ..) and raw tokens at raw0 + r, r < n_raw
+// (raw0 a multiple of 32).  Query j has seen vis = min(n_raw, vis0 + j) raw
+// tokens; of these the first bound(vis), a multiple of 128, have been
+// compressed by then, so it attends to decoded keys [0, dec0 + bound(vis)) and
+// raw keys [bound(vis), vis).  bound follows the ring: none below 256, then
+// 128 more every 128 tokens, at most ev_cap (dec0 and ev_cap multiples of
+// 128; ev_cap = 0: every key is raw).
+// Rows of one KV head (query j, head r % n_rep) are cut into blocks, a block's
+// 32-key tiles into ceil(tiles / unit) splits (at most n_split).  Blocks of one
+// split write out directly; split s of the others leaves the triple of (query
+// j, head hq) at part[((j * H_q + hq) * n_split + s) * 258].
 struct PrefillArgs {
     const __half* q;
     const __half* k;
     const __half* vt;
     float* part;
-    int ld_vt, n_k, n_q, vis0, h_kv, n_rep, n_split, keys_per_split;
-    float sc;
-    // Keys are indices [0, n_tot), n_tot >= n_k.  Queries j < q_b (the run
-    // before a compression event) lose [hole_lo, hole_hi) and see key
-    // ex_lo + i for position hole_lo + i (when that position is below their
-    // causal limit) instead: the raw copies of the compressed chunk, placed
-    // past n_k, while the main key space holds its decoded rows for the
-    // queries after the event.  q_b = 0: no such run.
-    int n_tot, q_b, hole_lo, hole_hi, ex_lo, ex_hi;
+    __half* out;  // NULL: every block leaves triples
+    int ld_vt, n_q, h_kv, n_rep, n_split, unit;
+    int vis0, n_raw, raw0, dec0, ev_cap;
+    float sc, eps;
+    __host__ __device__ int bound(int vis) const {
+        if (ev_cap <= 0 || vis < 256) return 0;
+        const int b = ((vis - 256) / 128 + 1) * 128;
+        return b < ev_cap ? b : ev_cap;
+    }
+    __host__ __device__ int vis_of(int j) const { return vis0 + j < n_raw ? vis0 + j : n_raw; }
+    // Tiles of a block of rows [row_first, row_last]: tile i is decoded tile i
+    // for i < nd, then raw tile u0 + i - nd.
+    __host__ __device__ int block_tiles(int row_first, int row_last, int* nd, int* u0) const {
+        const int vf = vis_of(row_first / n_rep), vl = vis_of(row_last / n_rep);
+        *nd = (dec0 + bound(vl)) / 32;
+        *u0 = bound(vf) / 32;
+        return *nd + (vl + 31) / 32 - *u0;
+    }
+    __host__ __device__ int block_splits(int tiles) const {
+        const int s = (tiles + unit - 1) / unit;
+        return s < n_split ? s : n_split;
+    }
 };
 hipError_t launch_decompress(const DecompArgs& a, hipStream_t st);
 hipError_t launch_ring_gather(const GatherArgs& a, hipStream_t st);
 // A decode and a gather whose outputs are disjoint, in one launch.
 hipError_t launch_decompress_gather(const DecompArgs& d, const GatherArgs& g, hipStream_t st);
 // A compression event (k, v: rows (token, KV head) of the chunk), the decode
-// of those rows (d: tok0 = key0, n_tok tokens, start_pos 0) and an optional
-// independent gather (chunk append or raw copy) in one launch.
+// of those rows (d: tok0 = key0, n_tok tokens, start_pos 0) and a gather
+// (disjoint from the decoded rows) in one launch.
 hipError_t launch_compress_decode(const CompressJob& k, const CompressJob& v, const DecompArgs& d,
-                                  const GatherArgs* g, hipStream_t st);
-int prefill_splits(int n_q, int n_rep, int h_kv, int n_k, int* keys_per_split);
+                                  const GatherArgs& g, hipStream_t st);
+// Several events' rows and a gather in one launch (no decode).
+hipError_t launch_compress_gather(const CompressJob& k, const CompressJob& v, const GatherArgs& g,
+                                  hipStream_t st);
+// Rows of one KV head a block of the prefill attention takes.
+int prefill_block_rows(int n_rows);
+// Fills a.n_split and a.unit for the current device.
+void prefill_plan(PrefillArgs& a);
 hipError_t launch_prefill_attn(const PrefillArgs& a, hipStream_t st);
-// Prefill attention plus merge and gate through the shared workspace; the
-// hole / extra ranges as in PrefillArgs (all zero: plain causal prefill);
-// merge = false: the attention launch alone (partials left in the workspace).
-int prefill_attn_run(const __half* q_gate, const __half* k, const __half* vt, int ld_vt, int n_k,
-                     int n_q, int vis0, int H_q, int H_kv, float scale, __half* out,
-                     hipStream_t stream, int q_b, int hole_lo, int hole_hi, int ex_lo, int ex_hi,
-                     bool merge = true);
-// Merge of n_split partial triples per row, / (den + eps), sigmoid gate from
-// q_gate row r (f16 [r][512], gate at 256..511): out f16 [r][256].
-hipError_t launch_prefill_merge(const float* part, const __half* q_gate, __half* out, int n_rows,
-                                int n_split, float eps, hipStream_t st);
+// Prefill attention plus merge and gate through the shared workspace: q, k, vt,
+// the shapes, the key runs and out set in a; with ring, its copy runs behind
+// the attention.  merge = false: the attention launch alone, every block's
+// triples left in the workspace.
+int prefill_attn_run(PrefillArgs a, const RingArgs* ring, hipStream_t stream, bool merge = true);
+// Merge of the split blocks' triples, / (den + eps), sigmoid gate from q_gate
+// row r (gate at 256..511), and the ring copy (ring may be NULL), in one launch.
+hipError_t launch_prefill_finish(const PrefillArgs& a, const RingArgs* ring, hipStream_t st);
 
 // Per-device launch set-up, cached per device index under a lock (a process
 // may drive several GPUs from several threads): the CU count of the current

@@ -19,14 +19,17 @@
 namespace khq {
 
 __global__ __launch_bounds__(256) void compress_kernel(CompressJob j, int is_v) {
+    __shared__ CompressLds lds;
     compress_block(j.x, j.d_vec, j.rotor, j.cents, j.vq, j.out_mask, j.out_norms, j.out_rn,
-                   j.out_pay, j.out_sm, j.n, j.ts, j.alpha, is_v, (int)blockIdx.x);
+                   j.out_pay, j.out_sm, j.n, j.ts, j.alpha, is_v, (int)blockIdx.x, &lds);
 }
 __global__ __launch_bounds__(256) void compress_v_rows_kernel(CompressJob j) {
-    compress_v_rows(j, (int)blockIdx.x);
+    __shared__ VRowsLds lds;
+    compress_v_rows(j, (int)blockIdx.x, &lds);
 }
 __global__ __launch_bounds__(256) void compress_k_rows_kernel(CompressJob j) {
-    compress_k_rows(j, (int)blockIdx.x);
+    __shared__ KRowsLds lds;
+    compress_k_rows(j, (int)blockIdx.x, &lds);
 }
 
 // K and V of one compression event in one launch: blocks [0, nb_k) run the K
@@ -34,12 +37,13 @@ __global__ __launch_bounds__(256) void compress_k_rows_kernel(CompressJob j) {
 // sets, is not written).
 __global__ __launch_bounds__(256) void compress_pair_kernel(CompressJob k, CompressJob v,
                                                             int nb_k) {
+    __shared__ CompressLds lds;
     if ((int)blockIdx.x < nb_k)
         compress_block(k.x, k.d_vec, k.rotor, k.cents, k.vq, k.out_mask, k.out_norms, k.out_rn,
-                       k.out_pay, nullptr, k.n, k.ts, k.alpha, 0, (int)blockIdx.x);
+                       k.out_pay, nullptr, k.n, k.ts, k.alpha, 0, (int)blockIdx.x, &lds);
     else
         compress_block(v.x, v.d_vec, v.rotor, v.cents, v.vq, v.out_mask, v.out_norms, v.out_rn,
-                       v.out_pay, v.out_sm, v.n, v.ts, v.alpha, 1, (int)blockIdx.x - nb_k);
+                       v.out_pay, v.out_sm, v.n, v.ts, v.alpha, 1, (int)blockIdx.x - nb_k, &lds);
 }
 
 // ------------------------------------------------- compressed-region parts
@@ -726,13 +730,14 @@ hipError_t launch_window_parts(const WinArgs& a, int n_rep, int h_kv, int waves,
     return hipGetLastError();
 }
 
+// Where several rows a wavefront overtake one (their blocks take 14 us however
+// few there are): V between 512 rows (12.1 us one row a block, 14.6 eight) and
+// 1024 (19.1, 14.8); K between 4096 (12.6, 14.2) and 8000 (20.6, 15.7).
+bool compress_v_many(int n) { return n >= 3 * device_cu_count(); }
+bool compress_k_many(int n) { return n >= 20 * device_cu_count(); }
+
 hipError_t launch_compress(const CompressJob& j, int is_v, hipStream_t st) {
-    // Where several rows a wavefront overtake one (their blocks take 14 us
-    // however few there are): V between 512 rows (12.1 us one row a block, 14.6
-    // eight) and 1024 (19.1, 14.8); K between 4096 (12.6, 14.2) and 8000
-    // (20.6, 15.7).
-    const int n_cu = device_cu_count();
-    if (j.n >= (is_v ? 3 : 20) * n_cu) {
+    if (is_v ? compress_v_many(j.n) : compress_k_many(j.n)) {
         if (is_v)
             hipLaunchKernelGGL(compress_v_rows_kernel, dim3((j.n + VR - 1) / VR), dim3(256), 0, st, j);
         else

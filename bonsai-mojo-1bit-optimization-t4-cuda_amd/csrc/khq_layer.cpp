@@ -25,6 +25,9 @@ constexpr int kWatermark = 256;  // :37
 constexpr int kChunk = 128;      // :38
 constexpr int kMaxSplits = 64;   // workspace bound of the reference-sequence path
 constexpr int kD = 256;
+// New tokens one prefill pass takes at most: 8,192 fill the chip 6 times over
+// (128 query rows a block) and their raw keys cost 34 MB a layer.
+constexpr int kPrefillMax = 8192;
 
 }  // namespace
 
@@ -40,11 +43,11 @@ struct khq_layer {
     __half *knorm = nullptr, *krn = nullptr, *vnorm = nullptr, *vrn = nullptr;
     float *ac = nullptr, *aw = nullptr, *ap = nullptr;
     int boundary = 0, write_pos = 0, n_events = 0;
-    // chunked prefill: dense fp16 keys [key][H_kv][256] and V^T [H_kv][256][ld]
-    // (key = token position), compressed tokens [0, dec_hi) already decoded,
-    // raw tokens [raw_lo, raw_hi) already copied (empty when raw_lo >= raw_hi)
+    // chunked prefill: dense fp16 keys [key][H_kv][256] and V^T [H_kv][256][ld];
+    // compressed token t at key t (tokens [0, dec_hi) decoded so far), then
+    // from key raw0 on the raw tokens of one call, at most raw_cap
     __half *dk = nullptr, *dvt = nullptr;
-    int d_keys = 0, d_ld = 0, dec_hi = 0, raw_lo = 0, raw_hi = 0;
+    int d_ld = 0, dec_hi = 0, raw0 = 0, raw_cap = 0;
     // calibration dumps of khq_layer_attention_step (not owned)
     khq_dump* dump = nullptr;
     int dump_layer = 0;
@@ -68,18 +71,23 @@ bool alloc_zero(T** p, size_t bytes) {
     return hipMemset(*p, 0, bytes) == hipSuccess;
 }
 
-// Compression event: ring slots [boundary % 256, + 128) -> payload rows of
-// tokens [boundary, boundary + 128) (ref runtime.mojo:494-552).
-void compress_jobs(const khq_layer* L, khq::CompressJob* kj, khq::CompressJob* vj) {
-    const int kv = L->H_kv * kD;
-    const int s0 = L->boundary % kRing;
+// Rows of tokens [boundary, ..) on: n_ring tokens in the ring from slot
+// boundary % 256 on, the rest in src.
+khq::RowSrc row_src(const khq_layer* L, const __half* ring, int n_ring, const __half* src) {
+    return khq::RowSrc{src, ring, n_ring * L->H_kv, L->boundary % kRing * L->H_kv,
+                       kRing * L->H_kv};
+}
+
+// Compression of n_tok tokens from boundary on (ref runtime.mojo:494-552).
+void compress_jobs(const khq_layer* L, int n_tok, const khq::RowSrc& k, const khq::RowSrc& v,
+                   khq::CompressJob* kj, khq::CompressJob* vj) {
     const size_t r0 = (size_t)L->boundary * L->H_kv;
-    const int n = kChunk * L->H_kv;
+    const int n = n_tok * L->H_kv;
     auto h = [](const void* p) { return static_cast<const __half*>(p); };
-    *kj = khq::CompressJob{khq::RowSrc{L->ring_u + (size_t)s0 * kv, nullptr, 0, 0, 1}, h(L->d_k), h(L->rotor_k), h(L->cents_k),
+    *kj = khq::CompressJob{k, h(L->d_k), h(L->rotor_k), h(L->cents_k),
                            h(L->cents_k), L->kmask + r0 * 16, L->knorm + r0, L->krn + r0,
                            L->kpay + r0 * 40, nullptr, n, L->ts_k, L->alpha_k};
-    *vj = khq::CompressJob{khq::RowSrc{L->ring_v + (size_t)s0 * kv, nullptr, 0, 0, 1}, h(L->d_v), h(L->rotor_v), h(L->cents_v),
+    *vj = khq::CompressJob{v, h(L->d_v), h(L->rotor_v), h(L->cents_v),
                            h(L->vq), L->kmask + r0 * 16, L->vnorm + r0, L->vrn + r0,
                            L->vpay + r0 * 104, L->vsm + r0 * 4, n, L->ts_v, L->alpha_v};
 }
@@ -87,7 +95,8 @@ void compress_jobs(const khq_layer* L, khq::CompressJob* kj, khq::CompressJob* v
 int compress_event(khq_layer* L, hipStream_t stream) {
     // K and V rows in one launch (the two jobs write disjoint outputs)
     khq::CompressJob kj, vj;
-    compress_jobs(L, &kj, &vj);
+    compress_jobs(L, kChunk, row_src(L, L->ring_u, kRing, nullptr),
+                  row_src(L, L->ring_v, kRing, nullptr), &kj, &vj);
     const hipError_t e = khq::launch_compress_pair(kj, vj, stream);
     if (e != hipSuccess) return (int)e;
     L->boundary += kChunk;
@@ -127,25 +136,6 @@ void decomp_args(const khq_layer* L, int d0, int nd, khq::DecompArgs* a) {
     a->a_k = L->alpha_k;
     a->a_v = L->alpha_v;
     a->rope_base = L->rope_base;
-}
-
-// Compression event whose rows are also decoded into the dense key space
-// (which holds every earlier row: dec_hi = boundary), with an optional
-// independent gather (the chunk append) in the same launch.
-int compress_event_decoded(khq_layer* L, const khq::GatherArgs* g, hipStream_t stream) {
-    const int c_a = L->boundary;
-    khq::CompressJob kj, vj;
-    compress_jobs(L, &kj, &vj);
-    khq::DecompArgs da{};
-    decomp_args(L, c_a, kChunk, &da);
-    const hipError_t e = khq::launch_compress_decode(kj, vj, da, g, stream);
-    if (e != hipSuccess) return (int)e;
-    L->boundary += kChunk;
-    L->n_events += 1;
-    L->dec_hi = c_a + kChunk;
-    // V^T columns up to the decode's last 16-column block are rewritten
-    L->raw_lo = std::max(L->raw_lo, c_a + (kChunk + 15) / 16 * 16);
-    return 0;
 }
 
 int split_count(int c_len, int splits) {  // ref runtime.mojo:211-222
@@ -216,7 +206,6 @@ int khq_layer_reset(khq_layer* L) {
     L->write_pos = 0;
     L->n_events = 0;
     L->dec_hi = 0;
-    L->raw_lo = L->raw_hi = 0;
     return 0;
 }
 
@@ -311,7 +300,6 @@ int khq_layer_attention_step(khq_layer* L, void* q_gate, void* k, const void* v,
 static int step_after_ring_write(khq_layer* L, const void* q_gate, void* out, float scale,
                                  hipStream_t stream) {
     int rc = 0;
-    L->raw_lo = L->raw_hi = 0;  // the dense key space does not get this token
     L->write_pos += 1;
     if (event_due(L, L->write_pos)) {
         rc = compress_event(L, stream);
@@ -358,28 +346,14 @@ int khq_layer_prefill(khq_layer* L, const void* q_gate, const void* k_roped, con
                       const void* k_unroped, void* out, int n, float scale, hipStream_t stream) {
     if (!L || !q_gate || !k_roped || !v || !k_unroped || !out || n <= 0) return -100;
     const int kv = L->H_kv * kD;
-    if (!L->dk) {  // dense key space for up to cap + 256 positions
-        // positions up to cap + ring, then the raw copy of one compressed
-        // chunk (the extra keys of a combined launch) past them
-        L->d_keys = L->cap + kRing + kChunk + 64;
-        L->d_ld = (L->d_keys + 63) / 64 * 64;
-        const size_t kb = (size_t)L->d_keys * kv * sizeof(__half);
-        const size_t vb = (size_t)L->H_kv * kD * L->d_ld * sizeof(__half);
+    if (!L->dk) {  // dense key space: cap decoded tokens, then one call's raw tokens
+        L->raw0 = (L->cap + 63) / 64 * 64;
+        L->raw_cap = kRing + std::min(kPrefillMax, (L->cap + kRing + 63) / 64 * 64);
+        L->d_ld = L->raw0 + L->raw_cap;
+        const size_t kb = (size_t)L->d_ld * kv * sizeof(__half);
         if (hipMalloc(reinterpret_cast<void**>(&L->dk), kb) != hipSuccess ||
-            hipMalloc(reinterpret_cast<void**>(&L->dvt), vb) != hipSuccess) {
+            hipMalloc(reinterpret_cast<void**>(&L->dvt), kb) != hipSuccess) {
             if (L->dk) (void)hipFree(L->dk);
-            L->dk = nullptr;
-            L->dvt = nullptr;
-            return -100;
-        }
-        // finite contents everywhere: padding keys of a launch get P = 0
-        if (hipMemsetAsync(L->dk, 0, kb, stream) != hipSuccess ||
-            hipMemsetAsync(L->dvt, 0, vb, stream) != hipSuccess) {
-            // leave no half-initialised dense key space behind: the next
-            // call allocates and clears it again
-            (void)hipStreamSynchronize(stream);
-            (void)hipFree(L->dk);
-            (void)hipFree(L->dvt);
             L->dk = nullptr;
             L->dvt = nullptr;
             return -100;
@@ -393,139 +367,80 @@ int khq_layer_prefill(khq_layer* L, const void* q_gate, const void* k_roped, con
     __half* o = static_cast<__half*>(out);
     int done = 0;
     while (done < n) {
-        // Sub-chunk whose ring writes overwrite no slot that any of its
-        // queries or compression events still reads.
-        const int m = std::min(n - done, kRing - (L->write_pos - L->boundary));
+        // One pass takes m tokens, whatever events fall among them.  Raw index
+        // r stands for token boundary + r: nw of the window, then the new ones.
+        // Events compress raw tokens [0, n_ev): as the steps would, 128 more
+        // whenever 256 raw tokens are seen, while the capacity lasts; past
+        // that the ring holds 256 more.
+        const int b0 = L->boundary, w0 = L->write_pos, nw = w0 - b0;
+        const int ev_cap = (L->cap - b0) / kChunk * kChunk;
+        const int m = std::min({n - done, ev_cap + kRing - nw, L->raw_cap - nw});
         if (m <= 0) return -102;
-        const int w0 = L->write_pos;
-        // An event due at the sub-chunk's last query and at none before it
-        // (the usual case: the sub-chunk fills the ring to the watermark):
-        // the event runs first and one attention launch serves every query;
-        // the earlier queries read the chunk's raw rows from a copy past the
-        // sub-chunk's keys instead of its decoded rows.
-        const bool combine = m >= 2 && event_due(L, w0 + m) && !event_due(L, w0 + m - 1);
-        const int c_a = L->boundary;
-        const int side0 = (w0 + m + 15) / 16 * 16;
-        // the sub-chunk's tokens go to their ring slots and to the dense key
-        // space in one launch (with the raw copy as a second job)
-        khq::GatherArgs cw{};
-        cw.out_k = L->dk;
-        cw.out_vt = L->dvt;
-        cw.h_kv = L->H_kv;
-        cw.win_start = w0 % kRing;
-        cw.n = m;
-        cw.ring_cap = kRing;
-        cw.key0 = w0;
-        cw.ld_vt = L->d_ld;
-        cw.src_k = kr + (size_t)done * kv;
-        cw.src_v = vv + (size_t)done * kv;
-        cw.src_u = ku + (size_t)done * kv;
-        cw.wr_k = L->ring_k;
-        cw.wr_v = L->ring_v;
-        cw.wr_u = L->ring_u;
-        if (combine) {
-            cw.side_n = kChunk;
-            cw.side_start = c_a % kRing;
-            cw.side_from_src = std::min(w0 - c_a, kChunk);
-            cw.side_key0 = side0;
-        }
-        // With the compressed chunk wholly before the sub-chunk (the steady
-        // state), the event reads no ring slot this launch writes: the append
-        // then rides in the decode launch below instead of a launch of its own.
-        const bool defer = combine && w0 >= c_a + kChunk && L->dec_hi < c_a + kChunk;
-        if (!defer) {
-            const hipError_t e = khq::launch_ring_gather(cw, stream);
-            if (e != hipSuccess) return (int)e;
-        }
-        if (L->raw_lo < L->raw_hi && L->raw_hi == w0)
-            L->raw_hi = w0 + m;
-        else {
-            L->raw_lo = w0;
-            L->raw_hi = w0 + m;
-        }
-        // decoded rows up to c_len, raw rows [c_len, n_k) in the dense key space
-        auto prepare = [&](int c_len, int n_k, const khq::GatherArgs* with) -> int {
-            if (L->dec_hi < c_len) {
-                const int d0 = L->dec_hi, nd = c_len - d0;
-                int rc;
-                if (with) {
-                    khq::DecompArgs da{};
-                    decomp_args(L, d0, nd, &da);
-                    const hipError_t de = khq::launch_decompress_gather(da, *with, stream);
-                    rc = de == hipSuccess ? 0 : (int)de;
-                } else {
-                    rc = khq_decompress_fp16(
-                        L->kpay, L->vpay, L->vsm, L->kmask, L->knorm, L->krn, L->vnorm, L->vrn,
-                        L->cents_k, L->cents_v, L->vq, L->rotor_k, L->rotor_v, L->d_k, L->d_v,
-                        L->H_kv, d0, nd, 0, L->alpha_k, L->alpha_v, L->rope_base, L->dk, d0,
-                        L->dvt, L->d_ld, stream);
-                }
-                if (rc) return rc;
-                L->dec_hi = c_len;
-                // V^T columns up to the decode's last 16-column block are rewritten
-                L->raw_lo = std::max(L->raw_lo, d0 + (nd + 15) / 16 * 16);
+        const __half* src_k = kr + (size_t)done * kv;
+        const __half* src_v = vv + (size_t)done * kv;
+        const __half* src_u = ku + (size_t)done * kv;
+        khq::PrefillArgs a{};
+        a.q = qg + (size_t)done * L->H_q * 2 * kD;
+        a.k = L->dk;
+        a.vt = L->dvt;
+        a.out = o + (size_t)done * L->H_q * kD;
+        a.ld_vt = L->d_ld;
+        a.n_q = m;
+        a.h_kv = L->H_kv;
+        a.n_rep = L->H_q / L->H_kv;
+        a.vis0 = nw + 1;
+        a.n_raw = nw + m;
+        a.raw0 = L->raw0;
+        a.dec0 = b0;
+        a.ev_cap = ev_cap;
+        a.sc = scale;
+        const int n_ev = a.bound(a.n_raw);
+        // ---- the raw run (window from the ring, then the new tokens), the
+        // events' rows and their decode
+        khq::GatherArgs g{};
+        g.k = row_src(L, L->ring_k, nw, src_k);
+        g.v = row_src(L, L->ring_v, nw, src_v);
+        g.out_k = L->dk;
+        g.out_vt = L->dvt;
+        g.h_kv = L->H_kv;
+        g.n = nw + m;
+        g.key0 = L->raw0;
+        g.ld_vt = L->d_ld;
+        khq::DecompArgs d{};
+        decomp_args(L, L->dec_hi, b0 + n_ev - L->dec_hi, &d);
+        hipError_t e;
+        if (n_ev == 0) {
+            e = khq::launch_decompress_gather(d, g, stream);
+        } else {
+            khq::CompressJob kj, vj;
+            compress_jobs(L, n_ev, row_src(L, L->ring_u, nw, src_u), g.v, &kj, &vj);
+            if (L->dec_hi == b0 && !khq::compress_v_many(vj.n)) {
+                // one event, every earlier row decoded: it decodes its own
+                e = khq::launch_compress_decode(kj, vj, d, g, stream);
+            } else {
+                e = khq::launch_compress_gather(kj, vj, g, stream);
+                if (e == hipSuccess) e = khq::launch_decompress(d, stream);
             }
-            // raw tokens [c_len, n_k): copied from the ring unless already
-            // there (with every raw token after them, so the copy's padded
-            // last block clobbers nothing still needed)
-            if (!(L->raw_lo <= c_len && L->raw_hi >= n_k && L->raw_lo < L->raw_hi)) {
-                const int g_hi = std::max(n_k, L->raw_lo < L->raw_hi && L->raw_lo <= n_k ? L->raw_hi : n_k);
-                khq::GatherArgs g{};
-                g.ring_k = L->ring_k;
-                g.ring_v = L->ring_v;
-                g.out_k = L->dk;
-                g.out_vt = L->dvt;
-                g.h_kv = L->H_kv;
-                g.win_start = c_len % kRing;
-                g.n = g_hi - c_len;
-                g.ring_cap = kRing;
-                g.key0 = c_len;
-                g.ld_vt = L->d_ld;
-                const hipError_t ge = khq::launch_ring_gather(g, stream);
-                if (ge != hipSuccess) return (int)ge;
-                L->raw_lo = c_len;
-                L->raw_hi = g_hi;
-            }
-            return 0;
-        };
-        if (combine) {
-            // steady state (every earlier row decoded): the event decodes its
-            // own rows, with the deferred append in the same launch
-            const bool fused = L->dec_hi == c_a;
-            int rc = fused ? compress_event_decoded(L, defer ? &cw : nullptr, stream)
-                           : compress_event(L, stream);
-            if (rc) return rc;
-            const int c_b = L->boundary;  // c_a + kChunk
-            const int n_k = w0 + m;
-            rc = prepare(c_b, n_k, defer && !fused ? &cw : nullptr);
-            if (rc) return rc;
-            rc = khq::prefill_attn_run(qg + (size_t)done * L->H_q * 2 * kD, L->dk, L->dvt,
-                                       L->d_ld, n_k, m, w0 + 1, L->H_q, L->H_kv, scale,
-                                       o + (size_t)done * L->H_q * kD, stream, m - 1, c_a, c_b,
-                                       side0, side0 + (c_b - c_a));
-            if (rc) return rc;
         }
-        int j = combine ? m : 0;
-        while (j < m) {
-            // query j appends position w0 + j; an event fires before its attention
-            if (event_due(L, w0 + j + 1)) {
-                const int rc = compress_event(L, stream);
-                if (rc) return rc;
-            }
-            int je = j + 1;
-            while (je < m && !event_due(L, w0 + je + 1)) je++;
-            // queries j .. je - 1 share c_len = boundary
-            const int c_len = L->boundary;
-            const int n_k = w0 + je;
-            if (n_k - c_len > kRing) return -102;
-            int rc = prepare(c_len, n_k, nullptr);
-            if (rc) return rc;
-            rc = khq_prefill_attn_fp16(qg + (size_t)(done + j) * L->H_q * 2 * kD, L->dk, L->dvt,
-                                       L->d_ld, n_k, je - j, w0 + j + 1, L->H_q, L->H_kv, scale,
-                                       o + (size_t)(done + j) * L->H_q * kD, stream);
-            if (rc) return rc;
-            j = je;
-        }
+        if (e != hipSuccess) return (int)e;
+        // ---- attention, then the ring takes the new tokens (all its readers
+        // are behind by then)
+        khq::RingArgs r{};
+        r.n = std::min(m, kRing);
+        const size_t skip = (size_t)(m - r.n) * kv;
+        r.src_k = src_k + skip;
+        r.src_v = src_v + skip;
+        r.src_u = src_u + skip;
+        r.ring_k = L->ring_k;
+        r.ring_v = L->ring_v;
+        r.ring_u = L->ring_u;
+        r.h_kv = L->H_kv;
+        r.slot0 = (w0 + m - r.n) % kRing;
+        r.ring_cap = kRing;
+        const int rc = khq::prefill_attn_run(a, &r, stream);
+        if (rc) return rc;
+        L->boundary = L->dec_hi = b0 + n_ev;
+        L->n_events += n_ev / kChunk;
         L->write_pos = w0 + m;
         done += m;
     }

@@ -9,20 +9,26 @@
 //                       qmv_sm75_kernel.cu:1608-1699 for K and :1739-1762,
 //                       1776-1826 for V, applied per token instead of being
 //                       folded into the running sums);
-//   ring_gather_kernel  raw ring slots -> the same K rows / V^T columns;
+//   ring_gather_kernel  raw tokens (ring slots, then the caller's) -> K rows
+//                       and V^T columns of the raw run;
 //   compress_decode_kernel  a compression event that decodes the rows it
-//                       packs into the key space (and appends new tokens);
+//                       packs into the key space (and gathers raw tokens);
+//   compress_gather_kernel  many events' rows (and the gather);
 //   prefill_attn_kernel, prefill_attn_rs_kernel  S^T = K Q^T and
 //                       O^T = V^T P^T on MFMA (fp16 in, fp32 accumulate),
-//                       online softmax, one split of the keys per block;
-//   prefill_merge_kernel  the splits' partial triples merged and gated.
-// Query j of a launch sees keys [0, vis0 + j): the sequential step semantics
-// (its own position included) when keys are positions.
+//                       online softmax, one split of a block's keys per block;
+//   prefill_finish_kernel  the splits' partial triples merged and gated, the
+//                       new tokens copied to their ring slots.
+// One launch serves queries on both sides of any number of compression events:
+// a block walks the decoded tiles its last query sees, then the raw tiles from
+// its first query's compressed bound on, and each row masks what it does not
+// see (PrefillArgs).
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
 #include <stdint.h>
 
 #include <algorithm>
+#include <cmath>
 
 #include "khq_internal.h"
 #include "khq_mfma_util.h"
@@ -34,55 +40,49 @@ namespace pf {
 
 using namespace mu;
 
-constexpr int TOK_BLK = 4;    // tokens per decompress / gather block: one per wavefront
-                              // (small blocks spread a short chunk over many CUs)
-constexpr int BLK_THR = 64 * TOK_BLK;
+constexpr int BLK_THR = 256;  // decompress / gather blocks: 4 wavefronts of TB / 4 tokens
 constexpr int VT_PAD = 8;     // halves of padding per LDS V^T row
+// Tokens per block TB: 4 spread a chunk over many CUs; 16 write V^T in 32-byte
+// runs and set a lane's constants up once for four tokens, but take 15 us
+// however few there are.
+constexpr int TB_LONG = 16;
 
-__device__ __forceinline__ uint32_t rd32(const uint8_t* p) {
-    return (uint32_t)p[0] | ((uint32_t)p[1] << 8) | ((uint32_t)p[2] << 16) | ((uint32_t)p[3] << 24);
-}
-
-// Writes the block's LDS V^T tile sv[256][TOK_BLK + VT_PAD] to vt columns
-// key0 .. key0 + TOK_BLK - 1 of KV head h (all TOK_BLK columns: the caller's
-// buffer is padded to a multiple of 64 keys), in 8-byte pieces (key0 is a
-// multiple of 4).
-__device__ __forceinline__ void store_vt(const _Float16 (*sv)[TOK_BLK + VT_PAD], __half* vt, int ld,
-                                         int h, int key0) {
-    for (int i = threadIdx.x; i < 256 * (TOK_BLK / 4); i += blockDim.x) {
-        const int d = i / (TOK_BLK / 4), part = i % (TOK_BLK / 4);
-        const uint2 v = *reinterpret_cast<const uint2*>(&sv[d][part * 4]);
-        *reinterpret_cast<uint2*>(vt + ((size_t)h * 256 + d) * ld + key0 + part * 4) = v;
-    }
-}
-
-// Writes columns key0 .. key0 + nc - 1 only (any alignment), 2 bytes each.
-__device__ __forceinline__ void store_vt_cols(const _Float16 (*sv)[TOK_BLK + VT_PAD], __half* vt,
-                                              int ld, int h, int key0, int nc) {
-    for (int i = threadIdx.x; i < 256 * TOK_BLK; i += blockDim.x) {
-        const int d = i / TOK_BLK, c = i % TOK_BLK;
-        if (c < nc)
-            reinterpret_cast<_Float16*>(vt)[((size_t)h * 256 + d) * ld + key0 + c] = sv[d][c];
+// Writes columns [0, nc) of the block's LDS V^T tile (nc <= TB a multiple of 4)
+// to vt columns key0 .. of KV head h, in pieces of 8 bytes (TB 4) or 16.
+template <int TB>
+__device__ __forceinline__ void store_vt(const _Float16 (*sv)[TB + VT_PAD], __half* vt, int ld,
+                                         int h, int key0, int nc) {
+    constexpr int W = TB < 8 ? 4 : 8;  // columns per piece
+    for (int i = threadIdx.x; i < 256 * (TB / W); i += BLK_THR) {
+        const int d = i / (TB / W), c = i % (TB / W) * W;
+        __half* dst = vt + ((size_t)h * 256 + d) * ld + key0 + c;
+        if (W == 8 && c + 8 <= nc)
+            *reinterpret_cast<uint4*>(dst) = *reinterpret_cast<const uint4*>(&sv[d][c]);
+        else if (c < nc)
+            *reinterpret_cast<uint2*>(dst) = *reinterpret_cast<const uint2*>(&sv[d][c]);
     }
 }
 
 // ------------------------------------------------------------- decompress
-// Block (16 tokens, KV head h), one wavefront per token (the decode of one
-// row is a chain of dependent loads: tokens in parallel hide it); lane p owns
-// patch p = dims 4 p .. 4 p + 3.
-__device__ __forceinline__ void decompress_block(const DecompArgs& a, int bx, int h) {
-    __shared__ __align__(16) _Float16 sv[256][TOK_BLK + VT_PAD];
+// Block (TB tokens, KV head h), a wavefront per TB / 4 tokens; lane p owns
+// patch p = dims 4 p .. 4 p + 3.  The decode of one row is a chain of dependent
+// loads: wavefronts in parallel hide it.
+template <int TB>
+using VtTile = _Float16[256][TB + VT_PAD];
+template <int TB>
+__device__ __forceinline__ void decompress_block(const DecompArgs& a, int bx, int h, void* lds) {
+    VtTile<TB>& sv = *static_cast<VtTile<TB>*>(lds);
     const int wv = threadIdx.x >> 6, p = threadIdx.x & 63;
-    const int t_blk = bx * TOK_BLK;
+    const int t_blk = bx * TB;
     dec::Consts cs;
     dec::load_consts(a, p, cs);
-    {
-        const int tl = wv;           // token within the block
+#pragma unroll 2
+    for (int tl = wv; tl < TB; tl += 4) {
         const int tok = t_blk + tl;
         if (tok >= a.n_tok) {        // uniform per wavefront
 #pragma unroll
             for (int c = 0; c < 4; c++) sv[4 * p + c][tl] = (_Float16)0.0f;
-            goto staged;
+            continue;
         }
         const size_t g = (size_t)(a.tok0 + tok) * a.h_kv + h;
         float y[4];
@@ -94,173 +94,179 @@ __device__ __forceinline__ void decompress_block(const DecompArgs& a, int bx, in
         // ---- V: patch fields, codebook, dim 3, inverse rotor, FWHT
         const uint8_t* vp = a.vpay + g * 104;
         const uint32_t grp = (uint32_t)p / 8, sub = (uint32_t)p % 8;
-        const uint64_t w0 = rd32(vp + (grp * 3 + 0) * 4), w1 = rd32(vp + (grp * 3 + 1) * 4),
-                       w2 = rd32(vp + (grp * 3 + 2) * 4);
+        const uint64_t w0 = dec::rd32(vp + (grp * 3 + 0) * 4), w1 = dec::rd32(vp + (grp * 3 + 1) * 4),
+                       w2 = dec::rd32(vp + (grp * 3 + 2) * 4);
         const uint64_t low64 = (w1 << 32) | w0, high64 = (w2 << 32) | w1;
         const uint32_t pvl = (sub < 4) ? (uint32_t)((low64 >> (sub * 12)) & 0xFFF)
                                        : (uint32_t)((high64 >> ((sub - 4) * 12 + 16)) & 0xFFF);
-        const uint32_t hb = (p < 32) ? ((rd32(vp + 96) >> p) & 1u) : ((rd32(vp + 100) >> (p - 32)) & 1u);
+        const uint32_t hb = (p < 32) ? ((dec::rd32(vp + 96) >> p) & 1u) : ((dec::rd32(vp + 100) >> (p - 32)) & 1u);
         dec::decode_v(a, cs, (pvl & 0x7Fu) | (hb << 7), pvl, __half2float(a.vnorm[g]),
-                      __half2float(a.vrn[g]), __uint_as_float(rd32(a.vsm + g * 4)), p, y);
+                      __half2float(a.vrn[g]), __uint_as_float(dec::rd32(a.vsm + g * 4)), p, y);
 #pragma unroll
         for (int c = 0; c < 4; c++) sv[4 * p + c][tl] = (_Float16)y[c];
     }
-staged:
     __syncthreads();
-    store_vt(sv, a.out_vt, a.ld_vt, h, a.key0 + t_blk);
+    store_vt<TB>(sv, a.out_vt, a.ld_vt, h, a.key0 + t_blk, min(TB, (a.n_tok - t_blk + 3) & ~3));
 }
 
-// ------------------------------------------------------------ ring gather
-// Block (16 keys, KV head h), one wavefront per key: K rows copied, V rows
-// transposed through LDS.  In chunk mode the keys come from the caller's new
-// tokens, which also go to their ring slots (one launch appends a chunk to
-// the ring and to the dense key space).
-__device__ __forceinline__ void gather_block(const GatherArgs& a, int bx, int h, int bz) {
-    __shared__ __align__(16) _Float16 sv[256][TOK_BLK + VT_PAD];
+// ------------------------------------------------------------- raw gather
+// Block (32 raw tokens, KV head h): K rows copied, V rows transposed through
+// LDS, every row of the block in flight at once.  Tokens past the last give
+// zero V^T columns.
+__device__ __forceinline__ void gather_block(const GatherArgs& a, int bx, int h, void* lds) {
+    VtTile<32>& sv = *static_cast<VtTile<32>*>(lds);
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int t_blk = bx * TOK_BLK;
-    // job 0: the gather / chunk write; job 1: the side copy (block-uniform)
-    const bool side = bz == 1;
-    const int n = side ? a.side_n : a.n;
-    const int key0 = side ? a.side_key0 : a.key0;
-    if (t_blk >= n) return;
-    {
-        const int tl = wv;
-        const int t = t_blk + tl;
-        if (t >= n) {
+    const int t_blk = bx * 32;
+    uint2 kw[8], vw[8];
 #pragma unroll
-            for (int c = 0; c < 4; c++) sv[4 * lane + c][tl] = (_Float16)0.0f;
-            goto staged;
-        }
-        uint2 kw, vw;
-        if (side) {
-            if (t >= a.side_from_src) {
-                const size_t cs = ((size_t)(t - a.side_from_src) * a.h_kv + h) * 256 + 4 * lane;
-                kw = *reinterpret_cast<const uint2*>(a.src_k + cs);
-                vw = *reinterpret_cast<const uint2*>(a.src_v + cs);
-            } else {
-                int slot = a.side_start + t;
-                slot = slot >= a.ring_cap ? slot - a.ring_cap : slot;
-                const size_t rs = ((size_t)slot * a.h_kv + h) * 256 + 4 * lane;
-                kw = *reinterpret_cast<const uint2*>(a.wr_k + rs);
-                vw = *reinterpret_cast<const uint2*>(a.wr_v + rs);
-            }
-        } else {
-            int slot = a.win_start + t;
-            slot = slot >= a.ring_cap ? slot - a.ring_cap : slot;
-            const size_t rs = ((size_t)slot * a.h_kv + h) * 256 + 4 * lane;
-            if (a.src_k) {
-                const size_t cs = ((size_t)t * a.h_kv + h) * 256 + 4 * lane;
-                kw = *reinterpret_cast<const uint2*>(a.src_k + cs);
-                vw = *reinterpret_cast<const uint2*>(a.src_v + cs);
-                *reinterpret_cast<uint2*>(a.wr_k + rs) = kw;
-                *reinterpret_cast<uint2*>(a.wr_v + rs) = vw;
-                if (a.wr_u) *reinterpret_cast<uint2*>(a.wr_u + rs) = *reinterpret_cast<const uint2*>(a.src_u + cs);
-            } else {
-                kw = *reinterpret_cast<const uint2*>(a.ring_k + rs);
-                vw = *reinterpret_cast<const uint2*>(a.ring_v + rs);
-            }
-        }
-        *reinterpret_cast<uint2*>(a.out_k + ((size_t)(key0 + t) * a.h_kv + h) * 256 + 4 * lane) = kw;
-        const h4 v = __builtin_bit_cast(h4, vw);
+    for (int i = 0; i < 8; i++) {
+        const int t = t_blk + wv + 4 * i;
+        const int r = min(t, a.n - 1) * a.h_kv + h;
+        kw[i] = *reinterpret_cast<const uint2*>(a.k.row(r) + 4 * lane);
+        vw[i] = *reinterpret_cast<const uint2*>(a.v.row(r) + 4 * lane);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const int tl = wv + 4 * i, t = t_blk + tl;
+        if (t < a.n)
+            *reinterpret_cast<uint2*>(a.out_k + ((size_t)(a.key0 + t) * a.h_kv + h) * 256 + 4 * lane) =
+                kw[i];
+        const h4 v = __builtin_bit_cast(h4, t < a.n ? vw[i] : uint2{0u, 0u});
 #pragma unroll
         for (int c = 0; c < 4; c++) sv[4 * lane + c][tl] = v[c];
     }
-staged:
     __syncthreads();
-    if (a.src_k)  // chunk mode: exactly the written columns (key0 is any position)
-        store_vt_cols(sv, a.out_vt, a.ld_vt, h, key0 + t_blk, min(TOK_BLK, n - t_blk));
-    else
-        store_vt(sv, a.out_vt, a.ld_vt, h, key0 + t_blk);
+    store_vt<32>(sv, a.out_vt, a.ld_vt, h, a.key0 + t_blk, 32);
 }
+// Flat block index of a gather: token block fastest, then the KV head.
+__device__ __forceinline__ void gather_flat(const GatherArgs& a, int b, void* lds) {
+    const int nx = (a.n + 31) / 32;
+    gather_block(a, b % nx, b / nx, lds);
+}
+// LDS of a launch whose blocks do one of several jobs: the largest job's.
+template <size_t... N>
+struct __align__(16) SharedLds {
+    static constexpr size_t bytes = std::max({N...});
+    unsigned char b[bytes];
+};
 
+template <int TB>
 __global__ __launch_bounds__(BLK_THR) void decompress_kernel(DecompArgs a) {
-    decompress_block(a, blockIdx.x, blockIdx.y);
+    __shared__ SharedLds<sizeof(VtTile<TB>)> lds;
+    decompress_block<TB>(a, blockIdx.x, blockIdx.y, &lds);
 }
 
 __global__ __launch_bounds__(BLK_THR) void ring_gather_kernel(GatherArgs a) {
-    gather_block(a, blockIdx.x, blockIdx.y, blockIdx.z);
+    __shared__ SharedLds<sizeof(VtTile<32>)> lds;
+    gather_flat(a, blockIdx.x, &lds);
 }
 
 // A decode and an independent gather (disjoint outputs, no data passed
-// between them) in one launch: blocks [0, nb_d) decode (x fastest, then the
-// KV head), the rest gather (x, then the KV head, then the job plane).
+// between them) in one launch: blocks [0, nx_d h_kv) decode (x fastest, then
+// the KV head), the rest gather.
+template <int TB>
 __global__ __launch_bounds__(BLK_THR) void decompress_gather_kernel(DecompArgs d, GatherArgs g,
-                                                                    int nx_d, int nx_g) {
-    const int nb_d = nx_d * d.h_kv;
-    int b = blockIdx.x;
-    if (b < nb_d) {
-        decompress_block(d, b % nx_d, b / nx_d);
-        return;
-    }
-    b -= nb_d;
-    const int per_plane = nx_g * g.h_kv;
-    const int bz = b / per_plane;
-    b -= bz * per_plane;
-    gather_block(g, b % nx_g, b / nx_g, bz);
+                                                                    int nx_d) {
+    __shared__ SharedLds<sizeof(VtTile<TB>), sizeof(VtTile<32>)> lds;
+    const int nb_d = nx_d * d.h_kv, b = blockIdx.x;
+    if (b < nb_d)
+        decompress_block<TB>(d, b % nx_d, b / nx_d, &lds);
+    else
+        gather_flat(g, b - nb_d, &lds);
 }
 
 // A compression event, the decode of its rows into the dense key space and
-// an independent gather (a chunk append or a raw copy, disjoint from the
-// rows compressed) in one launch: blocks [0, nb_k) compress and decode K rows
+// the raw gather in one launch: blocks [0, nb_k) compress and decode K rows
 // (four per block, the longest blocks, first), [nb_k, nb_k + n_v) V rows (one
-// per block), the rest gather (x, then the KV head, then the job plane;
-// nx_g = 0: no gather).
+// per block), the rest gather.
 __global__ __launch_bounds__(BLK_THR) void compress_decode_kernel(CompressJob k, CompressJob v,
                                                                   DecompArgs d, GatherArgs g,
-                                                                  int nb_k, int nx_g) {
+                                                                  int nb_k) {
+    __shared__ SharedLds<sizeof(CompressLds), sizeof(VtTile<32>)> lds;
     int b = blockIdx.x;
     if (b < nb_k) {
         compress_block<true>(k.x, k.d_vec, k.rotor, k.cents, k.vq, k.out_mask, k.out_norms,
-                             k.out_rn, k.out_pay, nullptr, k.n, k.ts, k.alpha, 0, b, &d);
+                             k.out_rn, k.out_pay, nullptr, k.n, k.ts, k.alpha, 0, b, &lds, &d);
         return;
     }
     b -= nb_k;
     if (b < v.n) {
         compress_block<true>(v.x, v.d_vec, v.rotor, v.cents, v.vq, v.out_mask, v.out_norms,
-                             v.out_rn, v.out_pay, v.out_sm, v.n, v.ts, v.alpha, 1, b, &d);
+                             v.out_rn, v.out_pay, v.out_sm, v.n, v.ts, v.alpha, 1, b, &lds, &d);
         return;
     }
-    b -= v.n;
-    const int per_plane = nx_g * g.h_kv;
-    const int bz = b / per_plane;
-    b -= bz * per_plane;
-    gather_block(g, b % nx_g, b / nx_g, bz);
+    gather_flat(g, b - v.n, &lds);
+}
+
+// The rows of several compression events and the raw gather in one launch:
+// K blocks (four rows each, or 4 KR with k_many), V blocks (VR rows), gather.
+__global__ __launch_bounds__(BLK_THR) void compress_gather_kernel(CompressJob k, CompressJob v,
+                                                                  GatherArgs g, int nb_k, int nb_v,
+                                                                  int k_many) {
+    __shared__ SharedLds<sizeof(CompressLds), sizeof(VRowsLds), sizeof(KRowsLds), sizeof(VtTile<32>)> lds;
+    int b = blockIdx.x;
+    if (b < nb_k) {
+        if (k_many)
+            compress_k_rows(k, b, &lds);
+        else
+            compress_block(k.x, k.d_vec, k.rotor, k.cents, k.vq, k.out_mask, k.out_norms, k.out_rn,
+                           k.out_pay, nullptr, k.n, k.ts, k.alpha, 0, b, &lds);
+        return;
+    }
+    b -= nb_k;
+    if (b < nb_v)
+        compress_v_rows(v, b, &lds);
+    else
+        gather_flat(g, b - nb_v, &lds);
 }
 
 // Visibility of the keys of one 32-key tile to one query row, as a bit mask
-// (bit i: key k0 + i): [0, vis) less the hole, plus the extra range (hole and
-// extra are empty for rows after a compression event).  Only vis and a lane
-// flag stay live; the hole and extra bounds are the launch's scalar arguments.
+// (bit i: key i of the tile): a decoded tile lies wholly below or wholly at or
+// past the row's compressed bound (both are multiples of 32), a raw tile wholly
+// before it or up to the row's causal end.  Only vis and the bound stay live.
 __device__ __forceinline__ uint32_t bits_below(int n) {  // bits [0, n) of 32
     return n >= 32 ? ~0u : (n <= 0 ? 0u : (1u << n) - 1u);
 }
 struct RowKeys {
-    const PrefillArgs& a;
-    int vis;
-    bool run_a;
-    __device__ __forceinline__ RowKeys(const PrefillArgs& a_, bool r_ok, int jq) : a(a_) {
-        // padding rows see every key: their scores are never written
-        vis = r_ok ? min(a.n_k, a.vis0 + jq) : a.n_tot;
-        run_a = r_ok && jq < a.q_b;
+    int vis, bnd, dec_end;
+    __device__ __forceinline__ RowKeys(const PrefillArgs& a, int jq)
+        : vis(a.vis_of(jq)), bnd(a.bound(a.vis_of(jq))), dec_end(0) {
+        dec_end = a.dec0 + bnd;
     }
-    __device__ __forceinline__ uint32_t tile(int k0) const {
+    // dec: decoded tile; base: its first token (decoded) or raw index
+    __device__ __forceinline__ uint32_t tile(bool dec, int base) const {
         // selects, no branch: a divergent branch here costs the 32-row
         // kernel about 45 registers (spilled to AGPRs)
-        const uint32_t hole = bits_below(a.hole_hi - k0) & ~bits_below(a.hole_lo - k0);
-        // extra key ex_lo + i stands for position hole_lo + i: visible below vis
-        const int ex_end = min(a.ex_hi, a.ex_lo + vis - a.hole_lo);
-        const uint32_t ex = bits_below(ex_end - k0) & ~bits_below(a.ex_lo - k0);
-        const uint32_t m = bits_below(vis - k0);
-        return run_a ? ((m & ~hole) | ex) : m;
+        const int end = dec ? dec_end : vis, lo = dec ? 0 : bnd;
+        const uint32_t m = bits_below(end - base);
+        return base >= lo ? m : 0u;
     }
 };
-// One past the last key any row of the block sees (rows are ordered by query).
-__device__ __forceinline__ int block_key_end(const PrefillArgs& a, int row_first, int row_last) {
-    int lim = min(a.n_k, a.vis0 + row_last / a.n_rep);
-    if (row_first / a.n_rep < a.q_b) lim = max(lim, a.ex_hi);
-    return lim;
-}
+// The block's tile list (PrefillArgs) and this split's part of it.
+struct BlockKeys {
+    int nd, u0, t_lo, t_hi, n_split;
+    __device__ __forceinline__ BlockKeys(const PrefillArgs& a, int row_first, int row_last, int split) {
+        const int n = a.block_tiles(row_first, row_last, &nd, &u0);
+        n_split = a.block_splits(n);
+        const int per = (n + n_split - 1) / n_split;
+        t_lo = min(n, split * per);
+        t_hi = min(n, t_lo + per);
+    }
+    __device__ __forceinline__ bool dec(int t) const { return t < nd; }
+    __device__ __forceinline__ int base(int t) const { return 32 * (t < nd ? t : u0 + t - nd); }
+};
+// Longest blocks first: the last query blocks see the most keys.  Block index =
+// ((reversed row block) * h_kv + head) * n_split + split.
+struct BlockPos {
+    int bx, h, split;
+    __device__ __forceinline__ BlockPos(const PrefillArgs& a, int n_blk) {
+        int b = blockIdx.x;
+        split = b % a.n_split;
+        b /= a.n_split;
+        h = b % a.h_kv;
+        bx = n_blk - 1 - b / a.h_kv;
+    }
+};
 
 // ----------------------------------------------------------- attention
 // Block = 4 wavefronts = 4 tiles of 16 query rows of one KV head, one key
@@ -283,26 +289,77 @@ constexpr int VS_LD = KT + 4;     // halves per LDS V^T row (rows 8-byte aligned
                                   // stored and read in 8-byte pieces)
 constexpr float GAP = 8.0f;
 
+// A wavefront's R rows (row0 on, of KV head h), left in LDS as floats (OUT_LD a
+// row), stored a row at a time: direct rows, already divided by their sums,
+// gated and rounded to the output; the others as the split's triples, with
+// m / l the row's maximum and sum in lane i (< R).  Each instruction writes a
+// whole row, 1 KB: the accumulators' own layout covers a 128-byte line in four
+// stores of 32 bytes, and with other lines' stores between those the 32 MB of
+// triples of a 128-query launch cost it 9 us more.
+constexpr int OUT_LD = 260;
+template <int R>
+__device__ __forceinline__ void store_rows(const PrefillArgs& a, const float* so, int row0, int h, int split,
+                                           bool direct, float m, float l, int lane) {
+    const int n = min(R, a.n_q * a.n_rep - row0), H_q = a.h_kv * a.n_rep;
+    auto row_of = [&](int r) { return (size_t)(r / a.n_rep) * H_q + h * a.n_rep + r % a.n_rep; };
+    if (direct) {
+        constexpr int G = 16;  // rows whose gates are in flight together
+#pragma unroll 1
+        for (int i0 = 0; i0 < n; i0 += G) {
+            uint2 g[G];
+#pragma unroll
+            for (int i = 0; i < G; i++)
+                g[i] = *reinterpret_cast<const uint2*>(a.q + row_of(row0 + min(i0 + i, n - 1)) * 512 + 256 + 4 * lane);
+#pragma unroll
+            for (int i = 0; i < G; i++) {
+                if (i0 + i >= n) break;  // uniform per wavefront
+                const h4 gh = __builtin_bit_cast(h4, g[i]);
+                const f4 v = *reinterpret_cast<const f4*>(&so[(i0 + i) * OUT_LD + 4 * lane]);
+                float o[4];
+#pragma unroll
+                for (int c = 0; c < 4; c++) o[c] = v[c] * (1.0f / (1.0f + expf(-(float)gh[c])));
+                *reinterpret_cast<uint2*>(a.out + row_of(row0 + i0 + i) * 256 + 4 * lane) =
+                    uint2{pk_rne(o[0], o[1]), pk_rne(o[2], o[3])};
+            }
+        }
+        return;
+    }
+    float* part = a.part + (size_t)split * 258;
+#pragma unroll 8
+    for (int i = 0; i < n; i++)
+        *reinterpret_cast<f4*>(part + row_of(row0 + i) * a.n_split * 258 + 4 * lane) =
+            *reinterpret_cast<const f4*>(&so[i * OUT_LD + 4 * lane]);
+    if (lane < n) {
+        float* ml = part + row_of(row0 + lane) * a.n_split * 258 + 256;
+        ml[0] = m;
+        ml[1] = l;
+    }
+}
+
 __global__ __launch_bounds__(256) void prefill_attn_kernel(PrefillArgs a) {
-    __shared__ __align__(16) _Float16 ks[2][KT][KS_LD];
-    __shared__ __align__(16) _Float16 vs[2][256][VS_LD];
-    const int h = blockIdx.y;
+    __shared__ union __align__(16) {
+        struct {
+            _Float16 ks[2][KT][KS_LD], vs[2][256][VS_LD];
+        } t;
+        float out[4][16][OUT_LD];
+    } lds;
+    auto& ks = lds.t.ks;
+    auto& vs = lds.t.vs;
     const int tid = threadIdx.x;
     const int wv = tid >> 6, lane = tid & 63;
     const int li = lane & 15, lg = lane >> 4;
     const int n_rows = a.n_q * a.n_rep;
-    const int row0 = (blockIdx.x * 4 + wv) * 16;
-    const int split = blockIdx.z;
-    const int k_lo = split * a.keys_per_split;
-    const int k_hi = min(a.n_tot, k_lo + a.keys_per_split);
+    const BlockPos pos(a, (n_rows + 63) / 64);
+    const int h = pos.h, split = pos.split;
+    const int row0 = (pos.bx * 4 + wv) * 16;
     const int H_q = a.h_kv * a.n_rep;
     const int r = row0 + li;
     const bool r_ok = r < n_rows;
     const int jq = r_ok ? r / a.n_rep : 0;
     const int hq = h * a.n_rep + (r_ok ? r % a.n_rep : 0);
-    const RowKeys vis(a, r_ok, jq);
-    const int b_last = min((int)blockIdx.x * 64 + 63, n_rows - 1);
-    const int kt_hi = min(k_hi, block_key_end(a, blockIdx.x * 64, b_last));
+    const RowKeys vis(a, jq);
+    const BlockKeys bk(a, pos.bx * 64, min(pos.bx * 64 + 63, n_rows - 1), split);
+    if (split >= bk.n_split) return;  // uniform per block
 
     h8 qb[8];
     {
@@ -326,8 +383,11 @@ __global__ __launch_bounds__(256) void prefill_attn_kernel(PrefillArgs a) {
     uint4 pk[4], pv[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) pk[i] = pv[i] = uint4{0u, 0u, 0u, 0u};
-    auto gload = [&](int k0) {
-        const int key = min(k0 + ld_key, a.n_tot - 1);
+    const int raw_end = a.raw0 + a.n_raw;
+    auto key_of = [&](int t) { return (bk.dec(t) ? 0 : a.raw0) + bk.base(t); };
+    auto gload = [&](int t) {
+        const int k0 = key_of(t);
+        const int key = bk.dec(t) ? k0 + ld_key : min(k0 + ld_key, raw_end - 1);
         const uint4* ksrc = reinterpret_cast<const uint4*>(kg + (size_t)key * a.h_kv * 256);
         const uint4* vsrc = reinterpret_cast<const uint4*>(vg + k0);
 #pragma unroll
@@ -336,13 +396,13 @@ __global__ __launch_bounds__(256) void prefill_attn_kernel(PrefillArgs a) {
             pv[i] = vsrc[i];
         }
     };
-    // V^T word w of a tile row holds keys 2 w, 2 w + 1; columns past n_k are
-    // padding and become zero
+    // V^T word w of a tile row holds keys 2 w, 2 w + 1; columns past the last
+    // raw key are padding and become zero
     auto vmask = [](uint32_t w, int i, int nv) {
         return 2 * i + 1 < nv ? w : (2 * i < nv ? (w & 0xFFFFu) : 0u);
     };
-    auto lstore = [&](int buf, int k0) {
-        const int nv = a.n_tot - k0;
+    auto lstore = [&](int buf, int t) {
+        const int nv = bk.dec(t) ? KT : a.n_raw - bk.base(t);
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             *reinterpret_cast<uint4*>(&ks[buf][ld_key][ld_off + 8 * i]) = pk[i];
@@ -355,16 +415,14 @@ __global__ __launch_bounds__(256) void prefill_attn_kernel(PrefillArgs a) {
         }
     };
 
-    const int n_tiles = k_lo < kt_hi ? (kt_hi - k_lo + KT - 1) / KT : 0;
-    if (n_tiles > 0) {
-        gload(k_lo);
-        lstore(0, k_lo);
-        if (n_tiles > 1) gload(k_lo + KT);
+    if (bk.t_lo < bk.t_hi) {
+        gload(bk.t_lo);
+        lstore(0, bk.t_lo);
+        if (bk.t_lo + 1 < bk.t_hi) gload(bk.t_lo + 1);
     }
     __syncthreads();
-    for (int t = 0; t < n_tiles; t++) {
-        const int buf = t & 1;
-        const int k0 = k_lo + t * KT;
+    for (int t = bk.t_lo; t < bk.t_hi; t++) {
+        const int buf = (t - bk.t_lo) & 1;
         // ---- S^T of both 16-key halves from LDS
         f4 s0 = f4{0.f, 0.f, 0.f, 0.f}, s1 = s0;
 #pragma unroll
@@ -376,7 +434,7 @@ __global__ __launch_bounds__(256) void prefill_attn_kernel(PrefillArgs a) {
         }
         float sc[8], lmax = -INFINITY;
         {
-            const uint32_t mb = vis.tile(k0) >> (4 * lg);
+            const uint32_t mb = vis.tile(bk.dec(t), bk.base(t)) >> (4 * lg);
 #pragma unroll
             for (int c = 0; c < 4; c++) {
                 sc[c] = (mb >> c) & 1u ? s0[c] * a.sc : -INFINITY;
@@ -421,26 +479,24 @@ __global__ __launch_bounds__(256) void prefill_attn_kernel(PrefillArgs a) {
             for (int i = 0; i < 4; i++) acc[m4 + i] = mfma32(vop[i], pb, acc[m4 + i]);
         }
         // ---- stage the next tile, load the one after
-        if (t + 1 < n_tiles) {
-            lstore(buf ^ 1, k0 + KT);
-            if (t + 2 < n_tiles) gload(k0 + 2 * KT);
+        if (t + 1 < bk.t_hi) {
+            lstore(buf ^ 1, t + 1);
+            if (t + 2 < bk.t_hi) gload(t + 2);
         }
         __syncthreads();
     }
-    // ---- partial triple of row li (dims 16 mt + 4 lg + c)
+    // ---- row li (dims 16 mt + 4 lg + c)
     float l_row = l_part + __shfl_xor(l_part, 16, 64);
     l_row += __shfl_xor(l_row, 32, 64);
-    if (r_ok) {
-        float* out = a.part + ((size_t)(jq * H_q + hq) * a.n_split + split) * 258;
-        const bool empty = (m_ref == -INFINITY);
+    const bool direct = bk.n_split == 1 && a.out;
+    const bool empty = m_ref == -INFINITY;
+    const float f = empty ? 0.0f : (direct ? 1.0f / (l_row + a.eps) : 1.0f);
 #pragma unroll
-        for (int mt = 0; mt < 16; mt++)
-            *reinterpret_cast<f4*>(&out[16 * mt + 4 * lg]) = empty ? f4{0.f, 0.f, 0.f, 0.f} : acc[mt];
-        if (lg == 0) {
-            out[256] = empty ? -1e20f : m_ref;
-            out[257] = empty ? 0.0f : l_row;
-        }
-    }
+    for (int mt = 0; mt < 16; mt++)  // every wavefront is past the tiles
+        *reinterpret_cast<f4*>(&lds.out[wv][li][16 * mt + 4 * lg]) = acc[mt] * f;
+    wave_sync();
+    store_rows<16>(a, &lds.out[wv][0][0], row0, h, split, direct, empty ? -1e20f : m_ref,
+                   empty ? 0.0f : l_row, lane);
 }
 
 // 32-row form: 32 query rows per wavefront pair on 32x32x16 MFMAs, so every
@@ -480,34 +536,41 @@ constexpr float GAP32 = 10.0f;
 // wavefront passes the same barriers).
 __global__ __launch_bounds__(512, 1) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void prefill_attn_rs_kernel(PrefillArgs a) {
-    __shared__ __align__(16) _Float16 ks[NKB][KT][KS2_LD];
-    __shared__ __align__(16) _Float16 vs[NKB][256][VS2_LD];
-    __shared__ __align__(16) f4 pss[2][4][4][64];     // masked scaled scores (slot, row group, quad, lane)
-    __shared__ float2 pmf[2][4][64];                   // (reference max, rescale factor) per slot
-    const int h = blockIdx.y;
+    __shared__ union __align__(16) {
+        struct {
+            _Float16 ks[NKB][KT][KS2_LD], vs[NKB][256][VS2_LD];
+            f4 pss[2][4][4][64];   // masked scaled scores (slot, row group, quad, lane)
+            float2 pmf[2][4][64];  // (reference max, rescale factor) per slot
+        } t;
+        float out[4][32][OUT_LD];
+    } lds;
+    auto& ks = lds.t.ks;
+    auto& vs = lds.t.vs;
+    auto& pss = lds.t.pss;
+    auto& pmf = lds.t.pmf;
     const int tid = threadIdx.x;
     const int wv = tid >> 6, lane = tid & 63;
     const int rg = wv & 3;           // row group
     const int t256 = tid & 255;      // staging thread within the role
     const int ln = lane & 31, hh = lane >> 5;
     const int n_rows = a.n_q * a.n_rep;
-    const int row0 = (blockIdx.x * 4 + rg) * 32;
-    const int split = blockIdx.z;
-    const int k_lo = split * a.keys_per_split;
-    const int k_hi = min(a.n_tot, k_lo + a.keys_per_split);
+    const BlockPos pos(a, (n_rows + 127) / 128);
+    const int h = pos.h, split = pos.split;
+    const int row0 = (pos.bx * 4 + rg) * 32;
     const int H_q = a.h_kv * a.n_rep;
     const int r = row0 + ln;
     const bool r_ok = r < n_rows;
     const int jq = r_ok ? r / a.n_rep : 0;
     const int hq = h * a.n_rep + (r_ok ? r % a.n_rep : 0);
-    const int b_last = min((int)blockIdx.x * 128 + 127, n_rows - 1);
-    const int kt_hi = min(k_hi, block_key_end(a, blockIdx.x * 128, b_last));
-    const int n_tiles = k_lo < kt_hi ? (kt_hi - k_lo + KT - 1) / KT : 0;
+    const BlockKeys bk(a, pos.bx * 128, min(pos.bx * 128 + 127, n_rows - 1), split);
+    if (split >= bk.n_split) return;  // uniform per block
+    const int n_tiles = bk.t_hi - bk.t_lo;
+    const int raw_end = a.raw0 + a.n_raw;
     const f32x16 zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 
     if (wv < 4) {
         // ================= score wavefront
-        const RowKeys vis(a, r_ok, jq);
+        const RowKeys vis(a, jq);
         h8 qb[16];
         {
             const __half* qrow = a.q + ((size_t)jq * H_q + hq) * 512;
@@ -523,8 +586,9 @@ void prefill_attn_rs_kernel(PrefillArgs a) {
         uint4 pk[4];
 #pragma unroll
         for (int i = 0; i < 4; i++) pk[i] = uint4{0u, 0u, 0u, 0u};
-        auto gload = [&](int k0) {
-            const int key = min(k0 + ld_key, a.n_tot - 1);
+        auto gload = [&](int i0) {  // tile i0 of the split
+            const int t = bk.t_lo + i0, b0 = bk.base(t);
+            const int key = bk.dec(t) ? b0 + ld_key : min(a.raw0 + b0 + ld_key, raw_end - 1);
             const uint4* ksrc = reinterpret_cast<const uint4*>(kg + (size_t)key * a.h_kv * 256);
 #pragma unroll
             for (int i = 0; i < 4; i++) pk[i] = ksrc[i];
@@ -540,14 +604,14 @@ void prefill_attn_rs_kernel(PrefillArgs a) {
                 kop[i] = *reinterpret_cast<const h8*>(&ks[buf][ln][16 * (8 * half + i) + 8 * hh]);
         };
         if (n_tiles > 0) {
-            gload(k_lo);
+            gload(0);
             lstore(0);
         }
         if (n_tiles > 1) {
-            gload(k_lo + KT);
+            gload(1);
             lstore(1);
         }
-        if (n_tiles > 2) gload(k_lo + 2 * KT);
+        if (n_tiles > 2) gload(2);
         __syncthreads();  // prologue: K tiles 0, 1 and V^T tile 0 staged
         float m_ref = -INFINITY;
         f32x16 s2[2];
@@ -563,7 +627,6 @@ void prefill_attn_rs_kernel(PrefillArgs a) {
         }
         for (int t = 0; t < n_tiles; t++) {
             const int nxt = (t + 1) % NKB;
-            const int k0 = k_lo + t * KT;
             float sc[16];
 #pragma unroll
             for (int e = 0; e < 16; e++) sc[e] = s2[0][e] + s2[1][e];
@@ -572,7 +635,8 @@ void prefill_attn_rs_kernel(PrefillArgs a) {
             // ---- S(t + 1), first half, under the mask and row maximum of tile t
             float lmax = -INFINITY;
             {
-                const uint32_t mb = vis.tile(k0) >> (4 * hh);
+                const uint32_t mb =
+                    vis.tile(bk.dec(bk.t_lo + t), bk.base(bk.t_lo + t)) >> (4 * hh);
 #pragma unroll
                 for (int i = 0; i < 8; i++) {
                     s2[i & 1] = mfma3232(kop[i], qb[i], i < 2 ? zero16 : s2[i & 1]);
@@ -605,7 +669,7 @@ void prefill_attn_rs_kernel(PrefillArgs a) {
             // ---- stage K tile t + 2 (its slot last held tile t - 1), load t + 3
             if (t + 2 < n_tiles) {
                 lstore((t + 2) % NKB);
-                if (t + 3 < n_tiles) gload(k0 + 3 * KT);
+                if (t + 3 < n_tiles) gload(t + 3);
             }
             __syncthreads();  // tile t
         }
@@ -620,22 +684,25 @@ void prefill_attn_rs_kernel(PrefillArgs a) {
         uint4 pv[4];
 #pragma unroll
         for (int i = 0; i < 4; i++) pv[i] = uint4{0u, 0u, 0u, 0u};
-        auto gload = [&](int k0) {
-            const uint4* vsrc = reinterpret_cast<const uint4*>(vg + k0);
+        auto gload = [&](int i0) {
+            const int t = bk.t_lo + i0;
+            const uint4* vsrc =
+                reinterpret_cast<const uint4*>(vg + (bk.dec(t) ? 0 : a.raw0) + bk.base(t));
 #pragma unroll
             for (int i = 0; i < 4; i++) pv[i] = vsrc[i];
         };
         auto vmask = [](uint32_t w, int i, int nv) {
             return 2 * i + 1 < nv ? w : (2 * i < nv ? (w & 0xFFFFu) : 0u);
         };
-        auto lstore = [&](int buf, int k0) {
-            const int nv = a.n_tot - k0;
+        auto lstore = [&](int buf, int i0) {
+            const int t = bk.t_lo + i0;
+            const int nv = bk.dec(t) ? KT : a.n_raw - bk.base(t);
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 *reinterpret_cast<uint2*>(&vs[buf][t256][8 * i]) = uint2{pv[i].x, pv[i].y};
                 *reinterpret_cast<uint2*>(&vs[buf][t256][8 * i + 4]) = uint2{pv[i].z, pv[i].w};
             }
-            if (nv < KT) {  // the key space's last tile: V^T columns past n_tot cleared
+            if (nv < KT) {  // the last raw tile: V^T columns past its keys cleared
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     const uint4 v = pv[i];
@@ -691,56 +758,48 @@ void prefill_attn_rs_kernel(PrefillArgs a) {
                 for (int t2 = 0; t2 < 8; t2++) acc[t2] = mfma3232(vop[sp][t2], pbv[sp], acc[t2]);
         };
         if (n_tiles > 0) {
-            gload(k_lo);
-            lstore(0, k_lo);
+            gload(0);
+            lstore(0, 0);
         }
-        if (n_tiles > 1) gload(k_lo + KT);
+        if (n_tiles > 1) gload(1);
         __syncthreads();  // prologue
         for (int t = 0; t < n_tiles; t++) {
             if (t >= 1) pv_tile(t - 1);
             // ---- stage V^T tile t + 1 (its slot last held tile t - 2), load t + 2
             if (t + 1 < n_tiles) {
-                lstore((t + 1) % NKB, k_lo + (t + 1) * KT);
-                if (t + 2 < n_tiles) gload(k_lo + (t + 2) * KT);
+                lstore((t + 1) % NKB, t + 1);
+                if (t + 2 < n_tiles) gload(t + 2);
             }
             __syncthreads();  // tile t
         }
         if (n_tiles > 0) pv_tile(n_tiles - 1);
         __syncthreads();  // last tile applied
         const float l_row = l_part + __shfl_xor(l_part, 32, 64);
-        // ---- partial triple of row ln (dims 32 t + 8 j + 4 hh + c)
-        if (r_ok) {
-            const float2 ml = float2{m_last, l_row};
-            float* out = a.part + ((size_t)(jq * H_q + hq) * a.n_split + split) * 258;
-            const bool empty = (ml.x == -INFINITY);
+        // ---- row ln: the output, or its partial triple (dims 32 t + 8 j + 4 hh + c)
+        const bool direct = bk.n_split == 1 && a.out;
+        const bool empty = m_last == -INFINITY;
+        const float f = empty ? 0.0f : (direct ? 1.0f / (l_row + a.eps) : 1.0f);
 #pragma unroll
-            for (int t2 = 0; t2 < 8; t2++)
+        for (int t2 = 0; t2 < 8; t2++)
 #pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const f4 v = f4{acc[t2][4 * j], acc[t2][4 * j + 1], acc[t2][4 * j + 2], acc[t2][4 * j + 3]};
-                    *reinterpret_cast<f4*>(&out[32 * t2 + 8 * j + 4 * hh]) = empty ? f4{0.f, 0.f, 0.f, 0.f} : v;
-                }
-            if (hh == 0) {
-                out[256] = empty ? -1e20f : ml.x;
-                out[257] = empty ? 0.0f : ml.y;
-            }
-        }
+            for (int j = 0; j < 4; j++)
+                *reinterpret_cast<f4*>(&lds.out[rg][ln][32 * t2 + 8 * j + 4 * hh]) =
+                    f4{acc[t2][4 * j], acc[t2][4 * j + 1], acc[t2][4 * j + 2], acc[t2][4 * j + 3]} * f;
+        wave_sync();
+        store_rows<32>(a, &lds.out[rg][0][0], row0, h, split, direct, empty ? -1e20f : m_last,
+                       empty ? 0.0f : l_row, lane);
     }
 }
 
 // Merge of the key splits, normalisation and gate: one wavefront per (query,
-// head) row, lane l owning dims 4 l .. 4 l + 3; lane s < n_split holds split
+// head) row of a block that was split (the others' rows are written already), lane l owning dims 4 l .. 4 l + 3; lane s < n_split holds split
 // s's (m, l) pair.  Each group of up to 16 splits has every load in flight
 // before the first is used (the first group's with the (m, l) loads, ahead of
 // the maximum); the sums run in split order.
 constexpr int MG = 16;  // splits per load group
-__global__ __launch_bounds__(256) void prefill_merge_kernel(const float* __restrict__ part,
-                                                            const __half* __restrict__ q_gate,
-                                                            __half* __restrict__ out, int n_rows,
-                                                            int n_split, float eps) {
-    const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (row >= n_rows) return;  // uniform per wavefront
-    const float* base = part + (size_t)row * n_split * 258;
+__device__ __forceinline__ void merge_row(const PrefillArgs& p, int row, int n_split) {
+    const int lane = threadIdx.x & 63;
+    const float* base = p.part + (size_t)row * p.n_split * 258;
     float2 a[MG][2];
     auto load_group = [&](int s0) {
 #pragma unroll
@@ -777,112 +836,185 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(const float* __restr
                 den += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(lw), s0 + j));
             }
     }
-    const uint2 gw = *reinterpret_cast<const uint2*>(q_gate + (size_t)row * 512 + 256 + 4 * lane);
+    const uint2 gw = *reinterpret_cast<const uint2*>(p.q + (size_t)row * 512 + 256 + 4 * lane);
     const h4 g = __builtin_bit_cast(h4, gw);
     float o[4];
 #pragma unroll
     for (int c = 0; c < 4; c++)
-        o[c] = num[c] / (den + eps) * (1.0f / (1.0f + expf(-(float)g[c])));
-    *reinterpret_cast<uint2*>(out + (size_t)row * 256 + 4 * lane) =
+        o[c] = num[c] / (den + p.eps) * (1.0f / (1.0f + expf(-(float)g[c])));
+    *reinterpret_cast<uint2*>(p.out + (size_t)row * 256 + 4 * lane) =
         uint2{pk_rne(o[0], o[1]), pk_rne(o[2], o[3])};
+}
+
+// Blocks [0, nb_m): rows 4 b .. + 3, one wavefront each; the rest copy new
+// tokens to the ring, 8 bytes a thread and tensor.
+__global__ __launch_bounds__(256) void prefill_finish_kernel(PrefillArgs a, RingArgs g, int nb_m,
+                                                             int block_rows) {
+    int b = blockIdx.x;
+    if (b < nb_m) {
+        const int H_q = a.h_kv * a.n_rep, row = b * 4 + (threadIdx.x >> 6);
+        if (row >= a.n_q * H_q) return;  // uniform per wavefront
+        const int r = row / H_q * a.n_rep + row % H_q % a.n_rep;  // row of its KV head
+        const int first = r / block_rows * block_rows;
+        int nd, u0;
+        const int ns = a.block_splits(
+            a.block_tiles(first, min(first + block_rows, a.n_q * a.n_rep) - 1, &nd, &u0));
+        if (ns > 1) merge_row(a, row, ns);
+        return;
+    }
+    b -= nb_m;
+    const int per = g.h_kv * 64;  // pieces per token
+    const long i = (long)b * 256 + threadIdx.x;
+    if (i >= (long)g.n * per) return;
+    const int t = (int)(i / per), e = (int)(i % per) * 4;
+    int slot = g.slot0 + t;
+    slot = slot >= g.ring_cap ? slot - g.ring_cap : slot;
+    const size_t src = (size_t)t * per * 4 + e, dst = (size_t)slot * per * 4 + e;
+    *reinterpret_cast<uint2*>(g.ring_k + dst) = *reinterpret_cast<const uint2*>(g.src_k + src);
+    *reinterpret_cast<uint2*>(g.ring_v + dst) = *reinterpret_cast<const uint2*>(g.src_v + src);
+    *reinterpret_cast<uint2*>(g.ring_u + dst) = *reinterpret_cast<const uint2*>(g.src_u + src);
 }
 
 }  // namespace pf
 
-hipError_t launch_prefill_merge(const float* part, const __half* q_gate, __half* out, int n_rows,
-                                int n_split, float eps, hipStream_t st) {
-    hipLaunchKernelGGL(pf::prefill_merge_kernel, dim3((n_rows + 3) / 4), dim3(256), 0, st, part,
-                       q_gate, out, n_rows, n_split, eps);
+namespace {
+int gather_blocks(const GatherArgs& g) { return g.n > 0 ? (g.n + 31) / 32 * g.h_kv : 0; }
+bool long_decode(const DecompArgs& a) {
+    // 4 KV heads, 4 / 16 tokens a block: 1,024 tokens 14.3 / 15.7 us, 2,000
+    // 21.9 / 19.3, 8,192 62.6 / 48.3 (32 a block: 25 us at least, 43.4)
+    return a.n_tok / pf::TB_LONG * a.h_kv >= 3 * device_cu_count() / 2;
+}
+}  // namespace
+
+hipError_t launch_prefill_finish(const PrefillArgs& a, const RingArgs* ring, hipStream_t st) {
+    const int nb_m = a.n_split > 1 ? (a.n_q * a.h_kv * a.n_rep + 3) / 4 : 0;
+    const RingArgs g = ring ? *ring : RingArgs{};
+    const int nb_g = ring ? (g.n * g.h_kv * 64 + 255) / 256 : 0;
+    if (nb_m + nb_g == 0) return hipSuccess;
+    hipLaunchKernelGGL(pf::prefill_finish_kernel, dim3(nb_m + nb_g), dim3(256), 0, st, a, g, nb_m,
+                       prefill_block_rows(a.n_q * a.n_rep));
     return hipGetLastError();
 }
 
 hipError_t launch_decompress(const DecompArgs& a, hipStream_t st) {
     if (a.n_tok <= 0) return hipSuccess;
-    hipLaunchKernelGGL(pf::decompress_kernel, dim3((a.n_tok + pf::TOK_BLK - 1) / pf::TOK_BLK, a.h_kv),
-                       dim3(pf::BLK_THR), 0, st, a);
+    if (long_decode(a))
+        hipLaunchKernelGGL(pf::decompress_kernel<pf::TB_LONG>,
+                           dim3((a.n_tok + pf::TB_LONG - 1) / pf::TB_LONG, a.h_kv),
+                           dim3(pf::BLK_THR), 0, st, a);
+    else
+        hipLaunchKernelGGL(pf::decompress_kernel<4>, dim3((a.n_tok + 3) / 4, a.h_kv),
+                           dim3(pf::BLK_THR), 0, st, a);
     return hipGetLastError();
 }
 
 hipError_t launch_decompress_gather(const DecompArgs& d, const GatherArgs& g, hipStream_t st) {
-    const int side = g.src_k && g.side_n > 0 ? 1 : 0;
-    const int n_g = std::max(g.n, side ? g.side_n : 0);
     if (d.n_tok <= 0) return launch_ring_gather(g, st);
-    if (n_g <= 0) return launch_decompress(d, st);
-    const int nx_d = (d.n_tok + pf::TOK_BLK - 1) / pf::TOK_BLK;
-    const int nx_g = (n_g + pf::TOK_BLK - 1) / pf::TOK_BLK;
-    hipLaunchKernelGGL(pf::decompress_gather_kernel,
-                       dim3(nx_d * d.h_kv + nx_g * g.h_kv * (1 + side)), dim3(pf::BLK_THR), 0, st,
-                       d, g, nx_d, nx_g);
+    if (g.n <= 0) return launch_decompress(d, st);
+    const int tb = long_decode(d) ? pf::TB_LONG : 4, nx_d = (d.n_tok + tb - 1) / tb;
+    const dim3 grid(nx_d * d.h_kv + gather_blocks(g));
+    if (tb == 4)
+        hipLaunchKernelGGL(pf::decompress_gather_kernel<4>, grid, dim3(pf::BLK_THR), 0, st, d, g, nx_d);
+    else
+        hipLaunchKernelGGL(pf::decompress_gather_kernel<pf::TB_LONG>, grid, dim3(pf::BLK_THR), 0, st,
+                           d, g, nx_d);
     return hipGetLastError();
 }
 
 hipError_t launch_compress_decode(const CompressJob& k, const CompressJob& v, const DecompArgs& d,
-                                  const GatherArgs* g, hipStream_t st) {
+                                  const GatherArgs& g, hipStream_t st) {
     // the decode covers exactly the compressed rows: token t, KV head h is row t h_kv + h
     if (k.n != v.n || d.n_tok * d.h_kv != k.n || d.tok0 != d.key0 || d.start_pos != 0)
         return hipErrorInvalidValue;
     const int nb_k = (k.n + 3) / 4;
-    int nx_g = 0, planes = 0;
-    GatherArgs ga{};
-    if (g) {
-        const int side = g->src_k && g->side_n > 0 ? 1 : 0;
-        const int n_g = std::max(g->n, side ? g->side_n : 0);
-        if (n_g > 0) {
-            nx_g = (n_g + pf::TOK_BLK - 1) / pf::TOK_BLK;
-            planes = 1 + side;
-            ga = *g;
-        }
-    }
-    hipLaunchKernelGGL(pf::compress_decode_kernel, dim3(v.n + nb_k + nx_g * ga.h_kv * planes),
-                       dim3(pf::BLK_THR), 0, st, k, v, d, ga, nb_k, nx_g);
+    hipLaunchKernelGGL(pf::compress_decode_kernel, dim3(v.n + nb_k + gather_blocks(g)),
+                       dim3(pf::BLK_THR), 0, st, k, v, d, g, nb_k);
+    return hipGetLastError();
+}
+
+hipError_t launch_compress_gather(const CompressJob& k, const CompressJob& v, const GatherArgs& g,
+                                  hipStream_t st) {
+    const int k_many = compress_k_many(k.n);
+    const int nb_k = k_many ? (k.n + 4 * KR - 1) / (4 * KR) : (k.n + 3) / 4;
+    const int nb_v = (v.n + VR - 1) / VR;
+    hipLaunchKernelGGL(pf::compress_gather_kernel, dim3(nb_k + nb_v + gather_blocks(g)),
+                       dim3(pf::BLK_THR), 0, st, k, v, g, nb_k, nb_v, k_many);
     return hipGetLastError();
 }
 
 hipError_t launch_ring_gather(const GatherArgs& a, hipStream_t st) {
-    const int side = a.src_k && a.side_n > 0 ? 1 : 0;
-    const int n = std::max(a.n, side ? a.side_n : 0);
-    if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(pf::ring_gather_kernel,
-                       dim3((n + pf::TOK_BLK - 1) / pf::TOK_BLK, a.h_kv, 1 + side),
-                       dim3(pf::BLK_THR), 0, st, a);
+    if (a.n <= 0) return hipSuccess;
+    hipLaunchKernelGGL(pf::ring_gather_kernel, dim3(gather_blocks(a)), dim3(pf::BLK_THR), 0, st, a);
     return hipGetLastError();
 }
 
 namespace {
-// Few query rows (a handful of queries, e.g. the one after a compression
-// event): the 16-row kernel, two blocks per CU (more, shorter splits); many:
-// the role-specialised 32-row kernel (half the LDS operand traffic per flop).
+// Few query rows (a handful of queries): the 16-row kernel, two blocks per CU
+// (more, shorter splits); many: the role-specialised 32-row kernel (half the
+// LDS operand traffic per flop).
 bool few_rows(int n_rows) { return n_rows <= 128; }
 }  // namespace
 
-int prefill_splits(int n_q, int n_rep, int h_kv, int n_k, int* keys_per_split) {
+int prefill_block_rows(int n_rows) { return few_rows(n_rows) ? 64 : 128; }
+
+void prefill_plan(PrefillArgs& a) {
     // Blocks that run at once: 2 per CU for the 16-row kernel (72 KB of LDS
-    // each), 1 for the 32-row kernel (142 KB).  The split count fills that
-    // many slots in one round: a few blocks past a round cost a whole round.
-    const int n_cu = device_cu_count();
-    const int n_rows = n_q * n_rep;
-    const bool few = few_rows(n_rows);
-    const int slots = few ? 2 * n_cu : n_cu;
-    const int blocks = (few ? ((n_rows + 15) / 16 + 3) / 4 : (n_rows + 127) / 128) * h_kv;
-    int ns = slots / blocks;
-    ns = std::max(1, std::min(ns, 64));
-    int per = (n_k + ns - 1) / ns;
-    per = (per + pf::KT - 1) / pf::KT * pf::KT;
-    ns = (n_k + per - 1) / per;
-    *keys_per_split = per;
-    return std::max(ns, 1);
+    // each), 1 for the 32-row kernel (142 KB).  With splits of at most `unit`
+    // tiles, the launch takes, in tiles of time:
+    //   one round of the longest block when they all fit at once;
+    //   else the work over the slots plus half a block of tail (they start
+    //   longest first), or whole rounds when the blocks are equally long (a
+    //   few blocks past a round cost a whole round).
+    // A block costs about 4 tiles beside its own (entry, first loads, output);
+    // splitting costs the finishing launch, about 4, and 0.045 a block for its
+    // triples (128 rows x 1 KB written and read).
+    const int n_rows = a.n_q * a.n_rep, br = prefill_block_rows(n_rows);
+    const int nb = (n_rows + br - 1) / br;
+    const int slots = (few_rows(n_rows) ? 2 : 1) * device_cu_count();
+    int t_max = 1, t_min = 1 << 30;
+    for (int b = 0; b < nb; b++) {
+        int nd, u0;
+        const int t = a.block_tiles(b * br, std::min(b * br + br, n_rows) - 1, &nd, &u0);
+        t_max = std::max(t_max, t);
+        t_min = std::min(t_min, t);
+    }
+    const bool even = t_max - t_min <= t_max / 8;
+    const int step = std::max(1, nb / 64);  // enough blocks to add up
+    float best = 0.0f;
+    int best_k = 1;
+    for (int k = 1; k <= std::min(64, t_max); k++) {
+        a.n_split = k;
+        a.unit = (t_max + k - 1) / k;
+        if (k > 1 && (size_t)a.n_q * a.h_kv * a.n_rep * k * 258 * 4 > (size_t)1 << 30) break;
+        float units = 0.0f, tiles = 0.0f;
+        for (int b = 0; b < nb; b += step) {
+            int nd, u0;
+            const int t = a.block_tiles(b * br, std::min(b * br + br, n_rows) - 1, &nd, &u0);
+            const float w = (float)std::min(step, nb - b) * a.h_kv;
+            units += w * a.block_splits(t);
+            tiles += w * t;
+        }
+        const float rounds = std::ceil(units / slots);
+        float est = rounds <= 1.0f || even ? rounds * (a.unit + 4)
+                                           : (tiles + 4 * units) / slots + 0.5f * a.unit;
+        if (k > 1) est += 4.0f + 0.045f * units;
+        if (k == 1 || est < best) {
+            best = est;
+            best_k = k;
+        }
+    }
+    a.n_split = best_k;
+    a.unit = (t_max + a.n_split - 1) / a.n_split;
+    a.n_split = (t_max + a.unit - 1) / a.unit;
 }
 
 hipError_t launch_prefill_attn(const PrefillArgs& a, hipStream_t st) {
-    const int n_rows = a.n_q * a.n_rep;
-    if (few_rows(n_rows)) {
-        const int mtiles = (n_rows + 15) / 16;
-        hipLaunchKernelGGL(pf::prefill_attn_kernel, dim3((mtiles + 3) / 4, a.h_kv, a.n_split),
-                           dim3(256), 0, st, a);
-    } else {
-        hipLaunchKernelGGL(pf::prefill_attn_rs_kernel, dim3((n_rows + 127) / 128, a.h_kv, a.n_split),
-                           dim3(512), 0, st, a);
-    }
+    const int n_rows = a.n_q * a.n_rep, br = prefill_block_rows(n_rows);
+    const dim3 grid((unsigned)((n_rows + br - 1) / br) * a.h_kv * a.n_split);
+    if (few_rows(n_rows))
+        hipLaunchKernelGGL(pf::prefill_attn_kernel, grid, dim3(256), 0, st, a);
+    else
+        hipLaunchKernelGGL(pf::prefill_attn_rs_kernel, grid, dim3(512), 0, st, a);
     return hipGetLastError();
 }
 

@@ -14,7 +14,7 @@ import torch
 
 import npref
 import oracle
-from khq import layer as KL
+from khq import synth, layer as KL
 from khq import ops
 from khqdata import (D, H_KV, H_Q, N_REP, SCALE, THETA, layer_consts, random_rows_np,
                      rope_fp16_rows, two_region_state)
@@ -280,6 +280,26 @@ def test_layer_prefill_decoded_rows_match_decode(device, chunks):
     assert np.array_equal(gv, wv)
 
 
+def test_decompress_long_matches_short(device):
+    """1,601 tokens in one call (16 a block, from 384 blocks on 256 CUs) against
+    the same tokens in calls of 400 (4 a block), bit for bit; columns past the
+    last token's group of four stay as they were."""
+    lc, _ = layer_consts(layer_id=2)
+    n, ld = 1601, 1664
+    cents, pay = ops.Centroids(lc, device), ops.Payload(n * H_KV, device)
+    synth.compressed_rows(pay, cents, seed=5)
+    outs = []
+    for step in (n, 400):
+        k = torch.zeros((n, H_KV, D), device=device, dtype=torch.float16)
+        vt = torch.full((H_KV, D, ld), 7.0, device=device, dtype=torch.float16)
+        for t0 in range(0, n, step):
+            ops.decompress(pay, cents, k, vt, H_kv=H_KV, tok0=t0, n_tok=min(step, n - t0), key0=t0,
+                           ld_vt=ld)
+        outs.append((k.cpu().numpy().view(np.uint16), vt.cpu().numpy().view(np.uint16)))
+    assert np.array_equal(outs[0][0], outs[1][0]) and np.array_equal(outs[0][1], outs[1][1])
+    assert (outs[0][1][:, :, 1604:] == np.float16(7.0).view(np.uint16)).all()
+
+
 def test_c5_chunk_vs_oracle(device):
     """Config 5: 8,192 tokens already appended (boundary 8,064, raw 8,064..
     8,191), then one chunk of 128 tokens at positions 8,192..8,319; the 128th
@@ -315,6 +335,75 @@ def test_c5_chunk_vs_oracle(device):
                                    ring_cap=256, H_q=H_Q, H_kv=H_KV, scale=SCALE)
         _, want = oracle.merge_gate(ac, aw, qj, H_q=H_Q, has_w=True)
         close(got[j], want)
+
+
+@pytest.mark.parametrize("cap,steps,calls,after", [
+    (2048, 0, (900,), 3),          # six events in one call
+    (2048, 0, (255, 1, 700), 0),   # ends just below / on the first event, then five
+    (2048, 130, (600,), 2),        # window in the ring, first compressed rows from it
+    (2048, 300, (21, 300), 0),     # earlier events stepped (nothing decoded yet), few rows
+    (300, 0, (600,), 0),           # capacity: two events, then the ring fills, then -102
+])
+def test_layer_prefill_one_call(device, cap, steps, calls, after):
+    """Calls that span several compression events (one attention launch with
+    rows on both sides of each) against the same tokens stepped: state, packed
+    bytes, ring contents, every output; steps after the call see its ring."""
+    lc, _ = layer_consts(layer_id=11)
+    opt = KL.KhqOptions(splits=8, fused=True)
+    st, pf = (KL.NativeKhqLayer(lc, H_q=H_Q, H_kv=H_KV, cap=cap, device=device, options=opt)
+              for _ in range(2))
+    n = steps + sum(calls) + after
+    k, kr, v, q = _tokens(n, seed=41)
+    qd, krd, vd, kd = t(q), t(kr), t(v), t(k)
+    o_st, o_pf = (torch.zeros((n, H_Q, D), device=device, dtype=torch.float16) for _ in range(2))
+    held = min(n, cap // 128 * 128 + 256)
+    for i in range(held):
+        assert st.step(qd[i], krd[i], vd[i], o_st[i], SCALE, k_unroped=kd[i])
+    for i in range(steps):
+        assert pf.step(qd[i], krd[i], vd[i], o_pf[i], SCALE, k_unroped=kd[i])
+    i = steps
+    for m in calls:
+        part = slice(i, i + m)
+        if i + m > held:
+            with pytest.raises(RuntimeError):
+                pf.prefill(qd[part], krd[part], vd[part], kd[part], o_pf[part], SCALE)
+        else:
+            assert pf.prefill(qd[part], krd[part], vd[part], kd[part], o_pf[part], SCALE) == m
+        i += m
+    for j in range(i, n):
+        assert pf.step(qd[j], krd[j], vd[j], o_pf[j], SCALE, k_unroped=kd[j])
+    torch.cuda.synchronize()
+    assert pf.state() == st.state()
+    a, ra = _payload_np(st, st.state()[0])
+    b, rb = _payload_np(pf, st.state()[0])
+    for name in a:
+        assert np.array_equal(a[name], b[name]), name
+    assert np.array_equal(ra[0], rb[0]) and np.array_equal(ra[1], rb[1])
+    got, want = o_pf.cpu().numpy(), o_st.cpu().numpy()
+    for j in range(n):
+        close(got[j], want[j])
+
+
+@pytest.mark.parametrize("n_q,n_k", [(21, 40), (22, 33), (700, 700), (3000, 3000)])
+def test_prefill_attn_plans_vs_float64(device, n_q, n_k):
+    """Both sides of the 16-row / 32-row switch (128 rows a KV head) and the
+    plans of long launches: blocks written out directly beside split ones, then
+    blocks past one round of the chip, none split."""
+    rng = np.random.default_rng(n_q)
+    q = rng.standard_normal((n_q, H_Q, 2 * D)).astype(np.float16)
+    K, V = (rng.standard_normal((n_k, H_KV, D)).astype(np.float16) for _ in range(2))
+    ld = ops.vt_ld(n_k)
+    vt = torch.full((H_KV, D, ld), float("nan"), device=device, dtype=torch.float16)
+    vt[:, :, :n_k] = t(V).permute(1, 2, 0)
+    out = torch.zeros((n_q, H_Q, D), device=device, dtype=torch.float16)
+    vis0 = n_k - n_q + 1
+    ops.prefill_attn(t(q), t(K), vt, out, ld_vt=ld, n_k=n_k, n_q=n_q, vis0=vis0, H_q=H_Q,
+                     H_kv=H_KV, scale=SCALE)
+    got = out.cpu().numpy()
+    rows = sorted({0, 1, 20, n_q // 2, n_q - 2, n_q - 1, *range(5, n_q, 97)} & set(range(n_q)))
+    for j in rows:
+        want = _dense_reference(q[j:j + 1], K.astype(np.float64), V.astype(np.float64), vis0 + j, n_k)
+        close(got[j:j + 1], want)
 
 
 def test_layer_prefill_mixed_with_steps(device):
