@@ -289,6 +289,14 @@ constexpr int VS_LD = KT + 4;     // halves per LDS V^T row (rows 8-byte aligned
                                   // stored and read in 8-byte pieces)
 constexpr float GAP = 8.0f;
 
+// l plus both halves of a packed weight pair (fp32 sum): row sums are taken over
+// the weights as the MFMAs use them, rounded to fp16, so a row's weights sum to
+// one exactly as applied and one rounding error does not become two.  Rows of
+// few keys gain the most; it is also half the adds.
+__device__ __forceinline__ float add_pair(uint32_t pw, float l) {
+    return __builtin_amdgcn_fdot2(__builtin_bit_cast(h2, pw), h2{(_Float16)1.0f, (_Float16)1.0f}, l, false);
+}
+
 // A wavefront's R rows (row0 on, of KV head h), left in LDS as floats (OUT_LD a
 // row), stored a row at a time: direct rows, already divided by their sums,
 // gated and rounded to the output; the others as the split's triples, with
@@ -458,12 +466,14 @@ __global__ __launch_bounds__(256) void prefill_attn_kernel(PrefillArgs a) {
         }
         float p[8];
 #pragma unroll
-        for (int e = 0; e < 8; e++) {
-            p[e] = sc[e] == -INFINITY ? 0.0f : __expf(sc[e] - m_ref);
-            l_part += p[e];
+        for (int e = 0; e < 8; e++) p[e] = sc[e] == -INFINITY ? 0.0f : __expf(sc[e] - m_ref);
+        uint32_t pw[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            pw[e] = pk_rne(p[2 * e], p[2 * e + 1]);
+            l_part = add_pair(pw[e], l_part);
         }
-        const h8 pb = __builtin_bit_cast(
-            h8, uint4{pk_rne(p[0], p[1]), pk_rne(p[2], p[3]), pk_rne(p[4], p[5]), pk_rne(p[6], p[7])});
+        const h8 pb = __builtin_bit_cast(h8, uint4{pw[0], pw[1], pw[2], pw[3]});
         // ---- O^T += V^T P^T (K = the 32 keys in the lane order above)
 #pragma unroll
         for (int m4 = 0; m4 < 16; m4 += 4) {  // 4 operand reads in flight, then 4 MFMAs
@@ -613,6 +623,12 @@ void prefill_attn_rs_kernel(PrefillArgs a) {
         }
         if (n_tiles > 2) gload(2);
         __syncthreads();  // prologue: K tiles 0, 1 and V^T tile 0 staged
+        // Weights are rounded to fp16 except a row's reference key's, which is 1.
+        // Blocks that run all their keys in one go raise the reference at every
+        // new maximum of the first 8 tiles, so a row of few keys (where one
+        // weight counts) has its largest one exact; splits had that from their
+        // several references.
+        const int n_eager = bk.n_split == 1 ? 8 : 0;
         float m_ref = -INFINITY;
         f32x16 s2[2];
         {
@@ -651,7 +667,7 @@ void prefill_attn_rs_kernel(PrefillArgs a) {
             // ---- raise the row's reference maximum only when needed; the
             // output wavefront rescales its accumulators and sums by fac
             float fac = 1.0f;
-            if (__ballot(lmax > m_ref + GAP32) != 0ull) {
+            if (__ballot(lmax > m_ref + (t < n_eager ? 0.0f : GAP32)) != 0ull) {
                 const float rmax = fmaxf(lmax, __shfl_xor(lmax, 32, 64));
                 const float m_new = fmaxf(m_ref, rmax);
                 if (m_new > m_ref) {
@@ -741,17 +757,17 @@ void prefill_attn_rs_kernel(PrefillArgs a) {
             }
             float p[16];
 #pragma unroll
-            for (int e = 0; e < 16; e++) {
-                p[e] = sc[e] == -INFINITY ? 0.0f : __expf(sc[e] - mf.x);
-                l_part += p[e];
+            for (int e = 0; e < 16; e++) p[e] = sc[e] == -INFINITY ? 0.0f : __expf(sc[e] - mf.x);
+            uint32_t pw[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                pw[e] = pk_rne(p[2 * e], p[2 * e + 1]);
+                l_part = add_pair(pw[e], l_part);
             }
             h8 pbv[2];
 #pragma unroll
             for (int sp = 0; sp < 2; sp++)
-                pbv[sp] = __builtin_bit_cast(h8, uint4{pk_rne(p[8 * sp], p[8 * sp + 1]),
-                                                       pk_rne(p[8 * sp + 2], p[8 * sp + 3]),
-                                                       pk_rne(p[8 * sp + 4], p[8 * sp + 5]),
-                                                       pk_rne(p[8 * sp + 6], p[8 * sp + 7])});
+                pbv[sp] = __builtin_bit_cast(h8, uint4{pw[4 * sp], pw[4 * sp + 1], pw[4 * sp + 2], pw[4 * sp + 3]});
 #pragma unroll
             for (int sp = 0; sp < 2; sp++)
 #pragma unroll
