@@ -528,7 +528,11 @@ constexpr int VS2_LD = KT + 4;    // halves per LDS V^T row
 
 constexpr int NKB = 3;            // LDS tile slots
 // Lazy-rescale gap of the 32-row form: weights stay <= e^10 (< fp16 max).
-constexpr float GAP32 = 10.0f;
+// Reference of a row that has seen no key: finite, so that a masked score less
+// it is -inf and its weight 0 without a test.
+constexpr float M_NONE = -1e30f;
+constexpr float LOG2E = 1.44269504f, LN2 = 0.693147181f;
+constexpr float GAP32 = 10.0f * LOG2E;  // in the kernel's log2 units
 
 // Role-specialised 32-row attention: per SIMD a score wavefront and an
 // output wavefront (8 wavefronts per block, 128 rows of one KV head).  The
@@ -629,7 +633,8 @@ void prefill_attn_rs_kernel(PrefillArgs a) {
         // weight counts) has its largest one exact; splits had that from their
         // several references.
         const int n_eager = bk.n_split == 1 ? 8 : 0;
-        float m_ref = -INFINITY;
+        const float sc2 = a.sc * LOG2E;  // scores in log2 units: a weight is one exp2
+        float m_ref = M_NONE;
         f32x16 s2[2];
         {
             h8 kop[8];
@@ -658,7 +663,7 @@ void prefill_attn_rs_kernel(PrefillArgs a) {
                     s2[i & 1] = mfma3232(kop[i], qb[i], i < 2 ? zero16 : s2[i & 1]);
 #pragma unroll
                     for (int e = 2 * i; e < 2 * i + 2; e++) {  // key k0 + 8 (e / 4) + 4 hh + e % 4
-                        sc[e] = (mb >> (8 * (e >> 2) + (e & 3))) & 1u ? sc[e] * a.sc : -INFINITY;
+                        sc[e] = (mb >> (8 * (e >> 2) + (e & 3))) & 1u ? sc[e] * sc2 : -INFINITY;
                         lmax = fmaxf(lmax, sc[e]);
                     }
                 }
@@ -671,7 +676,7 @@ void prefill_attn_rs_kernel(PrefillArgs a) {
                 const float rmax = fmaxf(lmax, __shfl_xor(lmax, 32, 64));
                 const float m_new = fmaxf(m_ref, rmax);
                 if (m_new > m_ref) {
-                    fac = __expf(m_ref - m_new);  // 0 when m_ref = -inf (the sums are still 0)
+                    fac = __builtin_amdgcn_exp2f(m_ref - m_new);  // 0 from M_NONE (the sums are still 0)
                     m_ref = m_new;
                 }
             }
@@ -730,7 +735,7 @@ void prefill_attn_rs_kernel(PrefillArgs a) {
             }
         };
         // O^T += V^T P^T for tile u: 8 tiles of 32 dims x 2 K-steps of 16 keys
-        float l_part = 0.0f, m_last = -INFINITY;
+        float l_part = 0.0f, m_last = M_NONE;
         auto pv_tile = [&](int u) {
             const int cur = u % NKB;
             // the tile's V^T operands first: their LDS latency runs under the
@@ -757,7 +762,7 @@ void prefill_attn_rs_kernel(PrefillArgs a) {
             }
             float p[16];
 #pragma unroll
-            for (int e = 0; e < 16; e++) p[e] = sc[e] == -INFINITY ? 0.0f : __expf(sc[e] - mf.x);
+            for (int e = 0; e < 16; e++) p[e] = __builtin_amdgcn_exp2f(sc[e] - mf.x);  // 0 where masked
             uint32_t pw[8];
 #pragma unroll
             for (int e = 0; e < 8; e++) {
@@ -793,7 +798,7 @@ void prefill_attn_rs_kernel(PrefillArgs a) {
         const float l_row = l_part + __shfl_xor(l_part, 32, 64);
         // ---- row ln: the output, or its partial triple (dims 32 t + 8 j + 4 hh + c)
         const bool direct = bk.n_split == 1 && a.out;
-        const bool empty = m_last == -INFINITY;
+        const bool empty = m_last == M_NONE;
         const float f = empty ? 0.0f : (direct ? 1.0f / (l_row + a.eps) : 1.0f);
 #pragma unroll
         for (int t2 = 0; t2 < 8; t2++)
@@ -802,7 +807,7 @@ void prefill_attn_rs_kernel(PrefillArgs a) {
                 *reinterpret_cast<f4*>(&lds.out[rg][ln][32 * t2 + 8 * j + 4 * hh]) =
                     f4{acc[t2][4 * j], acc[t2][4 * j + 1], acc[t2][4 * j + 2], acc[t2][4 * j + 3]} * f;
         wave_sync();
-        store_rows<32>(a, &lds.out[rg][0][0], row0, h, split, direct, empty ? -1e20f : m_last,
+        store_rows<32>(a, &lds.out[rg][0][0], row0, h, split, direct, empty ? -1e20f : m_last * LN2,
                        empty ? 0.0f : l_row, lane);
     }
 }
