@@ -251,6 +251,12 @@ struct BlockKeys {
         const int per = (n + n_split - 1) / n_split;
         t_lo = min(n, split * per);
         t_hi = min(n, t_lo + per);
+        // the divisions run on the vector ALU: back to scalars
+        nd = __builtin_amdgcn_readfirstlane(nd);
+        u0 = __builtin_amdgcn_readfirstlane(u0);
+        t_lo = __builtin_amdgcn_readfirstlane(t_lo);
+        t_hi = __builtin_amdgcn_readfirstlane(t_hi);
+        n_split = __builtin_amdgcn_readfirstlane(n_split);
     }
     __device__ __forceinline__ bool dec(int t) const { return t < nd; }
     __device__ __forceinline__ int base(int t) const { return 32 * (t < nd ? t : u0 + t - nd); }
@@ -265,6 +271,9 @@ struct BlockPos {
         b /= a.n_split;
         h = b % a.h_kv;
         bx = n_blk - 1 - b / a.h_kv;
+        bx = __builtin_amdgcn_readfirstlane(bx);
+        h = __builtin_amdgcn_readfirstlane(h);
+        split = __builtin_amdgcn_readfirstlane(split);
     }
 };
 
@@ -653,16 +662,28 @@ void prefill_attn_rs_kernel(PrefillArgs a) {
             for (int e = 0; e < 16; e++) sc[e] = s2[0][e] + s2[1][e];
             h8 kop[8];
             kread(nxt, 0, kop);
-            // ---- S(t + 1), first half, under the mask and row maximum of tile t
+            // ---- S(t + 1), first half, under the scaling, mask and row maximum
+            // of tile t; a tile every row of the wavefront sees whole (all but
+            // the last few of a block) skips the mask
             float lmax = -INFINITY;
-            {
-                const uint32_t mb =
-                    vis.tile(bk.dec(bk.t_lo + t), bk.base(bk.t_lo + t)) >> (4 * hh);
+            const uint32_t mask = vis.tile(bk.dec(bk.t_lo + t), bk.base(bk.t_lo + t));
+            if (__ballot(mask != ~0u) == 0ull) {
 #pragma unroll
                 for (int i = 0; i < 8; i++) {
                     s2[i & 1] = mfma3232(kop[i], qb[i], i < 2 ? zero16 : s2[i & 1]);
 #pragma unroll
-                    for (int e = 2 * i; e < 2 * i + 2; e++) {  // key k0 + 8 (e / 4) + 4 hh + e % 4
+                    for (int e = 2 * i; e < 2 * i + 2; e++) {
+                        sc[e] *= sc2;
+                        lmax = fmaxf(lmax, sc[e]);
+                    }
+                }
+            } else {
+                const uint32_t mb = mask >> (4 * hh);
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    s2[i & 1] = mfma3232(kop[i], qb[i], i < 2 ? zero16 : s2[i & 1]);
+#pragma unroll
+                    for (int e = 2 * i; e < 2 * i + 2; e++) {  // key 8 (e / 4) + 4 hh + e % 4
                         sc[e] = (mb >> (8 * (e >> 2) + (e & 3))) & 1u ? sc[e] * sc2 : -INFINITY;
                         lmax = fmaxf(lmax, sc[e]);
                     }
