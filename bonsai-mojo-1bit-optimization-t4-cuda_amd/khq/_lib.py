@@ -11,6 +11,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import struct
 
 from .build import LIB_PATH
 
@@ -81,6 +82,12 @@ class KhqSeq(ctypes.Structure):
         (n, I) for n in ("c_len", "win_start", "win_len", "ring_cap")]
 
 
+# the same layout for struct.pack_into: filling a KhqSeq field by field takes
+# 3 us a sequence
+SEQ_STRUCT = struct.Struct("=12Q4i")
+assert SEQ_STRUCT.size == ctypes.sizeof(KhqSeq)
+
+
 class KhqError(RuntimeError):
     """A launcher returned a nonzero code (-100 bad shape, -101 missing
     split buffer, > 0 a hipError_t)."""
@@ -117,12 +124,14 @@ def ptr(t) -> int | None:
 def stream_handle(stream=None) -> int | None:
     import torch
 
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return s.cuda_stream or None
+    if stream is not None:
+        return stream.cuda_stream or None
+    # the raw handle: a torch.cuda.Stream object per call costs about a microsecond
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()) or None
 
 
 def call(name: str, *args, check: bool = True) -> int:
-    rc = getattr(lib(), name)(*args)
+    rc = getattr(_lib or lib(), name)(*args)
     if check and rc != 0:
         raise KhqError(name, rc)
     return rc

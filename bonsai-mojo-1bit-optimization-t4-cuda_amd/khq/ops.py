@@ -19,6 +19,9 @@ ROW_BYTES = 220
 
 
 def _need(t: torch.Tensor, dtype, numel: int | None = None, name: str = "tensor"):
+    if (isinstance(t, torch.Tensor) and t.is_cuda and t.dtype == dtype and t.is_contiguous()
+            and (numel is None or t.numel() >= numel)):
+        return
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name}: expected a torch.Tensor")
     if not t.is_cuda:
@@ -195,21 +198,23 @@ def attn_step_batched(seqs, cents: Centroids, *, H_q: int, H_kv: int, scale: flo
     """khq_attn_step_batched_fp16 over a list of per-sequence dicts with keys
     q_gate, pay (Payload), ring_k, ring_v, out, c_len, win_start, win_len,
     ring_cap: every sequence's attention step in one library call."""
-    arr = (_lib.KhqSeq * len(seqs))()
+    f16, size = torch.float16, _lib.SEQ_STRUCT.size
+    buf = ctypes.create_string_buffer(max(1, len(seqs)) * size)
+    pack = _lib.SEQ_STRUCT.pack_into
     for i, s in enumerate(seqs):
-        pay = s["pay"]
-        _need(s["q_gate"], torch.float16, H_q * 2 * D, "q_gate")
-        _need(s["out"], torch.float16, H_q * D, "out")
-        if s["c_len"] * H_kv > pay.rows:
+        pay, q, out, rk, rv = s["pay"], s["q_gate"], s["out"], s["ring_k"], s["ring_v"]
+        c_len, win_len, cap = s["c_len"], s["win_len"], s["ring_cap"]
+        _need(q, f16, H_q * 2 * D, "q_gate")
+        _need(out, f16, H_q * D, "out")
+        if c_len * H_kv > pay.rows:
             raise ValueError("c_len exceeds payload rows")
-        if s["win_len"] > 0:
-            _need(s["ring_k"], torch.float16, s["ring_cap"] * H_kv * D, "ring_k")
-            _need(s["ring_v"], torch.float16, s["ring_cap"] * H_kv * D, "ring_v")
-        arr[i] = _lib.KhqSeq(ptr(s["q_gate"]), ptr(pay.kpay), ptr(pay.vpay), ptr(pay.vsm),
-                             ptr(pay.kmask), ptr(pay.knorm), ptr(pay.krn), ptr(pay.vnorm),
-                             ptr(pay.vrn), ptr(s["ring_k"]), ptr(s["ring_v"]), ptr(s["out"]),
-                             s["c_len"], s["win_start"], s["win_len"], s["ring_cap"])
-    return call("khq_attn_step_batched_fp16", ctypes.cast(arr, ctypes.c_void_p), len(seqs), ptr(cents.cents_k),
+        if win_len > 0:
+            _need(rk, f16, cap * H_kv * D, "ring_k")
+            _need(rv, f16, cap * H_kv * D, "ring_v")
+        pack(buf, i * size, q.data_ptr(), ptr(pay.kpay), ptr(pay.vpay), ptr(pay.vsm),
+             ptr(pay.kmask), ptr(pay.knorm), ptr(pay.krn), ptr(pay.vnorm), ptr(pay.vrn),
+             ptr(rk) or 0, ptr(rv) or 0, out.data_ptr(), c_len, s["win_start"], win_len, cap)
+    return call("khq_attn_step_batched_fp16", ctypes.addressof(buf), len(seqs), ptr(cents.cents_k),
                 ptr(cents.cents_v), ptr(cents.vq), ptr(cents.rotor_k), ptr(cents.rotor_v),
                 ptr(cents.d_k), ptr(cents.d_v), H_q, H_kv, scale, cents.alpha_k, cents.alpha_v,
                 rope_base, stream_handle(stream), check=check)
