@@ -333,10 +333,9 @@ int launch_khq_attn_fp16(const void* q, const void* k_payload, const void* v_pay
         a.split_subs = subs;
         e = khq::launch_attn_ws(a, tpc, nch, stream);
         if (e != hipSuccess) return rc_of(e);
-        if (subs > 1) {
-            e = khq::launch_lse_reduce(part, outp, num_queries * num_splits, subs, stream);
-            if (e != hipSuccess) return rc_of(e);
-        }
+        if (subs > 1)
+            return rc_of(khq::launch_split_reduce(part, outp, static_cast<float*>(out_attn),
+                                                  num_queries, num_splits, subs, stream));
         return rc_of(khq::launch_lse_reduce(outp, static_cast<float*>(out_attn), num_queries,
                                             num_splits, stream));
     }

@@ -123,6 +123,9 @@ hipError_t launch_attn_parts(const AttnArgs& a, int n_rep, dim3 grid, hipStream_
 hipError_t launch_window_parts(const WinArgs& a, int n_rep, int h_kv, int waves, hipStream_t st);
 hipError_t launch_lse_reduce(const float* part, float* out, int n_q, int n_parts,
                              hipStream_t st);
+// subs chunk triples per split -> split triples -> their merge (splits * subs <= 256).
+hipError_t launch_split_reduce(const float* part, float* out_partial, float* out, int n_q,
+                               int splits, int subs, hipStream_t st);
 hipError_t launch_combine_gate(const float* part, const __half* q_gate, __half* out, int H_q,
                                int n_parts, float eps, hipStream_t st);
 hipError_t launch_merge_gate(const float* ac, const float* aw, const __half* qg, __half* out,

@@ -557,6 +557,78 @@ __global__ __launch_bounds__(256) void lse_reduce_kernel(const float* __restrict
     }
 }
 
+// Both merges of a split partition in one launch: the subs chunk triples of each
+// split into out_partial [query][split], and those into out [query].  Block
+// (query, 64-dim slice) of 8 groups of 64 threads: the weights of all chunks
+// (n = splits * subs <= 256) are formed in LDS, then group g sums the chunks of
+// splits g, g + 8, ... , 16 rows in flight.  16 splits of 15 chunks at 12K
+// tokens: 4.2 us a launch twice -> 5.8 us once (bound by two round trips
+// to triples that have just been written).
+__global__ __launch_bounds__(512) void split_reduce_kernel(const float* __restrict__ part,
+                                                          float* __restrict__ out_partial,
+                                                          float* __restrict__ out, int splits,
+                                                          int subs) {
+    __shared__ float s_m[256], s_w[256], s_lw[256], s_M[256], s_f[256], s_D[256], s_acc[512];
+    const int t = threadIdx.x, g = t >> 6, d = blockIdx.y * 64 + (t & 63), n = splits * subs;
+    const size_t q = blockIdx.x;
+    const float* base = part + q * n * 258;
+    float m = 0.0f, l = 0.0f;
+    if (t < n) {
+        m = base[(size_t)t * 258 + 256];
+        l = base[(size_t)t * 258 + 257];
+        s_m[t] = m;
+    }
+    __syncthreads();
+    if (t < n) {
+        float M = -1e20f;
+        for (int u = 0, c = t / subs * subs; u < subs; u++) M = fmaxf(M, s_m[c + u]);
+        const float w = expf(m - M);
+        s_w[t] = w;
+        s_lw[t] = l * w;
+        if (t % subs == 0) s_M[t / subs] = M;
+    }
+    __syncthreads();
+    if (t < splits) {
+        float M = -1e20f, D = 0.0f;
+        for (int i = 0; i < splits; i++) M = fmaxf(M, s_M[i]);
+        for (int u = 0; u < subs; u++) D += s_lw[t * subs + u];
+        s_f[t] = expf(s_M[t] - M);
+        s_D[t] = D;
+        if (blockIdx.y == 0) {
+            float* o = out_partial + (q * splits + t) * 258;
+            o[256] = s_M[t];
+            o[257] = D;
+            if (t == 0) out[q * 258 + 256] = M;
+        }
+    }
+    __syncthreads();
+    float tot = 0.0f;
+    for (int sp = g; sp < splits; sp += 8) {
+        const float* row = base + (size_t)sp * subs * 258 + d;
+        float num = 0.0f;
+        for (int u0 = 0; u0 < subs; u0 += 16) {
+            float v[16];
+#pragma unroll
+            for (int u = 0; u < 16; u++) v[u] = row[(size_t)min(u0 + u, subs - 1) * 258];
+#pragma unroll
+            for (int u = 0; u < 16; u++)
+                if (u0 + u < subs) num = fmaf(v[u], s_w[sp * subs + u0 + u], num);
+        }
+        out_partial[(q * splits + sp) * 258 + d] = num;
+        tot = fmaf(num, s_f[sp], tot);
+    }
+    s_acc[t] = tot;
+    __syncthreads();
+    if (t < 64) {
+        for (int i = 1; i < 8; i++) tot += s_acc[64 * i + t];
+        out[q * 258 + d] = tot;
+    } else if (t == 64 && blockIdx.y == 0) {
+        float den = 0.0f;
+        for (int i = 0; i < splits; i++) den = fmaf(s_D[i], s_f[i], den);
+        out[q * 258 + 257] = den;
+    }
+}
+
 // Final merge of all parts of one head + normalise + sigmoid gate -> f16.
 __global__ __launch_bounds__(256) void combine_gate_kernel(const float* __restrict__ part,
                                                           const __half* __restrict__ q_gate,
@@ -759,6 +831,14 @@ hipError_t launch_lse_reduce(const float* part, float* out, int n_q, int n_parts
                              hipStream_t st) {
     if (n_parts > kMaxParts) return hipErrorInvalidValue;
     hipLaunchKernelGGL(lse_reduce_kernel, dim3(n_q, 4), dim3(256), 0, st, part, out, n_parts);
+    return hipGetLastError();
+}
+
+hipError_t launch_split_reduce(const float* part, float* out_partial, float* out, int n_q,
+                               int splits, int subs, hipStream_t st) {
+    if (splits * subs > 256) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(split_reduce_kernel, dim3(n_q, 4), dim3(512), 0, st, part, out_partial, out,
+                       splits, subs);
     return hipGetLastError();
 }
 
