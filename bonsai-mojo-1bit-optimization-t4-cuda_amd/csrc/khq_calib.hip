@@ -96,22 +96,6 @@ __global__ void rotate_kernel(const float* __restrict__ in, const float* __restr
     *reinterpret_cast<float4*>(out + i * 4) = o;
 }
 
-// inverse rotation back to the FWHT domain: dst[p][c] = sum_k src[p][k] rp[16p + 4c + k]
-__global__ void invrot_kernel(const float* __restrict__ src, const float* __restrict__ rp,
-                              float* __restrict__ dst, int rows) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (long)rows * NP) return;
-    const int p = (int)(i & 63);
-    const float4 v = *reinterpret_cast<const float4*>(src + i * 4);
-    const float* R = rp + p * 16;
-    float4 o;
-    o.x = v.x * R[0] + v.y * R[1] + v.z * R[2] + v.w * R[3];
-    o.y = v.x * R[4] + v.y * R[5] + v.z * R[6] + v.w * R[7];
-    o.z = v.x * R[8] + v.y * R[9] + v.z * R[10] + v.w * R[11];
-    o.w = v.x * R[12] + v.y * R[13] + v.z * R[14] + v.w * R[15];
-    *reinterpret_cast<float4*>(dst + i * 4) = o;
-}
-
 // ---- per-dim column statistics over rows (double accumulators)
 // acc[0][d] += x, acc[1][d] += |x|, acc[2][d] += (x - mean[d])^2 (pass 2)
 __global__ __launch_bounds__(256) void colsum_kernel(const float* __restrict__ x, int rows,
@@ -657,66 +641,6 @@ __global__ __launch_bounds__(256) void vq_hard_kernel(const float* __restrict__ 
     r[2] = c.z;
 }
 
-// dim 3 of rec: round half to even of rot * 16, / 16
-__global__ void dim3_kernel(const float* __restrict__ rot, float* __restrict__ rec, int rows) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (long)rows * NP) return;
-    rec[i * 4 + 3] = rintf(rot[i * 4 + 3] * 16.0f) / 16.0f;
-}
-
-// va = rec A (N x 8); dlt = rec + va B - v.  One wavefront per row.
-__global__ __launch_bounds__(256) void wtrm_fwd_kernel(const float* __restrict__ rec,
-                                                       const float* __restrict__ wa,
-                                                       const float* __restrict__ wb,
-                                                       const float* __restrict__ v,
-                                                       float* __restrict__ dlt, int rows) {
-    const int lane = threadIdx.x & 63;
-    const long n = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (n >= rows) return;
-    const float4 x = *reinterpret_cast<const float4*>(rec + n * D + 4 * lane);
-    const float xs[4] = {x.x, x.y, x.z, x.w};
-    float va[8];
-    for (int r = 0; r < 8; r++) {
-        float s = 0.0f;
-        for (int j = 0; j < 4; j++) s += xs[j] * wa[(4 * lane + j) * 8 + r];
-        va[r] = wsum(s);
-    }
-    const float4 vv = *reinterpret_cast<const float4*>(v + n * D + 4 * lane);
-    const float vs[4] = {vv.x, vv.y, vv.z, vv.w};
-    float o[4];
-    for (int j = 0; j < 4; j++) {
-        float s = xs[j];
-        for (int r = 0; r < 8; r++) s += va[r] * wb[r * D + 4 * lane + j];
-        o[j] = s - vs[j];
-    }
-    *reinterpret_cast<float4*>(dlt + n * D + 4 * lane) = make_float4(o[0], o[1], o[2], o[3]);
-}
-
-// grec = g + (g B^T) A^T per row (g = gradient w.r.t. dlt).  One wavefront per row.
-__global__ __launch_bounds__(256) void wtrm_bwd_kernel(const float* __restrict__ g,
-                                                       const float* __restrict__ wa,
-                                                       const float* __restrict__ wb,
-                                                       float* __restrict__ grec, int rows) {
-    const int lane = threadIdx.x & 63;
-    const long n = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (n >= rows) return;
-    const float4 x = *reinterpret_cast<const float4*>(g + n * D + 4 * lane);
-    const float xs[4] = {x.x, x.y, x.z, x.w};
-    float gb[8];
-    for (int r = 0; r < 8; r++) {
-        float s = 0.0f;
-        for (int j = 0; j < 4; j++) s += xs[j] * wb[r * D + 4 * lane + j];
-        gb[r] = wsum(s);
-    }
-    float o[4];
-    for (int j = 0; j < 4; j++) {
-        float s = xs[j];
-        for (int r = 0; r < 8; r++) s += gb[r] * wa[(4 * lane + j) * 8 + r];
-        o[j] = s;
-    }
-    *reinterpret_cast<float4*>(grec + n * D + 4 * lane) = make_float4(o[0], o[1], o[2], o[3]);
-}
-
 // C[b] (M x N) = alpha * op(A[b]) B[b]; row-major B (K x N, ldb) and C (ldc);
 // op(A) = A (M x K, lda) or A^T (A stored K x M, lda).
 // fp32 MFMA 32x32x2: a block owns a 64 x 64 tile, each of its four wavefronts a
@@ -822,38 +746,6 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const float* __restric
     out[i] = alpha * s;
 }
 
-// sum of squares (or of (a - b)^2, and the gradient 2 (a - b) / n) into a double
-__global__ __launch_bounds__(256) void sumsq_kernel(const float* __restrict__ a,
-                                                    const float* __restrict__ b,
-                                                    float* __restrict__ grad, long n, float gscale,
-                                                    double* __restrict__ out, int square) {
-    __shared__ double s[256];
-    double acc = 0.0;
-    for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long)gridDim.x * 256) {
-        const float df = b ? a[i] - b[i] : a[i];
-        acc += square ? (double)df * df : (double)df;
-        if (grad) grad[i] = gscale * df;
-    }
-    s[threadIdx.x] = acc;
-    __syncthreads();
-    for (int o = 128; o >= 1; o >>= 1) {
-        if (threadIdx.x < o) s[threadIdx.x] += s[threadIdx.x + o];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) atomicAdd(out, s[0]);
-}
-
-// gq[n][p][c] = sum_{d < 3} grec[n][4p + d] rp[16p + 4d + c], c < 3 (ref .cu:2300-2314)
-__global__ void rotbwd_kernel(const float* __restrict__ grec, const float* __restrict__ rp,
-                              float* __restrict__ gq, int rows) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (long)rows * NP) return;
-    const int p = (int)(i & 63);
-    const float* g = grec + i * 4;
-    for (int c = 0; c < 3; c++)
-        gq[i * 3 + c] = g[0] * rp[p * 16 + c] + g[1] * rp[p * 16 + 4 + c] + g[2] * rp[p * 16 + 8 + c];
-}
-
 // Codebook gradient (ref .cu:2339-2371) with w_k = softmax(-|v - c_k|^2 / temp)
 // and swg = sum_k w_k (gq . c_k): for every row
 //   gC[k] += w_k gq + (-w_k (gq . c_k - swg) / temp) * 2 (c_k - v)
@@ -936,34 +828,174 @@ __global__ __launch_bounds__(256) void soft_grad_kernel(const float* __restrict_
     o[2] = a2;
 }
 
-// gA = gW B^T (256 x 8), gB = A^T gW (8 x 256)
-__global__ void gwab_kernel(const float* __restrict__ gw, const float* __restrict__ wa,
-                            const float* __restrict__ wb, float* __restrict__ gwa,
-                            float* __restrict__ gwb) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < 2048) {
-        const int j = i >> 3, r = i & 7;
-        float s = 0.0f;
-        for (int d = 0; d < D; d++) s += gw[j * D + d] * wb[r * D + d];
-        gwa[i] = s;
-    } else if (i < 4096) {
-        const int r = (i - 2048) >> 8, d = (i - 2048) & 255;
-        float s = 0.0f;
-        for (int j = 0; j < D; j++) s += wa[j * 8 + r] * gw[j * D + d];
-        gwb[i - 2048] = s;
+// Row passes of one SmartVQ step, one wavefront per row, lane p = patch p (dims
+// 4 p .. 4 p + 3): each is bound by reading and writing its rows once (2 MB
+// arrays at 2048 rows), so what was six launches of 4 to 5 us (dim 3, inverse
+// rotation, transform forward and backward, rotation backward, dictionary sum)
+// is two.
+constexpr int ROWS_PER_BLOCK = 8;
+
+__device__ __forceinline__ void add_loss(double x, double* out) {  // block sum, one atomic
+    __shared__ double s_x[4];
+    for (int o = 32; o >= 1; o >>= 1) x += __shfl_xor(x, o, 64);
+    if ((threadIdx.x & 63) == 0) s_x[threadIdx.x >> 6] = x;
+    __syncthreads();
+    if (threadIdx.x == 0) atomicAdd(out, (s_x[0] + s_x[1]) + (s_x[2] + s_x[3]));
+    __syncthreads();
+}
+
+// Forward of a row: rec = (codeword, dim 3 rounded half to even to 1 / 16),
+// recf = its inverse rotation.  attn: va = recf A (8), dlt = recf + va B - v.
+// Otherwise the reconstruction loss, and with grad its gradient through the
+// rotation: gq[c] = sum_{d < 3} grec[d] rp[4 d + c], c < 3, grec = gscale
+// (recf - v) (ref .cu:2300-2314).
+__global__ __launch_bounds__(256) void svq_fwd_kernel(
+    const float* __restrict__ rot, const float* __restrict__ rec3, const float* __restrict__ dict,
+    const float* __restrict__ rp, const float* __restrict__ wa, const float* __restrict__ wb,
+    const float* __restrict__ v, float* __restrict__ recf, float* __restrict__ va_out,
+    float* __restrict__ dlt, float* __restrict__ gq, int rows, int attn, int grad, float gscale,
+    double* __restrict__ loss) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    float R[16];
+#pragma unroll
+    for (int i = 0; i < 16; i++) R[i] = rp[lane * 16 + i];
+    double sum = 0.0, dsum = 0.0;
+    for (int i = wave; i < ROWS_PER_BLOCK; i += 4) {
+        const long n = (long)blockIdx.x * ROWS_PER_BLOCK + i;
+        if (n >= rows) break;  // uniform per wavefront
+        const long at = n * D + 4 * lane;
+        const float4 q = *reinterpret_cast<const float4*>(rec3 + at);
+        const float w = rintf(rot[at + 3] * 16.0f) / 16.0f;
+        dsum += (double)dict[n * NP + lane];
+        float xs[4];
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+            xs[c] = q.x * R[4 * c] + q.y * R[4 * c + 1] + q.z * R[4 * c + 2] + w * R[4 * c + 3];
+        const float4 vv = *reinterpret_cast<const float4*>(v + at);
+        const float vs[4] = {vv.x, vv.y, vv.z, vv.w};
+        if (!attn) {
+            float g[4];
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                const float df = xs[c] - vs[c];
+                sum += (double)df * df;
+                g[c] = gscale * df;
+            }
+            if (grad)
+#pragma unroll
+                for (int c = 0; c < 3; c++)
+                    gq[(n * NP + lane) * 3 + c] = g[0] * R[c] + g[1] * R[4 + c] + g[2] * R[8 + c];
+            continue;
+        }
+        float va[8], o[4] = {xs[0], xs[1], xs[2], xs[3]};
+#pragma unroll
+        for (int r = 0; r < 8; r++) {
+            float x = 0.0f;
+#pragma unroll
+            for (int j = 0; j < 4; j++) x += xs[j] * wa[(4 * lane + j) * 8 + r];
+            va[r] = wsum(x);
+        }
+#pragma unroll
+        for (int r = 0; r < 8; r++) {
+            const float4 b = *reinterpret_cast<const float4*>(wb + r * D + 4 * lane);
+            o[0] += va[r] * b.x;
+            o[1] += va[r] * b.y;
+            o[2] += va[r] * b.z;
+            o[3] += va[r] * b.w;
+        }
+        *reinterpret_cast<float4*>(recf + at) = make_float4(xs[0], xs[1], xs[2], xs[3]);
+        *reinterpret_cast<float4*>(dlt + at) =
+            make_float4(o[0] - vs[0], o[1] - vs[1], o[2] - vs[2], o[3] - vs[3]);
+        if (lane == 0)
+#pragma unroll
+            for (int r = 0; r < 8; r++) va_out[n * 8 + r] = va[r];
+    }
+    add_loss(dsum, loss + 1);
+    if (!attn) add_loss(sum, loss);
+}
+
+// Backward of a row in attention mode, from gd = sum_h A_h^T A_h dlt: with
+// quad, the loss term dlt . gd (= sum_h |A_h dlt|^2 over the rows); with grad,
+// g = gscale gd, gb = g B^T (8), grec = g + gb A^T, gq as above.
+__global__ __launch_bounds__(256) void svq_bwd_kernel(
+    const float* __restrict__ gd, const float* __restrict__ dlt, const float* __restrict__ rp,
+    const float* __restrict__ wa, const float* __restrict__ wb, float* __restrict__ gb_out,
+    float* __restrict__ gq, int rows, int quad, int grad, float gscale, double* __restrict__ loss) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    double sum = 0.0;
+    for (int i = wave; i < ROWS_PER_BLOCK; i += 4) {
+        const long n = (long)blockIdx.x * ROWS_PER_BLOCK + i;
+        if (n >= rows) break;  // uniform per wavefront
+        const long at = n * D + 4 * lane;
+        const float4 x = *reinterpret_cast<const float4*>(gd + at);
+        if (quad) {
+            const float4 y = *reinterpret_cast<const float4*>(dlt + at);
+            sum += ((double)x.x * y.x + (double)x.y * y.y) + ((double)x.z * y.z + (double)x.w * y.w);
+        }
+        if (!grad) continue;
+        const float xs[4] = {gscale * x.x, gscale * x.y, gscale * x.z, gscale * x.w};
+        float gb[8], o[4] = {xs[0], xs[1], xs[2], xs[3]};
+#pragma unroll
+        for (int r = 0; r < 8; r++) {
+            const float4 b = *reinterpret_cast<const float4*>(wb + r * D + 4 * lane);
+            gb[r] = wsum(xs[0] * b.x + xs[1] * b.y + xs[2] * b.z + xs[3] * b.w);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int r = 0; r < 8; r++) o[j] += gb[r] * wa[(4 * lane + j) * 8 + r];
+#pragma unroll
+        for (int c = 0; c < 3; c++)
+            gq[(n * NP + lane) * 3 + c] =
+                o[0] * rp[lane * 16 + c] + o[1] * rp[lane * 16 + 4 + c] + o[2] * rp[lane * 16 + 8 + c];
+        if (lane == 0)
+#pragma unroll
+            for (int r = 0; r < 8; r++) gb_out[n * 8 + r] = gb[r];
+    }
+    if (quad) add_loss(sum, loss);
+}
+
+// Transform gradients from the rank-8 row factors, gA[j][r] = sum_n recf[n][j]
+// gb[n][r] and gB[r][d] = sum_n va[n][r] g[n][d]: the 256 x 256 product recf^T g
+// that they factor (11 us and two more launches) is never formed.  Thread j of
+// block b sums its range of rows into part[b][4096].
+__global__ __launch_bounds__(256) void gwab_kernel(const float* __restrict__ recf,
+                                                   const float* __restrict__ gd,
+                                                   const float* __restrict__ va,
+                                                   const float* __restrict__ gb, float gscale,
+                                                   float* __restrict__ part, int rows, int per) {
+    const int j = threadIdx.x;
+    const int lo = blockIdx.x * per, hi = min(rows, lo + per);
+    float a[8] = {}, b[8] = {};
+#pragma unroll 4
+    for (int n = lo; n < hi; n++) {
+        const float x = recf[(long)n * D + j], g = gscale * gd[(long)n * D + j];
+#pragma unroll
+        for (int r = 0; r < 8; r++) {
+            a[r] = fmaf(x, gb[(long)n * 8 + r], a[r]);
+            b[r] = fmaf(g, va[(long)n * 8 + r], b[r]);
+        }
+    }
+    float* o = part + (long)blockIdx.x * 4096;
+#pragma unroll
+    for (int r = 0; r < 8; r++) {
+        o[j * 8 + r] = a[r];
+        o[2048 + r * D + j] = b[r];
     }
 }
 
-// Adam with bias correction (ref .cu:2373-2385)
+// Adam with bias correction (ref .cu:2373-2385): parameters [0, CB) at rate lr
+// (the codebook), the rest (the transform) at 5 % of it.
 __global__ void adam_kernel(float* __restrict__ p, const float* __restrict__ g,
                             float* __restrict__ m, float* __restrict__ v, float lr, float bc1,
                             float bc2, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
+    const float rate = i < CB ? lr : lr * 0.05f;
     const float gi = g[i];
     m[i] = 0.9f * m[i] + 0.1f * gi;
     v[i] = 0.999f * v[i] + 0.001f * gi * gi;
-    p[i] -= lr * (m[i] / bc1) / (sqrtf(v[i] / bc2) + 1e-8f);
+    p[i] -= rate * (m[i] / bc1) / (sqrtf(v[i] / bc2) + 1e-8f);
 }
 
 // p = base + N(0,1) * scale, one Box-Muller draw from a per-entry xorshift
@@ -1139,32 +1171,42 @@ int tournament(bool is_k, const float* x32, const float* x16, const float* dv, c
 
 
 // ---------------------------------------------------------- SmartVQ host
+// Parameters of a seed, one block each: codebook [64][256][3], A [256][8],
+// B [8][256] (gradients and moments alike).
+constexpr int NPAR = CB + 4096;
 struct Seed {
-    Buf cb, wa, wb, mcb, vcb, mwa, vwa, mwb, vwb, bcb, bwa, bwb;
+    Buf buf;  // parameters, moments m and v, best parameters
+    float *par = nullptr, *m = nullptr, *v = nullptr, *best_par = nullptr;
     float best = 0.0f, lr_mult = 1.0f;
     int stagnant = 0, step = 0;
     unsigned seed = 0;
+    int alloc() {
+        CAL_TRY(buf.alloc(4 * NPAR * sizeof(float)));
+        par = buf.as<float>();
+        m = par + NPAR;
+        v = m + NPAR;
+        best_par = v + NPAR;
+        return 0;
+    }
+    float* cb() const { return par; }
+    float* wa() const { return par + CB; }
+    float* wb() const { return par + CB + 2048; }
     int init(const float* init_cb, unsigned sd, hipStream_t st) {
-        for (Buf* b : {&cb, &mcb, &vcb, &bcb}) CAL_TRY(b->alloc(CB * 4));
-        for (Buf* b : {&wa, &wb, &mwa, &vwa, &mwb, &vwb, &bwa, &bwb}) CAL_TRY(b->alloc(2048 * 4));
-        for (Buf* b : {&mcb, &vcb}) CAL_TRY(hipMemsetAsync(b->p, 0, CB * 4, st));
-        for (Buf* b : {&wa, &wb, &mwa, &vwa, &mwb, &vwb}) CAL_TRY(hipMemsetAsync(b->p, 0, 2048 * 4, st));
+        int rc = alloc();
+        if (rc) return rc;
+        CAL_TRY(hipMemsetAsync(wa(), 0, (4096 + 2 * NPAR) * 4, st));
         // A ~ N(0, 1) / 16, B = 0 (ref .cu:4503-4505)
-        hipLaunchKernelGGL(noise_kernel, dim3(8), dim3(256), 0, st, wa.as<float>(), wa.as<float>(),
+        hipLaunchKernelGGL(noise_kernel, dim3(8), dim3(256), 0, st, wa(), wa(),
                            sd * 2654435761u + 1u, 1.0f / 16.0f, 2048);
-        CAL_TRY(hipMemcpyAsync(cb.p, init_cb, CB * 4, hipMemcpyDeviceToDevice, st));
+        CAL_TRY(hipMemcpyAsync(cb(), init_cb, CB * 4, hipMemcpyDeviceToDevice, st));
         return keep_best(st);
     }
     int keep_best(hipStream_t st) {
-        CAL_TRY(hipMemcpyAsync(bcb.p, cb.p, CB * 4, hipMemcpyDeviceToDevice, st));
-        CAL_TRY(hipMemcpyAsync(bwa.p, wa.p, 2048 * 4, hipMemcpyDeviceToDevice, st));
-        CAL_TRY(hipMemcpyAsync(bwb.p, wb.p, 2048 * 4, hipMemcpyDeviceToDevice, st));
+        CAL_TRY(hipMemcpyAsync(best_par, par, NPAR * 4, hipMemcpyDeviceToDevice, st));
         return 0;
     }
     int restore_best(hipStream_t st) {
-        CAL_TRY(hipMemcpyAsync(cb.p, bcb.p, CB * 4, hipMemcpyDeviceToDevice, st));
-        CAL_TRY(hipMemcpyAsync(wa.p, bwa.p, 2048 * 4, hipMemcpyDeviceToDevice, st));
-        CAL_TRY(hipMemcpyAsync(wb.p, bwb.p, 2048 * 4, hipMemcpyDeviceToDevice, st));
+        CAL_TRY(hipMemcpyAsync(par, best_par, NPAR * 4, hipMemcpyDeviceToDevice, st));
         return 0;
     }
 };
@@ -1175,29 +1217,55 @@ struct Svq {
     const float* rp;    // [64][16]
     int N, T, H_q, H_kv;
     hipStream_t st;
-    Buf rot, rec, recf, dlt, idx, dict, y, gdl, grec, gw, gq, gcb, gwa, gwb, loss, part;
+    int passes;  // passes the caller will run
+    Buf buf, gram_buf;
+    float *rot, *rec, *recf, *dlt, *gd, *va, *gb, *dict, *gq, *grad, *part, *y, *gram;
+    int* idx;
+    double* loss;
+    // Every array from one allocation, the row rotation (the same in every
+    // pass) and, where it pays, the Gram matrices.
     int init() {
-        const size_t nd = (size_t)N * D * 4;
-        for (Buf* b : {&rot, &rec, &recf, &dlt, &grec, &gdl}) CAL_TRY(b->alloc(nd));
-        CAL_TRY(idx.alloc((size_t)N * NP * 4));
-        CAL_TRY(dict.alloc((size_t)N * NP * 4));
-        CAL_TRY(gq.alloc((size_t)N * NP * 3 * 4));
-        CAL_TRY(gw.alloc(D * D * 4));
-        CAL_TRY(gcb.alloc(CB * 4));
-        CAL_TRY(gwa.alloc(2048 * 4));
-        CAL_TRY(gwb.alloc(2048 * 4));
-        CAL_TRY(loss.alloc(2 * sizeof(double)));
+        const size_t nd = (size_t)N * D, np = (size_t)N * NP;
         int kp;
-        size_t np = (size_t)soft_ranges(N, &kp) * CB;
+        use_gram = attn && (long)T <= 512l * passes;
+        size_t n_part = std::max((size_t)soft_ranges(N, &kp) * CB, (size_t)GWAB * 4096);
         if (attn) {
-            CAL_TRY(y.alloc((size_t)H_q * T * D * 4));
-            const size_t p1 = (size_t)gemm_splits(T, D, H_q / H_kv * T, H_kv, &kp) * H_kv * T * D;
-            const size_t p2 = (size_t)gemm_splits(D, D, N, 1, &kp) * D * D;
-            np = std::max({np, p1, p2});
+            n_part = std::max(n_part, (size_t)gemm_splits(T, D, H_q / H_kv * T, H_kv, &kp) * H_kv * T * D);
+            if (use_gram) {
+                n_part = std::max(n_part, (size_t)gemm_splits(T, D, T, H_kv, &kp) * H_kv * T * D);
+                n_part = std::max(n_part, (size_t)gemm_splits(T, T, H_q / H_kv * T, H_kv, &kp) * H_kv * T * T);
+            }
         }
-        CAL_TRY(part.alloc(np * 4));
+        const size_t n_y = attn && !use_gram ? (size_t)H_q * T * D : 0;
+        const size_t n_gram = use_gram ? (size_t)H_kv * T * T : 0;
+        struct {
+            float** p;
+            size_t n;
+        } parts[] = {{&rot, nd}, {&rec, nd}, {&recf, nd}, {&dlt, nd}, {&gd, nd},
+                     {&va, (size_t)N * 8}, {&gb, (size_t)N * 8}, {&dict, np}, {&gq, 3 * np},
+                     {&grad, NPAR}, {&part, n_part}, {&y, n_y}, {&gram, n_gram},
+                     {reinterpret_cast<float**>(&idx), np}, {reinterpret_cast<float**>(&loss), 4}};
+        size_t total = 0;
+        for (auto& x : parts) total += (x.n + 63) / 64 * 64;
+        CAL_TRY(buf.alloc(total * sizeof(float)));
+        float* at = buf.as<float>();
+        for (auto& x : parts) {
+            *x.p = at;
+            at += (x.n + 63) / 64 * 64;
+        }
+        hipLaunchKernelGGL(rotate_kernel, dim3(blocks((long)N * NP, 256)), dim3(256), 0, st, v, rp,
+                           rot, N);
+        if (use_gram)  // gram_kv = sum_h A_h^T A_h, the group's heads stacked along K
+            gemm(attn, attn, gram, T, T, H_q / H_kv * T, T, T, (long)H_q / H_kv * T * T,
+                 (long)H_q / H_kv * T * T, H_kv, 1, 1, 1.0f, nullptr);
         return 0;
     }
+    // The loss and its gradient need only G = sum_h A_h^T A_h of each group:
+    // sum_h |A_h x|^2 = x . G x, and G x is the gradient.  G takes the products
+    // of T / 512 passes over the heads, G x a twelfth of one's.  512 tokens, 24
+    // / 4 heads: 117 us a pass over the heads -> 60 us once and 18 us a pass.
+    bool use_gram = false;
+    static constexpr int GWAB = 128;  // row ranges of the transform gradients
     // Splits of K: enough blocks for four a CU (a block's LDS and registers
     // let four share one and cover each other's barriers), at least 128 of K,
     // four slabs, each, and at most 16 partials to add.  The transform
@@ -1223,7 +1291,7 @@ struct Svq {
                    sumsq};
         if (!sumsq) g.splits = gemm_splits(M, Nn, K, batch, &g.k_per);
         if (g.splits > 1) {
-            g.C = part.as<float>();
+            g.C = part;
             g.alpha = 1.0f;
         }
         hipLaunchKernelGGL(gemm_kernel, dim3((Nn + 63) / 64, (M + 63) / 64, batch * g.splits),
@@ -1231,69 +1299,55 @@ struct Svq {
         if (g.splits > 1) {
             const long n = (long)batch * M * Nn;
             hipLaunchKernelGGL(gemm_reduce_kernel, dim3(blocks(n, 256)), dim3(256), 0, st,
-                               part.as<float>(), C, n, g.splits, alpha);
+                               part, C, n, g.splits, alpha);
         }
     }
     // One pass at temperature temp (ref .cu:2436-2467 forward, :2470-2530
     // with gradients): losses[0] = reconstruction (attention-weighted MSE of
     // the transformed residual, or plain MSE), losses[1] = dict term.
-    int pass(Seed& s, float temp, bool grad, double* losses) {
-        const int n_rep = H_q / H_kv;
-        CAL_TRY(hipMemsetAsync(loss.p, 0, 2 * sizeof(double), st));
-        hipLaunchKernelGGL(rotate_kernel, dim3(blocks((long)N * NP, 256)), dim3(256), 0, st, v, rp,
-                           rot.as<float>(), N);
-        hipLaunchKernelGGL(vq_hard_kernel, dim3(blocks(N, SR), NP), dim3(256), 0, st,
-                           rot.as<float>(), s.cb.as<float>(), rec.as<float>(), idx.as<int>(),
-                           dict.as<float>(), N);
-        hipLaunchKernelGGL(dim3_kernel, dim3(blocks((long)N * NP, 256)), dim3(256), 0, st,
-                           rot.as<float>(), rec.as<float>(), N);
-        hipLaunchKernelGGL(invrot_kernel, dim3(blocks((long)N * NP, 256)), dim3(256), 0, st,
-                           rec.as<float>(), rp, recf.as<float>(), N);
-        const long nd = (long)N * D;
-        double denom = (double)nd;
+    int pass(Seed& s, float temp, bool need_grad, double* losses) {
+        const int n_rep = attn ? H_q / H_kv : 1;
+        const double denom = attn ? (double)H_q * T * D : (double)N * D;
+        const float gscale = 2.0f / (float)denom;
+        const int row_blocks = blocks(N, ROWS_PER_BLOCK);
+        CAL_TRY(hipMemsetAsync(loss, 0, 2 * sizeof(double), st));
+        hipLaunchKernelGGL(vq_hard_kernel, dim3(blocks(N, SR), NP), dim3(256), 0, st, rot, s.cb(), rec,
+                           idx, dict, N);
+        hipLaunchKernelGGL(svq_fwd_kernel, dim3(row_blocks), dim3(256), 0, st, rot, rec, dict, rp,
+                           s.wa(), s.wb(), v, recf, va, dlt, gq, N, attn ? 1 : 0, need_grad ? 1 : 0,
+                           gscale, loss);
         if (attn) {
-            hipLaunchKernelGGL(wtrm_fwd_kernel, dim3(blocks(N, 4)), dim3(256), 0, st,
-                               recf.as<float>(), s.wa.as<float>(), s.wb.as<float>(), v,
-                               dlt.as<float>(), N);
-            const long ny = (long)H_q * T * D;
-            denom = (double)ny;
-            // y_h = A_h dlt_kv, every head in one launch
-            gemm(attn, dlt.as<float>(), y.as<float>(), T, D, T, T, D, (long)T * T, (long)T * D,
-                 H_q, n_rep, 0, 1.0f, loss.as<double>());
-            if (grad) {
-                const float g = 2.0f / (float)ny;
-                // gdlt_kv = g sum_h A_h^T y_h: the group's heads stacked along K
-                gemm(attn, y.as<float>(), gdl.as<float>(), T, D, n_rep * T, T, D,
-                     (long)n_rep * T * T, (long)n_rep * T * D, H_kv, 1, 1, g, nullptr);
-                hipLaunchKernelGGL(wtrm_bwd_kernel, dim3(blocks(N, 4)), dim3(256), 0, st,
-                                   gdl.as<float>(), s.wa.as<float>(), s.wb.as<float>(),
-                                   grec.as<float>(), N);
-                gemm(recf.as<float>(), gdl.as<float>(), gw.as<float>(), D, D, N, D, D, 0, 0, 1, 1, 1,
-                     1.0f, nullptr);  // gW = recf^T gdlt
-                hipLaunchKernelGGL(gwab_kernel, dim3(16), dim3(256), 0, st, gw.as<float>(),
-                                   s.wa.as<float>(), s.wb.as<float>(), gwa.as<float>(),
-                                   gwb.as<float>());
+            if (use_gram) {
+                gemm(gram, dlt, gd, T, D, T, T, D, (long)T * T, (long)T * D, H_kv, 1, 0, 1.0f, nullptr);
+            } else {
+                // y_h = A_h dlt_kv, every head in one launch, then sum_h A_h^T y_h
+                gemm(attn, dlt, y, T, D, T, T, D, (long)T * T, (long)T * D, H_q, n_rep, 0, 1.0f, loss);
+                if (need_grad)
+                    gemm(attn, y, gd, T, D, n_rep * T, T, D, (long)n_rep * T * T, (long)n_rep * T * D,
+                         H_kv, 1, 1, 1.0f, nullptr);
             }
-        } else {
-            hipLaunchKernelGGL(sumsq_kernel, dim3(256), dim3(256), 0, st, recf.as<float>(), v,
-                               grad ? grec.as<float>() : nullptr, nd, 2.0f / (float)nd,
-                               loss.as<double>(), 1);
+            if (use_gram || need_grad)
+                hipLaunchKernelGGL(svq_bwd_kernel, dim3(row_blocks), dim3(256), 0, st, gd, dlt, rp,
+                                   s.wa(), s.wb(), gb, gq, N, use_gram ? 1 : 0, need_grad ? 1 : 0,
+                                   gscale, loss);
+            if (need_grad) {
+                const int per = (N + GWAB - 1) / GWAB, n = (N + per - 1) / per;
+                hipLaunchKernelGGL(gwab_kernel, dim3(n), dim3(256), 0, st, recf, gd, va, gb, gscale,
+                                   part, N, per);
+                hipLaunchKernelGGL(gemm_reduce_kernel, dim3(16), dim3(256), 0, st, part, grad + CB,
+                                   4096l, n, 1.0f);
+            }
         }
-        hipLaunchKernelGGL(sumsq_kernel, dim3(64), dim3(256), 0, st, dict.as<float>(), nullptr,
-                           nullptr, (long)N * NP, 0.0f, loss.as<double>() + 1, 0);
-        if (grad) {
-            hipLaunchKernelGGL(rotbwd_kernel, dim3(blocks((long)N * NP, 256)), dim3(256), 0, st,
-                               grec.as<float>(), rp, gq.as<float>(), N);
+        if (need_grad) {
             int per;
             const int ranges = soft_ranges(N, &per);
-            hipLaunchKernelGGL(soft_grad_kernel, dim3(NP, ranges), dim3(256), 0, st,
-                               rot.as<float>(), s.cb.as<float>(), gq.as<float>(), idx.as<int>(),
-                               part.as<float>(), N, per, temp);
-            hipLaunchKernelGGL(gemm_reduce_kernel, dim3(blocks(CB, 256)), dim3(256), 0, st,
-                               part.as<float>(), gcb.as<float>(), (long)CB, ranges, 1.0f);
+            hipLaunchKernelGGL(soft_grad_kernel, dim3(NP, ranges), dim3(256), 0, st, rot, s.cb(), gq,
+                               idx, part, N, per, temp);
+            hipLaunchKernelGGL(gemm_reduce_kernel, dim3(blocks(CB, 256)), dim3(256), 0, st, part, grad,
+                               (long)CB, ranges, 1.0f);
         }
         double h[2];
-        CAL_TRY(hipMemcpyAsync(h, loss.p, sizeof(h), hipMemcpyDeviceToHost, st));
+        CAL_TRY(hipMemcpyAsync(h, loss, sizeof(h), hipMemcpyDeviceToHost, st));
         CAL_TRY(hipStreamSynchronize(st));
         losses[0] = h[0] / denom;
         losses[1] = h[1] / ((double)N * NP * 3);
@@ -1312,21 +1366,11 @@ struct Svq {
             double l[2];
             int rc = pass(s, temp, true, l);
             if (rc) return rc;
-            if (!attn) {  // no transform gradient without the attention loss
-                CAL_TRY(hipMemsetAsync(gwa.p, 0, 2048 * 4, st));
-                CAL_TRY(hipMemsetAsync(gwb.p, 0, 2048 * 4, st));
-            }
             s.step++;
             const float bc1 = 1.0f - powf(0.9f, (float)s.step), bc2 = 1.0f - powf(0.999f, (float)s.step);
-            hipLaunchKernelGGL(adam_kernel, dim3(blocks(CB, 256)), dim3(256), 0, st, s.cb.as<float>(),
-                               gcb.as<float>(), s.mcb.as<float>(), s.vcb.as<float>(), cur, bc1, bc2,
-                               CB);
-            hipLaunchKernelGGL(adam_kernel, dim3(8), dim3(256), 0, st, s.wa.as<float>(),
-                               gwa.as<float>(), s.mwa.as<float>(), s.vwa.as<float>(), cur * 0.05f,
-                               bc1, bc2, 2048);
-            hipLaunchKernelGGL(adam_kernel, dim3(8), dim3(256), 0, st, s.wb.as<float>(),
-                               gwb.as<float>(), s.mwb.as<float>(), s.vwb.as<float>(), cur * 0.05f,
-                               bc1, bc2, 2048);
+            // (without the attention loss the transform has no gradient)
+            hipLaunchKernelGGL(adam_kernel, dim3(blocks(NPAR, 256)), dim3(256), 0, st, s.par, grad, s.m,
+                               s.v, cur, bc1, bc2, attn ? NPAR : CB);
             // the loss of this step's forward pass (before the update), as the reference
             const float loss = (float)(l[0] + l[1]);
             if (loss < s.best - 1e-7f) {
@@ -1344,10 +1388,8 @@ struct Svq {
                     s.lr_mult = 3.0f;
                     const float ns = 1e-3f * expf(logf(0.01f) * (float)i / (float)max_it);
                     hipLaunchKernelGGL(noise_kernel, dim3(blocks(CB, 256)), dim3(256), 0, st,
-                                       s.bcb.as<float>(), s.cb.as<float>(), s.seed ^ (unsigned)i, ns,
-                                       CB);
-                    CAL_TRY(hipMemcpyAsync(s.wa.p, s.bwa.p, 2048 * 4, hipMemcpyDeviceToDevice, st));
-                    CAL_TRY(hipMemcpyAsync(s.wb.p, s.bwb.p, 2048 * 4, hipMemcpyDeviceToDevice, st));
+                                       s.best_par, s.cb(), s.seed ^ (unsigned)i, ns, CB);
+                    CAL_TRY(hipMemcpyAsync(s.wa(), s.best_par + CB, 4096 * 4, hipMemcpyDeviceToDevice, st));
                 }
                 s.stagnant = 0;
             }
@@ -1500,7 +1542,7 @@ int launch_cal_svq_train(const void* v, const void* attn, const void* init_cb, c
         return -100;
     n_seeds = std::max(1, std::min(3, n_seeds));
     Svq t{static_cast<const float*>(v), static_cast<const float*>(attn),
-          static_cast<const float*>(rp), N, T, H_q, H_kv, st};
+          static_cast<const float*>(rp), N, T, H_q, H_kv, st, n_seeds * (iterations + 2)};
     int rc = t.init();
     if (rc) return rc;
     const unsigned seeds[3] = {42u, 137u, 271u};
@@ -1536,10 +1578,10 @@ int launch_cal_svq_train(const void* v, const void* attn, const void* init_cb, c
     int win = order[0];
     for (int k = 0; k < n_seeds; k++)
         if (prox[order[k]] < prox[win]) win = order[k];
-    CAL_TRY(hipMemcpyAsync(out_cb, sd[win].bcb.p, CB * 4, hipMemcpyDeviceToDevice, st));
+    CAL_TRY(hipMemcpyAsync(out_cb, sd[win].best_par, CB * 4, hipMemcpyDeviceToDevice, st));
     if (out_wtrm)
-        hipLaunchKernelGGL(wtrm_compose_kernel, dim3(256), dim3(256), 0, st, sd[win].bwa.as<float>(),
-                           sd[win].bwb.as<float>(), static_cast<float*>(out_wtrm));
+        hipLaunchKernelGGL(wtrm_compose_kernel, dim3(256), dim3(256), 0, st, sd[win].best_par + CB,
+                           sd[win].best_par + CB + 2048, static_cast<float*>(out_wtrm));
     return (int)hipStreamSynchronize(st);
 }
 
@@ -1551,25 +1593,20 @@ int launch_cal_svq_pass(const void* v, const void* attn, const void* cb, const v
     if (attn && (T <= 0 || H_q <= 0 || H_kv <= 0 || H_q % H_kv != 0 || (long)H_kv * T != N))
         return -100;
     Svq t{static_cast<const float*>(v), static_cast<const float*>(attn),
-          static_cast<const float*>(rp), N, T, H_q, H_kv, st};
+          static_cast<const float*>(rp), N, T, H_q, H_kv, st, 1};
     int rc = t.init();
     if (rc) return rc;
     Seed s;
-    CAL_TRY(s.cb.alloc(CB * 4));
-    CAL_TRY(s.wa.alloc(2048 * 4));
-    CAL_TRY(s.wb.alloc(2048 * 4));
-    CAL_TRY(hipMemcpyAsync(s.cb.p, cb, CB * 4, hipMemcpyDeviceToDevice, st));
-    CAL_TRY(hipMemcpyAsync(s.wa.p, wa, 2048 * 4, hipMemcpyDeviceToDevice, st));
-    CAL_TRY(hipMemcpyAsync(s.wb.p, wb, 2048 * 4, hipMemcpyDeviceToDevice, st));
+    if ((rc = s.alloc())) return rc;
+    CAL_TRY(hipMemcpyAsync(s.cb(), cb, CB * 4, hipMemcpyDeviceToDevice, st));
+    CAL_TRY(hipMemcpyAsync(s.wa(), wa, 2048 * 4, hipMemcpyDeviceToDevice, st));
+    CAL_TRY(hipMemcpyAsync(s.wb(), wb, 2048 * 4, hipMemcpyDeviceToDevice, st));
     // without the attention loss the pass leaves the transform gradients alone
-    CAL_TRY(hipMemsetAsync(t.gwa.p, 0, 2048 * 4, st));
-    CAL_TRY(hipMemsetAsync(t.gwb.p, 0, 2048 * 4, st));
+    CAL_TRY(hipMemsetAsync(t.grad + CB, 0, 4096 * 4, st));
     double l[2];
     if ((rc = t.pass(s, temp, true, l))) return rc;
     float* g = static_cast<float*>(out_grad);
-    CAL_TRY(hipMemcpyAsync(g, t.gcb.p, CB * 4, hipMemcpyDeviceToDevice, st));
-    CAL_TRY(hipMemcpyAsync(g + CB, t.gwa.p, 2048 * 4, hipMemcpyDeviceToDevice, st));
-    CAL_TRY(hipMemcpyAsync(g + CB + 2048, t.gwb.p, 2048 * 4, hipMemcpyDeviceToDevice, st));
+    CAL_TRY(hipMemcpyAsync(g, t.grad, NPAR * 4, hipMemcpyDeviceToDevice, st));
     const float lf[2] = {(float)l[0], (float)l[1]};
     CAL_TRY(hipMemcpyAsync(out_loss, lf, sizeof(lf), hipMemcpyHostToDevice, st));
     return (int)hipStreamSynchronize(st);

@@ -231,11 +231,12 @@ def test_svq_pass_vs_restatement(device, mode):
         np.testing.assert_allclose(a, w, rtol=1e-3, atol=1e-4 * max(np.abs(w).max(), 1e-30))
 
 
-@pytest.mark.parametrize("T_,H_kv,H_q", [(1, 1, 1), (31, 2, 6), (65, 1, 5), (130, 2, 4)])
+@pytest.mark.parametrize("T_,H_kv,H_q", [(1, 1, 1), (31, 2, 6), (65, 1, 5), (130, 2, 4), (515, 1, 2)])
 def test_svq_pass_sizes(device, T_, H_kv, H_q):
     """The pass at sizes around the 64-wide matrix-product tiles, its 32-deep
-    slabs, the K splits (from 256 stacked rows on) and the 64-row blocks of the
-    codebook gradient, to the tolerance of test_svq_pass_vs_restatement."""
+    slabs, the K splits (from 256 stacked rows on), the 64-row blocks of the
+    codebook gradient and the switch from the heads' Gram matrices to the two
+    products per head (past 512 tokens a pass), to the tolerance of test_svq_pass_vs_restatement."""
     v, rp, cb, attn, N, Tn, H_q, H_kv = _svq_margin_case(T=T_, H_kv=H_kv, H_q=H_q, seed=31)
     rng = np.random.default_rng(32)
     wa = (rng.standard_normal((256, 8)) / 16).astype(np.float32)
