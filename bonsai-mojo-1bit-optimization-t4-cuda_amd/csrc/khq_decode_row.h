@@ -42,7 +42,7 @@ __device__ __forceinline__ void load_consts(const DecompArgs& a, int p, Consts& 
     c.cv1 = __half2float(a.cents_v[256 + 4 * p + 3]) * a.a_v;
     // RoPE frequencies of dims 4 (p & 7) + i (lanes 0..15 rotate dims 0..63)
 #pragma unroll
-    for (int i = 0; i < 4; i++) c.fr[i] = powf(a.rope_base, -2.0f * (float)(4 * (p & 7) + i) / 64.0f);
+    for (int i = 0; i < 4; i++) c.fr[i] = a.freq[4 * (p & 7) + i];
     c.below = (p == 0) ? 0ull : (~0ull >> (64 - p));
 }
 
@@ -109,11 +109,10 @@ __device__ __forceinline__ void decode_k(const DecompArgs& a, const Consts& c, u
     }
 }
 
-// V row: vc (decode_v) = the patch's 8-bit codebook index, pvl = its 12-bit field
-// (bit 7 the dim-3 centroid, bits 8..11 the dim-3 residual), nv / ec / smv =
-// the row's fp16 norm, fp16 energy ratio (as floats) and fp32 shared meta.
-// y = the decoded dims, 1 / (16 d_v) applied.
-// cbv = the patch's codebook entry (three fp16 values as floats).
+// V row: cbv = the patch's codebook entry (three fp16 values as floats), pvl =
+// its 12-bit field (bit 7 the dim-3 centroid, bits 8..11 the dim-3 residual),
+// nv / ec / smv = the row's fp16 norm, fp16 energy ratio (as floats) and fp32
+// shared meta.  y = the decoded dims, 1 / (16 d_v) applied.
 __device__ __forceinline__ void decode_v_cb(const DecompArgs& a, const Consts& c, const float (&cbv)[3],
                                             uint32_t pvl, float nv, float ec, float smv, int p,
                                             float (&y)[4]) {
@@ -135,15 +134,6 @@ __device__ __forceinline__ void decode_v_cb(const DecompArgs& a, const Consts& c
     mu::fwht256(y, p);
 #pragma unroll
     for (int i = 0; i < 4; i++) y[i] *= c.ldv[i];
-}
-
-__device__ __forceinline__ void decode_v(const DecompArgs& a, const Consts& c, uint32_t vc,
-                                         uint32_t pvl, float nv, float ec, float smv, int p,
-                                         float (&y)[4]) {
-    float cbv[3];
-#pragma unroll
-    for (int k = 0; k < 3; k++) cbv[k] = __half2float(a.vq[(size_t)p * 768 + vc * 3 + k]);
-    decode_v_cb(a, c, cbv, pvl, nv, ec, smv, p, y);
 }
 
 }  // namespace dec

@@ -82,7 +82,8 @@ hipError_t launch_step_finish(const FinishArgs& a, int H_q, hipStream_t st);
 // Copies bytes (a multiple of 16) from pinned host memory to device memory
 // with a one-block kernel on st.
 hipError_t launch_meta_upload(const void* host_src, void* dst, size_t bytes, hipStream_t st);
-hipError_t launch_step_finish_batched(const FinishArgs* args, int n_seq, int H_q,
+// max_parts: the largest part count of a sequence.
+hipError_t launch_step_finish_batched(const FinishArgs* args, int n_seq, int H_q, int max_parts,
                                       hipStream_t st);
 
 // Rows of 256 halves to compress: the first n_ring from a ring buffer of
@@ -196,6 +197,7 @@ struct DecompArgs {
     __half* out_vt;
     int h_kv, tok0, n_tok, start_pos, key0, ld_vt;
     float a_k, a_v, rope_base;
+    float freq[32];  // rope_base^(-2 i / 64), filled by the launchers
 };
 // n raw tokens (rows token * h_kv + head of k / v) -> the same key layout at
 // key0 + t (key0 a multiple of 32; V^T columns up to the next multiple of 32

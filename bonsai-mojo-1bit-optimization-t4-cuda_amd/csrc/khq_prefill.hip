@@ -26,6 +26,7 @@
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
 #include <stdint.h>
+#include <string.h>
 
 #include <algorithm>
 #include <cmath>
@@ -43,7 +44,7 @@ using namespace mu;
 constexpr int BLK_THR = 256;  // decompress / gather blocks: 4 wavefronts of TB / 4 tokens
 constexpr int VT_PAD = 8;     // halves of padding per LDS V^T row
 // Tokens per block TB: 4 spread a chunk over many CUs; 16 write V^T in 32-byte
-// runs and set a lane's constants up once for four tokens, but take 15 us
+// runs and set a lane's constants up once for four tokens, but take 12 us
 // however few there are.
 constexpr int TB_LONG = 16;
 
@@ -65,45 +66,76 @@ __device__ __forceinline__ void store_vt(const _Float16 (*sv)[TB + VT_PAD], __ha
 
 // ------------------------------------------------------------- decompress
 // Block (TB tokens, KV head h), a wavefront per TB / 4 tokens; lane p owns
-// patch p = dims 4 p .. 4 p + 3.  The decode of one row is a chain of dependent
-// loads: wavefronts in parallel hide it.
+// patch p = dims 4 p .. 4 p + 3.  Latency-bound: the decode of a row is a chain
+// of dependent reads (mask -> ordinals -> payload bytes, fields -> codebook), so
+// the block's packed rows come to LDS in one round trip first, and every
+// token's codebook entry is requested before the first row is decoded.
+// 8,000 rows 21.9 -> 15.8 us, 512 rows 7.1 -> 5.9 us, 130,560 rows 227 -> 121 us.
 template <int TB>
 using VtTile = _Float16[256][TB + VT_PAD];
 template <int TB>
+struct __align__(16) DecompLds {
+    VtTile<TB> sv;
+    uint32_t pay[TB][53];  // mask 16 words, K payload 10, V payload 26
+    float nrm[TB][5];      // K norm, residual scale; V norm, energy, shared meta
+};
+template <int TB>
 __device__ __forceinline__ void decompress_block(const DecompArgs& a, int bx, int h, void* lds) {
-    VtTile<TB>& sv = *static_cast<VtTile<TB>*>(lds);
+    DecompLds<TB>& L = *static_cast<DecompLds<TB>*>(lds);
+    auto& sv = L.sv;
     const int wv = threadIdx.x >> 6, p = threadIdx.x & 63;
     const int t_blk = bx * TB;
+    auto row_of = [&](int tl) { return (size_t)(a.tok0 + min(t_blk + tl, a.n_tok - 1)) * a.h_kv + h; };
+#pragma unroll
+    for (int i0 = 0; i0 < TB * 52; i0 += BLK_THR) {
+        const int i = i0 + threadIdx.x, tl = i / 52, w = i % 52;
+        if (i < TB * 52) {
+            const size_t g = row_of(tl);
+            const uint32_t* src = w < 16   ? a.kmask + g * 16 + w
+                                  : w < 26 ? reinterpret_cast<const uint32_t*>(a.kpay + g * 40) + w - 16
+                                           : reinterpret_cast<const uint32_t*>(a.vpay + g * 104) + w - 26;
+            L.pay[tl][w] = *src;
+        }
+    }
+    if (threadIdx.x < TB * 5) {
+        const int tl = threadIdx.x / 5, f = threadIdx.x % 5;
+        const size_t g = row_of(tl);
+        const __half* n = f == 0 ? a.knorm : f == 1 ? a.krn : f == 2 ? a.vnorm : a.vrn;
+        L.nrm[tl][f] = f == 4 ? __uint_as_float(*reinterpret_cast<const uint32_t*>(a.vsm + g * 4))
+                              : __half2float(n[g]);
+    }
     dec::Consts cs;
     dec::load_consts(a, p, cs);
-#pragma unroll 2
-    for (int tl = wv; tl < TB; tl += 4) {
-        const int tok = t_blk + tl;
-        if (tok >= a.n_tok) {        // uniform per wavefront
+    __syncthreads();
+    constexpr int TW = TB / 4;  // tokens per wavefront: wv, wv + 4, ...
+    uint32_t fld[TW];
+    float cbv[TW][3];
+    const uint32_t grp = (uint32_t)p / 8, bit = 12 * ((uint32_t)p % 8);
 #pragma unroll
-            for (int c = 0; c < 4; c++) sv[4 * p + c][tl] = (_Float16)0.0f;
-            continue;
-        }
-        const size_t g = (size_t)(a.tok0 + tok) * a.h_kv + h;
+    for (int i = 0; i < TW; i++) {
+        const uint32_t* vw = &L.pay[wv + 4 * i][26];
+        const uint32_t w = grp * 3 + (bit >> 5);  // (the words after the fields are there)
+        fld[i] = __builtin_amdgcn_alignbit(vw[w + 1], vw[w], bit & 31) & 0xFFFu;
+        const uint32_t code = (fld[i] & 0x7Fu) | (((vw[24 + (p >> 5)] >> (p & 31)) & 1u) << 7);
+#pragma unroll
+        for (int k = 0; k < 3; k++) cbv[i][k] = __half2float(a.vq[(size_t)p * 768 + code * 3 + k]);
+    }
+#pragma unroll
+    for (int i = 0; i < TW; i++) {
+        const int tl = wv + 4 * i, tok = t_blk + tl;
+        const bool ok = tok < a.n_tok;  // uniform per wavefront
+        const float* nr = L.nrm[tl];
         float y[4];
         // ---- K: codes, outlier ordinals (ballot prefix), values, RoPE
-        dec::decode_k(a, cs, a.kmask[g * 16 + (p >> 2)], a.kpay + g * 40, __half2float(a.knorm[g]),
-                      __half2float(a.krn[g]), (float)(a.start_pos + a.tok0 + tok), p, y);
-        *reinterpret_cast<uint2*>(a.out_k + ((size_t)(a.key0 + tok) * a.h_kv + h) * 256 + 4 * p) =
-            uint2{pk_rne(y[0], y[1]), pk_rne(y[2], y[3])};
-        // ---- V: patch fields, codebook, dim 3, inverse rotor, FWHT
-        const uint8_t* vp = a.vpay + g * 104;
-        const uint32_t grp = (uint32_t)p / 8, sub = (uint32_t)p % 8;
-        const uint64_t w0 = dec::rd32(vp + (grp * 3 + 0) * 4), w1 = dec::rd32(vp + (grp * 3 + 1) * 4),
-                       w2 = dec::rd32(vp + (grp * 3 + 2) * 4);
-        const uint64_t low64 = (w1 << 32) | w0, high64 = (w2 << 32) | w1;
-        const uint32_t pvl = (sub < 4) ? (uint32_t)((low64 >> (sub * 12)) & 0xFFF)
-                                       : (uint32_t)((high64 >> ((sub - 4) * 12 + 16)) & 0xFFF);
-        const uint32_t hb = (p < 32) ? ((dec::rd32(vp + 96) >> p) & 1u) : ((dec::rd32(vp + 100) >> (p - 32)) & 1u);
-        dec::decode_v(a, cs, (pvl & 0x7Fu) | (hb << 7), pvl, __half2float(a.vnorm[g]),
-                      __half2float(a.vrn[g]), __uint_as_float(dec::rd32(a.vsm + g * 4)), p, y);
+        dec::decode_k(a, cs, L.pay[tl][p >> 2], reinterpret_cast<const uint8_t*>(&L.pay[tl][16]), nr[0],
+                      nr[1], (float)(a.start_pos + a.tok0 + tok), p, y);
+        if (ok)
+            *reinterpret_cast<uint2*>(a.out_k + ((size_t)(a.key0 + tok) * a.h_kv + h) * 256 + 4 * p) =
+                uint2{pk_rne(y[0], y[1]), pk_rne(y[2], y[3])};
+        // ---- V: codebook, dim 3, inverse rotor, FWHT
+        dec::decode_v_cb(a, cs, cbv[i], fld[i], nr[2], nr[3], nr[4], p, y);
 #pragma unroll
-        for (int c = 0; c < 4; c++) sv[4 * p + c][tl] = (_Float16)y[c];
+        for (int c = 0; c < 4; c++) sv[4 * p + c][tl] = ok ? (_Float16)y[c] : (_Float16)0.0f;
     }
     __syncthreads();
     store_vt<TB>(sv, a.out_vt, a.ld_vt, h, a.key0 + t_blk, min(TB, (a.n_tok - t_blk + 3) & ~3));
@@ -152,7 +184,7 @@ struct __align__(16) SharedLds {
 
 template <int TB>
 __global__ __launch_bounds__(BLK_THR) void decompress_kernel(DecompArgs a) {
-    __shared__ SharedLds<sizeof(VtTile<TB>)> lds;
+    __shared__ SharedLds<sizeof(DecompLds<TB>)> lds;
     decompress_block<TB>(a, blockIdx.x, blockIdx.y, &lds);
 }
 
@@ -167,7 +199,7 @@ __global__ __launch_bounds__(BLK_THR) void ring_gather_kernel(GatherArgs a) {
 template <int TB>
 __global__ __launch_bounds__(BLK_THR) void decompress_gather_kernel(DecompArgs d, GatherArgs g,
                                                                     int nx_d) {
-    __shared__ SharedLds<sizeof(VtTile<TB>), sizeof(VtTile<32>)> lds;
+    __shared__ SharedLds<sizeof(DecompLds<TB>), sizeof(VtTile<32>)> lds;
     const int nb_d = nx_d * d.h_kv, b = blockIdx.x;
     if (b < nb_d)
         decompress_block<TB>(d, b % nx_d, b / nx_d, &lds);
@@ -920,11 +952,23 @@ __global__ __launch_bounds__(256) void prefill_finish_kernel(PrefillArgs a, Ring
 }  // namespace pf
 
 namespace {
+// RoPE frequencies by the host's powf, as the attention kernels' table has them
+// (four powf a lane on the GPU were more than a row's decode).
+DecompArgs with_rope(DecompArgs a) {
+    thread_local float last_base = -1.0f;
+    thread_local float freq[32];
+    if (a.rope_base != last_base) {
+        for (int i = 0; i < 32; i++) freq[i] = powf(a.rope_base, -2.0f * (float)i / 64.0f);
+        last_base = a.rope_base;
+    }
+    memcpy(a.freq, freq, sizeof(freq));
+    return a;
+}
 int gather_blocks(const GatherArgs& g) { return g.n > 0 ? (g.n + 31) / 32 * g.h_kv : 0; }
 bool long_decode(const DecompArgs& a) {
-    // 4 KV heads, 4 / 16 tokens a block: 1,024 tokens 14.3 / 15.7 us, 2,000
-    // 21.9 / 19.3, 8,192 62.6 / 48.3 (32 a block: 25 us at least, 43.4)
-    return a.n_tok / pf::TB_LONG * a.h_kv >= 3 * device_cu_count() / 2;
+    // 4 KV heads, 4 / 16 tokens a block: 1,024 tokens 11.3 / 12.6 us, 2,000
+    // 15.9 / 15.8, 8,192 39.6 / 37.0, 32,640 153 / 121
+    return a.n_tok / pf::TB_LONG * a.h_kv >= 2 * device_cu_count();
 }
 }  // namespace
 
@@ -938,8 +982,9 @@ hipError_t launch_prefill_finish(const PrefillArgs& a, const RingArgs* ring, hip
     return hipGetLastError();
 }
 
-hipError_t launch_decompress(const DecompArgs& a, hipStream_t st) {
-    if (a.n_tok <= 0) return hipSuccess;
+hipError_t launch_decompress(const DecompArgs& args, hipStream_t st) {
+    if (args.n_tok <= 0) return hipSuccess;
+    const DecompArgs a = with_rope(args);
     if (long_decode(a))
         hipLaunchKernelGGL(pf::decompress_kernel<pf::TB_LONG>,
                            dim3((a.n_tok + pf::TB_LONG - 1) / pf::TB_LONG, a.h_kv),
@@ -950,9 +995,10 @@ hipError_t launch_decompress(const DecompArgs& a, hipStream_t st) {
     return hipGetLastError();
 }
 
-hipError_t launch_decompress_gather(const DecompArgs& d, const GatherArgs& g, hipStream_t st) {
-    if (d.n_tok <= 0) return launch_ring_gather(g, st);
-    if (g.n <= 0) return launch_decompress(d, st);
+hipError_t launch_decompress_gather(const DecompArgs& args, const GatherArgs& g, hipStream_t st) {
+    if (args.n_tok <= 0) return launch_ring_gather(g, st);
+    if (g.n <= 0) return launch_decompress(args, st);
+    const DecompArgs d = with_rope(args);
     const int tb = long_decode(d) ? pf::TB_LONG : 4, nx_d = (d.n_tok + tb - 1) / tb;
     const dim3 grid(nx_d * d.h_kv + gather_blocks(g));
     if (tb == 4)
@@ -963,8 +1009,9 @@ hipError_t launch_decompress_gather(const DecompArgs& d, const GatherArgs& g, hi
     return hipGetLastError();
 }
 
-hipError_t launch_compress_decode(const CompressJob& k, const CompressJob& v, const DecompArgs& d,
+hipError_t launch_compress_decode(const CompressJob& k, const CompressJob& v, const DecompArgs& args,
                                   const GatherArgs& g, hipStream_t st) {
+    const DecompArgs d = with_rope(args);
     // the decode covers exactly the compressed rows: token t, KV head h is row t h_kv + h
     if (k.n != v.n || d.n_tok * d.h_kv != k.n || d.tok0 != d.key0 || d.start_pos != 0)
         return hipErrorInvalidValue;

@@ -281,11 +281,11 @@ def test_layer_prefill_decoded_rows_match_decode(device, chunks):
 
 
 def test_decompress_long_matches_short(device):
-    """1,601 tokens in one call (16 a block, from 384 blocks on 256 CUs) against
+    """2,113 tokens in one call (16 a block, from 512 blocks on 256 CUs) against
     the same tokens in calls of 400 (4 a block), bit for bit; columns past the
     last token's group of four stay as they were."""
     lc, _ = layer_consts(layer_id=2)
-    n, ld = 1601, 1664
+    n, ld = 2113, 2176
     cents, pay = ops.Centroids(lc, device), ops.Payload(n * H_KV, device)
     synth.compressed_rows(pay, cents, seed=5)
     outs = []
@@ -297,7 +297,7 @@ def test_decompress_long_matches_short(device):
                            ld_vt=ld)
         outs.append((k.cpu().numpy().view(np.uint16), vt.cpu().numpy().view(np.uint16)))
     assert np.array_equal(outs[0][0], outs[1][0]) and np.array_equal(outs[0][1], outs[1][1])
-    assert (outs[0][1][:, :, 1604:] == np.float16(7.0).view(np.uint16)).all()
+    assert (outs[0][1][:, :, 2116:] == np.float16(7.0).view(np.uint16)).all()
 
 
 def test_c5_chunk_vs_oracle(device):
