@@ -890,6 +890,23 @@ __device__ __forceinline__ void value_role(const AttnArgs& a, Smem& S, const Set
     PHASE(21);
 }
 
+// Appends the step's token for KV heads h0 .. h0 + nh - 1 (8-byte pieces, three
+// tensors) and makes it visible to the block: the heads' rows are read by this
+// block alone.  It saves the ring-write launch of a decode step for one round
+// trip in the window blocks, which end before the chunks do: a layer step at 300 /
+// 3,000 / 20,000 tokens takes 17.2 / 18.5 / 27.4 us, 18.9 / 20.8 / 29.0 with the
+// write apart.
+__device__ __forceinline__ void append_token(const RingNew& r, int h_kv, int h0, int nh) {
+    for (int i = threadIdx.x; i < 192 * nh; i += NTHR) {
+        const int t = i / (64 * nh), e = (h0 * 64 + i % (64 * nh)) * 4;
+        const __half* src = t == 0 ? r.k : t == 1 ? r.v : r.u;
+        __half* dst = t == 0 ? r.ring_k : t == 1 ? r.ring_v : r.ring_u;
+        if (src && dst) stg<uint2>(dst + (size_t)r.slot * h_kv * 256 + e, ldg<uint2>(src + e));
+    }
+    __threadfence_block();
+    __syncthreads();
+}
+
 // ------------------------------------------------------------ window blocks
 // The raw ring window (fp16, K already roped) of KV head hk, in one of four
 // blocks (one per KV head) after the last compressed chunk, used when the
@@ -1234,7 +1251,9 @@ __device__ __forceinline__ void ws_block(const AttnArgs& a, int chunk, int tiles
 #ifdef KHQ_PHASE_TIMING
         const unsigned long long wt0 = __builtin_amdgcn_s_memrealtime();
 #endif
-        if (a.win_blocks == NWIN)
+        const bool one = a.win_blocks != NWIN;  // one block for all heads
+        if (a.add.k) append_token(a.add, a.h_kv, one ? 0 : chunk - n_chunks, one ? a.h_kv : 1);
+        if (!one)
             window_block(a, S, a.part_offset + n_chunks, chunk - n_chunks);
         else
             window_block_all(a, S, a.part_offset + n_chunks);

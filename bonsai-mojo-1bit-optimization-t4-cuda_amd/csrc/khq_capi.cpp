@@ -522,7 +522,7 @@ static int attn_step_impl(const void* q_gate, const void* k_payload, const void*
                        const void* ring_v, void* out, int H_q, int H_kv, int c_len,
                        int win_start, int win_len, int ring_cap, float scale, float alpha_k,
                        float alpha_v, float rope_base, hipStream_t stream,
-                          bool noalloc) {
+                          bool noalloc, const khq::RingNew* add = nullptr) {
     if (c_len < 0 || win_len < 0 || (c_len == 0 && win_len == 0)) return -100;
     if (H_q <= 0 || H_kv <= 0 || H_q % H_kv != 0 || H_q / H_kv > 8) return -100;
     if (win_len > 0 && (ring_cap <= 0 || win_len > ring_cap || win_start < 0)) return -100;
@@ -534,9 +534,12 @@ static int attn_step_impl(const void* q_gate, const void* k_payload, const void*
     // finishing launch only merges; otherwise the finishing launch computes
     // the window too.  Longer windows: window partials + combine.
     const bool fused_tail = win_len <= 256 && npc <= 1000;
-    const bool win_in_ws = fused_tail && npc > 0 && win_len > 0 &&
-                           g_kernel_choice.load(std::memory_order_relaxed) == 0 &&
-                           use_mfma(n_rep, H_kv, 1);
+    const bool win_in_ws = fused_tail && khq::step_window_in_ws(H_q, H_kv, c_len, win_len);
+    if (add && !win_in_ws) {  // the kernel choice changed since the caller asked
+        const int rc = launch_khq_ring_write_fp16(add->ring_k, add->ring_v, add->u ? add->ring_u : nullptr,
+                                                  add->k, add->v, add->u, add->slot, H_kv * 256, stream);
+        if (rc) return rc;
+    }
     // (64 window parts at most: the fixed array of the no-allocation step holds those)
     const int npw = (win_len > 0 && !fused_tail) ? window_parts(win_len, H_kv, 4, 64) : (win_in_ws ? 1 : 0);
     const int np = npc + npw;
@@ -574,6 +577,7 @@ static int attn_step_impl(const void* q_gate, const void* k_payload, const void*
             a.win_start = win_start % ring;
             a.win_len = win_len;
             a.ring_cap = ring;
+            if (add) a.add = *add;
         }
         int used = 0;
         e = launch_compressed(a, n_rep, 1, &used, stream);
@@ -966,6 +970,18 @@ int khq_attn_step_batched_fp16(const khq_seq* seqs, int n_seq, const void* centr
 }  // extern "C"
 
 namespace khq {
+
+bool step_window_in_ws(int H_q, int H_kv, int c_len, int win_len) {
+    return H_kv > 0 && H_q % H_kv == 0 && c_len > 0 && win_len > 0 && win_len <= 256 &&
+           g_kernel_choice.load(std::memory_order_relaxed) == 0 && use_mfma(H_q / H_kv, H_kv, 1);
+}
+
+int attn_step_append(const AttnArgs& a, int H_q, __half* out, hipStream_t stream) {
+    return attn_step_impl(a.q, a.kpay, a.vpay, a.vsm, a.kmask, a.knorm, a.krn, a.vnorm, a.vrn,
+                          a.cents_k, a.cents_v, a.vq, a.rotor_k, a.rotor_v, a.dk, a.dv, a.ring_k,
+                          a.ring_v, out, H_q, a.h_kv, a.c_len, a.win_start, a.win_len, a.ring_cap,
+                          a.sc, a.a_k, a.a_v, a.rope_base, stream, false, &a.add);
+}
 
 int prefill_attn_run(PrefillArgs a, const RingArgs* ring, hipStream_t stream, bool merge) {
     prefill_plan(a);

@@ -9,6 +9,19 @@
 
 namespace khq {
 
+// The token of a decode step, to be appended to ring slot `slot` (rows
+// [h_kv][256]) by the launch that attends over it; k = NULL: none, u / ring_u
+// may be NULL.
+struct RingNew {
+    const __half* k;
+    const __half* v;
+    const __half* u;
+    __half* ring_k;
+    __half* ring_v;
+    __half* ring_u;
+    int slot;
+};
+
 // Compressed-region work: token range [0, c_len) of KV head blockIdx.y cut
 // into n_parts parts; the partial triple of query qid, part i lands at
 // part[(qid * part_stride + part_offset + i) * 258].
@@ -38,6 +51,7 @@ struct AttnArgs {
     const __half* ring_k;
     const __half* ring_v;
     int win_start, win_len, ring_cap;
+    RingNew add;     // appended by the window blocks before they read the window
     int win_blocks;  // window blocks after the chunks: 4 (one per KV head) or 1 (all heads)
     int chunk_tiles;  // batched launch: tiles per compressed chunk of this sequence
     // Bound of the key / value hand-off waits of the wavefront-specialised
@@ -147,6 +161,12 @@ hipError_t fault_status(int* out, int clear);
 // Hand-off wait bound used by the launchers (default 2^20 sleeps).
 extern std::atomic<int> g_spin_limit;
 size_t attn_ws_smem_bytes();
+// Whether khq_attn_step_fp16 computes this step's window inside the
+// compressed-region launch (which can then append the step's token to the ring).
+bool step_window_in_ws(int H_q, int H_kv, int c_len, int win_len);
+// khq_attn_step_fp16 with the token of the step appended first; only where
+// step_window_in_ws holds.
+int attn_step_append(const AttnArgs& a, int H_q, __half* out, hipStream_t stream);
 // Fills a.rope_tab from a.rope_base (host).
 void fill_rope_table(AttnArgs& a);
 hipError_t launch_attn_ws(const AttnArgs& a, int tiles_per_chunk, int n_chunks,

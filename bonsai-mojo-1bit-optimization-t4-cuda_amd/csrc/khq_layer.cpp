@@ -242,16 +242,33 @@ int khq_layer_capture_unroped(khq_layer* L, const void* k_unroped, hipStream_t s
 }
 
 // khq_step after the ring writes of the token (ref runtime.mojo:489-613).
+// With add, the fused attention launch writes the token to the ring; a step that
+// fails before that launch writes it apart, so it is in the ring either way.
 static int step_after_ring_write(khq_layer* L, const void* q_gate, void* out, float scale,
-                                 hipStream_t stream);
+                                 hipStream_t stream, const khq::RingNew* add = nullptr);
+
+static int ring_append(khq_layer* L, const khq::RingNew& t, hipStream_t stream) {
+    return launch_khq_ring_write_fp16(t.ring_k, t.ring_v, t.u ? t.ring_u : nullptr, t.k, t.v, t.u,
+                                      t.slot, L->H_kv * kD, stream);
+}
 
 int khq_layer_step(khq_layer* L, const void* q_gate, const void* k_roped, const void* v,
                    const void* k_unroped, void* out, float scale, hipStream_t stream) {
     if (!L || !q_gate || !k_roped || !v || !out) return -100;
-    const int kv = L->H_kv * kD;
     const int slot = L->write_pos % kRing;
-    int rc = launch_khq_ring_write_fp16(L->ring_k, L->ring_v, k_unroped ? L->ring_u : nullptr,
-                                        k_roped, v, k_unroped, slot, kv, stream);
+    const khq::RingNew add{static_cast<const __half*>(k_roped), static_cast<const __half*>(v),
+                           static_cast<const __half*>(k_unroped), L->ring_k, L->ring_v, L->ring_u,
+                           slot};
+    // A compression event of this step reads the 128 oldest raw tokens, never
+    // this one, so the ring write can wait for the attention launch (which
+    // copies 8-byte pieces).
+    const int c_len = L->boundary + (event_due(L, L->write_pos + 1) ? kChunk : 0);
+    const bool by8 = ((reinterpret_cast<uintptr_t>(k_roped) | reinterpret_cast<uintptr_t>(v) |
+                       reinterpret_cast<uintptr_t>(k_unroped)) & 7) == 0;
+    if (L->fused && by8 &&
+        khq::step_window_in_ws(L->H_q, L->H_kv, c_len, L->write_pos + 1 - c_len))
+        return step_after_ring_write(L, q_gate, out, scale, stream, &add);
+    const int rc = ring_append(L, add, stream);
     if (rc) return rc;
     return step_after_ring_write(L, q_gate, out, scale, stream);
 }
@@ -298,12 +315,15 @@ int khq_layer_attention_step(khq_layer* L, void* q_gate, void* k, const void* v,
 }
 
 static int step_after_ring_write(khq_layer* L, const void* q_gate, void* out, float scale,
-                                 hipStream_t stream) {
+                                 hipStream_t stream, const khq::RingNew* add) {
     int rc = 0;
     L->write_pos += 1;
     if (event_due(L, L->write_pos)) {
         rc = compress_event(L, stream);
-        if (rc) return rc;
+        if (rc) {
+            if (add) ring_append(L, *add, stream);
+            return rc;
+        }
     }
     const int c_len = L->boundary;
     const int win_len = L->write_pos - c_len;
@@ -312,6 +332,41 @@ static int step_after_ring_write(khq_layer* L, const void* q_gate, void* out, fl
     // (README:259); refuse instead.
     if (win_len > kRing) return -102;
     const int win_start = c_len % kRing;
+    if (add) {
+        khq::AttnArgs a{};
+        auto h = [](const void* p) { return static_cast<const __half*>(p); };
+        a.q = h(q_gate);
+        a.kpay = L->kpay;
+        a.vpay = L->vpay;
+        a.vsm = L->vsm;
+        a.kmask = L->kmask;
+        a.knorm = L->knorm;
+        a.krn = L->krn;
+        a.vnorm = L->vnorm;
+        a.vrn = L->vrn;
+        a.cents_k = h(L->cents_k);
+        a.cents_v = h(L->cents_v);
+        a.vq = h(L->vq);
+        a.rotor_k = h(L->rotor_k);
+        a.rotor_v = h(L->rotor_v);
+        a.dk = h(L->d_k);
+        a.dv = h(L->d_v);
+        a.ring_k = L->ring_k;
+        a.ring_v = L->ring_v;
+        a.h_kv = L->H_kv;
+        a.c_len = c_len;
+        a.win_start = win_start;
+        a.win_len = win_len;
+        a.ring_cap = kRing;
+        a.sc = scale;
+        a.a_k = L->alpha_k;
+        a.a_v = L->alpha_v;
+        a.rope_base = L->rope_base;
+        a.add = *add;
+        rc = khq::attn_step_append(a, L->H_q, static_cast<__half*>(out), stream);
+        if (rc) ring_append(L, *add, stream);
+        return rc ? rc : 1;
+    }
     if (L->fused) {
         rc = khq_attn_step_fp16(q_gate, L->kpay, L->vpay, L->vsm, L->kmask, L->knorm, L->krn,
                                 L->vnorm, L->vrn, L->cents_k, L->cents_v, L->vq, L->rotor_k,

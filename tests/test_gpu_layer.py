@@ -220,3 +220,39 @@ def test_runtime_loads_centroid_file(device, tmp_path):
     assert rt.layer(3) is L3 and L3.cap == 512
     with pytest.raises(KeyError):
         rt.layer(4)
+
+
+def _off_by_one(x):
+    """x at an address two bytes past an 8-byte boundary."""
+    flat = torch.empty(x.numel() + 1, device=x.device, dtype=x.dtype)[1:]
+    flat.copy_(x.reshape(-1))
+    return flat.view(x.shape)
+
+
+@pytest.mark.parametrize("n,steps", [(383, 262), (20479, 4)],
+                         ids=["per-head-window", "all-heads-window"])
+def test_step_ring_append_forms(device, n, steps):
+    """The token's ring write inside the attention launch against the write of
+    its own (unaligned rows take that one): same outputs and state, with and
+    without the unroped key, over an event (write_pos 384, 20,480), over the
+    event that compresses the appended tokens (640) and, at 20,224 compressed
+    tokens, one window block for all heads."""
+    lc, _ = layer_consts(7)
+    a, b = (KL.NativeKhqLayer(lc, H_q=H_Q, H_kv=H_KV, cap=20736, device=device,
+                              options=KL.KhqOptions(splits=8, fused=True)) for _ in range(2))
+    g = torch.Generator(device=device).manual_seed(n)
+
+    def rnd(*shape):
+        return torch.randn(*shape, generator=g, device=device).half()
+
+    q, k, v = rnd(n + steps, H_Q, 2 * D), rnd(n + steps, H_KV, D), rnd(n + steps, H_KV, D)
+    out = torch.zeros(n, H_Q, D, device=device, dtype=torch.float16)
+    for L in (a, b):
+        L.prefill(q[:n], k[:n], v[:n], k[:n], out, SCALE)
+    for i in range(n, n + steps):
+        ku = k[i] if i % 2 == 0 else None
+        oa, ob = (torch.zeros(H_Q, D, device=device, dtype=torch.float16) for _ in range(2))
+        assert a.step(q[i], k[i], v[i], oa, SCALE, k_unroped=ku)
+        assert b.step(q[i], _off_by_one(k[i]), _off_by_one(v[i]), ob, SCALE, k_unroped=ku)
+        assert torch.equal(oa, ob)
+        assert a.state() == b.state() and a.state()[1] == i + 1
