@@ -986,7 +986,7 @@ int attn_step_append(const AttnArgs& a, int H_q, __half* out, hipStream_t stream
 int prefill_attn_run(PrefillArgs a, const RingArgs* ring, hipStream_t stream, bool merge) {
     prefill_plan(a);
     a.eps = 1e-8f;
-    if (a.n_split > 1 || !a.out) {
+    if (a.n_split > 1 || a.apart) {
         const hipError_t e = workspace(
             (size_t)a.n_q * a.h_kv * a.n_rep * a.n_split * 258 * sizeof(float), stream, &a.part);
         if (e != hipSuccess) return rc_of(e);

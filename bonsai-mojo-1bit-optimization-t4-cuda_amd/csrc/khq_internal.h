@@ -249,15 +249,17 @@ struct RingArgs {
 // 128; ev_cap = 0: every key is raw).
 // Rows of one KV head (query j, head r % n_rep) are cut into blocks, a block's
 // 32-key tiles into ceil(tiles / unit) splits (at most n_split).  Blocks of one
-// split write out directly; split s of the others leaves the triple of (query
-// j, head hq) at part[((j * H_q + hq) * n_split + s) * 258].
+// split write out directly unless apart; split s of the others leaves the triple
+// of (query j, head hq) at part[((j * H_q + hq) * n_split + s) * 258].
 struct PrefillArgs {
     const __half* q;
     const __half* k;
     const __half* vt;
     float* part;
-    __half* out;  // NULL: every block leaves triples
+    __half* out;  // NULL: triples only (apart)
     int ld_vt, n_q, h_kv, n_rep, n_split, unit;
+    bool apart;    // every block leaves triples
+    bool uniform;  // every block has n_split splits
     int vis0, n_raw, raw0, dec0, ev_cap;
     float sc, eps;
     __host__ __device__ int bound(int vis) const {
@@ -293,7 +295,7 @@ hipError_t launch_compress_gather(const CompressJob& k, const CompressJob& v, co
                                   hipStream_t st);
 // Rows of one KV head a block of the prefill attention takes.
 int prefill_block_rows(int n_rows);
-// Fills a.n_split and a.unit for the current device.
+// Fills a.n_split, a.unit, a.apart and a.uniform for the current device.
 void prefill_plan(PrefillArgs& a);
 hipError_t launch_prefill_attn(const PrefillArgs& a, hipStream_t st);
 // Prefill attention plus merge and gate through the shared workspace: q, k, vt,

@@ -539,7 +539,7 @@ __global__ __launch_bounds__(256) void prefill_attn_kernel(PrefillArgs a) {
     // ---- row li (dims 16 mt + 4 lg + c)
     float l_row = l_part + __shfl_xor(l_part, 16, 64);
     l_row += __shfl_xor(l_row, 32, 64);
-    const bool direct = bk.n_split == 1 && a.out;
+    const bool direct = bk.n_split == 1 && !a.apart;
     const bool empty = m_ref == -INFINITY;
     const float f = empty ? 0.0f : (direct ? 1.0f / (l_row + a.eps) : 1.0f);
 #pragma unroll
@@ -568,12 +568,13 @@ constexpr int KS2_LD = 256 + 8;   // halves per LDS K row
 constexpr int VS2_LD = KT + 4;    // halves per LDS V^T row
 
 constexpr int NKB = 3;            // LDS tile slots
-// Lazy-rescale gap of the 32-row form: weights stay <= e^10 (< fp16 max).
 // Reference of a row that has seen no key: finite, so that a masked score less
 // it is -inf and its weight 0 without a test.
 constexpr float M_NONE = -1e30f;
 constexpr float LOG2E = 1.44269504f, LN2 = 0.693147181f;
-constexpr float GAP32 = 10.0f * LOG2E;  // in the kernel's log2 units
+// Lazy-rescale gap of the 32-row form, in its log2 units: weights stay <= e^10
+// (< fp16 max).
+constexpr float GAP32 = 10.0f * LOG2E;
 
 // Role-specialised 32-row attention: per SIMD a score wavefront and an
 // output wavefront (8 wavefronts per block, 128 rows of one KV head).  The
@@ -619,6 +620,7 @@ void prefill_attn_rs_kernel(PrefillArgs a) {
     const int hq = h * a.n_rep + (r_ok ? r % a.n_rep : 0);
     const BlockKeys bk(a, pos.bx * 128, min(pos.bx * 128 + 127, n_rows - 1), split);
     if (split >= bk.n_split) return;  // uniform per block
+    const bool direct = bk.n_split == 1 && !a.apart;
     const int n_tiles = bk.t_hi - bk.t_lo;
     const int raw_end = a.raw0 + a.n_raw;
     const f32x16 zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -850,7 +852,6 @@ void prefill_attn_rs_kernel(PrefillArgs a) {
         __syncthreads();  // last tile applied
         const float l_row = l_part + __shfl_xor(l_part, 32, 64);
         // ---- row ln: the output, or its partial triple (dims 32 t + 8 j + 4 hh + c)
-        const bool direct = bk.n_split == 1 && a.out;
         const bool empty = m_last == M_NONE;
         const float f = empty ? 0.0f : (direct ? 1.0f / (l_row + a.eps) : 1.0f);
 #pragma unroll
@@ -860,16 +861,23 @@ void prefill_attn_rs_kernel(PrefillArgs a) {
                 *reinterpret_cast<f4*>(&lds.out[rg][ln][32 * t2 + 8 * j + 4 * hh]) =
                     f4{acc[t2][4 * j], acc[t2][4 * j + 1], acc[t2][4 * j + 2], acc[t2][4 * j + 3]} * f;
         wave_sync();
-        store_rows<32>(a, &lds.out[rg][0][0], row0, h, split, direct, empty ? -1e20f : m_last * LN2,
-                       empty ? 0.0f : l_row, lane);
+        if (!direct)
+            store_rows<32>(a, &lds.out[rg][0][0], row0, h, split, false,
+                           empty ? -1e20f : m_last * LN2, empty ? 0.0f : l_row, lane);
+    }
+    if (direct) {  // uniform per block; gates and stores: half a row group each wavefront
+        __syncthreads();
+        const int half = tid < 256 ? 0 : 16;
+        store_rows<16>(a, &lds.out[rg][half][0], row0 + half, h, split, true, 0.0f, 0.0f, lane);
     }
 }
 
 // Merge of the key splits, normalisation and gate: one wavefront per (query,
-// head) row of a block that was split (the others' rows are written already), lane l owning dims 4 l .. 4 l + 3; lane s < n_split holds split
-// s's (m, l) pair.  Each group of up to 16 splits has every load in flight
-// before the first is used (the first group's with the (m, l) loads, ahead of
-// the maximum); the sums run in split order.
+// head) row of a block that was split (the others' rows are written already),
+// lane l owning dims 4 l .. 4 l + 3; lane s < n_split holds split s's (m, l)
+// pair.  Each group of up to 16 splits has every load in flight before the
+// first is used (the first group's with the (m, l) loads, ahead of the
+// maximum); the sums run in split order.
 constexpr int MG = 16;  // splits per load group
 __device__ __forceinline__ void merge_row(const PrefillArgs& p, int row, int n_split) {
     const int lane = threadIdx.x & 63;
@@ -930,10 +938,11 @@ __global__ __launch_bounds__(256) void prefill_finish_kernel(PrefillArgs a, Ring
         if (row >= a.n_q * H_q) return;  // uniform per wavefront
         const int r = row / H_q * a.n_rep + row % H_q % a.n_rep;  // row of its KV head
         const int first = r / block_rows * block_rows;
-        int nd, u0;
-        const int ns = a.block_splits(
-            a.block_tiles(first, min(first + block_rows, a.n_q * a.n_rep) - 1, &nd, &u0));
-        if (ns > 1) merge_row(a, row, ns);
+        int ns = a.n_split, nd, u0;
+        if (!a.uniform)
+            ns = a.block_splits(
+                a.block_tiles(first, min(first + block_rows, a.n_q * a.n_rep) - 1, &nd, &u0));
+        if (ns > 1 || a.apart) merge_row(a, row, ns);
         return;
     }
     b -= nb_m;
@@ -973,7 +982,7 @@ bool long_decode(const DecompArgs& a) {
 }  // namespace
 
 hipError_t launch_prefill_finish(const PrefillArgs& a, const RingArgs* ring, hipStream_t st) {
-    const int nb_m = a.n_split > 1 ? (a.n_q * a.h_kv * a.n_rep + 3) / 4 : 0;
+    const int nb_m = a.n_split > 1 || a.apart ? (a.n_q * a.h_kv * a.n_rep + 3) / 4 : 0;
     const RingArgs g = ring ? *ring : RingArgs{};
     const int nb_g = ring ? (g.n * g.h_kv * 64 + 255) / 256 : 0;
     if (nb_m + nb_g == 0) return hipSuccess;
@@ -1056,7 +1065,11 @@ void prefill_plan(PrefillArgs& a) {
     //   few blocks past a round cost a whole round).
     // A block costs about 4 tiles beside its own (entry, first loads, output);
     // splitting costs the finishing launch, about 4, and 0.045 a block for its
-    // triples (128 rows x 1 KB written and read).
+    // triples (128 rows x 1 KB written and read).  Where one round holds every
+    // block, gating the rows inside it (a.apart = false) is not free either: a
+    // wavefront gates up to 16 rows in turn, 0.29 each, with nothing else on its
+    // CU.  Left out, 48 queries over 200 tokens took 27.1 us unsplit against
+    // 17.4 in 8 splits, a 100-token prompt 29.5 against 22.4.
     const int n_rows = a.n_q * a.n_rep, br = prefill_block_rows(n_rows);
     const int nb = (n_rows + br - 1) / br;
     const int slots = (few_rows(n_rows) ? 2 : 1) * device_cu_count();
@@ -1068,6 +1081,7 @@ void prefill_plan(PrefillArgs& a) {
         t_min = std::min(t_min, t);
     }
     const bool even = t_max - t_min <= t_max / 8;
+    const float gate = 0.29f * std::min(16, n_rows);
     const int step = std::max(1, nb / 64);  // enough blocks to add up
     float best = 0.0f;
     int best_k = 1;
@@ -1086,15 +1100,23 @@ void prefill_plan(PrefillArgs& a) {
         const float rounds = std::ceil(units / slots);
         float est = rounds <= 1.0f || even ? rounds * (a.unit + 4)
                                            : (tiles + 4 * units) / slots + 0.5f * a.unit;
-        if (k > 1) est += 4.0f + 0.045f * units;
+        bool apart = !a.out;
+        if (k > 1 || (rounds <= 1.0f && gate > 4.0f + 0.045f * units)) {
+            est += 4.0f + 0.045f * units;
+            apart |= rounds <= 1.0f;
+        } else if (rounds <= 1.0f) {
+            est += gate;
+        }
         if (k == 1 || est < best) {
             best = est;
             best_k = k;
+            a.apart = apart;
         }
     }
     a.n_split = best_k;
     a.unit = (t_max + a.n_split - 1) / a.n_split;
     a.n_split = (t_max + a.unit - 1) / a.unit;
+    a.uniform = a.block_splits(t_min) == a.n_split;
 }
 
 hipError_t launch_prefill_attn(const PrefillArgs& a, hipStream_t st) {
