@@ -306,8 +306,9 @@ int khq_layer_step(khq_layer* layer, const void* q_gate, const void* k_roped, co
  * reproduces those steps' results).  q_gate f16 [n][H_q][512], k_roped / v /
  * k_unroped f16 [n][H_kv][256], out f16 [n][H_q][256].  Token i is appended,
  * any compression event fires, and query i attends to the compressed prefix
- * and its raw window, as in step i; queries between events share one launch
- * (dense fp16 keys decoded from the compressed rows, MFMA attention).
+ * and its raw window, as in step i; up to 8,192 queries, on both sides of any
+ * number of events, share one launch (dense fp16 keys decoded from the
+ * compressed rows, MFMA attention).
  * Returns n, -100 on bad arguments, -102 at capacity, else an error code. */
 int khq_layer_prefill(khq_layer* layer, const void* q_gate, const void* k_roped, const void* v,
                       const void* k_unroped, void* out, int n, float scale, hipStream_t stream);
