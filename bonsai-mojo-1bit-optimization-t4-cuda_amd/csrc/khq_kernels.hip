@@ -404,6 +404,16 @@ void window_part_kernel(WinArgs a) {
             if (li < NREP) s_w[wave][4 * lg + c][li] = w;
         }
         mu::wave_sync();
+        // slots past the window hold its last V row again: 0 x inf is not 0
+        if (const int n = a.win_len - WIN_TILE * t; n < WIN_TILE)
+#pragma unroll
+            for (int p = 0; p < WIN_TILE; p += 4)
+                if (n < p + 4)
+#pragma unroll
+                    for (int j = p; j < p + 4; j++) {
+                        const uint32_t in = n > j ? ~0u : 0u;
+                        vr[j] = make_uint2(vr[j].x & in, vr[j].y & in);
+                    }
 #pragma unroll
         for (int p = 0; p < WIN_TILE; p++) {
             const mu::h4 v = __builtin_bit_cast(mu::h4, vr[p]);
@@ -431,27 +441,35 @@ void window_part_kernel(WinArgs a) {
     // score (m_ref = -inf) weighs nothing
     float l_row = l_part + __shfl_xor(l_part, 16, 64);
     l_row += __shfl_xor(l_row, 32, 64);
-    if (lane < NREP) {
-        s_ml[wave][lane][0] = m_ref;
-        s_ml[wave][lane][1] = l_row;
-    }
-    __syncthreads();
     float M[NREP], den[NREP];
+    if constexpr (NW == 1) {
 #pragma unroll
-    for (int i = 0; i < NREP; i++) {
-        M[i] = -INFINITY;
-#pragma unroll
-        for (int w = 0; w < NW; w++) M[i] = fmaxf(M[i], s_ml[w][i][0]);
-        den[i] = 0.0f;
-#pragma unroll
-        for (int w = 0; w < NW; w++) {
-            const float m = s_ml[w][i][0];
-            den[i] = fmaf(s_ml[w][i][1], m == M[i] ? 1.0f : mu::fexp(m - M[i]), den[i]);
+        for (int i = 0; i < NREP; i++) {
+            M[i] = from_lane(m_ref, i);
+            den[i] = from_lane(l_row, i);
         }
-        const float m = s_ml[wave][i][0];
-        const float f = m == M[i] ? 1.0f : mu::fexp(m - M[i]);
+    } else {
+        if (lane < NREP) {
+            s_ml[wave][lane][0] = m_ref;
+            s_ml[wave][lane][1] = l_row;
+        }
+        __syncthreads();
 #pragma unroll
-        for (int c = 0; c < 4; c++) acc[i][c] *= f;
+        for (int i = 0; i < NREP; i++) {
+            M[i] = -INFINITY;
+#pragma unroll
+            for (int w = 0; w < NW; w++) M[i] = fmaxf(M[i], s_ml[w][i][0]);
+            den[i] = 0.0f;
+#pragma unroll
+            for (int w = 0; w < NW; w++) {
+                const float m = s_ml[w][i][0];
+                den[i] = fmaf(s_ml[w][i][1], m == M[i] ? 1.0f : mu::fexp(m - M[i]), den[i]);
+            }
+            const float m = s_ml[wave][i][0];
+            const float f = m == M[i] ? 1.0f : mu::fexp(m - M[i]);
+#pragma unroll
+            for (int c = 0; c < 4; c++) acc[i][c] *= f;
+        }
     }
 #pragma unroll
     for (int half = NW / 2; half >= 1; half /= 2) {

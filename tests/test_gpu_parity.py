@@ -574,6 +574,25 @@ def test_fp16_attention_minus_inf_scores(device):
     assert np.abs(got - want).max() <= 2e-5 and np.abs(got_lse - lse).max() <= 2e-5
 
 
+@pytest.mark.parametrize("length", [13, 17, 40])
+def test_fp16_attention_infinite_value(device, length):
+    """An infinite V entry in the window's last slot, with a last tile that is
+    not full, gives that infinity in its dim and leaves the others alone."""
+    rng = np.random.default_rng(length)
+    qg = rng.standard_normal((24, 512)).astype(np.float16)
+    k, v = (rng.standard_normal((length, 4, D)).astype(np.float16) for _ in range(2))
+    want, _ = _window_want(qg[:, :D], k, v, SCALE)
+    v[length - 1, :, 7], v[length - 1, :, 200] = np.inf, -np.inf
+    want[:, 7], want[:, 200] = np.inf, -np.inf
+    tri = torch.zeros((24, D + 2), device=device, dtype=torch.float32)
+    ops.window_attn(t(qg), t(k), t(v), tri, win_start=0, win_len=length, ring_cap=length, H_q=24,
+                    H_kv=4, scale=SCALE)
+    got = npref.triple_to_out(tri.cpu().numpy())[0]
+    assert np.array_equal(got[:, [7, 200]], want[:, [7, 200]])
+    fin = np.isfinite(want)
+    assert np.abs(got[fin] - want[fin]).max() <= 2e-5  # as test_fp16_attention_sizes
+
+
 def test_partial_rope_matches_oracle(device):
     H = 24
     j = np.arange(H * 512)
