@@ -305,7 +305,8 @@ __global__ __launch_bounds__(256) void attn_part_kernel(AttnArgs a) {
 //     the lane-per-patch form this replaces spent a six-step wavefront sum on
 //     every (slot, head).  Lane (head li, lg) gets slots 4 lg .. + 3.
 //   softmax: per-head reference maximum, raised only when a tile exceeds it by
-//     more than 8; the state lives in the head's lanes.
+//     more than 8; the state lives in the head's lanes.  Weights above the
+//     reference reach e^8, where __expf is off by 3e-7: exp32.
 //   P x V: fp32 weights broadcast through LDS (one read of the slot's heads),
 //     lane p owning dims 4 p .. + 3 of every V row (512 contiguous bytes a row);
 //     24 multiply-adds a slot leave the vector ALUs a quarter busy.
@@ -369,9 +370,13 @@ void window_part_kernel(WinArgs a) {
         load_v(t);
     }
     for (; t < t_hi; t += NW) {
-        mu::f4 s = mu::f4{0.f, 0.f, 0.f, 0.f};
+        mu::f4 s = mu::f4{0.f, 0.f, 0.f, 0.f}, s1 = s;
 #pragma unroll
-        for (int st = 0; st < 8; st++) s = mu::mfma32(__builtin_bit_cast(mu::h8, kr[st]), q[st], s);
+        for (int st = 0; st < 8; st += 2) {  // two chains: a block of one tile waits for this
+            s = mu::mfma32(__builtin_bit_cast(mu::h8, kr[st]), q[st], s);
+            s1 = mu::mfma32(__builtin_bit_cast(mu::h8, kr[st + 1]), q[st + 1], s1);
+        }
+        s += s1;
         if (t + NW < t_hi) load_k(t + NW);
         float sc[4], mx = -INFINITY;
 #pragma unroll
@@ -387,7 +392,7 @@ void window_part_kernel(WinArgs a) {
         mx = fmaxf(__uint_as_float(p32[0]), __uint_as_float(p32[1]));
         const bool need = mx > m_ref + 8.0f;
         if (__ballot(need) != 0ull) {
-            const float fac = need ? mu::fexp(m_ref - mx) : 1.0f;  // 0 when m_ref = -inf
+            const float fac = need ? (m_ref == -INFINITY ? 0.0f : mu::exp32(m_ref - mx)) : 1.0f;
             m_ref = need ? mx : m_ref;
             l_part *= fac;
 #pragma unroll
@@ -399,7 +404,7 @@ void window_part_kernel(WinArgs a) {
         }
 #pragma unroll
         for (int c = 0; c < 4; c++) {
-            const float w = sc[c] == -INFINITY ? 0.0f : mu::fexp(sc[c] - m_ref);
+            const float w = sc[c] == -INFINITY ? 0.0f : mu::exp32(sc[c] - m_ref);
             l_part += w;
             if (li < NREP) s_w[wave][4 * lg + c][li] = w;
         }
@@ -427,7 +432,7 @@ void window_part_kernel(WinArgs a) {
                     acc[i][c] = fmaf((float)v[c], w[i >> 2][i & 3], acc[i][c]);
             // sums of four slots complete before the next slots' weights are
             // read (all sixteen at once take 254 registers and spill at 8 heads)
-            if ((p & 3) == 3)
+            if (NREP > 4 && (p & 3) == 3)
 #pragma unroll
                 for (int i = 0; i < NREP; i++)
                     asm volatile("" : "+v"(acc[i][0]), "+v"(acc[i][1]), "+v"(acc[i][2]), "+v"(acc[i][3])
@@ -441,34 +446,21 @@ void window_part_kernel(WinArgs a) {
     // score (m_ref = -inf) weighs nothing
     float l_row = l_part + __shfl_xor(l_part, 16, 64);
     l_row += __shfl_xor(l_row, 32, 64);
-    float M[NREP], den[NREP];
-    if constexpr (NW == 1) {
-#pragma unroll
-        for (int i = 0; i < NREP; i++) {
-            M[i] = from_lane(m_ref, i);
-            den[i] = from_lane(l_row, i);
-        }
-    } else {
-        if (lane < NREP) {
-            s_ml[wave][lane][0] = m_ref;
-            s_ml[wave][lane][1] = l_row;
-        }
+    float m_row = m_ref;
+    if constexpr (NW > 1) {
+        const int head = min(li, NREP - 1);
+        if (lane < NREP) s_ml[wave][lane][0] = m_ref;
         __syncthreads();
 #pragma unroll
+        for (int w = 0; w < NW; w++) m_row = fmaxf(m_row, s_ml[w][head][0]);
+        // one exponential a lane, of its head, then to the others
+        const float f = m_ref == m_row ? 1.0f : m_ref == -INFINITY ? 0.0f : mu::exp32(m_ref - m_row);
+        if (lane < NREP) s_ml[wave][lane][1] = l_row * f;
+#pragma unroll
         for (int i = 0; i < NREP; i++) {
-            M[i] = -INFINITY;
+            const float fi = from_lane(f, i);
 #pragma unroll
-            for (int w = 0; w < NW; w++) M[i] = fmaxf(M[i], s_ml[w][i][0]);
-            den[i] = 0.0f;
-#pragma unroll
-            for (int w = 0; w < NW; w++) {
-                const float m = s_ml[w][i][0];
-                den[i] = fmaf(s_ml[w][i][1], m == M[i] ? 1.0f : mu::fexp(m - M[i]), den[i]);
-            }
-            const float m = s_ml[wave][i][0];
-            const float f = m == M[i] ? 1.0f : mu::fexp(m - M[i]);
-#pragma unroll
-            for (int c = 0; c < 4; c++) acc[i][c] *= f;
+            for (int c = 0; c < 4; c++) acc[i][c] *= fi;
         }
     }
 #pragma unroll
@@ -490,18 +482,24 @@ void window_part_kernel(WinArgs a) {
             }
         __syncthreads();
     }
+    if constexpr (NW > 1) {
+        l_row = 0.0f;
+#pragma unroll
+        for (int w = 0; w < NW; w++) l_row += s_ml[w][min(li, NREP - 1)][1];
+    }
     if (wave != 0) return;
 #pragma unroll
     for (int i = 0; i < NREP; i++) {
         const int h = hkv * NREP + i;
         float* out = a.part + ((size_t)h * a.part_stride + a.part_offset + part) * 258;
-        const bool empty = M[i] == -INFINITY;
         *reinterpret_cast<float2*>(out + 4 * lane) = make_float2(acc[i][0], acc[i][1]);
         *reinterpret_cast<float2*>(out + 4 * lane + 2) = make_float2(acc[i][2], acc[i][3]);
-        if (lane == 0) {
-            out[256] = empty ? -1e20f : M[i];
-            out[257] = empty ? 0.0f : den[i];
-        }
+    }
+    if (lane < NREP) {
+        const bool empty = m_row == -INFINITY;
+        float* ml = a.part + ((size_t)(hkv * NREP + lane) * a.part_stride + a.part_offset + part) * 258 + 256;
+        ml[0] = empty ? -1e20f : m_row;
+        ml[1] = empty ? 0.0f : l_row;
     }
 }
 

@@ -64,7 +64,16 @@ __device__ __forceinline__ void sincos_rev(float th, float& c, float& s) {
     s = __builtin_amdgcn_sinf(rf);
 }
 
+// e^x, finite x: __expf rounds x log2(e) to fp32 and is off by |x| 2^-24 for it.
 __device__ __forceinline__ float fexp(float x) { return __expf(x); }
+// e^x, finite x < 88, to about a unit in the last place (0 below e^-87):
+// 2^hi of the hardware times e^(ln2 lo), x log2(e) = hi + lo.
+__device__ __forceinline__ float exp32(float x) {
+    const float hi = x * 1.44269502f;
+    const float lo = fmaf(x, 1.92596303e-8f, fmaf(x, 1.44269502f, -hi));
+    const float y = __builtin_amdgcn_exp2f(hi);
+    return fmaf(y, lo * 0.693147181f, y);
+}
 
 // hi + lo fp16 split of two floats (hi truncated, lo carries the rest).
 __device__ __forceinline__ void split2(float x, float y, _Float16& xh, _Float16& yh,

@@ -593,6 +593,30 @@ def test_fp16_attention_infinite_value(device, length):
     assert np.abs(got[fin] - want[fin]).max() <= 2e-5  # as test_fp16_attention_sizes
 
 
+def test_fp16_attention_weight_rounding(device):
+    """Weights above a wavefront's reference maximum (it is raised only past
+    e^8) keep full fp32 precision: 64 heads whose later tiles score x in
+    (4, 7.9) over earlier ones at 0, each sum of weights against float64.  An
+    exponential rounded once and some ten fp32 additions give an rms error of
+    half a unit in the last place or so (2^-24 = 6e-8); one that rounds
+    x log2(e) first is off by up to 2^-21 ln 2 = 3.3e-7, rms 1.9e-7."""
+    H, length = 64, 16 * 36  # parts of 8 tiles: two a wavefront
+    x = np.random.default_rng(5).uniform(4, 7.9, H).astype(np.float16)
+    q = np.zeros((H, 512), np.float16)
+    q[:, 0] = 1
+    k, v = np.zeros((length, H, D), np.float16), np.ones((length, H, D), np.float16)
+    late = np.arange(length) // 16 % 8 >= 4
+    k[late, :, 0] = x
+    tri = torch.zeros((H, D + 2), device=device, dtype=torch.float32)
+    ops.window_attn(t(q), t(k), t(v), tri, win_start=0, win_len=length, ring_cap=length, H_q=H, H_kv=H,
+                    scale=1.0)
+    tr, xd = tri.cpu().numpy().astype(np.float64), x.astype(np.float64)
+    got = tr[:, D + 1] * np.exp(tr[:, D] - xd)
+    want = late.sum() + (~late).sum() * np.exp(-xd)
+    err = got / want - 1
+    assert np.sqrt(np.mean(err ** 2)) <= 1e-7, np.sqrt(np.mean(err ** 2))
+
+
 def test_partial_rope_matches_oracle(device):
     H = 24
     j = np.arange(H * 512)
