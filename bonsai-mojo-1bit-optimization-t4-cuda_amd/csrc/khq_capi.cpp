@@ -34,6 +34,7 @@ int rc_of(hipError_t e) { return e == hipSuccess ? 0 : static_cast<int>(e); }
 // allocated, so an earlier graph keeps replaying into memory it owns.  A
 // captured call that would need to grow the workspace fails instead
 // (hipErrorStreamCaptureUnsupported): reserve before capture.
+constexpr size_t kMinWorkspace = (size_t)4 << 20;
 struct Workspace {
     void* p = nullptr;
     size_t bytes = 0;
@@ -64,7 +65,7 @@ hipError_t workspace(size_t bytes, hipStream_t stream, float** out, bool use = t
         // growing under capture would bake a pointer that is freed later, and
         // the synchronisation it needs is illegal there: reserve beforehand
         if (cap) return hipErrorStreamCaptureUnsupported;
-        size_t want = std::max(bytes, (size_t)4 << 20);
+        size_t want = std::max(bytes, kMinWorkspace);
         if (w.p) {
             if (w.in_graph) {
                 // a graph captured earlier replays into the old buffer: keep
@@ -173,17 +174,27 @@ int compressed_parts(int c_len, int n_rep, int h_kv, int L_q) {
 
 // fp16 window work: 16-slot tiles, one per wavefront at a time.  While the
 // tiles fit two a CU each is a block of its own (one CU loads a tile's 16 KB
-// far slower than 256 do), at most max_parts a KV head; beyond that blocks of
-// 4 wavefronts, two a CU.
+// far slower than 256 do); beyond that blocks of 4 wavefronts, two a CU, or up
+// to a quarter more where that keeps a wavefront at one tile (32 KV heads of
+// one query head, 1,100 positions: 288 blocks 14.7 us, 576 13.2).
 int window_waves(int win_len, int h_kv) {
     return (win_len + 15) / 16 * h_kv <= 2 * khq::device_cu_count() ? 1 : 4;
 }
-int window_parts(int win_len, int h_kv, int waves, int max_parts = 1024) {
+// Parts a KV head, at most max_parts.
+int window_parts(int win_len, int h_kv, int waves, int max_parts) {
     const int groups = ((win_len + 15) / 16 + waves - 1) / waves;
-    const int cap = waves == 1 ? groups : 2 * khq::device_cu_count() / h_kv;
+    int cap = waves == 1 ? groups : 2 * khq::device_cu_count() / h_kv;
+    if (groups <= cap + cap / 4) cap = groups;
     const int want = std::max(1, std::min({groups, cap, max_parts}));
     const int per = (groups + want - 1) / want * waves;  // tiles a part
     return ((win_len + 15) / 16 + per - 1) / per;
+}
+// Part limits of the two fp16 entries: the merge has every load in flight up to
+// 256 parts (1 KV head, 8,192 positions: 512 parts 12.5 us, 256 7.7), and the
+// window entry's parts fit the smallest workspace there is, or are 64.
+constexpr int kMaxGqaParts = 256;
+int max_window_parts(int H_q) {
+    return std::max(64, std::min(256, (int)(kMinWorkspace / (H_q * 258 * sizeof(float)))));
 }
 
 khq::AttnArgs attn_args(const void* q, const void* k_payload, const void* v_payload,
@@ -371,7 +382,7 @@ int launch_khq_window_attn_fp16(const void* q, const void* ring_k, const void* r
         win_len > ring_cap || win_start < 0)
         return -100;
     const int waves = window_waves(win_len, H_kv);
-    const int np = window_parts(win_len, H_kv, waves);
+    const int np = window_parts(win_len, H_kv, waves, max_window_parts(H_q));
     float* ws = static_cast<float*>(out_attn);  // one part: the triple itself
     hipError_t e = hipSuccess;
     if (np > 1) e = workspace((size_t)H_q * np * 258 * sizeof(float), stream, &ws);
@@ -446,7 +457,7 @@ int launch_khq_gqa_attn_fp16(const void* q_gate, const void* k_cache, const void
         H_q / H_kv > 8)
         return -100;
     const int waves = window_waves(seq_len, H_kv);
-    const int np = window_parts(seq_len, H_kv, waves);
+    const int np = window_parts(seq_len, H_kv, waves, kMaxGqaParts);
     float* ws = nullptr;
     hipError_t e = workspace((size_t)H_q * np * 258 * sizeof(float), stream, &ws);
     if (e != hipSuccess) return rc_of(e);
