@@ -340,19 +340,19 @@ void window_part_kernel(WinArgs a) {
         const __half* qp = a.q + (size_t)(hkv * NREP + min(li, NREP - 1)) * 512 + 8 * lg;
 #pragma unroll
         for (int st = 0; st < 8; st++)
-            q[st] = __builtin_bit_cast(mu::h8, *reinterpret_cast<const uint4*>(qp + 32 * st));
+            q[st] = __builtin_bit_cast(mu::h8, *reinterpret_cast<const mu::u4h*>(qp + 32 * st));
     }
-    uint4 kr[8];
-    uint2 vr[WIN_TILE];
+    mu::u4h kr[8];
+    mu::u2h vr[WIN_TILE];
     auto load_k = [&](int t) {
         const __half* kp = kbase + slot_of(WIN_TILE * t + li) * row;
 #pragma unroll
-        for (int st = 0; st < 8; st++) kr[st] = *reinterpret_cast<const uint4*>(kp + 32 * st);
+        for (int st = 0; st < 8; st++) kr[st] = *reinterpret_cast<const mu::u4h*>(kp + 32 * st);
     };
     auto load_v = [&](int t) {
 #pragma unroll
         for (int i = 0; i < WIN_TILE; i++)
-            vr[i] = *reinterpret_cast<const uint2*>(vbase + slot_of(WIN_TILE * t + i) * row);
+            vr[i] = *reinterpret_cast<const mu::u2h*>(vbase + slot_of(WIN_TILE * t + i) * row);
     };
     float acc[NREP][4];
 #pragma unroll
@@ -417,7 +417,7 @@ void window_part_kernel(WinArgs a) {
 #pragma unroll
                     for (int j = p; j < p + 4; j++) {
                         const uint32_t in = n > j ? ~0u : 0u;
-                        vr[j] = make_uint2(vr[j].x & in, vr[j].y & in);
+                        vr[j] &= in;
                     }
 #pragma unroll
         for (int p = 0; p < WIN_TILE; p++) {
@@ -492,8 +492,8 @@ void window_part_kernel(WinArgs a) {
     for (int i = 0; i < NREP; i++) {
         const int h = hkv * NREP + i;
         float* out = a.part + ((size_t)h * a.part_stride + a.part_offset + part) * 258;
-        *reinterpret_cast<float2*>(out + 4 * lane) = make_float2(acc[i][0], acc[i][1]);
-        *reinterpret_cast<float2*>(out + 4 * lane + 2) = make_float2(acc[i][2], acc[i][3]);
+        *reinterpret_cast<mu::f2s*>(out + 4 * lane) = mu::f2s{acc[i][0], acc[i][1]};
+        *reinterpret_cast<mu::f2s*>(out + 4 * lane + 2) = mu::f2s{acc[i][2], acc[i][3]};
     }
     if (lane < NREP) {
         const bool empty = m_row == -INFINITY;

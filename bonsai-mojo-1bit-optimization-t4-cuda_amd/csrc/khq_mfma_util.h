@@ -17,6 +17,13 @@ typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 typedef _Float16 h4 __attribute__((ext_vector_type(4)));
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef float f4 __attribute__((ext_vector_type(4)));
+// The same widths at addresses with no more than their elements' alignment (a
+// caller's halves, triples of 258 floats): one load or store all the same.
+typedef uint32_t u4h __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t u2h __attribute__((ext_vector_type(2), aligned(2)));
+typedef float f4s __attribute__((ext_vector_type(4), aligned(4)));
+typedef float f2s __attribute__((ext_vector_type(2), aligned(4)));
+typedef uint32_t u1b __attribute__((aligned(1)));  // a word of packed bytes
 
 __device__ __forceinline__ f4 mfma32(h8 a, h8 b, f4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);

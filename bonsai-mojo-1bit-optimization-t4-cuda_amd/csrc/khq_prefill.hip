@@ -91,9 +91,9 @@ __device__ __forceinline__ void decompress_block(const DecompArgs& a, int bx, in
         const int i = i0 + threadIdx.x, tl = i / 52, w = i % 52;
         if (i < TB * 52) {
             const size_t g = row_of(tl);
-            const uint32_t* src = w < 16   ? a.kmask + g * 16 + w
-                                  : w < 26 ? reinterpret_cast<const uint32_t*>(a.kpay + g * 40) + w - 16
-                                           : reinterpret_cast<const uint32_t*>(a.vpay + g * 104) + w - 26;
+            const u1b* src = w < 16   ? reinterpret_cast<const u1b*>(a.kmask + g * 16) + w
+                             : w < 26 ? reinterpret_cast<const u1b*>(a.kpay + g * 40) + w - 16
+                                      : reinterpret_cast<const u1b*>(a.vpay + g * 104) + w - 26;
             L.pay[tl][w] = *src;
         }
     }
@@ -101,7 +101,7 @@ __device__ __forceinline__ void decompress_block(const DecompArgs& a, int bx, in
         const int tl = threadIdx.x / 5, f = threadIdx.x % 5;
         const size_t g = row_of(tl);
         const __half* n = f == 0 ? a.knorm : f == 1 ? a.krn : f == 2 ? a.vnorm : a.vrn;
-        L.nrm[tl][f] = f == 4 ? __uint_as_float(*reinterpret_cast<const uint32_t*>(a.vsm + g * 4))
+        L.nrm[tl][f] = f == 4 ? __uint_as_float(*reinterpret_cast<const u1b*>(a.vsm + g * 4))
                               : __half2float(n[g]);
     }
     dec::Consts cs;
@@ -376,7 +376,7 @@ __device__ __forceinline__ void store_rows(const PrefillArgs& a, const float* so
     float* part = a.part + (size_t)split * 258;
 #pragma unroll 8
     for (int i = 0; i < n; i++)
-        *reinterpret_cast<f4*>(part + row_of(row0 + i) * a.n_split * 258 + 4 * lane) =
+        *reinterpret_cast<f4s*>(part + row_of(row0 + i) * a.n_split * 258 + 4 * lane) =
             *reinterpret_cast<const f4*>(&so[i * OUT_LD + 4 * lane]);
     if (lane < n) {
         float* ml = part + row_of(row0 + lane) * a.n_split * 258 + 256;

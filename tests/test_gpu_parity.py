@@ -593,6 +593,32 @@ def test_fp16_attention_infinite_value(device, length):
     assert np.abs(got[fin] - want[fin]).max() <= 2e-5  # as test_fp16_attention_sizes
 
 
+@pytest.mark.parametrize("length", [7, 300, 2100])
+def test_fp16_attention_unaligned(device, length):
+    """q, K and V at odd half addresses and the triple at an odd float address:
+    the entries ask for no more than their elements' alignment, and the results
+    are those of aligned tensors bit for bit."""
+    rng = np.random.default_rng(length)
+    q = t(rng.standard_normal((24, 512)).astype(np.float16))
+    k, v = (t(rng.standard_normal((length, 4, D)).astype(np.float16)) for _ in range(2))
+
+    def odd(x):
+        flat = torch.empty(x.numel() + 1, device=device, dtype=x.dtype)[1:]
+        flat.copy_(x.reshape(-1))
+        return flat.view(x.shape)
+
+    res = []
+    for place in (lambda x: x, odd):
+        tri = place(torch.zeros((24, D + 2), device=device, dtype=torch.float32))
+        out = place(torch.zeros((24, D), device=device, dtype=torch.float16))
+        ops.window_attn(place(q), place(k), place(v), tri, win_start=3, win_len=length,
+                        ring_cap=length, H_q=24, H_kv=4, scale=SCALE)
+        ops.gqa_attn(place(q), place(k), place(v), out, seq_len=length, H_q=24, H_kv=4, scale=SCALE)
+        res.append((tri.cpu(), out.cpu()))
+    assert torch.equal(res[0][0], res[1][0]) and torch.equal(res[0][1], res[1][1])
+    assert res[0][0].abs().max() > 0 and res[0][1].abs().max() > 0
+
+
 def test_fp16_attention_weight_rounding(device):
     """Weights above a wavefront's reference maximum (it is raised only past
     e^8) keep full fp32 precision: 64 heads whose later tiles score x in

@@ -300,6 +300,30 @@ def test_decompress_long_matches_short(device):
     assert (outs[0][1][:, :, 2116:] == np.float16(7.0).view(np.uint16)).all()
 
 
+def test_decompress_unaligned_payload(device):
+    """Payload bytes at an odd address (they are bytes to the caller) and norms
+    at an odd half address decode to the same bits as aligned ones."""
+    lc, _ = layer_consts(layer_id=2)
+    n = 70
+    cents, pay = ops.Centroids(lc, device), ops.Payload(n * H_KV, device)
+    synth.compressed_rows(pay, cents, seed=6)
+    odd = ops.Payload(n * H_KV, device)
+    for name in ("kpay", "knorm", "krn", "vpay", "vnorm", "vrn", "vsm"):
+        x = getattr(pay, name)
+        flat = torch.empty(x.numel() + 1, device=device, dtype=x.dtype)[1:]
+        flat.copy_(x.reshape(-1))
+        setattr(odd, name, flat.view(x.shape))
+    odd.kmask.copy_(pay.kmask)
+    outs = []
+    for p in (pay, odd):
+        k = torch.zeros((n, H_KV, D), device=device, dtype=torch.float16)
+        vt = torch.zeros((H_KV, D, 128), device=device, dtype=torch.float16)
+        ops.decompress(p, cents, k, vt, H_kv=H_KV, tok0=0, n_tok=n, key0=0, ld_vt=128)
+        outs.append((k, vt))
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+    assert outs[0][0].abs().max() > 0 and outs[0][1].abs().max() > 0
+
+
 def test_c5_chunk_vs_oracle(device):
     """Config 5: 8,192 tokens already appended (boundary 8,064, raw 8,064..
     8,191), then one chunk of 128 tokens at positions 8,192..8,319; the 128th
