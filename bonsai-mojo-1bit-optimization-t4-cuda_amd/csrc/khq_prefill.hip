@@ -673,9 +673,11 @@ void prefill_attn_rs_kernel(PrefillArgs a) {
         // Weights are rounded to fp16 except a row's reference key's, which is 1.
         // Blocks that run all their keys in one go raise the reference at every
         // new maximum of the first 8 tiles, so a row of few keys (where one
-        // weight counts) has its largest one exact; splits had that from their
-        // several references.
-        const int n_eager = bk.n_split == 1 ? 8 : 0;
+        // weight counts) has its largest one exact; splits have that from their
+        // several references.  A layer's pass has fewer of them than one launch
+        // per event had, and raises it so too: 200 tokens after 300, 2.86e-4 from
+        // float64 without, 2.68e-4 with, 2.72e-4 in a launch per event.
+        const int n_eager = bk.n_split == 1 || a.ev_cap > 0 ? 8 : 0;
         const float sc2 = a.sc * LOG2E;  // scores in log2 units: a weight is one exp2
         float m_ref = M_NONE;
         f32x16 s2[2];
@@ -1083,12 +1085,18 @@ void prefill_plan(PrefillArgs& a) {
     const bool even = t_max - t_min <= t_max / 8;
     const float gate = 0.29f * std::min(16, n_rows);
     const int step = std::max(1, nb / 64);  // enough blocks to add up
+    // At least as many splits as one round holds: a weight is rounded to fp16
+    // but for its tile's largest where that sets the reference (a split's first
+    // tile), so short splits lose less.  16 queries over 900 tokens, whatever is
+    // faster (10 splits): 2.80e-4 from float64, 29 splits of a tile 2.53e-4, the
+    // output's own rounding being 2.07e-4.
+    const int k_min = std::max(1, std::min({64, t_max, slots / (nb * a.h_kv)}));
     float best = 0.0f;
-    int best_k = 1;
-    for (int k = 1; k <= std::min(64, t_max); k++) {
+    int best_k = k_min;
+    for (int k = k_min; k <= std::min(64, t_max); k++) {
         a.n_split = k;
         a.unit = (t_max + k - 1) / k;
-        if (k > 1 && (size_t)a.n_q * a.h_kv * a.n_rep * k * 258 * 4 > (size_t)1 << 30) break;
+        if (k > k_min && (size_t)a.n_q * a.h_kv * a.n_rep * k * 258 * 4 > (size_t)1 << 30) break;
         float units = 0.0f, tiles = 0.0f;
         for (int b = 0; b < nb; b += step) {
             int nd, u0;
@@ -1107,7 +1115,7 @@ void prefill_plan(PrefillArgs& a) {
         } else if (rounds <= 1.0f) {
             est += gate;
         }
-        if (k == 1 || est < best) {
+        if (k == k_min || est < best) {
             best = est;
             best_k = k;
             a.apart = apart;

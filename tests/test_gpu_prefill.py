@@ -430,6 +430,42 @@ def test_prefill_attn_plans_vs_float64(device, n_q, n_k):
         close(got[j:j + 1], want)
 
 
+@pytest.mark.parametrize("n_q,past", [(16, 900), (21, 200), (32, 900), (128, 60)])
+def test_prefill_attn_weight_rounding(device, n_q, past):
+    """Short launches run one tile of 32 keys a split, so each tile's largest
+    weight is exact (1 against the split's reference) and only the others are
+    rounded to fp16.  A rounding to fp16 is off by 2^-11 / sqrt(3) of the
+    mantissa's lower end, 2.07e-4 rms over its range (log-uniform), and with
+    random V the errors of the weights add up as the weights do: the relative
+    error is 2.07e-4 sqrt(2 - s), s the share of the exact weights in the sum of
+    squares.  A few per cent for the sampled rows."""
+    rng = np.random.default_rng(n_q)
+    n_k = past + n_q
+    q = rng.standard_normal((n_q, H_Q, 2 * D)).astype(np.float16)
+    K, V = (rng.standard_normal((n_k, H_KV, D)).astype(np.float16) for _ in range(2))
+    ld = ops.vt_ld(n_k)
+    vt = torch.zeros((H_KV, D, ld), device=device, dtype=torch.float16)
+    vt[:, :, :n_k] = t(V).permute(1, 2, 0)
+    out = torch.zeros((n_q, H_Q, D), device=device, dtype=torch.float16)
+    ops.prefill_attn(t(q), t(K), vt, out, ld_vt=ld, n_k=n_k, n_q=n_q, vis0=past + 1, H_q=H_Q, H_kv=H_KV,
+                     scale=SCALE)
+    got = out.cpu().numpy().astype(np.float64)
+    num = den = top = tot = 0.0
+    for j in sorted({0, n_q // 2, n_q - 1, *range(3, n_q, 11)}):
+        vis = past + 1 + j
+        for h in range(H_Q):
+            w = K[:vis, h // N_REP].astype(np.float64) @ q[j, h, :D].astype(np.float64) * SCALE
+            w = np.exp(w - w.max())
+            w /= w.sum()
+            want = (w @ V[:vis, h // N_REP].astype(np.float64)) * npref.sigmoid(q[j, h, D:].astype(np.float64))
+            num += ((got[j, h] - want) ** 2).sum()
+            den += (want ** 2).sum()
+            tot += (w ** 2).sum()
+            top += sum((w[i:i + 32].max()) ** 2 for i in range(0, vis, 32))
+    bound = 2.07e-4 * np.sqrt(2 - top / tot)
+    assert np.sqrt(num / den) <= 1.04 * bound, (np.sqrt(num / den), bound)
+
+
 def test_layer_prefill_mixed_with_steps(device):
     """Prefill chunks and single steps interleaved on one layer (the dense key
     space must not keep raw tokens the steps wrote only to the ring) against
