@@ -228,6 +228,25 @@ struct GatherArgs {
     __half* out_vt;
     int h_kv, n, key0, ld_vt;
 };
+// Division of any 32-bit n by a launch constant d: multiply and shift (Granlund
+// and Montgomery, 1994).  A block's index arithmetic is on the scalar unit with
+// it; the compiler's division by a variable is some 25 vector instructions.
+struct FastDiv {
+    uint32_t d, mul;
+    int s1, s2;
+    FastDiv() = default;
+    explicit FastDiv(uint32_t d_) : d(d_) {
+        int l = 0;
+        while (l < 32 && ((uint64_t)1 << l) < d) l++;
+        mul = (uint32_t)((((uint64_t)1 << 32) * (((uint64_t)1 << l) - d)) / d + 1);
+        s1 = l < 1 ? l : 1;
+        s2 = l > 1 ? l - 1 : 0;
+    }
+    __host__ __device__ int div(uint32_t n) const {
+        const uint32_t t = (uint32_t)(((uint64_t)mul * n) >> 32);
+        return (int)((t + ((n - t) >> s1)) >> s2);
+    }
+};
 // n tokens of src_k / src_v / src_u [t][h_kv][256] -> ring slots
 // (slot0 + t) % ring_cap (n <= ring_cap).
 struct RingArgs {
@@ -238,6 +257,7 @@ struct RingArgs {
     __half* ring_v;
     __half* ring_u;
     int h_kv, n, slot0, ring_cap;
+    FastDiv by_token;  // 8-byte pieces per token, filled by the launcher
 };
 // n_q queries (q_gate rows [n_q][H_q][512]) over two runs of dense keys:
 // decoded tokens at key indices [0, ..) and raw tokens at raw0 + r, r < n_raw
@@ -248,9 +268,9 @@ struct RingArgs {
 // 128 more every 128 tokens, at most ev_cap (dec0 and ev_cap multiples of
 // 128; ev_cap = 0: every key is raw).
 // Rows of one KV head (query j, head r % n_rep) are cut into blocks, a block's
-// 32-key tiles into ceil(tiles / unit) splits (at most n_split).  Blocks of one
-// split write out directly unless apart; split s of the others leaves the triple
-// of (query j, head hq) at part[((j * H_q + hq) * n_split + s) * 258].
+// 32-key tiles into splits of `unit` (at most n_split).  Blocks of one split write
+// out directly unless apart; split s of the others leaves the triple of (query j,
+// head hq) at part[((j * H_q + hq) * n_split + s) * 258].
 struct PrefillArgs {
     const __half* q;
     const __half* k;
@@ -259,27 +279,25 @@ struct PrefillArgs {
     __half* out;  // NULL: triples only (apart)
     int ld_vt, n_q, h_kv, n_rep, n_split, unit;
     bool apart;    // every block leaves triples
-    bool uniform;  // every block has n_split splits
+    bool uniform;  // every row has n_split triples
     int vis0, n_raw, raw0, dec0, ev_cap;
     float sc, eps;
+    FastDiv by_rep, by_hq, by_kv, by_split, by_unit;  // n_rep, H_q, h_kv, n_split, unit
     __host__ __device__ int bound(int vis) const {
         if (ev_cap <= 0 || vis < 256) return 0;
-        const int b = ((vis - 256) / 128 + 1) * 128;
+        const int b = (((vis - 256) >> 7) + 1) << 7;
         return b < ev_cap ? b : ev_cap;
     }
     __host__ __device__ int vis_of(int j) const { return vis0 + j < n_raw ? vis0 + j : n_raw; }
     // Tiles of a block of rows [row_first, row_last]: tile i is decoded tile i
     // for i < nd, then raw tile u0 + i - nd.
     __host__ __device__ int block_tiles(int row_first, int row_last, int* nd, int* u0) const {
-        const int vf = vis_of(row_first / n_rep), vl = vis_of(row_last / n_rep);
-        *nd = (dec0 + bound(vl)) / 32;
-        *u0 = bound(vf) / 32;
-        return *nd + (vl + 31) / 32 - *u0;
+        const int vf = vis_of(by_rep.div(row_first)), vl = vis_of(by_rep.div(row_last));
+        *nd = (dec0 + bound(vl)) >> 5;
+        *u0 = bound(vf) >> 5;
+        return *nd + ((vl + 31) >> 5) - *u0;
     }
-    __host__ __device__ int block_splits(int tiles) const {
-        const int s = (tiles + unit - 1) / unit;
-        return s < n_split ? s : n_split;
-    }
+    __host__ __device__ int block_splits(int tiles) const { return by_unit.div(tiles + unit - 1); }
 };
 hipError_t launch_decompress(const DecompArgs& a, hipStream_t st);
 hipError_t launch_ring_gather(const GatherArgs& a, hipStream_t st);

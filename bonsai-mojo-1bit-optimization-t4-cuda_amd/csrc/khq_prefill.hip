@@ -142,33 +142,37 @@ __device__ __forceinline__ void decompress_block(const DecompArgs& a, int bx, in
 }
 
 // ------------------------------------------------------------- raw gather
-// Block (32 raw tokens, KV head h): K rows copied, V rows transposed through
-// LDS, every row of the block in flight at once.  Tokens past the last give
-// zero V^T columns.
+// Block (32 raw tokens, KV head h), eight a wavefront: K rows copied, V rows
+// transposed through LDS, every row of the block in flight at once.  Tokens past
+// the last give zero V^T columns.  A lane's eight tokens go to LDS as one 16-byte
+// piece a dim: as single halves (32 stores a lane, 32 lanes to a bank) they took
+// 1.7 us of a short prompt.
 __device__ __forceinline__ void gather_block(const GatherArgs& a, int bx, int h, void* lds) {
     VtTile<32>& sv = *static_cast<VtTile<32>*>(lds);
-    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int t_blk = bx * 32;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int t0 = bx * 32 + wv * 8;
     uint2 kw[8], vw[8];
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-        const int t = t_blk + wv + 4 * i;
-        const int r = min(t, a.n - 1) * a.h_kv + h;
+        const int r = min(t0 + i, a.n - 1) * a.h_kv + h;
         kw[i] = *reinterpret_cast<const uint2*>(a.k.row(r) + 4 * lane);
         vw[i] = *reinterpret_cast<const uint2*>(a.v.row(r) + 4 * lane);
     }
+    h8 col[4];
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-        const int tl = wv + 4 * i, t = t_blk + tl;
+        const int t = t0 + i;
         if (t < a.n)
             *reinterpret_cast<uint2*>(a.out_k + ((size_t)(a.key0 + t) * a.h_kv + h) * 256 + 4 * lane) =
                 kw[i];
         const h4 v = __builtin_bit_cast(h4, t < a.n ? vw[i] : uint2{0u, 0u});
 #pragma unroll
-        for (int c = 0; c < 4; c++) sv[4 * lane + c][tl] = v[c];
+        for (int c = 0; c < 4; c++) col[c][i] = v[c];
     }
+#pragma unroll
+    for (int c = 0; c < 4; c++) *reinterpret_cast<h8*>(&sv[4 * lane + c][8 * wv]) = col[c];
     __syncthreads();
-    store_vt<32>(sv, a.out_vt, a.ld_vt, h, a.key0 + t_blk, 32);
+    store_vt<32>(sv, a.out_vt, a.ld_vt, h, a.key0 + bx * 32, 32);
 }
 // Flat block index of a gather: token block fastest, then the KV head.
 __device__ __forceinline__ void gather_flat(const GatherArgs& a, int b, void* lds) {
@@ -276,20 +280,9 @@ struct RowKeys {
 };
 // The block's tile list (PrefillArgs) and this split's part of it.
 struct BlockKeys {
-    int nd, u0, t_lo, t_hi, n_split;
-    __device__ __forceinline__ BlockKeys(const PrefillArgs& a, int row_first, int row_last, int split) {
-        const int n = a.block_tiles(row_first, row_last, &nd, &u0);
-        n_split = a.block_splits(n);
-        const int per = (n + n_split - 1) / n_split;
-        t_lo = min(n, split * per);
-        t_hi = min(n, t_lo + per);
-        // the divisions run on the vector ALU: back to scalars
-        nd = __builtin_amdgcn_readfirstlane(nd);
-        u0 = __builtin_amdgcn_readfirstlane(u0);
-        t_lo = __builtin_amdgcn_readfirstlane(t_lo);
-        t_hi = __builtin_amdgcn_readfirstlane(t_hi);
-        n_split = __builtin_amdgcn_readfirstlane(n_split);
-    }
+    int nd, u0, t_lo, t_hi;
+    __device__ __forceinline__ BlockKeys(const PrefillArgs& a, int nd_, int u0_, int n, int split)
+        : nd(nd_), u0(u0_), t_lo(min(n, split * a.unit)), t_hi(min(n, t_lo + a.unit)) {}
     __device__ __forceinline__ bool dec(int t) const { return t < nd; }
     __device__ __forceinline__ int base(int t) const { return 32 * (t < nd ? t : u0 + t - nd); }
 };
@@ -298,15 +291,16 @@ struct BlockKeys {
 struct BlockPos {
     int bx, h, split;
     __device__ __forceinline__ BlockPos(const PrefillArgs& a, int n_blk) {
-        int b = blockIdx.x;
-        split = b % a.n_split;
-        b /= a.n_split;
-        h = b % a.h_kv;
-        bx = n_blk - 1 - b / a.h_kv;
-        bx = __builtin_amdgcn_readfirstlane(bx);
-        h = __builtin_amdgcn_readfirstlane(h);
-        split = __builtin_amdgcn_readfirstlane(split);
+        const int b = blockIdx.x, rest = a.by_split.div(b), rev = a.by_kv.div(rest);
+        split = b - rest * a.n_split;
+        h = rest - rev * a.h_kv;
+        bx = n_blk - 1 - rev;
     }
+};
+// Row r of a KV head: its query and its head of the group.
+struct RowPos {
+    int j, g;
+    __device__ __forceinline__ RowPos(const PrefillArgs& a, int r) : j(a.by_rep.div(r)), g(r - j * a.n_rep) {}
 };
 
 // ----------------------------------------------------------- attention
@@ -350,15 +344,30 @@ template <int R>
 __device__ __forceinline__ void store_rows(const PrefillArgs& a, const float* so, int row0, int h, int split,
                                            bool direct, float m, float l, int lane) {
     const int n = min(R, a.n_q * a.n_rep - row0), H_q = a.h_kv * a.n_rep;
-    auto row_of = [&](int r) { return (size_t)(r / a.n_rep) * H_q + h * a.n_rep + r % a.n_rep; };
+    if (n <= 0) return;  // uniform per wavefront
+    const RowPos first(a, row0);
+    // output row of row0 + i, stepped: within the group, then to the next query
+    struct Step {
+        size_t row;
+        int g;
+    };
+    auto next = [&](Step& p) {
+        const bool wrap = ++p.g == a.n_rep;
+        p.row += wrap ? H_q - a.n_rep + 1 : 1;
+        p.g = wrap ? 0 : p.g;
+    };
+    Step p{(size_t)first.j * H_q + h * a.n_rep + first.g, first.g};
     if (direct) {
         constexpr int G = 16;  // rows whose gates are in flight together
 #pragma unroll 1
         for (int i0 = 0; i0 < n; i0 += G) {
             uint2 g[G];
+            Step q = p;
 #pragma unroll
-            for (int i = 0; i < G; i++)
-                g[i] = *reinterpret_cast<const uint2*>(a.q + row_of(row0 + min(i0 + i, n - 1)) * 512 + 256 + 4 * lane);
+            for (int i = 0; i < G; i++) {
+                g[i] = *reinterpret_cast<const uint2*>(a.q + q.row * 512 + 256 + 4 * lane);
+                if (i0 + i + 1 < n) next(q);
+            }
 #pragma unroll
             for (int i = 0; i < G; i++) {
                 if (i0 + i >= n) break;  // uniform per wavefront
@@ -367,48 +376,52 @@ __device__ __forceinline__ void store_rows(const PrefillArgs& a, const float* so
                 float o[4];
 #pragma unroll
                 for (int c = 0; c < 4; c++) o[c] = v[c] * (1.0f / (1.0f + expf(-(float)gh[c])));
-                *reinterpret_cast<uint2*>(a.out + row_of(row0 + i0 + i) * 256 + 4 * lane) =
+                *reinterpret_cast<uint2*>(a.out + p.row * 256 + 4 * lane) =
                     uint2{pk_rne(o[0], o[1]), pk_rne(o[2], o[3])};
+                next(p);
             }
         }
         return;
     }
     float* part = a.part + (size_t)split * 258;
-#pragma unroll 8
-    for (int i = 0; i < n; i++)
-        *reinterpret_cast<f4s*>(part + row_of(row0 + i) * a.n_split * 258 + 4 * lane) =
-            *reinterpret_cast<const f4*>(&so[i * OUT_LD + 4 * lane]);
+    const size_t ld = (size_t)a.n_split * 258;
     if (lane < n) {
-        float* ml = part + row_of(row0 + lane) * a.n_split * 258 + 256;
+        const RowPos r(a, row0 + lane);
+        float* ml = part + ((size_t)r.j * H_q + h * a.n_rep + r.g) * ld + 256;
         ml[0] = m;
         ml[1] = l;
     }
+#pragma unroll 8
+    for (int i = 0; i < n; i++) {
+        *reinterpret_cast<f4s*>(part + p.row * ld + 4 * lane) =
+            *reinterpret_cast<const f4*>(&so[i * OUT_LD + 4 * lane]);
+        next(p);
+    }
 }
 
-__global__ __launch_bounds__(256) void prefill_attn_kernel(PrefillArgs a) {
-    __shared__ union __align__(16) {
-        struct {
-            _Float16 ks[2][KT][KS_LD], vs[2][256][VS_LD];
-        } t;
-        float out[4][16][OUT_LD];
-    } lds;
-    auto& ks = lds.t.ks;
-    auto& vs = lds.t.vs;
+// Grid (row block, KV head, split), the tile lists of the at most two row blocks
+// worked out by the host: nothing but the arguments stands before the first
+// load.  A split past its block's tiles leaves an empty triple, so every row has
+// n_split of them.
+struct FewBlocks {
+    int nd[2], u0[2], n[2];
+};
+__global__ __launch_bounds__(256) void prefill_attn_kernel(PrefillArgs a, FewBlocks f) {
+    __shared__ __align__(16) _Float16 ks[2][KT][KS_LD];
+    __shared__ __align__(16) _Float16 vs[2][256][VS_LD];
     const int tid = threadIdx.x;
     const int wv = tid >> 6, lane = tid & 63;
     const int li = lane & 15, lg = lane >> 4;
     const int n_rows = a.n_q * a.n_rep;
-    const BlockPos pos(a, (n_rows + 63) / 64);
-    const int h = pos.h, split = pos.split;
-    const int row0 = (pos.bx * 4 + wv) * 16;
+    const int bx = blockIdx.x, h = blockIdx.y, split = blockIdx.z;
+    const int row0 = (bx * 4 + wv) * 16;
     const int H_q = a.h_kv * a.n_rep;
     const int r = row0 + li;
     const bool r_ok = r < n_rows;
-    const int jq = r_ok ? r / a.n_rep : 0;
-    const int hq = h * a.n_rep + (r_ok ? r % a.n_rep : 0);
+    const RowPos rp(a, r_ok ? r : 0);
+    const int jq = rp.j, hq = h * a.n_rep + rp.g;
     const RowKeys vis(a, jq);
-    const BlockKeys bk(a, pos.bx * 64, min(pos.bx * 64 + 63, n_rows - 1), split);
-    if (split >= bk.n_split) return;  // uniform per block
+    const BlockKeys bk(a, f.nd[bx], f.u0[bx], f.n[bx], split);
 
     h8 qb[8];
     {
@@ -536,18 +549,20 @@ __global__ __launch_bounds__(256) void prefill_attn_kernel(PrefillArgs a) {
         }
         __syncthreads();
     }
-    // ---- row li (dims 16 mt + 4 lg + c)
+    // ---- row li (dims 16 mt + 4 lg + c): its triple, in the accumulators' layout
+    // (a few rows: through LDS a whole row at a time takes 1 us more)
     float l_row = l_part + __shfl_xor(l_part, 16, 64);
     l_row += __shfl_xor(l_row, 32, 64);
-    const bool direct = bk.n_split == 1 && !a.apart;
+    if (!r_ok) return;
     const bool empty = m_ref == -INFINITY;
-    const float f = empty ? 0.0f : (direct ? 1.0f / (l_row + a.eps) : 1.0f);
+    float* out = a.part + ((size_t)(jq * H_q + hq) * a.n_split + split) * 258;
 #pragma unroll
-    for (int mt = 0; mt < 16; mt++)  // every wavefront is past the tiles
-        *reinterpret_cast<f4*>(&lds.out[wv][li][16 * mt + 4 * lg]) = acc[mt] * f;
-    wave_sync();
-    store_rows<16>(a, &lds.out[wv][0][0], row0, h, split, direct, empty ? -1e20f : m_ref,
-                   empty ? 0.0f : l_row, lane);
+    for (int mt = 0; mt < 16; mt++)
+        *reinterpret_cast<f4s*>(out + 16 * mt + 4 * lg) = empty ? f4{0.f, 0.f, 0.f, 0.f} : acc[mt];
+    if (lg == 0) {
+        out[256] = empty ? -1e20f : m_ref;
+        out[257] = empty ? 0.0f : l_row;
+    }
 }
 
 // 32-row form: 32 query rows per wavefront pair on 32x32x16 MFMAs, so every
@@ -616,11 +631,14 @@ void prefill_attn_rs_kernel(PrefillArgs a) {
     const int H_q = a.h_kv * a.n_rep;
     const int r = row0 + ln;
     const bool r_ok = r < n_rows;
-    const int jq = r_ok ? r / a.n_rep : 0;
-    const int hq = h * a.n_rep + (r_ok ? r % a.n_rep : 0);
-    const BlockKeys bk(a, pos.bx * 128, min(pos.bx * 128 + 127, n_rows - 1), split);
-    if (split >= bk.n_split) return;  // uniform per block
-    const bool direct = bk.n_split == 1 && !a.apart;
+    const RowPos rp(a, r_ok ? r : 0);
+    const int jq = rp.j, hq = h * a.n_rep + rp.g;
+    int nd, u0;
+    const int n_blk_tiles = a.block_tiles(pos.bx * 128, min(pos.bx * 128 + 127, n_rows - 1), &nd, &u0);
+    const int n_split = a.block_splits(n_blk_tiles);
+    if (split >= n_split) return;  // uniform per block
+    const BlockKeys bk(a, nd, u0, n_blk_tiles, split);
+    const bool direct = n_split == 1 && !a.apart;
     const int n_tiles = bk.t_hi - bk.t_lo;
     const int raw_end = a.raw0 + a.n_raw;
     const f32x16 zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -677,7 +695,7 @@ void prefill_attn_rs_kernel(PrefillArgs a) {
         // several references.  A layer's pass has fewer of them than one launch
         // per event had, and raises it so too: 200 tokens after 300, 2.86e-4 from
         // float64 without, 2.68e-4 with, 2.72e-4 in a launch per event.
-        const int n_eager = bk.n_split == 1 || a.ev_cap > 0 ? 8 : 0;
+        const int n_eager = n_split == 1 || a.ev_cap > 0 ? 8 : 0;
         const float sc2 = a.sc * LOG2E;  // scores in log2 units: a weight is one exp2
         float m_ref = M_NONE;
         f32x16 s2[2];
@@ -864,13 +882,14 @@ void prefill_attn_rs_kernel(PrefillArgs a) {
                     f4{acc[t2][4 * j], acc[t2][4 * j + 1], acc[t2][4 * j + 2], acc[t2][4 * j + 3]} * f;
         wave_sync();
         if (!direct)
-            store_rows<32>(a, &lds.out[rg][0][0], row0, h, split, false,
+            store_rows<32>(a, &lds.out[rg][0][0], __builtin_amdgcn_readfirstlane(row0), h, split, false,
                            empty ? -1e20f : m_last * LN2, empty ? 0.0f : l_row, lane);
     }
     if (direct) {  // uniform per block; gates and stores: half a row group each wavefront
         __syncthreads();
         const int half = tid < 256 ? 0 : 16;
-        store_rows<16>(a, &lds.out[rg][half][0], row0 + half, h, split, true, 0.0f, 0.0f, lane);
+        store_rows<16>(a, &lds.out[rg][half][0], __builtin_amdgcn_readfirstlane(row0 + half), h, split, true,
+                       0.0f, 0.0f, lane);
     }
 }
 
@@ -881,7 +900,14 @@ void prefill_attn_rs_kernel(PrefillArgs a) {
 // first is used (the first group's with the (m, l) loads, ahead of the
 // maximum); the sums run in split order.
 constexpr int MG = 16;  // splits per load group
-__device__ __forceinline__ void merge_row(const PrefillArgs& p, int row, int n_split) {
+struct MergeArgs {
+    const float* part;
+    const __half* q;
+    __half* out;
+    int n_rows, n_split, nb;  // rows, triples a row, merging blocks
+    float eps;
+};
+__device__ __forceinline__ void merge_row(const MergeArgs& p, int row, int n_split) {
     const int lane = threadIdx.x & 63;
     const float* base = p.part + (size_t)row * p.n_split * 258;
     float2 a[MG][2];
@@ -932,32 +958,43 @@ __device__ __forceinline__ void merge_row(const PrefillArgs& p, int row, int n_s
 
 // Blocks [0, nb_m): rows 4 b .. + 3, one wavefront each; the rest copy new
 // tokens to the ring, 8 bytes a thread and tensor.
-__global__ __launch_bounds__(256) void prefill_finish_kernel(PrefillArgs a, RingArgs g, int nb_m,
-                                                             int block_rows) {
-    int b = blockIdx.x;
-    if (b < nb_m) {
-        const int H_q = a.h_kv * a.n_rep, row = b * 4 + (threadIdx.x >> 6);
-        if (row >= a.n_q * H_q) return;  // uniform per wavefront
-        const int r = row / H_q * a.n_rep + row % H_q % a.n_rep;  // row of its KV head
-        const int first = r / block_rows * block_rows;
-        int ns = a.n_split, nd, u0;
-        if (!a.uniform)
-            ns = a.block_splits(
-                a.block_tiles(first, min(first + block_rows, a.n_q * a.n_rep) - 1, &nd, &u0));
-        if (ns > 1 || a.apart) merge_row(a, row, ns);
-        return;
-    }
-    b -= nb_m;
-    const int per = g.h_kv * 64;  // pieces per token
-    const long i = (long)b * 256 + threadIdx.x;
-    if (i >= (long)g.n * per) return;
-    const int t = (int)(i / per), e = (int)(i % per) * 4;
+__device__ __forceinline__ void ring_pieces(const RingArgs& g, int b) {
+    const int i = b * 256 + threadIdx.x, t = g.by_token.div(i);
+    if (t >= g.n) return;
+    const int per = g.h_kv * 64, e = (i - t * per) * 4;  // pieces per token
     int slot = g.slot0 + t;
     slot = slot >= g.ring_cap ? slot - g.ring_cap : slot;
     const size_t src = (size_t)t * per * 4 + e, dst = (size_t)slot * per * 4 + e;
     *reinterpret_cast<uint2*>(g.ring_k + dst) = *reinterpret_cast<const uint2*>(g.src_k + src);
     *reinterpret_cast<uint2*>(g.ring_v + dst) = *reinterpret_cast<const uint2*>(g.src_v + src);
     *reinterpret_cast<uint2*>(g.ring_u + dst) = *reinterpret_cast<const uint2*>(g.src_u + src);
+}
+__global__ __launch_bounds__(256) void prefill_finish_kernel(MergeArgs m, RingArgs g) {
+    const int b = blockIdx.x;
+    if (b >= m.nb) {
+        ring_pieces(g, b - m.nb);
+        return;
+    }
+    const int row = b * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (row < m.n_rows) merge_row(m, row, m.n_split);  // uniform per wavefront
+}
+// Blocks of unlike split counts, those of one split written out already:
+// block_rows (a power of two) rows of a KV head each.
+__global__ __launch_bounds__(256) void prefill_finish_ragged_kernel(MergeArgs m, RingArgs g, PrefillArgs a,
+                                                                    int block_rows) {
+    const int b = blockIdx.x;
+    if (b >= m.nb) {
+        ring_pieces(g, b - m.nb);
+        return;
+    }
+    const int row = b * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (row >= m.n_rows) return;
+    const int j = a.by_hq.div(row), hq = row - j * a.h_kv * a.n_rep;
+    const int first = (j * a.n_rep + RowPos(a, hq).g) & -block_rows;
+    int nd, u0;
+    const int ns = a.block_splits(
+        a.block_tiles(first, min(first + block_rows, a.n_q * a.n_rep) - 1, &nd, &u0));
+    if (ns > 1 || a.apart) merge_row(m, row, ns);
 }
 
 }  // namespace pf
@@ -984,12 +1021,18 @@ bool long_decode(const DecompArgs& a) {
 }  // namespace
 
 hipError_t launch_prefill_finish(const PrefillArgs& a, const RingArgs* ring, hipStream_t st) {
-    const int nb_m = a.n_split > 1 || a.apart ? (a.n_q * a.h_kv * a.n_rep + 3) / 4 : 0;
-    const RingArgs g = ring ? *ring : RingArgs{};
-    const int nb_g = ring ? (g.n * g.h_kv * 64 + 255) / 256 : 0;
-    if (nb_m + nb_g == 0) return hipSuccess;
-    hipLaunchKernelGGL(pf::prefill_finish_kernel, dim3(nb_m + nb_g), dim3(256), 0, st, a, g, nb_m,
-                       prefill_block_rows(a.n_q * a.n_rep));
+    const int n_rows = a.n_q * a.h_kv * a.n_rep;
+    const pf::MergeArgs m{a.part, a.q, a.out, n_rows, a.n_split,
+                          a.n_split > 1 || a.apart ? (n_rows + 3) / 4 : 0, a.eps};
+    RingArgs g = ring ? *ring : RingArgs{};
+    g.by_token = FastDiv(std::max(1, g.h_kv * 64));
+    const dim3 grid(m.nb + (g.n * g.h_kv * 64 + 255) / 256);
+    if (grid.x == 0) return hipSuccess;
+    if (a.uniform)
+        hipLaunchKernelGGL(pf::prefill_finish_kernel, grid, dim3(256), 0, st, m, g);
+    else
+        hipLaunchKernelGGL(pf::prefill_finish_ragged_kernel, grid, dim3(256), 0, st, m, g, a,
+                           prefill_block_rows(a.n_q * a.n_rep));
     return hipGetLastError();
 }
 
@@ -1059,81 +1102,98 @@ int prefill_block_rows(int n_rows) { return few_rows(n_rows) ? 64 : 128; }
 
 void prefill_plan(PrefillArgs& a) {
     // Blocks that run at once: 2 per CU for the 16-row kernel (72 KB of LDS
-    // each), 1 for the 32-row kernel (142 KB).  With splits of at most `unit`
-    // tiles, the launch takes, in tiles of time:
-    //   one round of the longest block when they all fit at once;
-    //   else the work over the slots plus half a block of tail (they start
-    //   longest first), or whole rounds when the blocks are equally long (a
-    //   few blocks past a round cost a whole round).
-    // A block costs about 4 tiles beside its own (entry, first loads, output);
-    // splitting costs the finishing launch, about 4, and 0.045 a block for its
-    // triples (128 rows x 1 KB written and read).  Where one round holds every
-    // block, gating the rows inside it (a.apart = false) is not free either: a
-    // wavefront gates up to 16 rows in turn, 0.29 each, with nothing else on its
-    // CU.  Left out, 48 queries over 200 tokens took 27.1 us unsplit against
-    // 17.4 in 8 splits, a 100-token prompt 29.5 against 22.4.
+    // each), 1 for the 32-row kernel (142 KB).
     const int n_rows = a.n_q * a.n_rep, br = prefill_block_rows(n_rows);
     const int nb = (n_rows + br - 1) / br;
-    const int slots = (few_rows(n_rows) ? 2 : 1) * device_cu_count();
+    const bool few = few_rows(n_rows);
+    const int slots = (few ? 2 : 1) * device_cu_count();
+    a.by_rep = FastDiv(a.n_rep);
+    a.by_hq = FastDiv(a.h_kv * a.n_rep);
+    a.by_kv = FastDiv(a.h_kv);
+    auto tiles_of = [&](int b) {
+        int nd, u0;
+        return a.block_tiles(b * br, std::min(b * br + br, n_rows) - 1, &nd, &u0);
+    };
+    auto set_splits = [&](int k, int t_max) {
+        a.unit = (t_max + k - 1) / k;
+        a.n_split = (t_max + a.unit - 1) / a.unit;
+        a.by_unit = FastDiv(a.unit);
+    };
     int t_max = 1, t_min = 1 << 30;
     for (int b = 0; b < nb; b++) {
-        int nd, u0;
-        const int t = a.block_tiles(b * br, std::min(b * br + br, n_rows) - 1, &nd, &u0);
+        const int t = tiles_of(b);
         t_max = std::max(t_max, t);
         t_min = std::min(t_min, t);
     }
-    const bool even = t_max - t_min <= t_max / 8;
-    const float gate = 0.29f * std::min(16, n_rows);
-    const int step = std::max(1, nb / 64);  // enough blocks to add up
     // At least as many splits as one round holds: a weight is rounded to fp16
     // but for its tile's largest where that sets the reference (a split's first
     // tile), so short splits lose less.  16 queries over 900 tokens, whatever is
     // faster (10 splits): 2.80e-4 from float64, 29 splits of a tile 2.53e-4, the
     // output's own rounding being 2.07e-4.
     const int k_min = std::max(1, std::min({64, t_max, slots / (nb * a.h_kv)}));
-    float best = 0.0f;
     int best_k = k_min;
-    for (int k = k_min; k <= std::min(64, t_max); k++) {
-        a.n_split = k;
-        a.unit = (t_max + k - 1) / k;
-        if (k > k_min && (size_t)a.n_q * a.h_kv * a.n_rep * k * 258 * 4 > (size_t)1 << 30) break;
-        float units = 0.0f, tiles = 0.0f;
-        for (int b = 0; b < nb; b += step) {
-            int nd, u0;
-            const int t = a.block_tiles(b * br, std::min(b * br + br, n_rows) - 1, &nd, &u0);
-            const float w = (float)std::min(step, nb - b) * a.h_kv;
-            units += w * a.block_splits(t);
-            tiles += w * t;
-        }
-        const float rounds = std::ceil(units / slots);
-        float est = rounds <= 1.0f || even ? rounds * (a.unit + 4)
-                                           : (tiles + 4 * units) / slots + 0.5f * a.unit;
-        bool apart = !a.out;
-        if (k > 1 || (rounds <= 1.0f && gate > 4.0f + 0.045f * units)) {
-            est += 4.0f + 0.045f * units;
-            apart |= rounds <= 1.0f;
-        } else if (rounds <= 1.0f) {
-            est += gate;
-        }
-        if (k == k_min || est < best) {
-            best = est;
-            best_k = k;
-            a.apart = apart;
+    if (few) {
+        a.apart = true;  // gating 16 rows in turn in the block takes longer than the finishing launch
+    } else {
+        // More where it is faster.  With splits of at most `unit` tiles, the
+        // launch takes, in tiles of time:
+        //   one round of the longest block when they all fit at once;
+        //   else the work over the slots plus half a block of tail (they start
+        //   longest first), or whole rounds when the blocks are equally long (a
+        //   few blocks past a round cost a whole round).
+        // A block costs about 4 tiles beside its own (entry, first loads, output);
+        // splitting costs the finishing launch, about 4, and 0.045 a block for its
+        // triples (128 rows x 1 KB written and read).  Where one round holds every
+        // block, gating the rows inside it (a.apart = false) is not free either: a
+        // wavefront gates up to 16 rows in turn, 0.29 each, with nothing else on its
+        // CU.
+        const bool even = t_max - t_min <= t_max / 8;
+        const float gate = 0.29f * std::min(16, n_rows);
+        const int step = std::max(1, nb / 64);  // enough blocks to add up
+        float best = 0.0f;
+        for (int k = k_min; k <= std::min(64, t_max); k++) {
+            set_splits(k, t_max);
+            if (k > k_min && (size_t)a.n_q * a.h_kv * a.n_rep * k * 258 * 4 > (size_t)1 << 30) break;
+            float units = 0.0f, tiles = 0.0f;
+            for (int b = 0; b < nb; b += step) {
+                const int t = tiles_of(b);
+                const float w = (float)std::min(step, nb - b) * a.h_kv;
+                units += w * a.block_splits(t);
+                tiles += w * t;
+            }
+            const float rounds = std::ceil(units / slots);
+            float est = rounds <= 1.0f || even ? rounds * (a.unit + 4)
+                                               : (tiles + 4 * units) / slots + 0.5f * a.unit;
+            bool apart = !a.out;
+            if (k > 1 || (rounds <= 1.0f && gate > 4.0f + 0.045f * units)) {
+                est += 4.0f + 0.045f * units;
+                apart |= rounds <= 1.0f;
+            } else if (rounds <= 1.0f) {
+                est += gate;
+            }
+            if (k == k_min || est < best) {
+                best = est;
+                best_k = k;
+                a.apart = apart;
+            }
         }
     }
-    a.n_split = best_k;
-    a.unit = (t_max + a.n_split - 1) / a.n_split;
-    a.n_split = (t_max + a.unit - 1) / a.unit;
-    a.uniform = a.block_splits(t_min) == a.n_split;
+    set_splits(best_k, t_max);
+    a.by_split = FastDiv(a.n_split);
+    a.uniform = few || a.block_splits(t_min) == a.n_split;
 }
 
 hipError_t launch_prefill_attn(const PrefillArgs& a, hipStream_t st) {
-    const int n_rows = a.n_q * a.n_rep, br = prefill_block_rows(n_rows);
-    const dim3 grid((unsigned)((n_rows + br - 1) / br) * a.h_kv * a.n_split);
-    if (few_rows(n_rows))
-        hipLaunchKernelGGL(pf::prefill_attn_kernel, grid, dim3(256), 0, st, a);
-    else
-        hipLaunchKernelGGL(pf::prefill_attn_rs_kernel, grid, dim3(512), 0, st, a);
+    const int n_rows = a.n_q * a.n_rep, br = prefill_block_rows(n_rows), nb = (n_rows + br - 1) / br;
+    if (few_rows(n_rows)) {
+        pf::FewBlocks f{};
+        for (int b = 0; b < nb; b++)
+            f.n[b] = a.block_tiles(b * br, std::min(b * br + br, n_rows) - 1, &f.nd[b], &f.u0[b]);
+        hipLaunchKernelGGL(pf::prefill_attn_kernel, dim3(nb, a.h_kv, a.n_split), dim3(256), 0, st, a, f);
+    } else {
+        hipLaunchKernelGGL(pf::prefill_attn_rs_kernel, dim3((unsigned)nb * a.h_kv * a.n_split), dim3(512), 0,
+                           st, a);
+    }
     return hipGetLastError();
 }
 

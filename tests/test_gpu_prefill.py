@@ -466,6 +466,31 @@ def test_prefill_attn_weight_rounding(device, n_q, past):
     assert np.sqrt(num / den) <= 1.04 * bound, (np.sqrt(num / den), bound)
 
 
+@pytest.mark.parametrize("H_q,H_kv", [(1, 1), (7, 7), (10, 2), (33, 3), (24, 1)])
+@pytest.mark.parametrize("n_q,past", [(3, 30), (40, 70), (300, 100)])
+def test_prefill_attn_head_groups(device, H_q, H_kv, n_q, past):
+    """Every row's query and head (divisions by the group size, the head count
+    and the split count) for group sizes that divide no block, in both kernels,
+    split and merged."""
+    rng = np.random.default_rng(H_q)
+    n_k = past + n_q
+    q = rng.standard_normal((n_q, H_q, 2 * D)).astype(np.float16)
+    K, V = (rng.standard_normal((n_k, H_kv, D)).astype(np.float16) for _ in range(2))
+    ld = ops.vt_ld(n_k)
+    vt = torch.zeros((H_kv, D, ld), device=device, dtype=torch.float16)
+    vt[:, :, :n_k] = t(V).permute(1, 2, 0)
+    out = torch.full((n_q, H_q, D), float("nan"), device=device, dtype=torch.float16)
+    ops.prefill_attn(t(q), t(K), vt, out, ld_vt=ld, n_k=n_k, n_q=n_q, vis0=past + 1, H_q=H_q, H_kv=H_kv,
+                     scale=SCALE)
+    got = out.cpu().numpy()
+    hidden = np.arange(n_k)[None] > past + np.arange(n_q)[:, None]
+    for h in range(H_q):
+        s = q[:, h, :D].astype(np.float64) @ K[:, h * H_kv // H_q].astype(np.float64).T * SCALE
+        w = np.exp(np.where(hidden, -np.inf, s - s.max(1, keepdims=True)))
+        want = w @ V[:, h * H_kv // H_q].astype(np.float64) / w.sum(1, keepdims=True)
+        close(got[:, h], want * npref.sigmoid(q[:, h, D:].astype(np.float64)))
+
+
 def test_layer_prefill_mixed_with_steps(device):
     """Prefill chunks and single steps interleaved on one layer (the dense key
     space must not keep raw tokens the steps wrote only to the ring) against
