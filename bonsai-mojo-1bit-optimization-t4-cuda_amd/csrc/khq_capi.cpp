@@ -104,6 +104,15 @@ hipError_t workspace(size_t bytes, hipStream_t stream, float** out, bool use = t
     return hipSuccess;
 }
 
+// What a launch on this stream may ask workspace() for.
+size_t workspace_limit(hipStream_t stream) {
+    int dev = 0;
+    if (!capturing(stream) || hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices)
+        return ~(size_t)0;
+    std::lock_guard<std::mutex> lk(g_ws_mu);
+    return g_ws[dev].bytes;  // a captured launch cannot grow it
+}
+
 std::mutex g_dev_mu;
 std::atomic<int> g_cu_count[kMaxDevices] = {};  // 0 until first queried
 struct LdsSet {
@@ -995,11 +1004,10 @@ int attn_step_append(const AttnArgs& a, int H_q, __half* out, hipStream_t stream
 }
 
 int prefill_attn_run(PrefillArgs a, const RingArgs* ring, hipStream_t stream, bool merge) {
-    prefill_plan(a);
+    prefill_plan(a, workspace_limit(stream));
     a.eps = 1e-8f;
     if (a.n_split > 1 || a.apart) {
-        const hipError_t e = workspace(
-            (size_t)a.n_q * a.h_kv * a.n_rep * a.n_split * 258 * sizeof(float), stream, &a.part);
+        const hipError_t e = workspace(a.triple_bytes(a.n_split), stream, &a.part);
         if (e != hipSuccess) return rc_of(e);
     }
     const hipError_t e = launch_prefill_attn(a, stream);

@@ -298,6 +298,9 @@ struct PrefillArgs {
         return *nd + ((vl + 31) >> 5) - *u0;
     }
     __host__ __device__ int block_splits(int tiles) const { return by_unit.div(tiles + unit - 1); }
+    size_t triple_bytes(int splits) const {
+        return (size_t)n_q * h_kv * n_rep * splits * 258 * sizeof(float);
+    }
 };
 hipError_t launch_decompress(const DecompArgs& a, hipStream_t st);
 hipError_t launch_ring_gather(const GatherArgs& a, hipStream_t st);
@@ -313,8 +316,9 @@ hipError_t launch_compress_gather(const CompressJob& k, const CompressJob& v, co
                                   hipStream_t st);
 // Rows of one KV head a block of the prefill attention takes.
 int prefill_block_rows(int n_rows);
-// Fills a.n_split, a.unit, a.apart and a.uniform for the current device.
-void prefill_plan(PrefillArgs& a);
+// Fills a.n_split, a.unit, a.apart and a.uniform for the current device, the
+// triples in at most max_bytes where that is possible.
+void prefill_plan(PrefillArgs& a, size_t max_bytes);
 hipError_t launch_prefill_attn(const PrefillArgs& a, hipStream_t st);
 // Prefill attention plus merge and gate through the shared workspace: q, k, vt,
 // the shapes, the key runs and out set in a; with ring, its copy runs behind

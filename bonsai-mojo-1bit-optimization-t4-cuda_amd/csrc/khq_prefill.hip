@@ -1100,7 +1100,7 @@ bool few_rows(int n_rows) { return n_rows <= 128; }
 
 int prefill_block_rows(int n_rows) { return few_rows(n_rows) ? 64 : 128; }
 
-void prefill_plan(PrefillArgs& a) {
+void prefill_plan(PrefillArgs& a, size_t max_bytes) {
     // Blocks that run at once: 2 per CU for the 16-row kernel (72 KB of LDS
     // each), 1 for the 32-row kernel (142 KB).
     const int n_rows = a.n_q * a.n_rep, br = prefill_block_rows(n_rows);
@@ -1130,7 +1130,8 @@ void prefill_plan(PrefillArgs& a) {
     // tile), so short splits lose less.  16 queries over 900 tokens, whatever is
     // faster (10 splits): 2.80e-4 from float64, 29 splits of a tile 2.53e-4, the
     // output's own rounding being 2.07e-4.
-    const int k_min = std::max(1, std::min({64, t_max, slots / (nb * a.h_kv)}));
+    int k_min = std::max(1, std::min({64, t_max, slots / (nb * a.h_kv)}));
+    while (k_min > 1 && a.triple_bytes(k_min) > max_bytes) k_min--;
     int best_k = k_min;
     if (few) {
         a.apart = true;  // gating 16 rows in turn in the block takes longer than the finishing launch
@@ -1153,7 +1154,8 @@ void prefill_plan(PrefillArgs& a) {
         float best = 0.0f;
         for (int k = k_min; k <= std::min(64, t_max); k++) {
             set_splits(k, t_max);
-            if (k > k_min && (size_t)a.n_q * a.h_kv * a.n_rep * k * 258 * 4 > (size_t)1 << 30) break;
+            // (the workspace stays: past 256 MB a finer tail is not worth it)
+            if (k > k_min && a.triple_bytes(k) > std::min(max_bytes, (size_t)256 << 20)) break;
             float units = 0.0f, tiles = 0.0f;
             for (int b = 0; b < nb; b += step) {
                 const int t = tiles_of(b);
@@ -1165,7 +1167,7 @@ void prefill_plan(PrefillArgs& a) {
             float est = rounds <= 1.0f || even ? rounds * (a.unit + 4)
                                                : (tiles + 4 * units) / slots + 0.5f * a.unit;
             bool apart = !a.out;
-            if (k > 1 || (rounds <= 1.0f && gate > 4.0f + 0.045f * units)) {
+            if (k > 1 || (rounds <= 1.0f && gate > 4.0f + 0.045f * units && a.triple_bytes(1) <= max_bytes)) {
                 est += 4.0f + 0.045f * units;
                 apart |= rounds <= 1.0f;
             } else if (rounds <= 1.0f) {
