@@ -651,12 +651,13 @@ __global__ __launch_bounds__(256) void vq_hard_kernel(const float* __restrict__ 
 // the LDS.  Scalar loads: T, and so lda, may be any size.  Grid z = batch x
 // splits; a split covers k_per of K and writes its own C (the partials are
 // added by gemm_reduce_kernel).
-// A 512-token calibration: 24 x (512 x 256 x 512) forward 376 us in four
-// launches of 94 -> 59 us (108 TFLOP/s of the 154 a large fp32 matrix product
-// reaches here); 4 x (512 x 256 x 3072) backward 2450 us in four launches of
-// 32 blocks -> 53 us with 8 splits and 5 us for their sum.
+// 512 tokens: 24 x (512 x 256 x 512) forward 376 us in four launches of 94 -> 59
+// us (55 TFLOP/s of the 154 a large fp32 matrix product reaches here); 4 x (512 x
+// 256 x 3072) backward 2450 us in four launches of 32 blocks -> 53 us with 8
+// splits and 5 us for their sum.
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr int GK = 32;   // K slab
+constexpr int LOSS_SLOTS = 32;  // a product's blocks add to as many sums in turn: 512 atomics on one take 5 us
 constexpr int GLD = 65;  // words per LDS row: the transposing stores hit 32 banks
 struct GemmArgs {
     const float *A, *B;
@@ -734,13 +735,111 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs g) {
     }
 }
 
+// C[b] (M x N) = A[b]^T B[b] in double: A stored K x M, B K x N, dense C; grid z
+// as gemm_kernel's.  fp64 MFMA 16x16x4 (A lane l: row l % 16, k l / 16; B lane l: k
+// l / 16, column l % 16; C register r: row l / 16 + 4 r, column l % 16), 2 x 2 of
+// them a wavefront over the same 64 x 64 tiles and slabs; fp32 operands are
+// widened as they leave LDS.  With dot, the sum of C .* B (M = K) is added to it.
+// It carries the Gram form of the loss, x . G x, whose terms cancel: with G and
+// G x in fp32 a loss over 512 tokens was off by 2.3e-7 (attention sinks), against
+// 3e-8 for the sum of squares over the heads.
+typedef double d4 __attribute__((ext_vector_type(4)));
+template <typename TA, typename TC>
+struct Gemm64Args {
+    const TA* A;
+    const float* B;
+    TC* C;
+    int M, N, K;
+    long sa, sb;
+    int batch, k_per;
+    double* dot;  // LOSS_SLOTS sums
+};
+template <typename TA, typename TC>
+__global__ __launch_bounds__(256) void gemm64_kernel(Gemm64Args<TA, TC> g) {
+    __shared__ TA sA[2][GK][GLD];
+    __shared__ float sB[2][GK][GLD];
+    const int b = blockIdx.z % g.batch, split = blockIdx.z / g.batch;
+    const TA* A = g.A + b * g.sa;
+    const float* B = g.B + b * g.sb;
+    TC* C = g.C + (long)blockIdx.z * g.M * g.N;
+    const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
+    const int k_lo = split * g.k_per, k_hi = min(g.K, k_lo + g.k_per);
+    const int t = threadIdx.x, wv = t >> 6, lane = t & 63, li = lane & 15, lg = lane >> 4;
+    const int wm = 32 * (wv & 1), wn = 32 * (wv >> 1);
+    const int gm = m0 + (t & 63), gn = n0 + (t & 63);
+    TA ra[8];
+    float rb[8];
+    auto load = [&](int k0) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int k = k0 + wv + 4 * i;
+            ra[i] = (gm < g.M && k < k_hi) ? A[(long)k * g.M + gm] : (TA)0;
+            rb[i] = (gn < g.N && k < k_hi) ? B[(long)k * g.N + gn] : 0.0f;
+        }
+    };
+    auto store = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            sA[buf][wv + 4 * i][lane] = ra[i];
+            sB[buf][wv + 4 * i][lane] = rb[i];
+        }
+    };
+    d4 acc[2][2] = {};
+    load(k_lo);
+    store(0);
+    int buf = 0;
+    for (int k0 = k_lo; k0 < k_hi; k0 += GK, buf ^= 1) {
+        __syncthreads();  // slab `buf` is staged, the other one is read out
+        const bool more = k0 + GK < k_hi;
+        if (more) load(k0 + GK);
+#pragma unroll
+        for (int kk = 0; kk < GK; kk += 4) {
+            double a[2], x[2];
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                a[i] = (double)sA[buf][kk + lg][wm + 16 * i + li];
+                x[i] = (double)sB[buf][kk + lg][wn + 16 * i + li];
+            }
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], x[j], acc[i][j], 0, 0, 0);
+        }
+        if (more) store(buf ^ 1);
+    }
+    double sum = 0.0;
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int m = m0 + wm + 16 * i + lg + 4 * r, n = n0 + wn + 16 * j + li;
+                if (m < g.M && n < g.N) {
+                    C[(long)m * g.N + n] = (TC)acc[i][j][r];
+                    if (g.dot) sum += acc[i][j][r] * (double)B[(long)m * g.N + n];
+                }
+            }
+    if (g.dot) {
+        __shared__ double s_sum[4];
+        for (int o = 32; o >= 1; o >>= 1) sum += __shfl_xor(sum, o, 64);
+        if (lane == 0) s_sum[wv] = sum;
+        __syncthreads();
+        if (t == 0)
+            atomicAdd(g.dot + (blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z)) % LOSS_SLOTS,
+                      (s_sum[0] + s_sum[1]) + (s_sum[2] + s_sum[3]));
+    }
+}
+
 // out[i] = alpha * (part[0][i] + part[1][i] + ...), in split order
-__global__ __launch_bounds__(256) void gemm_reduce_kernel(const float* __restrict__ part,
-                                                          float* __restrict__ out, long n,
+template <typename TC>
+__global__ __launch_bounds__(256) void gemm_reduce_kernel(const TC* __restrict__ part,
+                                                          TC* __restrict__ out, long n,
                                                           int splits, float alpha) {
     const long i = (long)blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
-    float s = 0.0f;
+    TC s = 0;
 #pragma unroll 8
     for (int k = 0; k < splits; k++) s += part[k * n + i];
     out[i] = alpha * s;
@@ -914,25 +1013,17 @@ __global__ __launch_bounds__(256) void svq_fwd_kernel(
     if (!attn) add_loss(sum, loss);
 }
 
-// Backward of a row in attention mode, from gd = sum_h A_h^T A_h dlt: with
-// quad, the loss term dlt . gd (= sum_h |A_h dlt|^2 over the rows); with grad,
-// g = gscale gd, gb = g B^T (8), grec = g + gb A^T, gq as above.
+// Backward of a row in attention mode, from gd = sum_h A_h^T A_h dlt: g = gscale
+// gd, gb = g B^T (8), grec = g + gb A^T, gq as above.
 __global__ __launch_bounds__(256) void svq_bwd_kernel(
-    const float* __restrict__ gd, const float* __restrict__ dlt, const float* __restrict__ rp,
-    const float* __restrict__ wa, const float* __restrict__ wb, float* __restrict__ gb_out,
-    float* __restrict__ gq, int rows, int quad, int grad, float gscale, double* __restrict__ loss) {
+    const float* __restrict__ gd, const float* __restrict__ rp, const float* __restrict__ wa,
+    const float* __restrict__ wb, float* __restrict__ gb_out, float* __restrict__ gq, int rows,
+    float gscale) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    double sum = 0.0;
     for (int i = wave; i < ROWS_PER_BLOCK; i += 4) {
         const long n = (long)blockIdx.x * ROWS_PER_BLOCK + i;
         if (n >= rows) break;  // uniform per wavefront
-        const long at = n * D + 4 * lane;
-        const float4 x = *reinterpret_cast<const float4*>(gd + at);
-        if (quad) {
-            const float4 y = *reinterpret_cast<const float4*>(dlt + at);
-            sum += ((double)x.x * y.x + (double)x.y * y.y) + ((double)x.z * y.z + (double)x.w * y.w);
-        }
-        if (!grad) continue;
+        const float4 x = *reinterpret_cast<const float4*>(gd + n * D + 4 * lane);
         const float xs[4] = {gscale * x.x, gscale * x.y, gscale * x.z, gscale * x.w};
         float gb[8], o[4] = {xs[0], xs[1], xs[2], xs[3]};
 #pragma unroll
@@ -952,7 +1043,6 @@ __global__ __launch_bounds__(256) void svq_bwd_kernel(
 #pragma unroll
             for (int r = 0; r < 8; r++) gb_out[n * 8 + r] = gb[r];
     }
-    if (quad) add_loss(sum, loss);
 }
 
 // Transform gradients from the rank-8 row factors, gA[j][r] = sum_n recf[n][j]
@@ -1218,33 +1308,34 @@ struct Svq {
     int N, T, H_q, H_kv;
     hipStream_t st;
     int passes;  // passes the caller will run
-    Buf buf, gram_buf;
-    float *rot, *rec, *recf, *dlt, *gd, *va, *gb, *dict, *gq, *grad, *part, *y, *gram;
+    Buf buf;
+    float *rot, *rec, *recf, *dlt, *gd, *va, *gb, *dict, *gq, *grad, *part, *y;
     int* idx;
-    double* loss;
+    double *loss, *gram;
     // Every array from one allocation, the row rotation (the same in every
     // pass) and, where it pays, the Gram matrices.
     int init() {
         const size_t nd = (size_t)N * D, np = (size_t)N * NP;
+        use_gram = attn && (long)T <= 256l * passes;
         int kp;
-        use_gram = attn && (long)T <= 512l * passes;
         size_t n_part = std::max((size_t)soft_ranges(N, &kp) * CB, (size_t)GWAB * 4096);
         if (attn) {
             n_part = std::max(n_part, (size_t)gemm_splits(T, D, H_q / H_kv * T, H_kv, &kp) * H_kv * T * D);
             if (use_gram) {
                 n_part = std::max(n_part, (size_t)gemm_splits(T, D, T, H_kv, &kp) * H_kv * T * D);
-                n_part = std::max(n_part, (size_t)gemm_splits(T, T, H_q / H_kv * T, H_kv, &kp) * H_kv * T * T);
+                n_part = std::max(n_part, (size_t)gemm_splits(T, T, H_q / H_kv * T, H_kv, &kp) * H_kv * T * T * 2);
             }
         }
         const size_t n_y = attn && !use_gram ? (size_t)H_q * T * D : 0;
-        const size_t n_gram = use_gram ? (size_t)H_kv * T * T : 0;
+        const size_t n_gram = use_gram ? 2 * (size_t)H_kv * T * T : 0;
         struct {
             float** p;
             size_t n;
         } parts[] = {{&rot, nd}, {&rec, nd}, {&recf, nd}, {&dlt, nd}, {&gd, nd},
                      {&va, (size_t)N * 8}, {&gb, (size_t)N * 8}, {&dict, np}, {&gq, 3 * np},
-                     {&grad, NPAR}, {&part, n_part}, {&y, n_y}, {&gram, n_gram},
-                     {reinterpret_cast<float**>(&idx), np}, {reinterpret_cast<float**>(&loss), 4}};
+                     {&grad, NPAR}, {&part, n_part}, {&y, n_y},
+                     {reinterpret_cast<float**>(&gram), n_gram}, {reinterpret_cast<float**>(&idx), np},
+                     {reinterpret_cast<float**>(&loss), 2 * (2 + LOSS_SLOTS)}};
         size_t total = 0;
         for (auto& x : parts) total += (x.n + 63) / 64 * 64;
         CAL_TRY(buf.alloc(total * sizeof(float)));
@@ -1256,20 +1347,21 @@ struct Svq {
         hipLaunchKernelGGL(rotate_kernel, dim3(blocks((long)N * NP, 256)), dim3(256), 0, st, v, rp,
                            rot, N);
         if (use_gram)  // gram_kv = sum_h A_h^T A_h, the group's heads stacked along K
-            gemm(attn, attn, gram, T, T, H_q / H_kv * T, T, T, (long)H_q / H_kv * T * T,
-                 (long)H_q / H_kv * T * T, H_kv, 1, 1, 1.0f, nullptr);
+            gemm64(attn, attn, gram, T, T, H_q / H_kv * T, nullptr);
         return 0;
     }
     // The loss and its gradient need only G = sum_h A_h^T A_h of each group:
-    // sum_h |A_h x|^2 = x . G x, and G x is the gradient.  G takes the products
-    // of T / 512 passes over the heads, G x a twelfth of one's.  512 tokens, 24
-    // / 4 heads: 117 us a pass over the heads -> 60 us once and 18 us a pass.
+    // sum_h |A_h x|^2 = x . G x, and G x is the gradient.  The terms of x . G x
+    // cancel, so G and both products are in double (gemm64_kernel), at half the
+    // fp32 rate: G costs as much as T / 256 passes over the heads, G x about a
+    // fifth of one's.  512 tokens, 24 / 4 heads: 117 us a pass over the heads ->
+    // 137 us once and 26 us a pass.
     bool use_gram = false;
     static constexpr int GWAB = 128;  // row ranges of the transform gradients
     // Splits of K: enough blocks for four a CU (a block's LDS and registers
     // let four share one and cover each other's barriers), at least 128 of K,
-    // four slabs, each, and at most 16 partials to add.  The transform
-    // gradient, 16 tiles of K 2048: 410 us unsplit, 11 + 5 us in 16 splits.
+    // four slabs, each, and at most 16 partials to add (4 x (512 x 256 x 3072), 128
+    // tiles: 53 + 5 us in 8 splits).
     static int gemm_splits(int M, int Nn, int K, int batch, int* k_per) {
         const int tiles = ((Nn + 63) / 64) * ((M + 63) / 64) * batch;
         int s = std::max(1, std::min({1024 / tiles, K / 128, 16}));
@@ -1298,8 +1390,22 @@ struct Svq {
                            dim3(256), 0, st, g);
         if (g.splits > 1) {
             const long n = (long)batch * M * Nn;
-            hipLaunchKernelGGL(gemm_reduce_kernel, dim3(blocks(n, 256)), dim3(256), 0, st,
+            hipLaunchKernelGGL(gemm_reduce_kernel<float>, dim3(blocks(n, 256)), dim3(256), 0, st,
                                part, C, n, g.splits, alpha);
+        }
+    }
+    // The Gram products: dense batches of A (K x M) and B (K x Nn) for each KV head
+    template <typename TA, typename TC>
+    void gemm64(const TA* A, const float* B, TC* C, int M, int Nn, int K, double* dot) {
+        Gemm64Args<TA, TC> g{A, B, C, M, Nn, K, (long)K * M, (long)K * Nn, H_kv, 0, dot};
+        const int splits = gemm_splits(M, Nn, K, H_kv, &g.k_per);
+        if (splits > 1) g.C = reinterpret_cast<TC*>(part);
+        hipLaunchKernelGGL((gemm64_kernel<TA, TC>), dim3((Nn + 63) / 64, (M + 63) / 64, H_kv * splits),
+                           dim3(256), 0, st, g);
+        if (splits > 1) {
+            const long n = (long)H_kv * M * Nn;
+            hipLaunchKernelGGL(gemm_reduce_kernel<TC>, dim3(blocks(n, 256)), dim3(256), 0, st, g.C, C, n,
+                               splits, 1.0f);
         }
     }
     // One pass at temperature temp (ref .cu:2436-2467 forward, :2470-2530
@@ -1310,7 +1416,7 @@ struct Svq {
         const double denom = attn ? (double)H_q * T * D : (double)N * D;
         const float gscale = 2.0f / (float)denom;
         const int row_blocks = blocks(N, ROWS_PER_BLOCK);
-        CAL_TRY(hipMemsetAsync(loss, 0, 2 * sizeof(double), st));
+        CAL_TRY(hipMemsetAsync(loss, 0, (2 + LOSS_SLOTS) * sizeof(double), st));
         hipLaunchKernelGGL(vq_hard_kernel, dim3(blocks(N, SR), NP), dim3(256), 0, st, rot, s.cb(), rec,
                            idx, dict, N);
         hipLaunchKernelGGL(svq_fwd_kernel, dim3(row_blocks), dim3(256), 0, st, rot, rec, dict, rp,
@@ -1318,7 +1424,7 @@ struct Svq {
                            gscale, loss);
         if (attn) {
             if (use_gram) {
-                gemm(gram, dlt, gd, T, D, T, T, D, (long)T * T, (long)T * D, H_kv, 1, 0, 1.0f, nullptr);
+                gemm64(gram, dlt, gd, T, D, T, loss + 2);  // (G is its own transpose)
             } else {
                 // y_h = A_h dlt_kv, every head in one launch, then sum_h A_h^T y_h
                 gemm(attn, dlt, y, T, D, T, T, D, (long)T * T, (long)T * D, H_q, n_rep, 0, 1.0f, loss);
@@ -1326,15 +1432,14 @@ struct Svq {
                     gemm(attn, y, gd, T, D, n_rep * T, T, D, (long)n_rep * T * T, (long)n_rep * T * D,
                          H_kv, 1, 1, 1.0f, nullptr);
             }
-            if (use_gram || need_grad)
-                hipLaunchKernelGGL(svq_bwd_kernel, dim3(row_blocks), dim3(256), 0, st, gd, dlt, rp,
-                                   s.wa(), s.wb(), gb, gq, N, use_gram ? 1 : 0, need_grad ? 1 : 0,
-                                   gscale, loss);
+            if (need_grad)
+                hipLaunchKernelGGL(svq_bwd_kernel, dim3(row_blocks), dim3(256), 0, st, gd, rp, s.wa(),
+                                   s.wb(), gb, gq, N, gscale);
             if (need_grad) {
                 const int per = (N + GWAB - 1) / GWAB, n = (N + per - 1) / per;
                 hipLaunchKernelGGL(gwab_kernel, dim3(n), dim3(256), 0, st, recf, gd, va, gb, gscale,
                                    part, N, per);
-                hipLaunchKernelGGL(gemm_reduce_kernel, dim3(16), dim3(256), 0, st, part, grad + CB,
+                hipLaunchKernelGGL(gemm_reduce_kernel<float>, dim3(16), dim3(256), 0, st, part, grad + CB,
                                    4096l, n, 1.0f);
             }
         }
@@ -1343,12 +1448,13 @@ struct Svq {
             const int ranges = soft_ranges(N, &per);
             hipLaunchKernelGGL(soft_grad_kernel, dim3(NP, ranges), dim3(256), 0, st, rot, s.cb(), gq,
                                idx, part, N, per, temp);
-            hipLaunchKernelGGL(gemm_reduce_kernel, dim3(blocks(CB, 256)), dim3(256), 0, st, part, grad,
+            hipLaunchKernelGGL(gemm_reduce_kernel<float>, dim3(blocks(CB, 256)), dim3(256), 0, st, part, grad,
                                (long)CB, ranges, 1.0f);
         }
-        double h[2];
+        double h[2 + LOSS_SLOTS];
         CAL_TRY(hipMemcpyAsync(h, loss, sizeof(h), hipMemcpyDeviceToHost, st));
         CAL_TRY(hipStreamSynchronize(st));
+        for (int i = 0; i < LOSS_SLOTS; i++) h[0] += h[2 + i];
         losses[0] = h[0] / denom;
         losses[1] = h[1] / ((double)N * NP * 3);
         return 0;

@@ -252,6 +252,34 @@ def test_svq_pass_sizes(device, T_, H_kv, H_q):
         np.testing.assert_allclose(a, w, rtol=1e-3, atol=1e-4 * max(np.abs(w).max(), 1e-30))
 
 
+@pytest.mark.parametrize("T_,H_kv,H_q", [(256, 1, 8), (256, 1, 2), (512, 1, 8)])
+def test_svq_pass_loss_precision(device, T_, H_kv, H_q):
+    """The attention-weighted loss to fp32's own rounding (2^-24 on the way out,
+    and sums in fp32 of random errors before it) with attention sinks, where the
+    sum of squares over the heads is small against its terms in the Gram form:
+    an fp32 Gram matrix is off by 1.4e-7 in the mean here, 3e-7 at most."""
+    errs = []
+    for seed in range(4):
+        v, rp, cb, attn, N, Tn, H_q, H_kv = _svq_margin_case(T=T_, H_kv=H_kv, H_q=H_q, seed=seed)
+        rng = np.random.default_rng(seed)
+        s = rng.standard_normal((H_q, Tn, Tn)) + np.triu(np.full((Tn, Tn), -1e9), 1)[None]
+        s[:, :, 0] += 4 if H_q == 8 else 8
+        a = np.exp(s - s.max(-1, keepdims=True))
+        attn = (a / a.sum(-1, keepdims=True)).astype(np.float32)
+        # unit rows the codebook does not fit, as the trainer meets them
+        v = rng.standard_normal(v.shape)
+        v = (v / np.linalg.norm(v, axis=1, keepdims=True)).astype(np.float32)
+        wa = (rng.standard_normal((256, 8)) / 16).astype(np.float32)
+        wb = (rng.standard_normal((8, 256)) / 64).astype(np.float32)
+        g, l = new(49152 + 4096), new(2)
+        calib.svq_pass(T(v), T(attn), T(cb), T(wa), T(wb), T(rp), g, l, N=N, T=Tn, H_q=H_q, H_kv=H_kv,
+                       temp=0.3)
+        want = R.svq_pass(v, attn, cb, wa, wb, rp, Tn, H_q, H_kv, 0.3, grad=False)[0]
+        errs.append(abs(float(l[0]) / want - 1))
+    print("loss error", errs)
+    assert np.sqrt(np.mean(np.square(errs))) <= 6e-8
+
+
 def test_svq_train_vs_restatement(device):
     """The whole trainer (3 seeds, Adam steps, best tracking, the proxy
     tournament) against the float64 restatement; with no rate the output
