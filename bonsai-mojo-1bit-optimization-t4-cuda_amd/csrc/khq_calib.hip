@@ -1317,14 +1317,18 @@ struct Svq {
     int init() {
         const size_t nd = (size_t)N * D, np = (size_t)N * NP;
         use_gram = attn && (long)T <= 256l * passes;
+        // partials, where a product is split (in floats; Gram ones are doubles)
         int kp;
         size_t n_part = std::max((size_t)soft_ranges(N, &kp) * CB, (size_t)GWAB * 4096);
-        if (attn) {
-            n_part = std::max(n_part, (size_t)gemm_splits(T, D, H_q / H_kv * T, H_kv, &kp) * H_kv * T * D);
-            if (use_gram) {
-                n_part = std::max(n_part, (size_t)gemm_splits(T, D, T, H_kv, &kp) * H_kv * T * D);
-                n_part = std::max(n_part, (size_t)gemm_splits(T, T, H_q / H_kv * T, H_kv, &kp) * H_kv * T * T * 2);
-            }
+        auto need = [&](int M, int Nn, int K, size_t floats) {
+            const int splits = gemm_splits(M, Nn, K, H_kv, &kp);
+            if (splits > 1) n_part = std::max(n_part, splits * floats * H_kv * M * Nn);
+        };
+        if (use_gram) {
+            need(T, T, H_q / H_kv * T, 2);
+            need(T, D, T, 1);
+        } else if (attn) {
+            need(T, D, H_q / H_kv * T, 1);
         }
         const size_t n_y = attn && !use_gram ? (size_t)H_q * T * D : 0;
         const size_t n_gram = use_gram ? 2 * (size_t)H_kv * T * T : 0;

@@ -4,6 +4,7 @@ and the khq.calib driver) against the CPU restatement oracle/calib_ref.py
 mathematics fixes: orthonormal rotors, Lloyd fixed points, the deploy
 validator's checks on the written file, loss decrease of SmartVQ."""
 import os
+import threading
 
 import numpy as np
 import pytest
@@ -278,6 +279,42 @@ def test_svq_pass_loss_precision(device, T_, H_kv, H_q):
         errs.append(abs(float(l[0]) / want - 1))
     print("loss error", errs)
     assert np.sqrt(np.mean(np.square(errs))) <= 6e-8
+
+
+def test_svq_train_memory(device):
+    """A training over 4,096 tokens holds one T x T Gram matrix (134 MB in
+    double) and its row arrays: the product that forms it is not split at this
+    size and needs no partials."""
+    Tn = 4096
+    g = torch.Generator(device=device).manual_seed(1)
+    v = torch.randn((Tn, 256), generator=g, device=device)
+    v /= v.norm(dim=1, keepdim=True)
+    attn = torch.softmax(torch.randn((1, Tn, Tn), generator=g, device=device), -1)
+    cb, rp = torch.randn((64, 256, 3), generator=g, device=device) * 0.06, T(C.quaternion_rotors(
+        np.random.default_rng(1)).astype(np.float32))
+    out = new(64, 256, 3)
+
+    def train(n):
+        calib.svq_train(v, attn, cb, rp, out, N=Tn, T=Tn, H_q=1, H_kv=1, iterations=n, n_seeds=1)
+
+    train(16)
+    torch.cuda.synchronize()
+    before, least, done = torch.cuda.mem_get_info()[0], [], threading.Event()
+
+    def watch():
+        while not done.is_set():
+            least.append(torch.cuda.mem_get_info()[0])
+
+    th = threading.Thread(target=watch)
+    th.start()
+    train(60)
+    done.set()
+    th.join()
+    used = before - min(least)
+    rows = Tn * (5 * 256 + 2 * 8 + 5 * 64) * 4  # the row arrays, and ...
+    fixed = 64 * 49152 * 4 + 5 * 53248 * 4      # gradient partials, parameters
+    print(f"{len(least)} samples, {used / 2 ** 20:.0f} MB held")
+    assert Tn * Tn * 8 <= used <= Tn * Tn * 8 + rows + fixed + (16 << 20)
 
 
 def test_svq_train_vs_restatement(device):
