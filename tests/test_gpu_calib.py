@@ -339,6 +339,22 @@ def test_svq_train_vs_restatement(device):
             assert np.abs(want_cb - cb).max() > 0.5 * lr
 
 
+@pytest.mark.parametrize("T_,it", [(530, 2), (1480, 4)], ids=["ragged-split", "unsplit"])
+def test_svq_train_long(device, T_, it):
+    """The trainer in its Gram form past 512 tokens, ragged against the 64-wide
+    tiles, with the T x T product split over K and (24 x 24 tiles) in one piece,
+    to the tolerance of test_svq_train_vs_restatement."""
+    v, rp, cb, attn, N, Tn, H_q, H_kv = _svq_margin_case(T=T_, H_kv=1, H_q=2, seed=41, shift=4e-3)
+    lr = 1e-3
+    out, wt = new(64, 256, 3), new(256, 256)
+    calib.svq_train(T(v), T(attn), T(cb), T(rp), out, N=N, T=Tn, H_q=H_q, H_kv=H_kv, iterations=it,
+                    n_seeds=1, lr=lr, out_wtrm=wt)
+    want_cb, want_w = R.svq_train(v, attn, cb, rp, Tn, H_q, H_kv, iterations=it, n_seeds=1, lr=lr)
+    np.testing.assert_allclose(out.cpu().numpy(), want_cb, atol=1e-3 * lr)
+    np.testing.assert_allclose(wt.cpu().numpy(), want_w, atol=1e-3 * lr)
+    assert np.abs(want_cb - cb).max() > 0.5 * lr
+
+
 def _write_attn(path, H_q, n, H_kv, rng):
     with open(path, "wb") as f:
         import struct
