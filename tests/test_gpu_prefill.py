@@ -408,6 +408,62 @@ def test_layer_prefill_one_call(device, cap, steps, calls, after):
         close(got[j], want[j])
 
 
+def test_layer_prefill_long_call(device):
+    """One call of 8,900 tokens: two passes (the cut falls where the layer's raw
+    keys end, between events), several rows a wavefront for K and V, 16-token
+    decode blocks, rows decoded and events far into the space.  Packed bytes of
+    every event against compress on the same rows, the dense key space against
+    decompress, and sampled output rows (around the first event, the pass cut and
+    late events, and the last) against float64 attention over the decoded prefix
+    and the raw tokens as the sequential steps see them."""
+    lc, _ = layer_consts(layer_id=9)
+    n = 8900
+    L = KL.NativeKhqLayer(lc, H_q=H_Q, H_kv=H_KV, cap=9216, device=device,
+                          options=KL.KhqOptions(splits=8, fused=True))
+    tok = synth.tokens(n, H_KV, 77, device)
+    kr, v, k = tok["k_roped"], tok["v"], tok["k"]
+    g = torch.Generator(device=device).manual_seed(78)
+    q = torch.randn((n, H_Q, 2 * D), generator=g, device=device).half()
+    out = torch.full((n, H_Q, D), float("nan"), device=device, dtype=torch.float16)
+    assert L.prefill(q, kr, v, k, out, SCALE) == n
+    held = ((n - 256) // 128 + 1) * 128
+    assert L.state() == (held, n, held // 128)
+    pay, cents = ops.Payload(held * H_KV, device), ops.Centroids(lc, device)
+    for i in range(0, held, 128):  # short calls: one row a wavefront
+        r = slice(i, i + 128)
+        ops.compress(k[r].reshape(-1, D), cents, pay, i * H_KV, is_v=False)
+        ops.compress(v[r].reshape(-1, D), cents, pay, i * H_KV, is_v=True)
+    got, ring = _payload_np(L, held)
+    for name, x in got.items():
+        assert np.array_equal(x.view(np.uint8), getattr(pay, name).cpu().numpy().view(np.uint8).reshape(
+            x.view(np.uint8).shape)), name
+    for x, src in zip(ring, (kr, v)):
+        for i in range(n - 256, n):
+            assert np.array_equal(x.reshape(256, H_KV, D)[i % 256], src[i].cpu().numpy()), i
+    dk = torch.zeros((held, H_KV, D), device=device, dtype=torch.float16)
+    dvt = torch.zeros((H_KV, D, ops.vt_ld(held)), device=device, dtype=torch.float16)
+    for i in range(0, held, 512):  # 4-token blocks
+        ops.decompress(pay, cents, dk, dvt, H_kv=H_KV, tok0=i, n_tok=min(512, held - i), key0=i,
+                       ld_vt=dvt.shape[2])
+    kp, vtp, ld, n_dec = L.dense()
+    assert n_dec == held
+    gk, gvt = torch.empty_like(dk), torch.empty((H_KV, D, ld), device=device, dtype=torch.float16)
+    assert _hip_d2d(gk.data_ptr(), kp, gk.numel() * 2) == 0
+    assert _hip_d2d(gvt.data_ptr(), vtp, gvt.numel() * 2) == 0
+    assert torch.equal(gk.view(torch.int16), dk.view(torch.int16))
+    assert torch.equal(gvt[:, :, :held].view(torch.int16), dvt[:, :, :held].view(torch.int16))
+    dv = dvt[:, :, :held].permute(2, 0, 1)
+    cut = 256 + 8192  # raw keys of a pass
+    rows = [0, 254, 255, 256, 383, 384, 4991, 4992, 5000, cut - 1, cut, cut + 1, held - 1, held, n - 1]
+    for j in rows:
+        b = ((j + 1 - 256) // 128 + 1) * 128 if j + 1 >= 256 else 0
+        K = torch.cat([dk[:b], kr[b:j + 1]]).double()
+        V = torch.cat([dv[:b], v[b:j + 1]]).double()
+        s = torch.matmul(q[j, :, :D].double().reshape(H_KV, N_REP, D), K.permute(1, 2, 0).contiguous()) * SCALE
+        want = torch.matmul(torch.softmax(s, -1), V.permute(1, 0, 2).contiguous()).reshape(H_Q, D)
+        close(out[j].cpu().numpy(), (want * torch.sigmoid(q[j, :, D:].double())).cpu().numpy())
+
+
 @pytest.mark.parametrize("n_q,n_k", [(21, 40), (22, 33), (700, 700), (3000, 3000)])
 def test_prefill_attn_plans_vs_float64(device, n_q, n_k):
     """Both sides of the 16-row / 32-row switch (128 rows a KV head) and the
@@ -464,6 +520,33 @@ def test_prefill_attn_weight_rounding(device, n_q, past):
             top += sum((w[i:i + 32].max()) ** 2 for i in range(0, vis, 32))
     bound = 2.07e-4 * np.sqrt(2 - top / tot)
     assert np.sqrt(num / den) <= 1.04 * bound, (np.sqrt(num / den), bound)
+
+
+@pytest.mark.parametrize("n_q", [16, 128, 1400])
+@pytest.mark.parametrize("gap", [10.0, 12.0, 14.0])
+def test_prefill_attn_sink_key(device, n_q, gap):
+    """One key dominates and thousands of others, e^-gap each, are below the
+    smallest normal fp16 weight (6.1e-5): numerator (matrix cores) and row sum
+    (packed dot products) both have to keep them, in a split and in blocks of all
+    their keys.  V is 0 at the sink and 1 elsewhere, so the output is half the
+    others' share s; a weight is rounded by 2^-25 at most, the same one in both,
+    and the output to fp16."""
+    n_k = 6800 + n_q
+    q = torch.zeros((n_q, H_Q, 2 * D), device=device, dtype=torch.float16)
+    q[:, :, 0] = 1
+    K = torch.zeros((n_k, H_KV, D), device=device, dtype=torch.float16)
+    K[1:, :, 0] = -gap
+    ld = ops.vt_ld(n_k)
+    vt = torch.ones((H_KV, D, ld), device=device, dtype=torch.float16)
+    vt[:, :, 0] = 0
+    out = torch.zeros((n_q, H_Q, D), device=device, dtype=torch.float16)
+    ops.prefill_attn(q, K, vt, out, ld_vt=ld, n_k=n_k, n_q=n_q, vis0=6801, H_q=H_Q, H_kv=H_KV, scale=1.0)
+    w = np.exp(-gap)
+    m = (6800 + np.arange(n_q))[:, None, None] * w
+    s = m / (1 + m)
+    want = 0.5 * s
+    bound = 0.5 * 2.0 ** -25 / w * s * (1 - s) + 2.0 ** -11 * want + 1e-6
+    assert (np.abs(out.cpu().numpy() - want) <= bound).all()
 
 
 @pytest.mark.parametrize("H_q,H_kv", [(1, 1), (7, 7), (10, 2), (33, 3), (24, 1)])
