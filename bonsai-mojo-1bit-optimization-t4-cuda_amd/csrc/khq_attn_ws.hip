@@ -1463,7 +1463,7 @@ int attn_ws_tiles_per_chunk(int c_len, int* n_chunks) {
 void fill_rope_table(AttnArgs& a) {
     // freq = powf(base, -2 m / 64) as the oracle and the portable kernels
     // compute it; the 16-token rotation in double, rounded once
-    thread_local float last_base = -1.0f;
+    thread_local float last_base = NAN;  // unlike every base
     thread_local float tab[96];
     if (a.rope_base != last_base) {
         for (int g = 0; g < 4; g++)

@@ -1003,7 +1003,7 @@ namespace {
 // RoPE frequencies by the host's powf, as the attention kernels' table has them
 // (four powf a lane on the GPU were more than a row's decode).
 DecompArgs with_rope(DecompArgs a) {
-    thread_local float last_base = -1.0f;
+    thread_local float last_base = NAN;  // unlike every base
     thread_local float freq[32];
     if (a.rope_base != last_base) {
         for (int i = 0; i < 32; i++) freq[i] = powf(a.rope_base, -2.0f * (float)i / 64.0f);

@@ -8,6 +8,8 @@ against the oracle's sequential steps.
 Bars: decoded K / V within fp16 rounding (2^-10 of the row block's largest
 magnitude); attention outputs within max-abs 2e-3 and rel 1e-3.
 """
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -298,6 +300,34 @@ def test_decompress_long_matches_short(device):
         outs.append((k.cpu().numpy().view(np.uint16), vt.cpu().numpy().view(np.uint16)))
     assert np.array_equal(outs[0][0], outs[1][0]) and np.array_equal(outs[0][1], outs[1][1])
     assert (outs[0][1][:, :, 2116:] == np.float16(7.0).view(np.uint16)).all()
+
+
+def test_rope_table_first_use(device):
+    """The first call of a thread computes its rotary frequencies whatever the
+    base: base -1 (odd powers of a negative number: NaN) as it does later on."""
+    lc, _ = layer_consts(layer_id=2)
+    n = 64
+    cents, pay = ops.Centroids(lc, device), ops.Payload(n * H_KV, device)
+    synth.compressed_rows(pay, cents, seed=8)
+    q = torch.ones((H_Q, 2 * D), device=device, dtype=torch.float16)
+    ring = torch.zeros((256, H_KV, D), device=device, dtype=torch.float16)
+    res = []
+
+    def run(base):
+        k = torch.zeros((n, H_KV, D), device=device, dtype=torch.float16)
+        vt = torch.zeros((H_KV, D, 64), device=device, dtype=torch.float16)
+        out = torch.zeros((H_Q, D), device=device, dtype=torch.float16)
+        ops.decompress(pay, cents, k, vt, H_kv=H_KV, tok0=0, n_tok=n, key0=0, ld_vt=64, rope_base=base)
+        ops.attn_step(q, pay, cents, ring, ring, out, H_q=H_Q, H_kv=H_KV, c_len=n, win_start=0, win_len=0,
+                      ring_cap=256, scale=SCALE, rope_base=base)
+        res.append((k.cpu().numpy(), out.cpu().numpy()))
+
+    th = threading.Thread(target=lambda: [run(b) for b in (-1.0, THETA, -1.0)])
+    th.start()
+    th.join()
+    for first, later in zip(res[0], res[2]):
+        assert np.array_equal(first, later, equal_nan=True)
+    assert np.isnan(res[0][0]).any() and not np.isnan(res[1][0]).any()
 
 
 def test_decompress_unaligned_payload(device):
