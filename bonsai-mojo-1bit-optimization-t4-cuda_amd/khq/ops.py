@@ -8,6 +8,7 @@ meaning follow the reference's FFI wrappers (ref:src/ops.mojo:1101-1279).
 from __future__ import annotations
 
 import ctypes
+import struct
 
 import torch
 
@@ -211,9 +212,15 @@ def attn_step_batched(seqs, cents: Centroids, *, H_q: int, H_kv: int, scale: flo
         if win_len > 0:
             _need(rk, f16, cap * H_kv * D, "ring_k")
             _need(rv, f16, cap * H_kv * D, "ring_v")
-        pack(buf, i * size, q.data_ptr(), ptr(pay.kpay), ptr(pay.vpay), ptr(pay.vsm),
-             ptr(pay.kmask), ptr(pay.knorm), ptr(pay.krn), ptr(pay.vnorm), ptr(pay.vrn),
-             ptr(rk) or 0, ptr(rv) or 0, out.data_ptr(), c_len, s["win_start"], win_len, cap)
+        tail = (c_len, s["win_start"], win_len, cap)
+        try:
+            pack(buf, i * size, q.data_ptr(), ptr(pay.kpay), ptr(pay.vpay), ptr(pay.vsm),
+                 ptr(pay.kmask), ptr(pay.knorm), ptr(pay.krn), ptr(pay.vnorm), ptr(pay.vrn),
+                 ptr(rk), ptr(rv), out.data_ptr(), *tail)
+        except struct.error:  # a null pointer (None) among them
+            ptrs = (q, pay.kpay, pay.vpay, pay.vsm, pay.kmask, pay.knorm, pay.krn, pay.vnorm,
+                    pay.vrn, rk, rv, out)
+            pack(buf, i * size, *(ptr(x) or 0 for x in ptrs), *tail)
     return call("khq_attn_step_batched_fp16", ctypes.addressof(buf), len(seqs), ptr(cents.cents_k),
                 ptr(cents.cents_v), ptr(cents.vq), ptr(cents.rotor_k), ptr(cents.rotor_v),
                 ptr(cents.d_k), ptr(cents.d_v), H_q, H_kv, scale, cents.alpha_k, cents.alpha_v,

@@ -7,6 +7,8 @@ Bar: attention outputs within max-abs 2e-3 and rel 1e-3 of the oracle; the
 single-step comparison uses the same tolerance (the two calls partition the
 tokens differently, so their fp32 sums round differently).
 """
+import types
+
 import numpy as np
 import pytest
 import torch
@@ -66,6 +68,27 @@ def test_batched_matches_oracle(device, order):
     torch.cuda.synchronize()
     for st, s in zip(states, seqs):
         close(s["out"].cpu().numpy(), _oracle_out(st))
+
+
+def test_batched_window_only_without_payload(device):
+    """A sequence with nothing compressed may come without payload pointers
+    (None, as to the single-sequence step), and one without a window without
+    rings."""
+    lc, h = layer_consts()
+    rng = np.random.default_rng(14)
+    st = _seq_state(rng, lc, h, 0, 0, 200, seed=21)
+    none = types.SimpleNamespace(rows=0, **{k: None for k in (
+        "kmask", "kpay", "knorm", "krn", "vpay", "vnorm", "vrn", "vsm")})
+    comp = _seq_state(rng, lc, h, 64, 64, 0, seed=22)
+    seqs = [dict(q_gate=t(x["q_gate"]), pay=p, ring_k=rk, ring_v=rv,
+                 out=torch.zeros((H_Q, D), device=device, dtype=torch.float16), c_len=x["c_len"],
+                 win_start=x["win_start"], win_len=x["win_len"], ring_cap=256)
+            for x, p, rk, rv in (
+                (st, none, t(st["ring_k"]), t(st["ring_v"])),
+                (comp, payload_from_rows(comp["rows"], comp["rows"]["kmask"].shape[0]), None, None))]
+    ops.attn_step_batched(seqs, ops.Centroids(lc, device), H_q=H_Q, H_kv=H_KV, scale=SCALE)
+    for x, q in zip((st, comp), seqs):
+        close(q["out"].cpu().numpy(), _oracle_out(x))
 
 
 def test_batched_back_to_back_calls(device):
