@@ -126,8 +126,12 @@ def stream_handle(stream=None) -> int | None:
 
     if stream is not None:
         return stream.cuda_stream or None
-    # the raw handle: a torch.cuda.Stream object per call costs about a microsecond
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()) or None
+    # the raw handle where this torch has it: a torch.cuda.Stream object per
+    # call costs about a microsecond
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is None:
+        return torch.cuda.current_stream().cuda_stream or None
+    return raw(torch.cuda.current_device()) or None
 
 
 def call(name: str, *args, check: bool = True) -> int:

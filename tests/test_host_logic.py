@@ -60,3 +60,17 @@ def test_capacity_stops_compression():
         if win_len > RING and over is None:
             over = w
     assert b == 512 and over == 512 + RING + 1
+
+
+def test_stream_handle_without_raw_entry(monkeypatch):
+    """The current stream's handle does not depend on torch's private entry."""
+    import types
+
+    import torch
+
+    from khq import _lib
+
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream", raising=False)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: types.SimpleNamespace(cuda_stream=4660))
+    assert _lib.stream_handle() == 4660
+    assert _lib.stream_handle(types.SimpleNamespace(cuda_stream=0)) is None
