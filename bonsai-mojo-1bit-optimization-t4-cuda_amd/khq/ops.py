@@ -212,15 +212,14 @@ def attn_step_batched(seqs, cents: Centroids, *, H_q: int, H_kv: int, scale: flo
         if win_len > 0:
             _need(rk, f16, cap * H_kv * D, "ring_k")
             _need(rv, f16, cap * H_kv * D, "ring_v")
-        tail = (c_len, s["win_start"], win_len, cap)
         try:
             pack(buf, i * size, q.data_ptr(), ptr(pay.kpay), ptr(pay.vpay), ptr(pay.vsm),
                  ptr(pay.kmask), ptr(pay.knorm), ptr(pay.krn), ptr(pay.vnorm), ptr(pay.vrn),
-                 ptr(rk), ptr(rv), out.data_ptr(), *tail)
+                 ptr(rk), ptr(rv), out.data_ptr(), c_len, s["win_start"], win_len, cap)
         except struct.error:  # a null pointer (None) among them
             ptrs = (q, pay.kpay, pay.vpay, pay.vsm, pay.kmask, pay.knorm, pay.krn, pay.vnorm,
                     pay.vrn, rk, rv, out)
-            pack(buf, i * size, *(ptr(x) or 0 for x in ptrs), *tail)
+            pack(buf, i * size, *(ptr(x) or 0 for x in ptrs), c_len, s["win_start"], win_len, cap)
     return call("khq_attn_step_batched_fp16", ctypes.addressof(buf), len(seqs), ptr(cents.cents_k),
                 ptr(cents.cents_v), ptr(cents.vq), ptr(cents.rotor_k), ptr(cents.rotor_v),
                 ptr(cents.d_k), ptr(cents.d_v), H_q, H_kv, scale, cents.alpha_k, cents.alpha_v,
