@@ -268,9 +268,9 @@ struct RingArgs {
 // 128 more every 128 tokens, at most ev_cap (dec0 and ev_cap multiples of
 // 128; ev_cap = 0: every key is raw).
 // Rows of one KV head (query j, head r % n_rep) are cut into blocks, a block's
-// 32-key tiles into splits of `unit` (at most n_split).  Blocks of one split write
-// out directly unless apart; split s of the others leaves the triple of (query j,
-// head hq) at part[((j * H_q + hq) * n_split + s) * 258].
+// 32-key tiles into ceil(tiles / unit) splits (at most n_split).  Blocks of one
+// split write out directly unless apart; split s of the others leaves the triple of
+// (query j, head hq) at part[((j * H_q + hq) * n_split + s) * 258].
 struct PrefillArgs {
     const __half* q;
     const __half* k;

@@ -494,7 +494,8 @@ def test_layer_prefill_long_call(device):
         close(out[j].cpu().numpy(), (want * torch.sigmoid(q[j, :, D:].double())).cpu().numpy())
 
 
-@pytest.mark.parametrize("n_q,n_k", [(21, 40), (22, 33), (700, 700), (3000, 3000)])
+@pytest.mark.parametrize("n_q,n_k", [(21, 40), (22, 33), (400, 400), (550, 650), (700, 700), (700, 1600),
+                                     (3000, 3000)])
 def test_prefill_attn_plans_vs_float64(device, n_q, n_k):
     """Both sides of the 16-row / 32-row switch (128 rows a KV head) and the
     plans of long launches: blocks written out directly beside split ones, then
