@@ -1148,7 +1148,8 @@ void prefill_plan(PrefillArgs& a, size_t max_bytes) {
         //   one round of the longest block when they all fit at once;
         //   else the work over the slots plus half a block of tail (they start
         //   longest first), or whole rounds when the blocks are equally long (a
-        //   few blocks past a round cost a whole round).
+        //   few blocks past a round cost a whole round); the fullest engine's work
+        //   where they split unlike and are few.
         // A block costs about 4 tiles beside its own (entry, first loads, output);
         // splitting costs the finishing launch, about 4, and 0.045 a block for its
         // triples (128 rows x 1 KB written and read).  Where one round holds every
@@ -1156,6 +1157,25 @@ void prefill_plan(PrefillArgs& a, size_t max_bytes) {
         // wavefront gates up to 16 rows in turn, 0.29 each, with nothing else on its
         // CU.
         const bool even = t_max - t_min <= t_max / 8;
+        // Blocks go to the shader engines (8 CUs) in turn: where they split unlike,
+        // the fullest engine counts, with every fourth or eighth index in use or
+        // fewer (400 queries of a prompt, 160 blocks in up to 4 splits: two rounds,
+        // 33.6 us; 140 in up to 3: 26.3), and the last eighth of the slots is not
+        // filled in one round (550 over 100 tokens: 228 blocks 36.7 us, 164 32.5).
+        const int engines = std::min(64, std::max(1, slots / 8));
+        auto engine_time = [&](int units) {
+            int most = 0, n[64] = {};
+            float load = 0.0f, w[64] = {};
+            for (int b = 0, i = 0; b < nb; b++) {
+                const int t = tiles_of(nb - 1 - b), s = a.block_splits(t), per = (t + s - 1) / s;
+                for (int h = 0; h < a.h_kv; h++, i += a.n_split)
+                    for (int e = i; e < i + s; e++) {
+                        most = std::max(most, ++n[e % engines]);
+                        load = std::max(load, w[e % engines] += per + 4);
+                    }
+            }
+            return most <= 8 && units <= slots - slots / 8 ? a.unit + 4.0f : load / 8 + 0.5f * a.unit;
+        };
         const float gate = 0.29f * std::min(16, n_rows);
         const int step = std::max(1, nb / 64);  // enough blocks to add up
         float best = 0.0f;
@@ -1170,9 +1190,13 @@ void prefill_plan(PrefillArgs& a, size_t max_bytes) {
                 units += w * a.block_splits(t);
                 tiles += w * t;
             }
+            const float least = (tiles + 4 * units) / slots;
+            if (k > k_min && least + 4.0f + 0.045f * units >= best) break;  // and so any finer
+            const bool alike = a.block_splits(t_min) == a.n_split;
             const float rounds = std::ceil(units / slots);
-            float est = rounds <= 1.0f || even ? rounds * (a.unit + 4)
-                                               : (tiles + 4 * units) / slots + 0.5f * a.unit;
+            float est = alike && (rounds <= 1.0f || even) ? rounds * (a.unit + 4)
+                        : alike || rounds > 4.0f          ? least + 0.5f * a.unit
+                                                          : engine_time((int)units);
             bool apart = !a.out;
             if (k > 1 || (rounds <= 1.0f && gate > 4.0f + 0.045f * units && a.triple_bytes(1) <= max_bytes)) {
                 est += 4.0f + 0.045f * units;
