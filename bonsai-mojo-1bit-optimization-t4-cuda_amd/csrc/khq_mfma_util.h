@@ -23,6 +23,7 @@ typedef uint32_t u4h __attribute__((ext_vector_type(4), aligned(2)));
 typedef uint32_t u2h __attribute__((ext_vector_type(2), aligned(2)));
 typedef float f4s __attribute__((ext_vector_type(4), aligned(4)));
 typedef float f2s __attribute__((ext_vector_type(2), aligned(4)));
+typedef uint32_t u4q __attribute__((ext_vector_type(4), aligned(8)));  // pieces of 4 halves
 typedef uint32_t u1b __attribute__((aligned(1)));  // a word of packed bytes
 
 __device__ __forceinline__ f4 mfma32(h8 a, h8 b, f4 c) {

@@ -58,7 +58,7 @@ __device__ __forceinline__ void store_vt(const _Float16 (*sv)[TB + VT_PAD], __ha
         const int d = i / (TB / W), c = i % (TB / W) * W;
         __half* dst = vt + ((size_t)h * 256 + d) * ld + key0 + c;
         if (W == 8 && c + 8 <= nc)
-            *reinterpret_cast<uint4*>(dst) = *reinterpret_cast<const uint4*>(&sv[d][c]);
+            *reinterpret_cast<u4q*>(dst) = *reinterpret_cast<const u4q*>(&sv[d][c]);
         else if (c < nc)
             *reinterpret_cast<uint2*>(dst) = *reinterpret_cast<const uint2*>(&sv[d][c]);
     }

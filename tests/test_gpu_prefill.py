@@ -302,6 +302,23 @@ def test_decompress_long_matches_short(device):
     assert (outs[0][1][:, :, 2116:] == np.float16(7.0).view(np.uint16)).all()
 
 
+def test_decompress_vt_at_eight_bytes(device):
+    """V^T rows at an address 8 bytes off a 16-byte boundary, in the form that
+    writes eight columns at a time: the bits of an aligned call."""
+    lc, _ = layer_consts(layer_id=2)
+    n = 2113
+    cents, pay = ops.Centroids(lc, device), ops.Payload(n * H_KV, device)
+    synth.compressed_rows(pay, cents, seed=9)
+    res = []
+    ld = ops.vt_ld(n)
+    for off in (0, 4):
+        k = torch.zeros((n, H_KV, D), device=device, dtype=torch.float16)
+        vt = torch.zeros(H_KV * D * ld + 4, device=device, dtype=torch.float16)[off:off + H_KV * D * ld]
+        ops.decompress(pay, cents, k, vt, H_kv=H_KV, tok0=0, n_tok=n, key0=0, ld_vt=ld)
+        res.append(vt.clone())
+    assert torch.equal(res[0], res[1]) and res[0].abs().max() > 0
+
+
 def test_rope_table_first_use(device):
     """The first call of a thread computes its rotary frequencies whatever the
     base: base -1 (odd powers of a negative number: NaN) as it does later on."""
