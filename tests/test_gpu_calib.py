@@ -237,7 +237,7 @@ def test_svq_pass_sizes(device, T_, H_kv, H_q):
     """The pass at sizes around the 64-wide matrix-product tiles, its 32-deep
     slabs, the K splits (from 256 stacked rows on), the 64-row blocks of the
     codebook gradient and the switch from the heads' Gram matrices to the two
-    products per head (past 512 tokens a pass), to the tolerance of test_svq_pass_vs_restatement."""
+    products per head (past 256 tokens a pass), to the tolerance of test_svq_pass_vs_restatement."""
     v, rp, cb, attn, N, Tn, H_q, H_kv = _svq_margin_case(T=T_, H_kv=H_kv, H_q=H_q, seed=31)
     rng = np.random.default_rng(32)
     wa = (rng.standard_normal((256, 8)) / 16).astype(np.float32)
