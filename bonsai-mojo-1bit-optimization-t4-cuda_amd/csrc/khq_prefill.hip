@@ -913,6 +913,8 @@ struct MergeArgs {
     __half* out;
     int n_rows, n_split, nb;  // rows, triples a row, merging blocks
     float eps;
+    int h_kv, n_rep;
+    FastDiv by_kv, by_rep;
 };
 __device__ __forceinline__ void merge_row(const MergeArgs& p, int row, int n_split) {
     const int lane = threadIdx.x & 63;
@@ -976,6 +978,61 @@ __device__ __forceinline__ void ring_pieces(const RingArgs& g, int b) {
     *reinterpret_cast<uint2*>(g.ring_v + dst) = *reinterpret_cast<const uint2*>(g.src_v + src);
     *reinterpret_cast<uint2*>(g.ring_u + dst) = *reinterpret_cast<const uint2*>(g.src_u + src);
 }
+// A block for a row of many splits: each wavefront sums a quarter of them, every
+// load and the gate in flight, and the four meet in LDS.  One wavefront takes 64
+// splits in four round trips and the gate in a fifth: 120 rows 8.3 us, 504 rows
+// 9.1; this way 4.3 and 6.8.  Blocks take the KV heads in turn, as the 16-row
+// kernel's blocks do: with 8 of them a row is merged on the XCD whose L2 holds its
+// triples (16 queries of 32 / 8 heads over 900 tokens: 10.9 us, 17.4 row by row).
+__device__ __forceinline__ void merge_row_wide(const MergeArgs& p, int row) {
+    __shared__ __align__(16) float s_num[4][256];
+    __shared__ float s_den[4];
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const float* base = p.part + (size_t)row * p.n_split * 258;
+    const int per = (p.n_split + 3) / 4, lo = wv * per, n = min(per, p.n_split - lo);  // per <= MG
+    float2 a[MG][2];
+#pragma unroll
+    for (int j = 0; j < MG; j++)
+        if (j < n) {
+            const float* pp = base + (size_t)(lo + j) * 258 + 4 * lane;
+            a[j][0] = *reinterpret_cast<const float2*>(pp);
+            a[j][1] = *reinterpret_cast<const float2*>(pp + 2);
+        }
+    const float2 ml = *reinterpret_cast<const float2*>(base + (size_t)min(lane, p.n_split - 1) * 258 + 256);
+    const float gate = __half2float(p.q[(size_t)row * 512 + 256 + threadIdx.x]);
+    float M = ml.x;
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) M = fmaxf(M, __shfl_xor(M, o, 64));
+    const float w = __expf(ml.x - M), lw = ml.y * w;  // lanes past the splits repeat the last
+    float num[4] = {0.f, 0.f, 0.f, 0.f}, den = 0.0f;
+#pragma unroll
+    for (int j = 0; j < MG; j++)
+        if (j < n) {
+            const float ws = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), lo + j));
+            num[0] = fmaf(a[j][0].x, ws, num[0]);
+            num[1] = fmaf(a[j][0].y, ws, num[1]);
+            num[2] = fmaf(a[j][1].x, ws, num[2]);
+            num[3] = fmaf(a[j][1].y, ws, num[3]);
+            den += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(lw), lo + j));
+        }
+    *reinterpret_cast<float4*>(&s_num[wv][4 * lane]) = make_float4(num[0], num[1], num[2], num[3]);
+    if (lane == 0) s_den[wv] = den;
+    __syncthreads();
+    const int t = threadIdx.x;
+    const float v = (s_num[0][t] + s_num[1][t]) + (s_num[2][t] + s_num[3][t]);
+    const float d = (s_den[0] + s_den[1]) + (s_den[2] + s_den[3]);
+    p.out[(size_t)row * 256 + t] = __float2half(v / (d + p.eps) * (1.0f / (1.0f + expf(-gate))));
+}
+__global__ __launch_bounds__(256) void prefill_finish_wide_kernel(MergeArgs m, RingArgs g) {
+    const int b = blockIdx.x;
+    if (b >= m.nb) {
+        ring_pieces(g, b - m.nb);
+        return;
+    }
+    const int r = m.by_kv.div(b), h = b - r * m.h_kv;  // row of the KV head
+    const int j = m.by_rep.div(r);
+    merge_row_wide(m, j * m.h_kv * m.n_rep + h * m.n_rep + r - j * m.n_rep);
+}
 __global__ __launch_bounds__(256) void prefill_finish_kernel(MergeArgs m, RingArgs g) {
     const int b = blockIdx.x;
     if (b >= m.nb) {
@@ -1029,13 +1086,20 @@ bool long_decode(const DecompArgs& a) {
 
 hipError_t launch_prefill_finish(const PrefillArgs& a, const RingArgs* ring, hipStream_t st) {
     const int n_rows = a.n_q * a.h_kv * a.n_rep;
+    // (wide at up to 16 splits: 1 query over 200 tokens 8.0 -> 7.7 us, 48 over 900, 1,152
+    // rows of 15 splits, 22.2 -> 21.2; 6,144 rows of 5 splits the other way, 48.5 -> 50.3)
+    const bool wide = a.uniform && (a.n_split > pf::MG ||
+                                    (a.n_split > 4 && n_rows <= 8 * device_cu_count()));
     const pf::MergeArgs m{a.part, a.q, a.out, n_rows, a.n_split,
-                          a.n_split > 1 || a.apart ? (n_rows + 3) / 4 : 0, a.eps};
+                          wide ? n_rows : a.n_split > 1 || a.apart ? (n_rows + 3) / 4 : 0, a.eps,
+                          a.h_kv, a.n_rep, a.by_kv, a.by_rep};
     RingArgs g = ring ? *ring : RingArgs{};
     g.by_token = FastDiv(std::max(1, g.h_kv * 64));
     const dim3 grid(m.nb + (g.n * g.h_kv * 64 + 255) / 256);
     if (grid.x == 0) return hipSuccess;
-    if (a.uniform)
+    if (wide)
+        hipLaunchKernelGGL(pf::prefill_finish_wide_kernel, grid, dim3(256), 0, st, m, g);
+    else if (a.uniform)
         hipLaunchKernelGGL(pf::prefill_finish_kernel, grid, dim3(256), 0, st, m, g);
     else
         hipLaunchKernelGGL(pf::prefill_finish_ragged_kernel, grid, dim3(256), 0, st, m, g, a,

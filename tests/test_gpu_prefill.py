@@ -570,6 +570,31 @@ def test_prefill_attn_weight_rounding(device, n_q, past):
     assert np.sqrt(num / den) <= 1.04 * bound, (np.sqrt(num / den), bound)
 
 
+@pytest.mark.parametrize("tiles", [2, 4, 5, 6, 7, 13, 16, 17, 31, 33, 61, 64, 65])
+@pytest.mark.parametrize("n_q,H_q,H_kv", [(1, 24, 4), (3, 5, 1)])
+def test_prefill_merge_splits(device, tiles, n_q, H_q, H_kv):
+    """Few rows over `tiles` tiles of 32 keys, one split each up to 64: both forms
+    of the merge (a wavefront or a block a row, from 5 splits on) at counts that
+    four wavefronts share evenly, unevenly and with one left empty."""
+    rng = np.random.default_rng(tiles)
+    n_k = 32 * tiles - 3
+    q = rng.standard_normal((n_q, H_q, 2 * D)).astype(np.float16)
+    K, V = (rng.standard_normal((n_k, H_kv, D)).astype(np.float16) for _ in range(2))
+    ld = ops.vt_ld(n_k)
+    vt = torch.zeros((H_kv, D, ld), device=device, dtype=torch.float16)
+    vt[:, :, :n_k] = t(V).permute(1, 2, 0)
+    out = torch.full((n_q, H_q, D), float("nan"), device=device, dtype=torch.float16)
+    ops.prefill_attn(t(q), t(K), vt, out, ld_vt=ld, n_k=n_k, n_q=n_q, vis0=n_k - n_q + 1, H_q=H_q, H_kv=H_kv,
+                     scale=SCALE)
+    got = out.cpu().numpy()
+    hidden = np.arange(n_k)[None] > n_k - n_q + np.arange(n_q)[:, None]
+    for h in range(H_q):
+        s = q[:, h, :D].astype(np.float64) @ K[:, h * H_kv // H_q].astype(np.float64).T * SCALE
+        w = np.exp(np.where(hidden, -np.inf, s - s.max(1, keepdims=True)))
+        want = w @ V[:, h * H_kv // H_q].astype(np.float64) / w.sum(1, keepdims=True)
+        close(got[:, h], want * npref.sigmoid(q[:, h, D:].astype(np.float64)))
+
+
 @pytest.mark.parametrize("n_q", [16, 128, 1400])
 @pytest.mark.parametrize("gap", [10.0, 12.0, 14.0])
 def test_prefill_attn_sink_key(device, n_q, gap):
