@@ -268,21 +268,24 @@ struct RingArgs {
 // 128 more every 128 tokens, at most ev_cap (dec0 and ev_cap multiples of
 // 128; ev_cap = 0: every key is raw).
 // Rows of one KV head (query j, head r % n_rep) are cut into blocks, a block's
-// 32-key tiles into ceil(tiles / unit) splits (at most n_split).  Blocks of one
-// split write out directly unless apart; split s of the others leaves the triple of
-// (query j, head hq) at part[((j * H_q + hq) * n_split + s) * 258].
+// 32-key tiles into ceil(tiles / unit) splits (at most n_split; with uniform, into
+// n_split).  Blocks of one split write out directly unless apart; split s of the
+// others leaves the triple of (query j, head hq) at
+// part[((j * H_q + hq) * n_split + s) * 258].
 struct PrefillArgs {
     const __half* q;
     const __half* k;
     const __half* vt;
     float* part;
     __half* out;  // NULL: triples only (apart)
-    int ld_vt, n_q, h_kv, n_rep, n_split, unit;
+    int ld_vt, n_q, h_kv, n_rep, n_split;
+    int round_up;  // unit - 1, or with uniform what makes by_unit's quotient n_split
     bool apart;    // every block leaves triples
-    bool uniform;  // every row has n_split triples
+    bool uniform;  // every block has n_split splits
     int vis0, n_raw, raw0, dec0, ev_cap;
     float sc, eps;
     FastDiv by_rep, by_hq, by_kv, by_split, by_unit;  // n_rep, H_q, h_kv, n_split, unit
+    int unit;  // tiles of a split
     __host__ __device__ int bound(int vis) const {
         if (ev_cap <= 0 || vis < 256) return 0;
         const int b = (((vis - 256) >> 7) + 1) << 7;
@@ -297,7 +300,7 @@ struct PrefillArgs {
         *u0 = bound(vf) >> 5;
         return *nd + ((vl + 31) >> 5) - *u0;
     }
-    __host__ __device__ int block_splits(int tiles) const { return by_unit.div(tiles + unit - 1); }
+    __host__ __device__ int block_splits(int tiles) const { return by_unit.div(tiles + round_up); }
     size_t triple_bytes(int splits) const {
         return (size_t)n_q * h_kv * n_rep * splits * 258 * sizeof(float);
     }
