@@ -913,7 +913,7 @@ struct MergeArgs {
     __half* out;
     int n_rows, n_split, nb;  // rows, triples a row, merging blocks
     float eps;
-    int h_kv, n_rep;
+    int h_kv, n_rep;  // row order of the wide form: heads in turn, or 1 and H_q
     FastDiv by_kv, by_rep;
 };
 __device__ __forceinline__ void merge_row(const MergeArgs& p, int row, int n_split) {
@@ -981,9 +981,10 @@ __device__ __forceinline__ void ring_pieces(const RingArgs& g, int b) {
 // A block for a row of many splits: each wavefront sums a quarter of them, every
 // load and the gate in flight, and the four meet in LDS.  One wavefront takes 64
 // splits in four round trips and the gate in a fifth: 120 rows 8.3 us, 504 rows
-// 9.1; this way 4.3 and 6.8.  Blocks take the KV heads in turn, as the 16-row
-// kernel's blocks do: with 8 of them a row is merged on the XCD whose L2 holds its
-// triples (16 queries of 32 / 8 heads over 900 tokens: 10.9 us, 17.4 row by row).
+// 9.1; this way 4.3 and 6.8.  With 8 KV heads blocks take them in turn, as the
+// 16-row kernel's blocks do, and a row is merged on the XCD whose L2 holds its
+// triples (16 queries of 32 / 8 heads over 900 tokens: 12.7 us, 17.4 row by row; of
+// 24 / 4 heads 15.1, 14.5 row by row).
 __device__ __forceinline__ void merge_row_wide(const MergeArgs& p, int row) {
     __shared__ __align__(16) float s_num[4][256];
     __shared__ float s_den[4];
@@ -1090,9 +1091,11 @@ hipError_t launch_prefill_finish(const PrefillArgs& a, const RingArgs* ring, hip
     // rows of 15 splits, 22.2 -> 21.2; 6,144 rows of 5 splits the other way, 48.5 -> 50.3)
     const bool wide = a.uniform && (a.n_split > pf::MG ||
                                     (a.n_split > 4 && n_rows <= 8 * device_cu_count()));
+    const bool turn = a.h_kv % 8 == 0;  // XCDs
     const pf::MergeArgs m{a.part, a.q, a.out, n_rows, a.n_split,
                           wide ? n_rows : a.n_split > 1 || a.apart ? (n_rows + 3) / 4 : 0, a.eps,
-                          a.h_kv, a.n_rep, a.by_kv, a.by_rep};
+                          turn ? a.h_kv : 1, turn ? a.n_rep : a.h_kv * a.n_rep,
+                          turn ? a.by_kv : FastDiv(1), turn ? a.by_rep : a.by_hq};
     RingArgs g = ring ? *ring : RingArgs{};
     g.by_token = FastDiv(std::max(1, g.h_kv * 64));
     const dim3 grid(m.nb + (g.n * g.h_kv * 64 + 255) / 256);

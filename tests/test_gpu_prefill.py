@@ -571,7 +571,7 @@ def test_prefill_attn_weight_rounding(device, n_q, past):
 
 
 @pytest.mark.parametrize("tiles", [2, 4, 5, 6, 7, 13, 16, 17, 31, 33, 61, 64, 65])
-@pytest.mark.parametrize("n_q,H_q,H_kv", [(1, 24, 4), (3, 5, 1)])
+@pytest.mark.parametrize("n_q,H_q,H_kv", [(1, 24, 4), (3, 5, 1), (3, 24, 8)])
 def test_prefill_merge_splits(device, tiles, n_q, H_q, H_kv):
     """Few rows over `tiles` tiles of 32 keys, one split each up to 64: both forms
     of the merge (a wavefront or a block a row, from 5 splits on) at counts that
